@@ -77,10 +77,13 @@ JL_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
 #endif
 }
 
-// Philox4x32-10, general counter and key.
-JL_HD u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
+// Rounds FIRST .. 9 of Philox4x32-10 (FIRST = 0: all of it), general counter and key.
+template <int FIRST>
+JL_HD u32x4 philox_rounds(u32x4 c, uint32_t k0, uint32_t k1) {
+    k0 += (uint32_t)FIRST * kPhiloxW0;
+    k1 += (uint32_t)FIRST * kPhiloxW1;
 #pragma unroll
-    for (int r = 0; r < 10; ++r) {
+    for (int r = FIRST; r < 10; ++r) {
         const uint64_t p0 = (uint64_t)kPhiloxM0 * c.x;
         const uint64_t p1 = (uint64_t)kPhiloxM1 * c.z;
         u32x4 n;
@@ -98,7 +101,38 @@ JL_HD u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
 // Block n of the stream named s: counter (n, s, 0, 0), key (seed, 0).
 JL_HD u32x4 stream_block(uint32_t seed, uint32_t s, uint32_t n) {
     u32x4 c = {n, s, 0u, 0u};
-    return philox4x32_10(c, seed, 0u);
+    return philox_rounds<0>(c, seed, 0u);
+}
+
+// The same block in two parts.  The counter (n, s, 0, 0) has two zero words, so after three of the ten rounds
+// most of the state depends on the block number n alone or on the stream's name s alone:
+//   round 1  (s ^ seed, 0, hi(M0 n), lo(M0 n))
+//   round 2  x, y from n;  z = hi(M0 (s ^ seed)) ^ (from n);  w = lo(M0 (s ^ seed))
+//   round 3  w and a part of x and z from n
+// BlockRounds holds what comes from n (one value for all the streams of a kernel's columns), NameRounds
+// what comes from s (one value for all the blocks of a stream); finish_block puts them together: 15 multiplies per
+// block instead of 20.
+struct BlockRounds {
+    uint32_t z2, x3, z3, w3;  // xored into the words of these names (round keys included); w3: the word itself
+};
+struct NameRounds {
+    uint32_t hi, lo;  // of M0 * (s ^ seed)
+};
+JL_HD BlockRounds block_rounds(uint32_t seed, uint32_t n) {
+    const uint64_t p = (uint64_t)kPhiloxM0 * n;
+    const uint64_t q = (uint64_t)kPhiloxM1 * (uint32_t)(p >> 32);
+    const uint64_t r = (uint64_t)kPhiloxM0 * ((uint32_t)(q >> 32) ^ (seed + kPhiloxW0));
+    return {(uint32_t)p ^ kPhiloxW1, (uint32_t)q ^ (seed + 2u * kPhiloxW0), (uint32_t)(r >> 32) ^ (2u * kPhiloxW1),
+            (uint32_t)r};
+}
+JL_HD NameRounds name_rounds(uint32_t seed, uint32_t s) {
+    const uint64_t p = (uint64_t)kPhiloxM0 * (s ^ seed);
+    return {(uint32_t)(p >> 32), (uint32_t)p};
+}
+JL_HD u32x4 finish_block(uint32_t seed, const NameRounds& s, const BlockRounds& b) {
+    const uint64_t p = (uint64_t)kPhiloxM1 * (s.hi ^ b.z2);
+    u32x4 c = {(uint32_t)(p >> 32) ^ b.x3, (uint32_t)p, s.lo ^ b.z3, b.w3};
+    return philox_rounds<3>(c, seed, 0u);
 }
 
 JL_HD uint32_t word_of(const u32x4& b, uint32_t i) {

@@ -848,10 +848,6 @@ typedef unsigned short ushort2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kRadiusEntries = 1 << jl::kRadiusBits;
 constexpr int kAngleEntries = 1 << jl::kAngleBits;
-#ifndef JL_NORMAL_UNROLL
-#define JL_NORMAL_UNROLL 1
-#endif
-constexpr int kNormalUnroll = JL_NORMAL_UNROLL;  // MFMA steps of the hot loop unrolled together
 
 template <int IN>
 struct NormalTraits;
@@ -990,6 +986,12 @@ __device__ __forceinline__ uint32_t normal_pair(uint32_t w, const char* r_tab, c
     return __builtin_bit_cast(uint32_t, z);
 }
 
+// The value that lane 16 (lane / 16) + L holds (DPP row_newbcast).
+template <int L>
+__device__ __forceinline__ uint32_t row_lane(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + L, 0xF, 0xF, true);
+}
+
 // GPW = 32-column groups per wave: 4 (workgroup = 1024 columns) or 2 (512 columns, for projection
 // dimensions that are an odd multiple of 512).  RB = 32-row blocks per pass: 2 for fp16 / bf16 gradients
 // when the batch has more than 32 rows - every generated entry then feeds two MFMAs, which is worth
@@ -1094,9 +1096,9 @@ __global__ __launch_bounds__(64 * W) void jl_project_normal_kernel(
         const uint64_t nf_lo = f_lo + tile_size;
         const uint64_t nf_hi = (nf_lo + tile_size < P) ? nf_lo + tile_size : P;
 
-        uint32_t sname[GPW];
+        jl::NameRounds name[GPW];
 #pragma unroll
-        for (int j = 0; j < GPW; ++j) sname[j] = jl::stream_name(seed, col0 + 32u * j, tile);
+        for (int j = 0; j < GPW; ++j) name[j] = jl::name_rounds(seed, jl::stream_name(seed, col0 + 32u * j, tile));
 
         for (uint32_t s = s_begin; s < chunks; ++s) {
             const bool more_here = s + 1 < chunks;
@@ -1129,19 +1131,26 @@ __global__ __launch_bounds__(64 * W) void jl_project_normal_kernel(
                 }
             }
 
-            // Philox block of (column, offset o): o / 8 with o = 256 s + 128 h + 8 q
-            const uint32_t n0 = 32u * s + 16u * h;
-#pragma unroll kNormalUnroll
-            for (int q = 0; q < 16; ++q) {
+            // Philox block of (column, offset o): o / 8 with o = 256 s + 128 h + 8 q.  What its first rounds make of the
+            // block's number is the same for all columns: lane 16 x + q of a half-wave works it out for q, once per
+            // chunk, and step q reads it from there through DPP (row_newbcast, an operand modifier of the xors that
+            // use it).  Issue slots per MFMA 68 -> 62; the LDS, 88 % busy with the look-ups, is what binds then:
+            // [32, 109 482 240] bf16 in chunks -> 4096 99.5 -> 98.7 ms, [64, 3 000 000] bf16 -> 4096 3.24 -> 3.10 ms,
+            // [8, 3 000 000] fp16 -> 512 0.362 -> 0.344 ms.  (The same values through an LDS table: 103 ms.)
+            const jl::BlockRounds mine = jl::block_rounds(seed, 32u * s + 16u * h + (lane & 15u));
+            auto do_step = [&](auto q_c) __attribute__((always_inline)) {
+                constexpr int q = decltype(q_c)::value;
                 uint4 a[RB][kPlanes];
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
                     for (int pl = 0; pl < kPlanes; ++pl)
                         a[rb][pl] = *reinterpret_cast<const uint4*>(a_base + rb * 32 * kLdsRow + pl * kPlaneElems + 8 * q);
+                const jl::BlockRounds shared = {row_lane<q>(mine.z2), row_lane<q>(mine.x3), row_lane<q>(mine.z3),
+                                                row_lane<q>(mine.w3)};
 #pragma unroll
                 for (int j = 0; j < GPW; ++j) {
-                    const jl::u32x4 blk = jl::stream_block(seed, sname[j], n0 + (uint32_t)q);
+                    const jl::u32x4 blk = jl::finish_block(seed, name[j], shared);
                     const uint4 b = {normal_pair(blk.x, rt, ct), normal_pair(blk.y, rt, ct),
                                      normal_pair(blk.z, rt, ct), normal_pair(blk.w, rt, ct)};
 #pragma unroll
@@ -1149,7 +1158,9 @@ __global__ __launch_bounds__(64 * W) void jl_project_normal_kernel(
 #pragma unroll
                         for (int pl = 0; pl < kPlanes; ++pl) acc[rb][j] = mfma16(a[rb][pl], b, acc[rb][j], false);
                 }
-            }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            for_each_step(do_step, std::make_integer_sequence<int, 16>{});
 
             last = cur;
             if (kBuffers == 2) {
