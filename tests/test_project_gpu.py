@@ -615,6 +615,29 @@ def test_many_rows(gpu, c_oracle, proj_type, dtype, B):
     assert torch.equal(out[:32], head)   # same launch shape, same matrix, same order of additions
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,k,P,tiles", [(1, 512, 700, 3), (8, 1024, 9_001, 4), (15, 1536, 5_130, 5), (16, 1024, 2_049, 2)])
+def test_passes_of_up_to_sixteen_rows(gpu, c_oracle, dtype, B, k, P, tiles):
+    """The 16-row instance of the Rademacher kernel at both ends of its rows, with two, three and four column groups
+    per wave: one-hot rows read the matrix back exactly (both half-waves, chunk and tile ends, the last feature),
+    the gathered form gives the bits of the dense one, and 16-bit rows have the bits they have in a batch of 32 (the
+    16x16x32 MFMA adds the two k ranges of its two 32x32x16 counterparts one after the other)."""
+    seed = 29
+    e = torch.zeros(B, P, dtype=dtype, device=gpu)
+    feats = [P - 1, 0, 7, 8, 127, 128, 255, 256, 136, 383, 511, 512, 650, 15, 16, 640][:B]
+    e[torch.arange(B), torch.tensor(feats)] = 1.0
+    got = fn(R)(e, k, seed, tiles).cpu().numpy()
+    for r, f in enumerate(feats):
+        assert np.array_equal(got[r], c_oracle.materialize(seed, tiles, P, f, 1, 0, k, R)[0]), (r, f)
+    g = (torch.randn(B, P, generator=torch.Generator().manual_seed(B)) * 1e-2).to(dtype).to(gpu)
+    out = fn(R)(g, k, seed, tiles)
+    pieces = [g[:, lo:hi].contiguous() for lo, hi in ((0, 1), (1, 300), (300, 303), (303, P))]
+    assert torch.equal(fast_jl.project_gather(pieces, k, seed, tiles, "rademacher"), out)
+    if dtype != torch.float32:
+        wide = torch.cat([g, torch.ones(32 - B, P, dtype=dtype, device=gpu)])
+        assert torch.equal(fn(R)(wide, k, seed, tiles)[:B], out)
+
+
 def test_many_rows_gather(gpu):
     from trak_amd import vectorize
 

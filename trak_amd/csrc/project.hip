@@ -42,11 +42,11 @@ using trakhip::store4;
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // A workgroup has 8 waves (one workgroup per CU, two waves per SIMD) and stages every gradient
 // chunk once for all its columns.
 constexpr int kColsMultiple = 512;                    // proj dim granularity (fast_jl_kernel.cuh:113)
-constexpr int kPieces = 32 * 32;                      // 16-byte pieces of a [32 x 256] chunk of 16-bit values
 constexpr int kChunk = 256;                           // features per staged chunk
 constexpr int kLdsRow = kChunk + 8;                   // 16-bit elements; 528 B keeps b128 reads conflict free
 constexpr int kPlaneElems = 32 * kLdsRow;
@@ -99,6 +99,14 @@ __device__ __forceinline__ floatx16 mfma16(const uint4& a, const uint4& b, float
                                                   __builtin_bit_cast(half8, b), c, 0, 0, 0);
 }
 
+// the same for 16 rows and columns and 32 values of k
+__device__ __forceinline__ floatx4 mfma16(const uint4& a, const uint4& b, floatx4 c, bool bf16) {
+    if (bf16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                       0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
+}
+
 // ---- staging of a [32 x 256] gradient chunk ------------------------------------------------
 
 // 16-bit inputs: every thread moves N = ROWS / (2 W) 16-byte pieces, 2 W rows apart (ROWS = 32, or 64
@@ -125,6 +133,22 @@ struct Stage16 {
             const Raw16 r = gload<Raw16>(p + i * piece_pitch);
             v[i] = {r.x, r.y, r.z, r.w};
         }
+    }
+    // the same for a pass with fewer than ROWS rows: the missing ones read as zero
+    __device__ __forceinline__ void load_pieces(const char* p, uint64_t piece_pitch, uint32_t rows, int tid) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            v[i] = {0u, 0u, 0u, 0u};
+            if ((uint32_t)(tid >> 5) + 2 * W * i < rows) {
+                const Raw16 r = gload<Raw16>(p + i * piece_pitch);
+                v[i] = {r.x, r.y, r.z, r.w};
+            }
+        }
+    }
+    __device__ __forceinline__ void load_whole(const uint16_t* __restrict__ g, uint64_t ld, uint32_t rows, uint64_t f_begin,
+                                               int tid) {
+        load_pieces(reinterpret_cast<const char*>(g + (uint64_t)(tid >> 5) * ld + f_begin + 8u * (tid & 31)),
+                    (uint64_t)(2 * W) * ld * 2, rows, tid);
     }
     __device__ __forceinline__ void load(const uint16_t* __restrict__ g, uint64_t ld, uint32_t rows,
                                          uint64_t f_begin, uint64_t f_end, int tid) {
@@ -169,14 +193,30 @@ struct Stage16 {
     }
 };
 
-// fp32 inputs: every thread moves N = 32 / W pieces of 4 floats, W rows apart, and splits each float into
+// fp32 inputs: every thread moves N = ROWS / W pieces of 4 floats, W rows apart, and splits each float into
 // three bf16 terms by truncation (x = b1 + b2 + b3 exactly).
-template <int W>
+template <int W, int ROWS = 32>
 struct Stage32 {
-    static constexpr int N = 2 * kPieces / (64 * W);
+    static constexpr int N = ROWS / W;
     static constexpr int kThreads = 64 * W;
     uint4 v[N];
 
+    // the whole chunk in range; rows beyond `rows` read as zero
+    __device__ __forceinline__ void load_whole(const float* __restrict__ g, uint64_t ld, uint32_t rows, uint64_t f_begin,
+                                               int tid) {
+        load_pieces(reinterpret_cast<const char*>(g + (uint64_t)(tid >> 6) * ld + f_begin + 4u * (tid & 63)),
+                    (uint64_t)W * ld * 4, rows, tid);
+    }
+    __device__ __forceinline__ void load_pieces(const char* p, uint64_t piece_pitch, uint32_t rows, int tid) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            v[i] = {0u, 0u, 0u, 0u};
+            if ((uint32_t)(tid >> 6) + W * i < rows) {
+                const Raw16f r = gload<Raw16f>(p + i * piece_pitch);
+                v[i] = {r.x, r.y, r.z, r.w};
+            }
+        }
+    }
     __device__ __forceinline__ void load(const float* __restrict__ g, uint64_t ld, uint32_t rows,
                                          uint64_t f_begin, uint64_t f_end, int tid) {
 #pragma unroll
@@ -223,7 +263,7 @@ struct Stage32 {
 #pragma unroll
             for (int pl = 0; pl < 3; ++pl) {
                 uint2 o = {a[0][pl] | (a[1][pl] << 16), a[2][pl] | (a[3][pl] << 16)};
-                *reinterpret_cast<uint2*>(lds + pl * kPlaneElems + row * kLdsRow + 4 * sg) = o;
+                *reinterpret_cast<uint2*>(lds + pl * ROWS * kLdsRow + row * kLdsRow + 4 * sg) = o;
             }
         }
     }
@@ -295,12 +335,15 @@ __device__ __noinline__ uint4 gather_piece(const trakhip_segment* segs, uint32_t
 // The segment the workgroup's current chunk starts in, as uniform values (scalar registers): when the
 // whole chunk lies inside it, the chunk is loaded like a chunk of a dense matrix, without the per-thread
 // cursors below.
-// 16-bit elements; a thread's pieces are at row tid / 32 + row_step * i, features 8 (tid % 32) .. + 7 of the chunk.
+// ESZ = element size; 16-bit elements: a thread's pieces are at row tid / 32 + row_step * i, features 8 (tid % 32) .. + 7
+// of the chunk; 32-bit elements: at row tid / 64 + row_step * i, features 4 (tid % 64) .. + 3.
+template <int ESZ>
 struct UniformSeg {
+    static constexpr int kLanes = 16 * ESZ, kElems = 16 / ESZ;  // threads per row, elements per piece
     uint32_t idx;
     uint32_t first, end;   // feature range of segs[idx] (P < 2^32)
     uint64_t piece_pitch;  // bytes from one piece of a thread to its next (row_step rows)
-    const char* tbase;     // per thread: tbase + 2 f = address of its first piece of the chunk that starts at feature f
+    const char* tbase;     // per thread: tbase + ESZ f = address of its first piece of the chunk that starts at feature f
     __device__ __forceinline__ void set(const trakhip_segment* segs, uint32_t i, int tid, uint32_t row_step) {
         const trakhip_segment sg = segs[i];
         // the same values in every lane; said so, they live in scalar registers (a load that follows a
@@ -308,10 +351,11 @@ struct UniformSeg {
         idx = i;
         first = __builtin_amdgcn_readfirstlane((uint32_t)sg.first);
         end = __builtin_amdgcn_readfirstlane((uint32_t)(sg.first + sg.numel));
-        const uint64_t pp = (uint64_t)row_step * sg.ld * 2;
+        const uint64_t pp = (uint64_t)row_step * sg.ld * ESZ;
         piece_pitch = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(pp >> 32)) << 32) |
                       __builtin_amdgcn_readfirstlane((uint32_t)pp);
-        tbase = static_cast<const char*>(sg.ptr) + ((uint64_t)(tid >> 5) * sg.ld + 8u * (tid & 31)) * 2 - sg.first * 2;
+        tbase = static_cast<const char*>(sg.ptr) +
+                ((uint64_t)(tid / kLanes) * sg.ld + (uint32_t)(kElems * (tid % kLanes))) * ESZ - sg.first * ESZ;
     }
     __device__ __forceinline__ void seek(const trakhip_segment* segs, uint32_t n, uint32_t f, int tid, uint32_t row_step) {
         uint32_t lo = 0, hi = n - 1;
@@ -381,10 +425,10 @@ struct Gather16 : Stage16<W, ROWS> {
     }
 };
 
-template <int W>
-struct Gather32 : Stage32<W> {
-    static constexpr int N = Stage32<W>::N;
-    using Stage32<W>::v;
+template <int W, int ROWS = 32>
+struct Gather32 : Stage32<W, ROWS> {
+    static constexpr int N = Stage32<W, ROWS>::N;
+    using Stage32<W, ROWS>::v;
     SegCursor<N> cur;
     __device__ __forceinline__ void init(const trakhip_segment* segs, uint32_t n, uint64_t f_begin, uint64_t P,
                                          int tid) {
@@ -396,9 +440,23 @@ struct Gather32 : Stage32<W> {
         const uint32_t n = (uint32_t)n64;
         const uint64_t f64 = f_begin + 4u * (tid & 63);
         const bool live = f64 < f_end;
+        if (live) cur.advance(segs, n, (uint32_t)f64, tid >> 6, W, 4);
+        load_at(segs, n, cur, rows, f64, f_end, live, tid);
+    }
+    // as Gather16::load_from
+    __device__ __forceinline__ void load_from(const trakhip_segment* segs, uint32_t n, uint32_t start, uint32_t rows,
+                                              uint64_t f_begin, uint64_t f_end, int tid) {
+        const uint64_t f64 = f_begin + 4u * (tid & 63);
+        const bool live = f64 < f_end;
+        SegCursor<N> c;
+        c.set(segs, start, tid >> 6, W, 4);
+        if (live) c.advance(segs, n, (uint32_t)f64, tid >> 6, W, 4);
+        load_at(segs, n, c, rows, f64, f_end, live, tid);
+    }
+    __device__ __forceinline__ void load_at(const trakhip_segment* segs, uint32_t n, const SegCursor<N>& c, uint32_t rows,
+                                            uint64_t f64, uint64_t f_end, bool live, int tid) {
         const uint32_t f = (uint32_t)f64;
-        if (live) cur.advance(segs, n, f, tid >> 6, W, 4);
-        const uint32_t lim = (uint32_t)f_end < cur.end ? (uint32_t)f_end : cur.end;
+        const uint32_t lim = (uint32_t)f_end < c.end ? (uint32_t)f_end : c.end;  // f_end <= P < 2^32
         const bool whole = live && f + 4u <= lim && f + 4u > f;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -406,10 +464,10 @@ struct Gather32 : Stage32<W> {
             uint4 val = {0u, 0u, 0u, 0u};
             if (live && row < rows) {
                 if (whole) {
-                    const Raw16f r = gload<Raw16f>(cur.base[i] + (uint64_t)f * 4);
+                    const Raw16f r = gload<Raw16f>(c.base[i] + (uint64_t)f * 4);
                     val = {r.x, r.y, r.z, r.w};
                 } else {
-                    val = gather_piece<uint32_t, 4>(segs, n, cur.idx, row, f64, f_end);
+                    val = gather_piece<uint32_t, 4>(segs, n, c.idx, row, f64, f_end);
                 }
             }
             v[i] = val;
@@ -424,7 +482,7 @@ struct StageOf {
 };
 template <int W, int ROWS>
 struct StageOf<TRAKHIP_F32, false, W, ROWS> {
-    typedef Stage32<W> type;
+    typedef Stage32<W, ROWS> type;
     typedef float elem;
 };
 template <int W, int ROWS>
@@ -439,7 +497,7 @@ struct StageOf<TRAKHIP_BF16, true, W, ROWS> {
 };
 template <int W, int ROWS>
 struct StageOf<TRAKHIP_F32, true, W, ROWS> {
-    typedef Gather32<W> type;
+    typedef Gather32<W, ROWS> type;
     typedef trakhip_segment elem;
 };
 
@@ -478,35 +536,44 @@ __device__ __forceinline__ uint32_t sign_entry_address(uint32_t word, int q, uin
     return __builtin_amdgcn_perm(word, lane_base, sel);
 }
 
-// Half of a Philox round on one column group's state: half 0 is the multiply of c.x (gives z, w
-// of the next state), half 1 the multiply of c.z (gives x, y).  The empty asm statements tie the
-// instructions to the place in the instruction stream where the call stands: without them the
+// The generator of a chunk is cut into operations of one 64-bit multiply and one or two xors each
+// (see jl::block_rounds, jl::name_rounds): three on what the block's number alone decides (once for all column
+// groups), two per column group for its first three rounds, then two per round and group.  The empty asm statements
+// tie the instructions to the place in the instruction stream where the call stands: without them the
 // compiler moves all the generator arithmetic of a chunk in front of its first MFMA.
 //
 // In two parts, so that other instructions of the step can stand between the asm that ties down the
 // inputs and the multiply: the compiler assumes that a register written by inline asm may not be read
 // by the very next vector instruction (one wait state on this target) and would put an s_nop there.
-struct PhiloxHalfIn {
+struct MulIn {
     uint32_t m, o;  // the word that is multiplied and the word that is xored into the high half
 };
-__device__ __forceinline__ PhiloxHalfIn philox_half_in(const jl::u32x4& c, int half) {
-    PhiloxHalfIn in = {half == 0 ? c.x : c.z, half == 0 ? c.w : c.y};
+struct MulOut {
+    uint32_t hi, lo;  // high half ^ o ^ key, low half
+};
+__device__ __forceinline__ MulIn mul_in(uint32_t m, uint32_t o) {
+    MulIn in = {m, o};
     asm volatile("" : "+v"(in.m), "+v"(in.o));
     return in;
 }
-__device__ __forceinline__ void philox_half_out(const PhiloxHalfIn& in, jl::u32x4& next, int half, uint32_t k0,
-                                                uint32_t k1) {
-    if (half == 0) {
-        const uint64_t p0 = (uint64_t)jl::kPhiloxM0 * in.m;
-        next.z = jl::xor3((uint32_t)(p0 >> 32), in.o, k1);
-        next.w = (uint32_t)p0;
-        asm volatile("" : "+v"(next.z), "+v"(next.w));
-    } else {
-        const uint64_t p1 = (uint64_t)jl::kPhiloxM1 * in.m;
-        next.x = jl::xor3((uint32_t)(p1 >> 32), in.o, k0);
-        next.y = (uint32_t)p1;
-        asm volatile("" : "+v"(next.x), "+v"(next.y));
-    }
+__device__ __forceinline__ MulOut mul_out(uint32_t factor, const MulIn& in, uint32_t key) {
+    const uint64_t p = (uint64_t)factor * in.m;
+    MulOut out = {jl::xor3((uint32_t)(p >> 32), in.o, key), (uint32_t)p};
+    asm volatile("" : "+v"(out.hi), "+v"(out.lo));
+    return out;
+}
+
+// A block's sixteen bytes for passes of 16 rows.  The lower half-wave needs the even bytes of every block, the upper one
+// the odd bytes, of the blocks that both of them hold: each keeps the bytes it needs of its own block and sends
+// the others across (one v_permlane32_swap_b32 for two words).  Result: words 0, 1 = bytes of the lower
+// half-wave's blocks (side 0), words 2, 3 = of the upper one's (side 1), in the order of p.
+__device__ __forceinline__ jl::u32x4 pack_sides(const jl::u32x4& w) {
+    const uint32_t kEven = 0x06040200u, kOdd = 0x07050301u;
+    const auto a = __builtin_amdgcn_permlane32_swap(__builtin_amdgcn_perm(w.y, w.x, kEven),
+                                                    __builtin_amdgcn_perm(w.y, w.x, kOdd), false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(__builtin_amdgcn_perm(w.w, w.z, kEven),
+                                                    __builtin_amdgcn_perm(w.w, w.z, kOdd), false, false);
+    return {a[0], b[0], a[1], b[1]};
 }
 
 // f(integral_constant<int, 0>), f(integral_constant<int, 1>), ... in this order
@@ -520,41 +587,61 @@ __device__ __forceinline__ void for_each_step(F& f, std::integer_sequence<int, S
 // columns), or for projection dimensions that are an odd multiple of 512: 3 (768 columns) when 768
 // divides the dimension, else 2 (512 columns).
 //
-// The main loop is written out step by step.  A chunk is 16 * GPW steps (q, j): one table lookup
-// and one MFMA (three for fp32 gradients) for column group j and features 8q..8q+7 of the lane's
-// half of the chunk.  Under them runs the generator for the NEXT chunk, one half round or two per
-// step (nine rounds x GPW groups x two halves spread over the steps; the first round has scalar
-// operands and is done at the top of the chunk), and the operand reads run kAhead steps ahead of
+// The main loop is written out step by step.  A chunk is 16 * GPW steps: one table lookup
+// and one MFMA (three for fp32 gradients) for one column group and eight features per lane.
+// Under them runs the generator for the NEXT chunk, one operation (one 64-bit multiply) or two per
+// step (67 per chunk with four groups: what the block's number alone decides is worked out once for all groups, 72
+// half rounds when every group did it for itself: 1 % of the call at 32 rows), and the operand reads run kAhead steps ahead of
 // the MFMA that uses them.  The matrix pipe stays busy only if the vector instructions between two
 // MFMAs of a wave fit into the time of one MFMA of each of the two waves of the SIMD (8 issue
 // slots of 4 cycles each, two of them for a 64-bit multiply), which is why the generator is cut
 // that fine.
 //
-// RB = 32-row blocks per pass: 1, or 2 for 16-bit gradients when the batch has more than 32 rows - every
-// looked-up operand (and the generator behind it) then feeds two MFMAs.
-template <int IN, bool GATHER, int GPW, int RB>
+// ROWS = rows of a pass:
+//   32  step = (q, j), MFMA 32x32x16: column group j, features 8q..8q+7 of the lane's half of the chunk;
+//   64  16-bit gradients, batches of more than 32 rows: two 32-row blocks - every looked-up operand (and the
+//       generator behind it) feeds two MFMAs;
+//   16  batches of up to 16 rows, for which half or more of a 32-row MFMA multiplies zero rows: MFMA 16x16x32 in
+//       half the time.  Step = (p, j, side), columns 32 j + 16 side ..+15, k slots 0..15 = the features of q = 2p and
+//       16..31 those of q = 2p + 1 of the 32-row step: the matrix pipe adds the two halves one after the other, so a row's
+//       result has the bits that it has in a 32-row pass.  A lane generates the block of (column 32 j + lane % 16 +
+//       16 (lane / 32), half (lane / 16) % 2), as in the 32-row kernel; a step needs bytes 2p of a block in the lower lanes
+//       and bytes 2p + 1 of the same block in the upper ones, so once per block and chunk the two half-waves trade
+//       odd bytes for even ones (pack_sides: six instructions for sixteen steps).
+//       The step's time is then the issue slots (5.8 per step), not the matrix pipe: [8, 11 689 512] fp16 -> 2048 811 ->
+//       671 us, [16, 1 048 576] fp32 -> 512 (three MFMAs per step) 67 -> 43 us, [12, 3 000 001] fp32 -> 2048 596 -> 375 us.
+//       Sixteen waves of half the columns each take the same time (681 us).
+template <int IN, bool GATHER, int GPW, int ROWS>
 __global__ __launch_bounds__(512) void jl_project_kernel(
     const void* __restrict__ g_in, uint64_t ld, uint32_t rows, uint64_t P, uint32_t k,
     uint32_t seed, uint32_t tiles, uint64_t tile_size, uint32_t chunks_per_tile,
     uint32_t chunks_per_group, uint32_t groups, float* __restrict__ partial) {
     constexpr int W = 8;
     typedef InTraits<IN> Tr;
-    typedef typename StageOf<IN, GATHER, W, 32 * RB>::type Stage;
-    typedef typename StageOf<IN, GATHER, W, 32 * RB>::elem Elem;
+    typedef typename StageOf<IN, GATHER, W, ROWS>::type Stage;
+    typedef typename StageOf<IN, GATHER, W, ROWS>::elem Elem;
+    constexpr bool kSmall = ROWS == 16;
+    constexpr int RB = ROWS == 64 ? 2 : 1;          // row blocks of an MFMA's rows
     constexpr int kColsPerWG = W * GPW * 32;
     constexpr bool kBf = Tr::bf16;
     constexpr int kPlanes = Tr::planes;
+    constexpr int kEsz = IN == TRAKHIP_F32 ? 4 : 2;
+    constexpr uint32_t kRowStep = kEsz == 2 ? 2 * W : W;  // rows between two pieces of a thread
     static_assert(RB == 1 || kPlanes == 1, "two row blocks: 16-bit gradients only (LDS)");
-    // 16-bit inputs: two LDS buffers, one barrier per chunk.  fp32 inputs (three planes) keep one
+    // Two LDS buffers, one barrier per chunk; 32 rows of fp32 inputs (three planes) keep one
     // buffer and two barriers: two buffers of three planes do not fit next to the table.
-    constexpr int kBuffers = kPlanes == 1 ? 2 : 1;
-    constexpr int kPlaneElems = RB * kPlaneElems32;  // this kernel's plane: 32 RB rows
+    constexpr int kBuffers = kPlanes == 1 || kSmall ? 2 : 1;
+    constexpr int kPlaneElems = ROWS * kLdsRow;
     constexpr int kBufElems = kPlanes * kPlaneElems;
     constexpr int kSteps = 16 * GPW;
-    constexpr int kAhead = 3;                       // operand reads in flight
-    constexpr int kHalfRounds = 9 * GPW * 2;        // rounds 1..9 of the next chunk's blocks
+    constexpr int kAhead = kSmall ? 7 : 3;          // operand reads in flight
+    constexpr int kOps = 3 + 16 * GPW;              // generator operations per chunk
+    // The operations are spread over the first kSpan steps, one per step and two in kExtra evenly spaced ones: all blocks are
+    // complete when the first look-up for the next chunk is issued, kAhead steps before the end.
+    constexpr int kSpan = kSteps - kAhead - (kSmall ? GPW : 0);
+    constexpr int kExtra = kOps - kSpan, kEvery = kSpan / kExtra;
     static_assert(kSteps % (kAhead + 1) == 0, "the operand ring must close over a chunk");
-    static_assert(kHalfRounds >= kSteps && kHalfRounds <= 2 * kSteps, "one or two half rounds per step");
+    static_assert(kExtra >= 0 && kExtra * kEvery <= kSpan, "one or two generator operations per step");
 
     // the table comes first: a DS instruction adds a 16-bit immediate to the address register, and
     // a table entry's address is built without adding a base
@@ -574,7 +661,9 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
-    const uint32_t n = lane & 31, h = lane >> 5;
+    // column (of a 32-column group) and half of the chunk whose blocks the lane generates; ROWS = 16: the MFMA operands
+    // are of columns lane % 16
+    const uint32_t n = kSmall ? (lane & 15) + 16 * (lane >> 5) : lane & 31, h = kSmall ? (lane >> 4) & 1 : lane >> 5;
     const uint32_t col0 = cb * kColsPerWG + wave * (GPW * 32) + n;
 
     {
@@ -589,16 +678,19 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
         }
     }
 
-    floatx16 acc[RB][GPW];
+    typedef typename std::conditional<kSmall, floatx4, floatx16>::type Acc;
+    constexpr int kAccs = kSmall ? 2 * GPW : GPW;   // MFMA results per row block
+    Acc acc[RB][kAccs];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int j = 0; j < GPW; ++j)
+        for (int j = 0; j < kAccs; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[rb][j][r] = 0.0f;
+            for (int r = 0; r < (kSmall ? 4 : 16); ++r) acc[rb][j][r] = 0.0f;
 
     const Elem* g = reinterpret_cast<const Elem*>(g_in);
-    const uint32_t a_off = n * kLdsRow + 128 * h;  // row block rb: + 32 rb rows
+    // row block rb: + 32 rb rows; ROWS = 16: the upper half-wave takes the odd q
+    const uint32_t a_off = kSmall ? (lane & 15) * kLdsRow + 128 * h + 8 * (lane >> 5) : n * kLdsRow + 128 * h;
     const uint32_t lane_base = (uint32_t)(lane & 15) << 4;
 
     // Position of a chunk of the run: tile, chunk in tile, first feature, end of the tile's features and
@@ -625,48 +717,55 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
             c.f += kChunk;
         }
     };
-    const bool full_rows = rows == 32u * RB;
+    // passes of 16 rows seldom have all their rows: the loads test the row
+    const bool full_rows = kSmall || kPlanes == 3 || rows == (uint32_t)ROWS;
     Stage st;
-    UniformSeg useg = {0u, 0u, 0u, 0u, nullptr};  // GATHER, 16-bit gradients
+    UniformSeg<kEsz> useg = {0u, 0u, 0u, 0u, nullptr};  // GATHER
     auto load_chunk = [&](const Cursor& c) {
-        if constexpr (!GATHER && kPlanes == 1) {
-            if (full_rows && c.s < c.whole)
-                st.load_whole(g, ld, c.f, tid);
-            else
-                st.load_edge(g, ld, rows, c.f, c.hi, tid);
-        } else if constexpr (GATHER && kPlanes == 1) {
-            const uint32_t f32 = (uint32_t)c.f;  // P < 2^32 with segments; beyond P: c.whole is 0
-            useg.advance(g, (uint32_t)ld, f32, tid, 2 * W);
-            if (full_rows && c.s < c.whole && f32 >= useg.first && f32 + (uint32_t)kChunk <= useg.end)
-                st.load_pieces(useg.tbase + 2 * (uint64_t)f32, useg.piece_pitch);
-            else  // chunks that cross a segment or tile end: per-thread cursors, set up for this chunk only
-                st.load_from(g, (uint32_t)ld, useg.idx, rows, c.f, c.hi, tid);
+        if constexpr (!GATHER) {
+            if (full_rows && c.s < c.whole) {
+                if constexpr (kSmall || kPlanes == 3)
+                    st.load_whole(g, ld, rows, c.f, tid);
+                else
+                    st.load_whole(g, ld, c.f, tid);
+            } else {
+                if constexpr (kPlanes == 1)
+                    st.load_edge(g, ld, rows, c.f, c.hi, tid);
+                else
+                    st.load(g, ld, rows, c.f, c.hi, tid);
+            }
         } else {
-            st.load(g, ld, rows, c.f, c.hi, tid);
+            const uint32_t f32 = (uint32_t)c.f;  // P < 2^32 with segments; beyond P: c.whole is 0
+            useg.advance(g, (uint32_t)ld, f32, tid, kRowStep);
+            if (full_rows && c.s < c.whole && f32 >= useg.first && f32 + (uint32_t)kChunk <= useg.end) {
+                if constexpr (kSmall || kPlanes == 3)
+                    st.load_pieces(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch, rows, tid);
+                else
+                    st.load_pieces(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch);
+            } else {  // chunks that cross a segment or tile end: per-thread cursors, set up for this chunk only
+                st.load_from(g, (uint32_t)ld, useg.idx, rows, c.f, c.hi, tid);
+            }
         }
     };
     const uint32_t n_chunks = (uint32_t)(c_end - c_begin);
 
-    // Two LDS buffers (16-bit gradients): the chunk loop is one uninterrupted stream of steps.  Chunk
+    // Two LDS buffers: the chunk loop is one uninterrupted stream of steps.  Chunk
     // i + 1 is stored to the other buffer in the middle of chunk i (it was loaded in the middle of chunk
     // i - 1: one chunk time, about 2 us, in flight), the loads of chunk i + 2 follow the store into the
-    // same registers, the one barrier of the chunk stands in front of the first step of its last q -
+    // same registers, the one barrier of the chunk stands in front of the first step that uses its last A operand -
     // every wave has finished reading the current buffer by then, and the other one is published for the
     // operand reads of the next chunk, which start right there: the rings of A and B operands run on
-    // across the chunk boundary.  One buffer (fp32 gradients): store between two barriers at the top of
+    // across the chunk boundary.  One buffer (32 rows of fp32 gradients): store between two barriers at the top of
     // the chunk, the rings start anew.
     constexpr bool kRing = kBuffers == 2;
-    constexpr int kSyncStep = 15 * GPW;
+    constexpr int kQSteps = kSmall ? 2 * GPW : GPW;   // steps per A operand
+    constexpr int kQ = kSteps / kQSteps;              // A operands per chunk
+    constexpr int kSyncStep = kSteps - kQSteps;
     constexpr int kStoreStep = 10 * GPW, kLoadStep = kStoreStep + 1;
     Cursor nx = {t0, s0, 0u, 0u, 0u};  // the chunk after the current one (tile and s: its generator blocks)
     open_tile(nx);
     Cursor ld2 = nx;                   // kRing: the chunk after that (the next one to load)
-    if constexpr (GATHER) {
-        if constexpr (kPlanes == 1)
-            useg.seek(g, (uint32_t)ld, (uint32_t)(nx.f < P ? nx.f : P - 1), tid, 2 * W);
-        else
-            st.init(g, (uint32_t)ld, nx.f, P, tid);
-    }
+    if constexpr (GATHER) useg.seek(g, (uint32_t)ld, (uint32_t)(nx.f < P ? nx.f : P - 1), tid, kRowStep);
     load_chunk(nx);
     advance(nx);
     if (kRing) {
@@ -677,12 +776,13 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
     }
     __syncthreads();  // publishes the table (and the first chunk)
 
-    // the first two words of a block are bytes 0..7 = MFMA steps q = 0..7, the other two q = 8..15
-    uint32_t wd[GPW][4];
+    // 32 and 64 rows: the first two words of a block are bytes 0..7 = MFMA steps q = 0..7, the other two q = 8..15.
+    // 16 rows: words 0, 1 are the sixteen bytes of side 0 (p = 0..7), words 2, 3 those of side 1.
+    jl::u32x4 wd[GPW];
 #pragma unroll
     for (int j = 0; j < GPW; ++j) {
-        const jl::u32x4 w = jl::stream_block(seed, jl::stream_name(seed, col0 + 32u * j, t0), 2u * s0 + h);
-        wd[j][0] = w.x, wd[j][1] = w.y, wd[j][2] = w.z, wd[j][3] = w.w;
+        wd[j] = jl::stream_block(seed, jl::stream_name(seed, col0 + 32u * j, t0), 2u * s0 + h);
+        if constexpr (kSmall) wd[j] = pack_sides(wd[j]);
     }
 
     uint4 bq[kAhead + 1];       // B operands (sign look-ups), read kAhead steps ahead
@@ -692,14 +792,19 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
             for (int pl = 0; pl < kPlanes; ++pl)
-                a[slot][rb][pl] = *reinterpret_cast<const uint4*>(base + rb * 32 * kLdsRow + pl * kPlaneElems + 8 * q);
+                a[slot][rb][pl] = *reinterpret_cast<const uint4*>(base + rb * 32 * kLdsRow + pl * kPlaneElems +
+                                                                  (kSmall ? 16 : 8) * q);
     };
-    auto lookup = [&](uint32_t word, int q) -> uint4 {
-        return *reinterpret_cast<const uint4*>(smem + sign_entry_address(word, q, lane_base));
+    // the B operand of step t of the chunk whose blocks are w
+    auto lookup = [&](const jl::u32x4 (&w)[GPW], auto t_c) -> uint4 {
+        constexpr int t = decltype(t_c)::value, q = t / kQSteps;
+        constexpr int j = kSmall ? (t % kQSteps) / 2 : t % kQSteps;
+        constexpr int word = kSmall ? 2 * (t % 2) + q / 4 : q / 4;
+        return *reinterpret_cast<const uint4*>(smem + sign_entry_address(jl::word_of(w[j], word), q, lane_base));
     };
+    auto lookup_first = [&](auto t_c) { bq[decltype(t_c)::value] = lookup(wd, t_c); };
     if (kRing) {
-#pragma unroll
-        for (int p = 0; p < kAhead; ++p) bq[p] = lookup(wd[p % GPW][0], p / GPW);
+        for_each_step(lookup_first, std::make_integer_sequence<int, kAhead>{});
         read_a(lds + a_off, 0, 0);
     }
 
@@ -715,24 +820,63 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
         const uint16_t* a_base = lds + kCur * kBufElems + a_off;
         const uint16_t* a_next = lds + (kCur ^ 1) * kBufElems + a_off;
 
-        // The next chunk's blocks: first round now - its counter is (block, stream name, 0, 0) and
-        // the block number is the same for the GPW groups, so it is one multiply for all of them
-        // and one xor per group - the other nine under the MFMAs below.
-        jl::u32x4 pc[GPW], pn[GPW];
-        {
-            const uint64_t q0 = (uint64_t)jl::kPhiloxM0 * (2u * nx.s + h);
-#pragma unroll
-            for (int j = 0; j < GPW; ++j) {
-                pc[j].x = jl::stream_name(seed, col0 + 32u * j, nx.tile) ^ seed;
-                pc[j].y = 0u;
-                pc[j].z = (uint32_t)(q0 >> 32);
-                pc[j].w = (uint32_t)q0;
+        // The next chunk's blocks.  Operations 0..2: what the block's number decides (shared), then two per group that
+        // put it together with what the stream's name decides, then rounds 4..10, two per round and group.
+        jl::u32x4 pc[GPW];              // state of a group
+        MulOut half[GPW];               // its first half of a round, kept until the second is done
+        jl::BlockRounds shared;
+        uint32_t chain;                 // from operation 0 to 1 to 2
+        auto op_in = [&](auto u_c) __attribute__((always_inline)) -> MulIn {
+            constexpr int u = decltype(u_c)::value;
+            if constexpr (u == 0)
+                return mul_in(2u * nx.s + h, 0u);
+            else if constexpr (u < 3)
+                return mul_in(chain, 0u);
+            else if constexpr (u < 3 + GPW)
+                return mul_in(jl::stream_name(seed, col0 + 32u * (u - 3), nx.tile) ^ seed, shared.z2);
+            else if constexpr (u < 3 + 2 * GPW)
+                return mul_in(pc[u - 3 - GPW].z, shared.x3);
+            else {
+                constexpr int v = u - 3 - 2 * GPW, j = (v / 2) % GPW;
+                return v % 2 == 0 ? mul_in(pc[j].x, pc[j].w) : mul_in(pc[j].z, pc[j].y);
             }
-        }
+        };
+        auto op_out = [&](auto u_c, const MulIn& in) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_c)::value;
+            if constexpr (u == 0) {
+                const MulOut o = mul_out(jl::kPhiloxM0, in, 0u);
+                chain = o.hi;
+                shared.z2 = o.lo ^ jl::kPhiloxW1;
+            } else if constexpr (u == 1) {
+                const MulOut o = mul_out(jl::kPhiloxM1, in, seed + jl::kPhiloxW0);
+                chain = o.hi;
+                shared.x3 = o.lo ^ (seed + 2u * jl::kPhiloxW0);
+            } else if constexpr (u == 2) {
+                const MulOut o = mul_out(jl::kPhiloxM0, in, 2u * jl::kPhiloxW1);
+                shared.z3 = o.hi;
+                shared.w3 = o.lo;
+            } else if constexpr (u < 3 + GPW) {
+                const MulOut o = mul_out(jl::kPhiloxM0, in, 0u);
+                pc[u - 3].z = o.hi;
+                pc[u - 3].w = o.lo;
+            } else if constexpr (u < 3 + 2 * GPW) {
+                constexpr int j = u - 3 - GPW;
+                const MulOut o = mul_out(jl::kPhiloxM1, in, 0u);
+                pc[j] = {o.hi, o.lo, pc[j].w ^ shared.z3, shared.w3};
+            } else {
+                constexpr int v = u - 3 - 2 * GPW, j = (v / 2) % GPW;
+                constexpr uint32_t r = 3u + (uint32_t)(v / (2 * GPW));
+                if constexpr (v % 2 == 0) {
+                    half[j] = mul_out(jl::kPhiloxM0, in, r * jl::kPhiloxW1);
+                } else {
+                    const MulOut o = mul_out(jl::kPhiloxM1, in, seed + r * jl::kPhiloxW0);
+                    pc[j] = {o.hi, o.lo, half[j].hi, half[j].lo};
+                }
+            }
+        };
 
         if (!kRing) {
-#pragma unroll
-            for (int p = 0; p < kAhead; ++p) bq[p] = lookup(wd[p % GPW][(p / GPW) >> 2], p / GPW);
+            for_each_step(lookup_first, std::make_integer_sequence<int, kAhead>{});
             read_a(a_base, 0, 0);
         }
         // one step; the step number is a constant (the steps are written out through for_each_step, which
@@ -740,50 +884,41 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
         auto do_step = [&](auto step_c) __attribute__((always_inline)) {
             {
                 constexpr int step = decltype(step_c)::value;
-                constexpr int q = step / GPW, j = step % GPW;
+                constexpr int q = step / kQSteps;
                 if constexpr (kRing && step == kSyncStep) __syncthreads();
-                // half rounds number first .. first + count - 1 of the kHalfRounds; number
-                // i is half i % 2 of round 1 + i / (2 GPW) of group (i / 2) % GPW.  They are
-                // spread over the first kSpan steps, one per step and two in every kEvery-th:
-                // group g's block must be complete when its first look-up for the next chunk
-                // is issued, kAhead steps before the end.
-                constexpr int kSpan = GPW == 4 ? kSteps : kSteps - 4;
-                constexpr int kExtra = kHalfRounds - kSpan;        // steps that take two
-                constexpr int kEvery = kSpan / kExtra;
-                static_assert(kExtra * kEvery <= kSpan, "half-round schedule");
+                // generator operations first .. first + count - 1
                 constexpr int twos = (step + kEvery - 1) / kEvery;     // steps < step that took two
                 constexpr int first = step + (twos < kExtra ? twos : kExtra);
                 constexpr int count = step >= kSpan ? 0 : (step % kEvery == 0 && step / kEvery < kExtra) ? 2 : 1;
-                PhiloxHalfIn hin0 = {0u, 0u}, hin1 = {0u, 0u};
-                if constexpr (count >= 1) hin0 = philox_half_in(pc[(first / 2) % GPW], first % 2);
-                if constexpr (count == 2) hin1 = philox_half_in(pc[((first + 1) / 2) % GPW], (first + 1) % 2);
+                MulIn in0 = {0u, 0u}, in1 = {0u, 0u};
+                // where the second operation of a step may need the result of the first, it is taken in after that is out
+                constexpr bool kChained = count == 2 && first < 3 + 2 * GPW;
+                if constexpr (count >= 1) in0 = op_in(std::integral_constant<int, first>{});
+                if constexpr (count == 2 && !kChained) in1 = op_in(std::integral_constant<int, first + 1>{});
                 {
                     constexpr int t = step + kAhead;  // the look-up issued now; beyond this chunk: the next one's
                     if constexpr (t < kSteps)
-                        bq[t % (kAhead + 1)] = lookup(wd[t % GPW][(t / GPW) >> 2], t / GPW);
+                        bq[t % (kAhead + 1)] = lookup(wd, std::integral_constant<int, t>{});
                     else if constexpr (kRing)
-                        bq[t % (kAhead + 1)] = lookup(pc[(t - kSteps) % GPW].x, (t - kSteps) / GPW);
+                        bq[t % (kAhead + 1)] = lookup(pc, std::integral_constant<int, t - kSteps>{});
                 }
-                if constexpr (j == 0) {
-                    if constexpr (q + 1 < 16)
+                if constexpr (step % kQSteps == 0) {
+                    if constexpr (q + 1 < kQ)
                         read_a(a_base, (q + 1) & 1, q + 1);
                     else if constexpr (kRing)
                         read_a(a_next, 0, 0);
                 }
-                auto half_out = [&](const PhiloxHalfIn& in, int u) {
-                    const int r = 1 + u / (2 * GPW), g4 = (u / 2) % GPW;
-                    philox_half_out(in, pn[g4], u % 2, seed + (uint32_t)r * jl::kPhiloxW0, (uint32_t)r * jl::kPhiloxW1);
-                };
-                if constexpr (count >= 1) half_out(hin0, first);
-                if constexpr (count == 2) half_out(hin1, first + 1);
-#pragma unroll
-                for (int u = first; u < first + count; ++u)
-                    if (u % 2 == 1) pc[(u / 2) % GPW] = pn[(u / 2) % GPW];
+                if constexpr (count >= 1) op_out(std::integral_constant<int, first>{}, in0);
+                if constexpr (kChained) in1 = op_in(std::integral_constant<int, first + 1>{});
+                if constexpr (count == 2) op_out(std::integral_constant<int, first + 1>{}, in1);
+                if constexpr (kSmall && step >= kSpan && step < kSpan + GPW) pc[step - kSpan] = pack_sides(pc[step - kSpan]);
                 if constexpr (kRing && step == kStoreStep) {
                     if (i + 1 < n_chunks) st.store(lds + (kCur ^ 1) * kBufElems, tid);
                 }
                 if constexpr (kRing && step == kLoadStep) {
                     if (i + 2 < n_chunks) load_chunk(ld2);
+                    // (the operations that read nx, the first 3 + GPW, are behind)
+                    static_assert(kOps - 16 * GPW + GPW <= kLoadStep, "nx is read before it moves");
                     nx.tile = ld2.tile;
                     nx.s = ld2.s;
                     advance(ld2);
@@ -792,14 +927,16 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                    for (int pl = 0; pl < kPlanes; ++pl)
+                    for (int pl = 0; pl < kPlanes; ++pl) {
+                        constexpr int j = step % kQSteps;
                         acc[rb][j] = mfma16(a[q & 1][rb][pl], bq[step % (kAhead + 1)], acc[rb][j], kBf);
+                    }
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
         for_each_step(do_step, std::make_integer_sequence<int, kSteps>{});
 #pragma unroll
-        for (int j = 0; j < GPW; ++j) wd[j][0] = pc[j].x, wd[j][1] = pc[j].y, wd[j][2] = pc[j].z, wd[j][3] = pc[j].w;
+        for (int j = 0; j < GPW; ++j) wd[j] = pc[j];
         if (!kRing) advance(nx);
     };
     for (uint32_t i = 0; i < n_chunks; i += 2) {
@@ -808,16 +945,29 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
     }
 
     // D[m][n] of a 32x32 MFMA: lane holds column n = lane % 32 and, in register r, row
-    // m = 8*(r/4) + 4*(lane/32) + r%4.
+    // m = 8*(r/4) + 4*(lane/32) + r%4; of a 16x16 MFMA: column lane % 16, row 4*(lane/16) + r.
     float* out = partial + (uint64_t)group * rows * k;
+    if constexpr (kSmall) {
+        const uint32_t col = cb * kColsPerWG + wave * (GPW * 32) + (lane & 15);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
+        for (int j = 0; j < kAccs; ++j) {
 #pragma unroll
-        for (int j = 0; j < GPW; ++j) {
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t m = 4u * (lane >> 4) + r;
+                if (m < rows) out[(uint64_t)m * k + col + 16u * j] = acc[0][j][r];
+            }
+        }
+        return;
+    } else {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t m = 32u * rb + 8u * (r >> 2) + 4u * h + (r & 3);
-                if (m < rows) out[(uint64_t)m * k + col0 + 32u * j] = acc[rb][j][r];
+        for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+            for (int j = 0; j < GPW; ++j) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t m = 32u * rb + 8u * (r >> 2) + 4u * h + (r & 3);
+                    if (m < rows) out[(uint64_t)m * k + col0 + 32u * j] = acc[rb][j][r];
+                }
             }
         }
     }
@@ -1334,18 +1484,19 @@ hipError_t launch_rademacher(const void* in, uint64_t ld, uint32_t rows, uint64_
                              const Plan& pl, float* partial, hipStream_t s) {
     const uint64_t wgs = plan_workgroups(pl);
     if (wgs > 0x7FFFFFFFull) return hipErrorInvalidValue;
-    if (rows > 32) {
+    void (*kernel)(const void*, uint64_t, uint32_t, uint64_t, uint32_t, uint32_t, uint32_t, uint64_t, uint32_t, uint32_t,
+                   uint32_t, float*) = jl_project_kernel<IN, GATHER, GPW, 32>;
+    if (rows <= 16) {
+        kernel = jl_project_kernel<IN, GATHER, GPW, 16>;
+    } else if (rows > 32) {
         // two 32-row blocks per pass (16-bit gradients only)
-        if constexpr (IN == TRAKHIP_F32) {
+        if constexpr (IN == TRAKHIP_F32)
             return hipErrorInvalidValue;
-        } else {
-            hipLaunchKernelGGL((jl_project_kernel<IN, GATHER, GPW, 2>), dim3((uint32_t)wgs), dim3(512), 0, s, in, ld, rows,
-                               P, k, seed, pl.tl.tiles, pl.tl.tile_size, pl.chunks_per_tile, pl.chunks_per_group, pl.groups, partial);
-        }
-    } else {
-        hipLaunchKernelGGL((jl_project_kernel<IN, GATHER, GPW, 1>), dim3((uint32_t)wgs), dim3(512), 0, s, in, ld, rows, P,
-                           k, seed, pl.tl.tiles, pl.tl.tile_size, pl.chunks_per_tile, pl.chunks_per_group, pl.groups, partial);
+        else
+            kernel = jl_project_kernel<IN, GATHER, GPW, 64>;
     }
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)wgs), dim3(512), 0, s, in, ld, rows, P, k, seed, pl.tl.tiles, pl.tl.tile_size,
+                       pl.chunks_per_tile, pl.chunks_per_group, pl.groups, partial);
     return hipGetLastError();
 }
 
