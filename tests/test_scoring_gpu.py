@@ -111,6 +111,27 @@ def test_spd_inverse(gpu, n, lam):
     assert np.abs(prod - np.eye(n)).max() < 1e-3
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 127, 129, 191, 256, 320, 641, 1100])
+def test_spd_inverse_at_the_edges_of_its_tiles(gpu, n):
+    # 64 x 64 tiles, k ranges cut to whole 128-blocks of the triangular factor, rows of a larger matrix
+    gen = torch.Generator(device="cpu").manual_seed(n)
+    x = torch.randn(4 * n + 8, n, generator=gen) / math.sqrt(4 * n)
+    full = torch.full((n, n + 5), float("nan"))
+    full[:, :n] = x.T @ x
+    a = full.to(gpu)[:, :n]
+    a64 = full[:, :n].double().numpy() + 0.125 * np.eye(n)
+    want = np.linalg.inv((a64 + a64.T) / 2)
+    inv, mean_abs = spd_inverse(a, lambda_reg=0.125)
+    assert torch.equal(inv, inv.T)
+    # backward error n * 2^-24 of the factor's and the products' sums (2-norm), times the condition number
+    bound = 4 * (n + 8) * 2.0**-24 * np.linalg.cond(a64) * np.linalg.norm(want, 2)
+    assert np.linalg.norm(inv.double().cpu().numpy() - want, 2) <= bound
+    # n^2 terms added in fp32, 1024 partial sums of rows
+    assert abs(mean_abs.item() / inv.double().abs().mean().item() - 1) <= 64 * 2.0**-24
+    scaled, _ = spd_inverse(a, lambda_reg=0.125, normalize=True)
+    assert (scaled.double() * mean_abs.double() - inv.double()).abs().max() <= 4 * 2.0**-24 * inv.abs().max()
+
+
 def test_spd_inverse_many_blocks(gpu):
     # 67 diagonal blocks: more tree nodes of one shape than one batched launch takes, odd block counts
     n, lam = 8500, 1e-2

@@ -11,9 +11,9 @@
 //      matrix gets  W -= panel * panel^T   (MFMA products; the trailing update and the next
 //      diagonal block share one launch, see spd_step_kernel);
 //   3. L^-1 by recursive halving: inv([[A,0],[B,C]]) = [[A^-1,0],[-C^-1 B A^-1, C^-1]]
-//      (two GEMMs per node of the recursion tree);
-//   4. inverse = L^-T L^-1 (one GEMM), then the mean of |.| by a two-stage reduction in a
-//      fixed order and a scaling pass.
+//      (two products per node of the recursion tree);
+//   4. inverse = L^-T L^-1 (one product), then the mean of |.| by a two-stage reduction in a
+//      fixed order and a scaling pass (the products of 3 and 4: tri_product_kernel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -29,21 +29,25 @@ namespace {
 constexpr int NB = 128;
 constexpr int kSumBlocks = 1024;
 
+// W = A + lambda I padded with an identity block, the 128-blocks on and below the diagonal only: nothing above them
+// is read, and every block of L and Li that is read is written first.  A workgroup takes 1024 columns of one row
+// (one scalar division per workgroup; with a 64-bit division per element the pass took 12 us at np = 2048 and 55 us
+// at 4096, with Li cleared alongside).
+constexpr int kInitCols = 1024;
+
 __global__ __launch_bounds__(256) void spd_init_kernel(const float* __restrict__ A, uint64_t lda, float lambda,
-                                                       uint64_t n, uint64_t np, float* __restrict__ W,
-                                                       float* __restrict__ Li, int32_t* __restrict__ status) {
-    const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx == 0 && status) *status = 0;
-    if (idx >= np * np) return;
-    const uint64_t i = idx / np, j = idx % np;
-    float v;
-    if (i < n && j < n)
-        v = A[i * lda + j] + (i == j ? lambda : 0.0f);
-    else
-        v = (i == j) ? 1.0f : 0.0f;
-    W[idx] = v;
-    Li[idx] = 0.0f;  // the blocks above the diagonal stay zero: the final product reads all of Li
-    // (every block of L that is read later - diagonal blocks, panels - is written first)
+                                                       uint32_t n, uint32_t np, uint32_t segments,
+                                                       float* __restrict__ W, int32_t* __restrict__ status) {
+    const uint32_t row = blockIdx.x / segments, seg = blockIdx.x % segments;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && status) *status = 0;
+    const uint32_t end = (row / NB + 1) * NB;  // the row's blocks up to the diagonal one
+    for (uint32_t c = 0; c < kInitCols; c += 256) {
+        const uint32_t col = seg * kInitCols + c + threadIdx.x;
+        if (col >= end) return;
+        float v = row == col ? 1.0f : 0.0f;
+        if (row < n && col < n) v = A[(uint64_t)row * lda + col] + (row == col ? lambda : 0.0f);
+        W[(uint64_t)row * np + col] = v;
+    }
 }
 
 // One workgroup of four waves: Cholesky of the 128x128 diagonal block at W (lower triangle used),
@@ -336,48 +340,182 @@ __global__ __launch_bounds__(256, 1) void spd_step_kernel(float* __restrict__ Wt
     }
 }
 
-__global__ __launch_bounds__(256) void abs_sum_kernel(const float* __restrict__ M, uint64_t ld, uint64_t n,
+__device__ __forceinline__ float workgroup_sum(float s) {
+    __shared__ float red[256];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        __syncthreads();
+    }
+    return red[0];
+}
+
+// Workgroup b adds up |M| over rows b, b + 1024, ... (partial[b] = 0 where there is none).
+__global__ __launch_bounds__(256) void abs_sum_kernel(const float* __restrict__ M, uint64_t ld, uint32_t n,
                                                       float* __restrict__ partial) {
-    __shared__ float red[256];
-    const uint64_t total = n * n;
-    const uint64_t per = (total + kSumBlocks - 1) / kSumBlocks;
-    const uint64_t lo = (uint64_t)blockIdx.x * per;
-    const uint64_t hi = lo + per < total ? lo + per : total;
     float s = 0.0f;
-    for (uint64_t e = lo + threadIdx.x; e < hi; e += 256) s += fabsf(M[(e / n) * ld + (e % n)]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+    for (uint32_t row = blockIdx.x; row < n; row += kSumBlocks) {
+        const float* m = M + (uint64_t)row * ld;
+        for (uint32_t col = threadIdx.x; col < n; col += 256) s += fabsf(m[col]);
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+    s = workgroup_sum(s);
+    if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-__global__ __launch_bounds__(256) void mean_kernel(const float* __restrict__ partial, uint64_t n,
-                                                   float* __restrict__ mean_out, float* __restrict__ mean_user) {
-    __shared__ float red[256];
+// The mean from the partial sums - every workgroup works it out for itself (4 KB from L2) instead of waiting for a
+// launch that does only that - and M /= mean, rows b, b + gridDim.x, ... for workgroup b.
+__global__ __launch_bounds__(256) void mean_scale_kernel(const float* __restrict__ partial, float* __restrict__ M,
+                                                         uint64_t ld, uint32_t n, int normalize,
+                                                         float* __restrict__ mean_user) {
     float s = 0.0f;
-    for (int e = threadIdx.x; e < kSumBlocks; e += 256) s += partial[e];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const float mean = red[0] / ((float)n * (float)n);
-        *mean_out = mean;
-        if (mean_user) *mean_user = mean;
+#pragma unroll
+    for (int e = 0; e < kSumBlocks; e += 256) s += partial[e + threadIdx.x];
+    const float mean = workgroup_sum(s) / ((float)n * (float)n);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && mean_user) *mean_user = mean;
+    if (!normalize) return;
+    const float inv = 1.0f / mean;
+    for (uint32_t row = blockIdx.x; row < n; row += gridDim.x) {
+        float* m = M + (uint64_t)row * ld;
+        for (uint32_t col = threadIdx.x; col < n; col += 256) m[col] *= inv;
     }
 }
 
-__global__ __launch_bounds__(256) void scale_kernel(float* __restrict__ M, uint64_t ld, uint64_t n,
-                                                    const float* __restrict__ mean) {
-    const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= n * n) return;
-    const float inv = 1.0f / *mean;
-    M[(idx / n) * ld + (idx % n)] *= inv;
+int divide_by_mean(float* M, uint64_t ld, uint64_t n, int normalize, float* partial, float* mean_user, hipStream_t s) {
+    if (!normalize && !mean_user) return TRAKHIP_OK;
+    hipLaunchKernelGGL(abs_sum_kernel, dim3(kSumBlocks), dim3(256), 0, s, M, ld, (uint32_t)n, partial);
+    const uint32_t rows = normalize ? (uint32_t)(n < 2048 ? n : 2048) : 1;
+    hipLaunchKernelGGL(mean_scale_kernel, dim3(rows), dim3(256), 0, s, partial, M, ld, (uint32_t)n, normalize, mean_user);
+    return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+}
+
+// ---- products with a triangular operand ---------------------------------------------------------------------
+//
+// fp32 MFMA products of the triangular inverse and the final L^-T L^-1.  Bound: the latency of the global loads at
+// the sizes of the recursion (a [1024 x 1024] node has 2 GFLOP for the whole chip), the fp32 MFMA at the largest.
+// So: 64 x 64 tiles (256 workgroups where 128 x 128 tiles gave 64), four k steps of 32 in flight in registers while
+// one is multiplied from LDS, and k ranges cut to the part where the triangular operand is not zero (rounded to
+// 128, so a range is whole chunks of four steps), tiles with the longest range first.
+enum class Tri { kLowerB, kLowerA, kGram };
+//   kLowerB  C = alpha A B    A row-major along k, B lower triangular (k down the rows): k from the tile's columns on
+//   kLowerA  C = alpha A B    A lower triangular: k up to the tile's rows
+//   kGram    C = A^T A        A lower triangular, lower tiles + mirror image: k from the tile's rows on; n x n stored
+// Operands have whole 128-blocks (row pitch np).  A wave owns one 32 x 32 tile, two accumulators (even and odd
+// sub-steps) that are added at the end: error of the inverse against 64 bits 9.4e-7 at n = 2048, 1.26e-6 with one
+// accumulator over the whole range in the earlier kernels.  Measured: the recursion 415 -> 112 us at n = 2048 and
+// 824 -> 350 us at 4096 (128 x 128 tiles over the full k range), L^-T L^-1 240 -> 66 us and 516 -> 277 us (256 x 256 tiles of the
+// six-term bf16 product, planes included).  The staging registers are vector types (arrays of HIP's float4 stayed in
+// scratch) and all fragment reads of a step stand before its first MFMA: without these two the same products took
+// twice as long.
+constexpr int kTriTile = 64, kTriStep = 32, kTriDepth = NB / kTriStep;
+constexpr int kRowPitch = kTriStep + 4;   // row-k tile, 64 rows: 144-byte rows, conflict-free 16-byte reads
+constexpr int kColPitch = kTriTile + 8;   // k-row tile, 32 rows: the half-waves (4 rows apart) read other banks
+constexpr int kTriFloats = kTriTile * kRowPitch;
+static_assert(kTriStep * kColPitch == kTriFloats, "both operand layouts take the same room");
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+template <bool KROW>
+__device__ __forceinline__ void tri_load(const float* __restrict__ p, uint64_t ld, uint32_t x0, uint32_t k0, int tid,
+                                         floatx4 (&r)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int id = tid + 256 * i;
+        const uint64_t at = KROW ? (uint64_t)(k0 + (id >> 4)) * ld + x0 + 4 * (id & 15)
+                                 : (uint64_t)(x0 + (id >> 3)) * ld + k0 + 4 * (id & 7);
+        r[i] = *reinterpret_cast<const floatx4*>(p + at);
+    }
+}
+
+template <bool KROW>
+__device__ __forceinline__ void tri_store(float* lds, int tid, const floatx4 (&r)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int id = tid + 256 * i;
+        float* q = KROW ? lds + (id >> 4) * kColPitch + 4 * (id & 15) : lds + (id >> 3) * kRowPitch + 4 * (id & 7);
+        *reinterpret_cast<floatx4*>(q) = r[i];
+    }
+}
+
+// the values k = 8 s + 4 h + t, t = 0..3, of row or column x: lane half h's operands of four MFMAs
+template <bool KROW>
+__device__ __forceinline__ floatx4 tri_frag(const float* lds, int x, int h, int s) {
+    if (!KROW) return *reinterpret_cast<const floatx4*>(lds + x * kRowPitch + 8 * s + 4 * h);
+    const float* q = lds + (8 * s + 4 * h) * kColPitch + x;
+    return floatx4{q[0], q[kColPitch], q[2 * kColPitch], q[3 * kColPitch]};
+}
+
+template <Tri KIND>
+__global__ __launch_bounds__(256, 2) void tri_product_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                             float* __restrict__ C, uint64_t np, uint64_t ldc,
+                                                             uint32_t M, uint32_t N, uint32_t K, float alpha,
+                                                             trakhip::GemmBatch batch) {
+    constexpr bool kKrowA = KIND == Tri::kGram;
+    __shared__ __attribute__((aligned(16))) float lds[2][2][kTriFloats];
+    const uint32_t tiles_m = M / kTriTile, tiles_n = N / kTriTile;
+    uint32_t tm, tn, k_begin = 0, k_end = K;
+    if (KIND == Tri::kGram) {
+        short_k::triangle_tile(blockIdx.x, tm, tn);
+        k_begin = tm * kTriTile / NB * NB;
+    } else if (KIND == Tri::kLowerB) {
+        tn = blockIdx.x / tiles_m, tm = blockIdx.x % tiles_m;
+        k_begin = tn * kTriTile / NB * NB;
+    } else {
+        tm = tiles_m - 1 - blockIdx.x / tiles_n, tn = blockIdx.x % tiles_n;
+        k_end = (tm * kTriTile / NB + 1) * NB;
+    }
+    const uint32_t m0 = tm * kTriTile, n0 = tn * kTriTile;
+    const uint32_t y = blockIdx.y;
+    if (KIND != Tri::kGram) A += batch.a[y], B += batch.b[y], C += batch.c[y];
+
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int x = lane & 31, h = lane >> 5;
+    const int wm = 32 * (wave >> 1), wn = 32 * (wave & 1);
+    floatx4 ra[kTriDepth][2], rb[kTriDepth][2];
+#pragma unroll
+    for (int u = 0; u < kTriDepth; ++u) {
+        tri_load<kKrowA>(A, np, m0, k_begin + kTriStep * u, tid, ra[u]);
+        tri_load<true>(B, np, n0, k_begin + kTriStep * u, tid, rb[u]);
+    }
+    floatx16 acc[2] = {tile_zero(), tile_zero()};
+    for (uint32_t k0 = k_begin; k0 < k_end; k0 += NB) {
+        const bool more = k0 + NB < k_end;
+#pragma unroll
+        for (int u = 0; u < kTriDepth; ++u) {
+            // a buffer is written again two steps later, behind the barrier that follows its reads
+            tri_store<kKrowA>(lds[u & 1][0], tid, ra[u]);
+            tri_store<true>(lds[u & 1][1], tid, rb[u]);
+            if (more) {
+                tri_load<kKrowA>(A, np, m0, k0 + NB + kTriStep * u, tid, ra[u]);
+                tri_load<true>(B, np, n0, k0 + NB + kTriStep * u, tid, rb[u]);
+            }
+            __syncthreads();
+            floatx4 fa[kTriStep / 8], fb[kTriStep / 8];
+#pragma unroll
+            for (int s = 0; s < kTriStep / 8; ++s) {
+                fa[s] = tri_frag<kKrowA>(lds[u & 1][0], wm + x, h, s);
+                fb[s] = tri_frag<true>(lds[u & 1][1], wn + x, h, s);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // all reads of the step in flight before its first MFMA waits
+#pragma unroll
+            for (int s = 0; s < kTriStep / 8; ++s)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[s & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[s][t], fb[s][t], acc[s & 1], 0, 0, 0);
+        }
+    }
+    const uint32_t col = n0 + wn + x;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const uint32_t row = m0 + wm + mfma_row(r, h);
+        const float v = acc[0][r] + acc[1][r];
+        if (KIND != Tri::kGram) {
+            C[(uint64_t)row * ldc + col] = alpha * v;
+        } else if (row < M && col <= row) {
+            C[(uint64_t)row * ldc + col] = v;
+            C[(uint64_t)col * ldc + row] = v;
+        }
+    }
 }
 
 struct Ctx {
@@ -433,9 +571,12 @@ int tri_inverse_impl(Ctx& c, uint64_t nblk) {
                 out_of_t.b[y] = below;                              // T      in W
                 out_of_t.c[y] = below;                              // result in Li
             }
-            int e = trakhip::gemm_nn_batched(c.L, np, c.Li, np, c.W, np, r, q, q, 1.0f, 0.0f, t_of_b, c.s);
-            if (!e) e = trakhip::gemm_nn_batched(c.Li, np, c.W, np, c.Li, np, r, q, r, -1.0f, 0.0f, out_of_t, c.s);
-            if (e) return e;
+            const dim3 grid((uint32_t)(r / kTriTile * (q / kTriTile)), t_of_b.count);
+            hipLaunchKernelGGL(tri_product_kernel<Tri::kLowerB>, grid, dim3(256), 0, c.s, c.L, c.Li, c.W, np, np,
+                               (uint32_t)r, (uint32_t)q, (uint32_t)q, 1.0f, t_of_b);
+            hipLaunchKernelGGL(tri_product_kernel<Tri::kLowerA>, grid, dim3(256), 0, c.s, c.Li, c.W, c.Li, np, np,
+                               (uint32_t)r, (uint32_t)q, (uint32_t)r, -1.0f, out_of_t);
+            if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
         }
     }
     return TRAKHIP_OK;
@@ -454,17 +595,11 @@ int tri_inverse(Ctx& c, uint64_t nblk) {
 
 namespace trakhip {
 
-// Workspace: three np x np matrices (W, L, Li), the reduction scratch, and for small n a tail for the
-// split planes of Li^T (for np >= 384 they fit into W and L, which are free by then).
-static size_t planes_tail_bytes(uint64_t n, uint64_t np) {
-    const size_t planes = split_bytes(n, n, TRAKHIP_F32), free_front = (size_t)(2 * np * np) * sizeof(float);
-    return planes > free_front ? planes : 0;
-}
-
+// Workspace: three np x np matrices (W, L, Li) and the reduction scratch.
 size_t spd_inverse_workspace_bytes(uint64_t n) {
     if (n == 0) return 0;
     const uint64_t np = (n + NB - 1) / NB * NB;
-    return (size_t)(3 * np * np + kSumBlocks + 4) * sizeof(float) + planes_tail_bytes(n, np);
+    return (size_t)(3 * np * np + kSumBlocks) * sizeof(float);
 }
 
 int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t ldi, uint64_t n, int normalize,
@@ -479,11 +614,10 @@ int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t
     float* L = W + np * np;
     float* Li = L + np * np;
     float* partial = Li + np * np;
-    float* mean_dev = partial + kSumBlocks;
 
-    const uint64_t total = np * np;
-    hipLaunchKernelGGL(spd_init_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, A, lda, lambda, n,
-                       np, W, Li, status);
+    const uint32_t segments = (uint32_t)((np + kInitCols - 1) / kInitCols);
+    hipLaunchKernelGGL(spd_init_kernel, dim3((uint32_t)np * segments), dim3(256), 0, s, A, lda, lambda, (uint32_t)n,
+                       (uint32_t)np, segments, W, status);
     if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
 
     // Diagonal block 0 alone; then per block column j: the panel below it, and one launch that holds both
@@ -519,23 +653,12 @@ int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t
     int e = tri_inverse(c, nblk);
     if (e) return e;
 
-    // inverse = Li^T * Li (rows of Li at or beyond n do not reach the leading n x n block): the
-    // symmetric product of the split operand Li^T, lower-triangle tiles mirrored, so the result is
-    // exactly symmetric.  The planes go where W and L were (or behind the scratch for small n).
-    void* planes = planes_tail_bytes(n, np) ? static_cast<void*>(mean_dev + 4) : static_cast<void*>(W);
-    e = split_rows(Li, TRAKHIP_F32, np, n, n, 1, planes, split_bytes(n, n, TRAKHIP_F32), s);
-    if (!e) e = gram_split(planes, n, n, TRAKHIP_F32, inv, ldi, 1.0f, 0.0f, nullptr, 0, s);
-    if (e) return e;
-
-    if (normalize || mean_abs) {
-        hipLaunchKernelGGL(abs_sum_kernel, dim3(kSumBlocks), dim3(256), 0, s, inv, ldi, n, partial);
-        hipLaunchKernelGGL(mean_kernel, dim3(1), dim3(256), 0, s, partial, n, mean_dev, mean_abs);
-        if (normalize)
-            hipLaunchKernelGGL(scale_kernel, dim3((uint32_t)((n * n + 255) / 256)), dim3(256), 0, s, inv, ldi, n,
-                               mean_dev);
-        if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
-    }
-    return TRAKHIP_OK;
+    // inverse = Li^T * Li: lower-triangle tiles and their mirror image, so the result is exactly symmetric
+    const uint64_t tiles = (n + kTriTile - 1) / kTriTile;
+    hipLaunchKernelGGL(tri_product_kernel<Tri::kGram>, dim3((uint32_t)(tiles * (tiles + 1) / 2)), dim3(256), 0, s, Li, Li,
+                       inv, np, ldi, (uint32_t)n, (uint32_t)n, (uint32_t)np, 1.0f, GemmBatch{});
+    if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
+    return divide_by_mean(inv, ldi, n, normalize, partial, mean_abs, s);
 }
 
 }  // namespace trakhip
@@ -963,7 +1086,7 @@ constexpr uint64_t kGeneralInverseMaxN = 12288;
 size_t general_inverse_workspace_bytes(uint64_t n) {
     if (n == 0 || n > kGeneralInverseMaxN) return 0;
     const uint64_t np = (n + NB - 1) / NB * NB;
-    return (size_t)(2 * np * np + 2 * np * kGjOb + kSumBlocks + 4) * sizeof(float) + (kGjOb / 8) * sizeof(GjStep);
+    return (size_t)(2 * np * np + 2 * np * kGjOb + kSumBlocks) * sizeof(float) + (kGjOb / 8) * sizeof(GjStep);
 }
 
 int general_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t ldi, uint64_t n, int normalize,
@@ -977,8 +1100,7 @@ int general_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint
     float* W = static_cast<float*>(ws);
     float* Y = W + 2 * np * np;  // kGjOb x 2 np: L^-1 * (pivot rows) of the block at work
     float* partial = Y + 2 * np * kGjOb;
-    float* mean_dev = partial + kSumBlocks;
-    GjStep* steps = reinterpret_cast<GjStep*>(mean_dev + 4);
+    GjStep* steps = reinterpret_cast<GjStep*>(partial + kSumBlocks);
     hipLaunchKernelGGL(gj_init_kernel, dim3((uint32_t)((2 * np * np + 255) / 256)), dim3(256), 0, s, A, lda, lambda, n,
                        np, W, status);
     if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
@@ -990,14 +1112,8 @@ int general_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint
     if (e) return e;
     hipLaunchKernelGGL(gj_copy_out_kernel, dim3((uint32_t)((n * n + 255) / 256)), dim3(256), 0, s, W, 2 * np, np, n, inv,
                        ldi);
-    if (normalize || mean_abs) {
-        hipLaunchKernelGGL(abs_sum_kernel, dim3(kSumBlocks), dim3(256), 0, s, inv, ldi, n, partial);
-        hipLaunchKernelGGL(mean_kernel, dim3(1), dim3(256), 0, s, partial, n, mean_dev, mean_abs);
-        if (normalize)
-            hipLaunchKernelGGL(scale_kernel, dim3((uint32_t)((n * n + 255) / 256)), dim3(256), 0, s, inv, ldi, n,
-                               mean_dev);
-    }
-    return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+    if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
+    return divide_by_mean(inv, ldi, n, normalize, partial, mean_abs, s);
 }
 
 }  // namespace trakhip
