@@ -749,3 +749,32 @@ def test_gram_shares_the_k_range_over_idle_cus(gpu, fmt, N, K):
     wide = torch.full((N, N + 3), 7.0, device=gpu)
     gram_split(make(), out=wide[:, :N])
     assert torch.equal(wide[:, :N], g) and bool((wide[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("fmt,N,K", [("fp32", 512, 2000), ("fp16", 512, 64 * 8 * 16), ("fp32", 257, 16 * 33), ("bf16", 2048, 5000)])
+def test_gram_takes_the_shares_that_its_scratch_holds(gpu, fmt, N, K):
+    """No scratch, scratch for two or five shares and for all of them: the same product, exactly symmetric."""
+    import ctypes
+
+    from trak_amd import _lib
+
+    dtype = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}[fmt]
+    code = {"fp32": _lib.F32, "fp16": _lib.F16, "bf16": _lib.BF16}[fmt]
+    gen = torch.Generator(device=gpu).manual_seed(N + K)
+    x = torch.randn(K, N, generator=gen, device=gpu).to(dtype)
+    operand = split_rows(x, transposed=True)
+    want = (x.double().T @ x.double()).cpu().numpy()
+    lib = _lib.load()
+    share = 4 * N * N
+    full = lib.trakhip_gram_split_workspace_most(N, operand.K, code, 0)
+    assert full % share == 0 and full // share >= 2
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for size in {0, share + 4, 2 * share, min(5 * share, full), full}:
+        ws = torch.full((size // 4 + 64,), float("nan"), device=gpu)
+        out = torch.zeros(N, N, device=gpu)
+        rc = lib.trakhip_gram_split(ctypes.c_void_p(operand.planes.data_ptr()), N, operand.K, code,
+                                    ctypes.c_void_p(out.data_ptr()), N, 1.0, 0.0, ctypes.c_void_p(ws.data_ptr()), size,
+                                    stream)
+        assert rc == 0 and torch.equal(out, out.T)
+        assert rel_max(out.cpu().numpy(), want) < gemm_tol(K)
+        assert ws[size // 4:].isnan().all()                                   # nothing written behind the scratch

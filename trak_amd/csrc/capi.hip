@@ -128,7 +128,11 @@ int trakhip_gemm_nt_split(const void* A_planes_dev, uint64_t M, const void* B_pl
 }
 
 size_t trakhip_gram_split_workspace(uint64_t N, uint64_t K, int dtype, int two_planes) {
-    return trakhip::gram_split_workspace_bytes(N, K, dtype, two_planes);
+    return trakhip::gram_split_workspace_bytes(N, K, dtype, two_planes, false);
+}
+
+size_t trakhip_gram_split_workspace_most(uint64_t N, uint64_t K, int dtype, int two_planes) {
+    return trakhip::gram_split_workspace_bytes(N, K, dtype, two_planes, true);
 }
 
 int trakhip_gram_split(const void* A_planes_dev, uint64_t N, uint64_t K, int dtype, float* C_dev, uint64_t ldc,

@@ -705,24 +705,64 @@ __global__ __launch_bounds__(256) void gram_combine_kernel(const float* __restri
     __shared__ float t[32][33];
     const uint32_t bi = blockIdx.y, bj = blockIdx.x;  // 32 x 32 block (bi, bj) on or under the diagonal
     if (bj > bi) return;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    // A thread adds up four columns of one row, eight shares' loads in flight (a share that does not exist is read
+    // from the last one and not added).  A block on the diagonal also adds what lies above it (the 256-row tiles hold
+    // it) and does not store that.  Bound by the latency of its loads: seven shares of 2048 x 2048 take 24 us, fifteen
+    // of 512 x 512 5 us (12 us with four rows per thread, one column wide, one after the other).
+    const int r = threadIdx.x >> 3, c = 4 * (threadIdx.x & 7);
+    const uint64_t row = (uint64_t)bi * 32 + r, col = (uint64_t)bj * 32 + c;
+    const bool whole = row < n && col + 4 <= n;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (whole) {
+        const float* q = P + row * n + col;
+        for (uint32_t p = 0; p < parts; p += 8) {
+            float4u s[8];
 #pragma unroll
-    for (int r = ty; r < 32; r += 8) {
-        const uint64_t row = (uint64_t)bi * 32 + r, col = (uint64_t)bj * 32 + tx;
-        float v = 0.0f;
-        if (row < n && col <= row) {
-            for (uint32_t p = 0; p < parts; ++p) v += P[(uint64_t)p * part_stride + row * n + col];
-            v *= alpha;
-            if (beta != 0.0f) v += beta * C[row * ldc + col];
-            C[row * ldc + col] = v;
+            for (uint32_t i = 0; i < 8; ++i)
+                s[i] = *reinterpret_cast<const float4u*>(q + (uint64_t)(p + i < parts ? p + i : parts - 1) * part_stride);
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += p + i < parts ? s[i][e] : 0.0f;
         }
-        t[r][tx] = v;
+    } else if (row < n) {
+        for (uint32_t p = 0; p < parts; ++p)
+            for (int e = 0; e < 4; ++e)
+                if (col + e < n) v[e] += P[(uint64_t)p * part_stride + row * n + col + e];
     }
-    __syncthreads();
+    float* out = C + row * ldc + col;
+    if (whole && bj < bi) {
+        float4u old = {0.0f, 0.0f, 0.0f, 0.0f}, sum;
+        if (beta != 0.0f) old = *reinterpret_cast<const float4u*>(out);
 #pragma unroll
-    for (int r = ty; r < 32; r += 8) {
-        const uint64_t row = (uint64_t)bj * 32 + r, col = (uint64_t)bi * 32 + tx;  // the mirror image
-        if (row < n && col < n && col > row) C[row * ldc + col] = t[tx][r];
+        for (int e = 0; e < 4; ++e) {
+            v[e] = alpha * v[e];
+            if (beta != 0.0f) v[e] += beta * old[e];
+            sum[e] = v[e];
+        }
+        *reinterpret_cast<float4u*>(out) = sum;
+    } else if (row < n) {
+        for (int e = 0; e < 4; ++e) {
+            if (col + e > row || col + e >= n) continue;
+            v[e] = alpha * v[e];
+            if (beta != 0.0f) v[e] += beta * out[e];
+            out[e] = v[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[r][c + e] = v[e];
+    __syncthreads();
+    // the mirror image: four columns of row 32 bj + r, from column c .. c + 3 of the transpose
+    const uint64_t mrow = (uint64_t)bj * 32 + r, mcol = (uint64_t)bi * 32 + c;
+    float* mirror = C + mrow * ldc + mcol;
+    if (bj < bi && mcol + 4 <= n) {  // (mrow < mcol then)
+        float4u o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = t[c + e][r];
+        *reinterpret_cast<float4u*>(mirror) = o;
+    } else {
+        for (int e = 0; e < 4; ++e)
+            if (mrow < n && mcol + e < n && mcol + e > mrow) mirror[e] = t[c + e][r];
     }
 }
 
@@ -830,23 +870,40 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
     return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
 }
 
-// A symmetric product has (tiles + 1) tiles / 2 workgroups' worth of work; up to 170 of them leave a third of
-// the CUs idle, and the k range is long enough to share out: three shares, a round and a half of
-// workgroups of a third of the work each.
-constexpr uint32_t kGramParts = 3;
+// A symmetric product has (tiles + 1) tiles / 2 workgroups' worth of work; up to 170 of them leave a third of the
+// CUs idle, and the k range is long enough to share out.  The number of shares is the one whose estimate is
+// smallest: rounds of workgroups over the 256 CUs times the steps of a share (1.7 us each, whatever the operand
+// format; 5 us for a workgroup's first loads and its stores), plus the pass that adds the shares up (its reads at about
+// 3 TB/s).  N = 2048 takes seven (36 tiles: 252 workgroups; three gave 108), N = 512 at 2000 values of k fifteen,
+// N = 4096 seven (952 workgroups, 3.7 rounds; three leave the second of two rounds 60 % full).  A share has at
+// least eight steps, and the shares together at most 512 MB.  Measured against three shares, X^T X of [50 000, 2048]
+// fp16: 438 -> 228 us, of [2000, 512] fp32: 80 -> 25 us.
+constexpr uint32_t kGramPartsMax = 16, kGramPartsFew = 3, kGramTilesMax = 170;
 uint32_t gram_parts(uint64_t N, uint64_t K, int dtype, bool two_planes) {
     const uint64_t tiles = (N + BM - 1) / BM, lower = tiles * (tiles + 1) / 2;
     const uint64_t steps = octets(K) / (2 * sub_steps(dtype, two_planes));
-    return (lower <= 170 && steps >= 8 * kGramParts) ? kGramParts : 1;
+    if (lower > kGramTilesMax || steps < 8 * kGramPartsFew) return 1;
+    constexpr uint64_t kCus = 256;
+    const double share_mb = 4e-6 * (double)N * (double)N;
+    uint32_t best = 1;
+    double best_us = 0;
+    for (uint32_t p = 1; p <= kGramPartsMax; ++p) {
+        if (p > 1 && (steps < 8 * p || p * share_mb > 512.0)) break;
+        const uint64_t rounds = (lower * p + kCus - 1) / kCus;
+        const double us = (double)rounds * (1.7 * (double)((steps + p - 1) / p) + 5.0) + (p > 1 ? 0.18 * p * share_mb : 0.0);
+        if (p == 1 || us < best_us) best = p, best_us = us;
+    }
+    return best;
 }
 
 int gram_impl(const void* A_planes, const float* a_scales, uint64_t N, uint64_t K, int dtype, float* C, uint64_t ldc,
               float alpha, float beta, void* ws, size_t ws_bytes, hipStream_t s) {
     if (N == 0) return TRAKHIP_OK;
     const bool two_planes = a_scales != nullptr;
-    const uint32_t parts = gram_parts(N, K, dtype, two_planes);
-    const size_t need = (size_t)parts * N * N * sizeof(float);
-    if (parts > 1 && ws && ws_bytes >= need && reinterpret_cast<uintptr_t>(ws) % 16 == 0) {
+    uint32_t parts = gram_parts(N, K, dtype, two_planes);
+    const size_t fit = ws_bytes / ((size_t)N * N * sizeof(float));  // a smaller scratch takes fewer shares
+    if (fit < parts) parts = (uint32_t)fit;
+    if (parts > 1 && ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0) {
         if (!C) return TRAKHIP_ERR_NULL;
         if (ldc < N) return TRAKHIP_ERR_SHAPE;
         float* shares = static_cast<float*>(ws);
@@ -925,9 +982,13 @@ int gemm_nt_split2(const void* A_planes, const float* a_scales, uint64_t M, cons
                         b_scales);
 }
 
-size_t gram_split_workspace_bytes(uint64_t N, uint64_t K, int dtype, int two_planes) {
+size_t gram_split_workspace_bytes(uint64_t N, uint64_t K, int dtype, int two_planes, bool most) {
     if (N == 0 || K == 0 || !known_dtype(dtype)) return 0;
-    const uint32_t parts = gram_parts(N, K, dtype, two_planes != 0);
+    uint32_t parts = gram_parts(N, K, dtype, two_planes != 0);
+    if (!most) {
+        const uint64_t tiles = (N + BM - 1) / BM, steps = octets(K) / (2 * sub_steps(dtype, two_planes != 0));
+        parts = (tiles * (tiles + 1) / 2 <= kGramTilesMax && steps >= 8 * kGramPartsFew) ? kGramPartsFew : 1;
+    }
     return parts > 1 ? (size_t)parts * N * N * sizeof(float) : 0;
 }
 

@@ -341,7 +341,7 @@ def gram_split(a, out=None, alpha=1.0, beta=0.0):
         stream = torch.cuda.current_stream(a.device).cuda_stream
         # scratch that lets a product with few tiles share its k range out over the idle CUs
         two = a.scales is not None
-        ws_bytes = lib.trakhip_gram_split_workspace(N, a.K, _STORE_DTYPES[a.dtype], int(two))
+        ws_bytes = lib.trakhip_gram_split_workspace_most(N, a.K, _STORE_DTYPES[a.dtype], int(two))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
         ws_ptr = ctypes.c_void_p(ws.data_ptr()) if ws is not None else None
         if two:
