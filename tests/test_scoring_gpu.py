@@ -132,6 +132,17 @@ def test_spd_inverse_at_the_edges_of_its_tiles(gpu, n):
     assert (scaled.double() * mean_abs.double() - inv.double()).abs().max() <= 4 * 2.0**-24 * inv.abs().max()
 
 
+@pytest.mark.parametrize("first", [0, 31, 32, 70, 127, 128, 159, 255, 299])
+@pytest.mark.parametrize("value", [-1.0, 0.0, float("nan")])
+def test_spd_inverse_names_the_first_bad_pivot(gpu, first, value):
+    a = torch.eye(300)
+    a[first, first] = value
+    if first < 290:
+        a[first + 9, first + 9] = -3.0
+    with pytest.raises(torch.linalg.LinAlgError, match=rf"pivot {first} "):
+        spd_inverse(a.to(gpu))
+
+
 def test_spd_inverse_many_blocks(gpu):
     # 67 diagonal blocks: more tree nodes of one shape than one batched launch takes, odd block counts
     n, lam = 8500, 1e-2

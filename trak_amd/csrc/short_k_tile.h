@@ -26,16 +26,16 @@ __device__ __forceinline__ void triangle_tile(uint32_t t, uint32_t& tile_m, uint
 
 // C[ROWS x 128 tile (tile_m, tile_n)] = alpha * A[M, K] * B[N, K]^T + beta * C.  Both operand tiles are
 // loaded whole (one global round trip, one barrier), the MFMAs run back to back, the old values of C
-// are fetched under them.  16-byte aligned rows, K <= 128 and a multiple of 8; 256 threads;
+// are fetched under them.  16-byte aligned rows, K <= 128 and a multiple of 8; THREADS threads;
 // `lds` holds lds_floats<ROWS>() floats, 16-byte aligned.
-// ROWS = 128: 2 x 2 waves of 64 x 64.  ROWS = 32: 1 x 4 waves of 32 x 32.
-template <int ROWS>
+// ROWS = 128: 2 x 2 waves of 64 x 64, or with 512 threads 4 x 2 waves of 32 x 64.  ROWS = 32: 1 x 4 waves of 32 x 32.
+template <int ROWS, int THREADS = kThreads>
 __device__ __forceinline__ void tile(const float* __restrict__ A, uint64_t lda, const float* __restrict__ B,
                                      uint64_t ldb, float* __restrict__ C, uint64_t ldc, uint64_t M, uint64_t N,
                                      uint32_t K, float alpha, float beta, uint32_t tile_m, uint32_t tile_n,
                                      float* __restrict__ lds) {
     constexpr int BM = kCols, kShortK = kMaxK, kShortStride = kStride;
-    constexpr int WM = ROWS >= 64 ? 2 : 1, WNV = 4 / WM;           // wave grid
+    constexpr int WM = ROWS >= 64 ? THREADS / 128 : 1, WNV = THREADS / 64 / WM;  // wave grid
     constexpr int IT = ROWS / WM / 32, JT = BM / WNV / 32;          // 32 x 32 MFMA tiles per wave
     const uint64_t m0 = (uint64_t)tile_m * ROWS, n0 = (uint64_t)tile_n * BM;
     const int tid = threadIdx.x;
@@ -44,18 +44,18 @@ __device__ __forceinline__ void tile(const float* __restrict__ A, uint64_t lda, 
     const int x = lane & 31, h = lane >> 5;
 
     // rows x 32 float4 per operand, all loads in flight at once
-    constexpr int kPiecesA = ROWS * (kShortK / 4) / kThreads, kPiecesB = BM * (kShortK / 4) / kThreads;
+    constexpr int kPiecesA = ROWS * (kShortK / 4) / THREADS, kPiecesB = BM * (kShortK / 4) / THREADS;
     float4 ra[kPiecesA], rb[kPiecesB];
 #pragma unroll
     for (int i = 0; i < kPiecesA; ++i) {
-        const int id = tid + kThreads * i;
+        const int id = tid + THREADS * i;
         const uint32_t row = id >> 5, k4 = 4 * (id & 31);
         ra[i] = (m0 + row < M && k4 < K) ? *reinterpret_cast<const float4*>(A + (m0 + row) * lda + k4)
                                          : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
     for (int i = 0; i < kPiecesB; ++i) {
-        const int id = tid + kThreads * i;
+        const int id = tid + THREADS * i;
         const uint32_t row = id >> 5, k4 = 4 * (id & 31);
         rb[i] = (n0 + row < N && k4 < K) ? *reinterpret_cast<const float4*>(B + (n0 + row) * ldb + k4)
                                          : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -64,12 +64,12 @@ __device__ __forceinline__ void tile(const float* __restrict__ A, uint64_t lda, 
     float* bs = lds + ROWS * kShortStride;
 #pragma unroll
     for (int i = 0; i < kPiecesA; ++i) {
-        const int id = tid + kThreads * i;
+        const int id = tid + THREADS * i;
         *reinterpret_cast<float4*>(as + (id >> 5) * kShortStride + 4 * (id & 31)) = ra[i];
     }
 #pragma unroll
     for (int i = 0; i < kPiecesB; ++i) {
-        const int id = tid + kThreads * i;
+        const int id = tid + THREADS * i;
         *reinterpret_cast<float4*>(bs + (id >> 5) * kShortStride + 4 * (id & 31)) = rb[i];
     }
     __syncthreads();

@@ -50,25 +50,30 @@ __global__ __launch_bounds__(256) void spd_init_kernel(const float* __restrict__
     }
 }
 
-// One workgroup of four waves: Cholesky of the 128x128 diagonal block at W (lower triangle used),
+// One workgroup of eight waves: Cholesky of the 128x128 diagonal block at W (lower triangle used),
 // L block to Lout (upper part zero), its inverse to Linv_out.
 //
-// The block is handled as 4 x 4 sub-blocks of 32 in LDS (row pitch 129 floats: conflict free by rows
-// and by columns).  For sub-block column p:
-//   - ONE WAVE factors the 32 x 32 diagonal sub-block and inverts the factor, registers only, values of
-//     other lanes through v_readlane: no barriers and no LDS round trips inside this strictly
-//     sequential part (see factor_sub_block);
-//   - the sub-blocks below become L = A X^T and the trailing sub-blocks get A -= L L^T, both on
-//     v_mfma_f32_32x32x2_f32, one 32 x 32 tile per wave at a time.
-// The off-diagonal sub-blocks of the inverse follow by halving, [A 0; B C]^-1 = [A^-1 0; -C^-1 B A^-1 C^-1],
-// two levels (32 -> 64 -> 128), again on the MFMA.  About 1200 vector instructions per sub-block on one
-// wave and a dozen workgroup barriers, against 128 barriers (and an LDS round trip
-// each) for a column-at-a-time loop over the whole block.
+// The block is handled as 4 x 4 sub-blocks of 32 in LDS.  ONE WAVE factors a 32 x 32 diagonal sub-block and inverts
+// the factor, registers only, values of other lanes through DPP: no barriers and no LDS round trips inside this
+// strictly sequential part (see factor_sub_block).  Everything else is products of 16 x 32 strips on
+// v_mfma_f32_16x16x4_f32, and what the next factorization does not wait for runs on waves of the other SIMDs beside it:
+//
+//   phase p   wave 0: factor and invert (p, p)         six waves: the other trailing updates by column p - 1, and
+//                                                      T_j = sum over m of L[p][m] X[m][j], j < p
+//             L[t][p] = A[t][p] X_pp^T for t > p, X[p][j] = -X_pp T_j for j < p            (six strips)
+//             A[p+1][p+1] -= L[p+1][p] L[p+1][p]^T                                        (two strips)
+//
+// so the inverse of the factor grows row by row with the factorization and is complete one product after the last
+// sub-block.  Bound: the four sub-blocks in sequence (32 000 of 51 000 cycles, the loads 4 300, a block's own
+// trailing update 13 700 more).  With four waves, one 32 x 32 tile at a time and the inverse behind the factorization a
+// step of the factorization (this beside the trailing update) took 43 us, now 30.
 constexpr int kSub = 32;
-constexpr int kPitch = NB + 1;
-constexpr int kTPitch = 2 * kSub + 1;
+constexpr int kPitch = NB + 4;            // 528-byte rows: 16-byte reads, conflict free over 16 rows
+constexpr int kTPitch = 3 * kSub + 4;
+constexpr int kDiagThreads = 512, kDiagWaves = kDiagThreads / 64;
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float lane_value(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
@@ -82,49 +87,95 @@ __device__ __forceinline__ int mfma_row(int r, int h) { return 8 * (r >> 2) + 4 
 // starts as the identity (v[j] = X[j][c]).  Step k scales v[k] by s = 1 / sqrt(A[k][k]) in every lane
 // (lower half: column k of L; upper half: the finished row k of X = L^-1), then for j > k every lane
 // does v[j] -= v[k] L[j][k] with L[j][k] read from lane j: the trailing update of A in the lower half,
-// forward elimination of the identity in the upper half - one lane read and one multiply-add per (k, j).
+// forward elimination of the identity in the upper half.  What a lane holds right of its own row (x < j) is never
+// used.
+//
+// L[j][k] sits in lane j of t.  Two copies of t are made per step, one with lanes 0-15 and one with lanes 16-31 in every
+// row of 16 lanes (v_permlane16_swap, v_permlane32_swap); a multiply-add then takes lane j of its row as a DPP operand
+// (row_newbcast), one instruction per (k, j).  Bound: the chain from pivot to pivot (scale, lane read, multiply-add,
+// reciprocal root, Newton step, lane read), 250 cycles per step; the other multiply-adds pass beside it.  7950 cycles per
+// sub-block; with a v_readlane into a scalar register per (k, j) in front of the multiply-add, and the test of each
+// pivot inside the chain, 8900.
+// (As assembly: the compiler folds a DPP move into v_fmac_f32 only where it had made one of the fma before, which it
+// does too late.  A register written by a vector instruction may be read through DPP two wait states later: s_nop 1.)
+template <int LANE>
+__device__ __forceinline__ void multiply_add_row(float& v, float bcast, float m) {  // v += (lane LANE of bcast's row) * m
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(v)
+        : "v"(bcast), "v"(m), "i"(LANE));
+}
+
+template <int LANE>
+__device__ __forceinline__ void multiply_add_rows4(float* v, float bcast, float m) {  // four lanes and values in a row
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])
+        : "v"(bcast), "v"(m), "i"(LANE), "i"(LANE + 1), "i"(LANE + 2), "i"(LANE + 3));
+}
+
+template <class F, int... S>
+__device__ __forceinline__ void for_each_index(F& f, std::integer_sequence<int, S...>) {
+    (f(std::integral_constant<int, S>{}), ...);
+}
+
 __device__ __forceinline__ void factor_sub_block(float* As, float* Xs, int base, int lane, int32_t first_index,
                                                  int32_t* status) {
     const int x = lane & 31;
     const bool lower = lane < kSub;
     float v[kSub];
-    int32_t bad = 0;  // 1 + index of the first pivot that is not positive
-    // every lane reads its row (the upper half-wave the same one again): 32 loads in flight, no
+    // every lane reads its row (the upper half-wave the same one again): eight 16-byte loads in flight, no
     // branch per element around them
-    float row[kSub];
+    floatx4 row[kSub / 4];
 #pragma unroll
-    for (int j = 0; j < kSub; ++j) row[j] = As[(base + x) * kPitch + base + j];
+    for (int j = 0; j < kSub / 4; ++j) row[j] = *reinterpret_cast<const floatx4*>(As + (base + x) * kPitch + base + 4 * j);
 #pragma unroll
-    for (int j = 0; j < kSub; ++j) {
-        asm volatile("" : "+v"(row[j]));
-        v[j] = lower ? row[j] : (j == x ? 1.0f : 0.0f);
-    }
-#pragma unroll
-    for (int k = 0; k < kSub; ++k) {
-        float d = lane_value(v[k], k);
-        // a pivot that is not positive is recorded and replaced, without a branch: the 32 steps stay one
-        // straight line of code
-        const bool ok = d > 0.0f;
-        bad = (ok || bad != 0) ? bad : 1 + first_index + k;
-        d = ok ? d : 1.0f;
-        float s = __builtin_amdgcn_rsqf(d);
-        s = s * __builtin_fmaf(-0.5f * d * s, s, 1.5f);  // one Newton step on the 1 ulp hardware value
+    for (int j = 0; j < kSub; ++j) v[j] = lower ? row[j / 4][j % 4] : (j == x ? 1.0f : 0.0f);
+    // 1 / sqrt of pivot k, which lane k holds: every lane works on its own value (one Newton step on the 1 ulp hardware
+    // value) and lane k's result is the one that counts.  The pivots are kept, lane k's in lane k, and looked at once at
+    // the end: one that is not positive makes everything behind it NaN.
+    float pivots = 1.0f;
+    auto pivot_scale = [&](int k) __attribute__((always_inline)) {
+        const float d = v[k], r = __builtin_amdgcn_rsqf(d);
+        pivots = lane == k ? d : pivots;
+        return lane_value(r * __builtin_fmaf(-0.5f * d * r, r, 1.5f), k);
+    };
+    float s = pivot_scale(0);
+    // (written out through compile-time sequences: DPP controls are immediates)
+    auto step_k = [&](auto k_const) __attribute__((always_inline)) {
+        constexpr int k = decltype(k_const)::value;
         const float t = v[k] * s;
         v[k] = t;
-        // All lane reads first, then the multiply-adds: a scalar register written by a vector
-        // instruction cannot be read by the next one.  The empty volatile statement and the fences pin
-        // each step between its neighbours (otherwise lane reads of later steps drift up here and
-        // their scalar results spill).
-        __builtin_amdgcn_sched_barrier(0);
-        float lj[kSub];
-#pragma unroll
-        for (int j = k + 1; j < kSub; ++j) lj[j] = lane_value(t, j);
-#pragma unroll
-        for (int j = k + 1; j < kSub; ++j) v[j] = __builtin_fmaf(-t, lj[j], v[j]);
-        if (k + 1 < kSub) asm volatile("" : "+v"(v[k + 1]));
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (bad != 0 && lane == 0 && status && *status == 0) *status = bad;
+        if constexpr (k + 1 < kSub) {
+            const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
+            const float lo = __uint_as_float(__builtin_amdgcn_permlane32_swap(rows[0], rows[0], false, false)[0]);
+            const float hi = __uint_as_float(__builtin_amdgcn_permlane32_swap(rows[1], rows[1], false, false)[0]);
+            const float minus_t = -t;
+            // The next pivot needs only the first multiply-add: its chain (lane read, reciprocal root, Newton
+            // step) passes under the others, single ones up to a multiple of four, then four at a time.  The empty
+            // volatile statement and the fence pin each step between its neighbours.
+            constexpr int j1 = k + 1, j4 = (k + 5) / 4 * 4;
+            v[j1] = __builtin_fmaf(lane_value(t, j1), minus_t, v[j1]);  // (a scalar operand: sooner there than lo and hi)
+            s = pivot_scale(j1);
+            auto single = [&](auto i_const) __attribute__((always_inline)) {
+                constexpr int j = j1 + 1 + decltype(i_const)::value;
+                multiply_add_row<j % 16>(v[j], j < 16 ? lo : hi, minus_t);
+            };
+            for_each_index(single, std::make_integer_sequence<int, j4 - j1 - 1>{});
+            auto four = [&](auto i_const) __attribute__((always_inline)) {
+                constexpr int j = j4 + 4 * decltype(i_const)::value;
+                multiply_add_rows4<j % 16>(v + j, j < 16 ? lo : hi, minus_t);
+            };
+            for_each_index(four, std::make_integer_sequence<int, (kSub - j4) / 4>{});
+            asm volatile("" : "+v"(v[k + 1]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for_each_index(step_k, std::make_integer_sequence<int, kSub>{});
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(!(pivots > 0.0f));
+    if (bad != 0 && lane == 0 && status && *status == 0) *status = 1 + first_index + __builtin_ctzll(bad);
     // lower half: row x of L (zero above the diagonal); upper half: X[j][x], zero above the diagonal by
     // construction.  One store per j for the whole wave.
     float* dst = lower ? As + (base + x) * kPitch + base : Xs + base * kPitch + base + x;
@@ -133,43 +184,72 @@ __device__ __forceinline__ void factor_sub_block(float* As, float* Xs, int base,
     for (int j = 0; j < kSub; ++j) dst[j * step] = (lower && j > x) ? 0.0f : v[j];
 }
 
-// acc += sign * A[32 x K] * op(B): A rows at `a` (pitch pa, k contiguous); B^T rows at `b` (B_T: pitch
-// pb, k contiguous) or B rows at `b` (k down the rows, pitch pb).  LDS operands.
+// acc[q] += sign * A[16 x K] * op(B)[:, 16 q .. 16 q + 15], q = 0, 1: a strip of 16 rows and 32 columns.  A rows at `a`
+// (pitch pa, k contiguous); B^T rows at `b` (B_T: pitch pb, k contiguous) or B rows at `b` (k down the rows).  K a
+// multiple of 32.  Quarter g of the wave (lane / 16) takes k = 16 s + 4 g + t for the t-th MFMA of sub-step s, so that
+// an operand whose k is contiguous is one 16-byte LDS read per four MFMAs.
 template <bool B_T>
-__device__ __forceinline__ floatx16 tile_product(const float* a, int pa, const float* b, int pb, int K, float sign,
-                                                 floatx16 acc, int lane) {
-    const int x = lane & 31, h = lane >> 5;
-    for (int k2 = 0; k2 < K; k2 += 2) {  // the half-wave h takes k2 + h
-        const int k = k2 + h;
-        const float av = sign * a[x * pa + k];
-        const float bv = B_T ? b[x * pb + k] : b[k * pb + x];
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
+__device__ __forceinline__ void strip_product(const float* a, int pa, const float* b, int pb, int K, float sign,
+                                              floatx4 (&acc)[2], int lane) {
+    const int x = lane & 15, g = lane >> 4;
+    for (int k0 = 0; k0 < K; k0 += 32) {
+        floatx4 fa[2], fb[2][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int k = k0 + 16 * s + 4 * g;
+            fa[s] = *reinterpret_cast<const floatx4*>(a + x * pa + k);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (B_T) {
+                    fb[s][q] = *reinterpret_cast<const floatx4*>(b + (16 * q + x) * pb + k);
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) fb[s][q][t] = b[(k + t) * pb + 16 * q + x];
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * fa[s][t], fb[s][q][t], acc[q], 0, 0, 0);
     }
-    return acc;
 }
 
-__device__ __forceinline__ floatx16 tile_load(const float* c, int pc, int lane) {
-    const int x = lane & 31, h = lane >> 5;
-    floatx16 acc;
+// Row 4 (lane / 16) + r of a 16 x 16 MFMA result is in register r; its column is lane % 16.
+__device__ __forceinline__ void strip_load(const float* c, int pc, floatx4 (&acc)[2], int lane) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = c[mfma_row(r, h) * pc + x];
-    return acc;
-}
-
-__device__ __forceinline__ void tile_store(float* c, int pc, const floatx16& acc, int lane) {
-    const int x = lane & 31, h = lane >> 5;
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) c[mfma_row(r, h) * pc + x] = acc[r];
+        for (int r = 0; r < 4; ++r) acc[q][r] = c[(4 * (lane >> 4) + r) * pc + 16 * q + (lane & 15)];
 }
 
-__device__ __forceinline__ floatx16 tile_zero() {
-    floatx16 acc;
+__device__ __forceinline__ void strip_store(float* c, int pc, const floatx4 (&acc)[2], int lane) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    return acc;
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[(4 * (lane >> 4) + r) * pc + 16 * q + (lane & 15)] = acc[q][r];
 }
 
-constexpr int kDiagLdsFloats = 2 * NB * kPitch + 2 * kSub * kTPitch;  // 148 736 bytes
+__device__ __forceinline__ void strip_zero(floatx4 (&acc)[2]) {
+    acc[0] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    acc[1] = acc[0];
+}
+
+// A[ti][tj] -= P[ti] P[tj]^T, rows 16 half .. 16 half + 15 of the sub-block; P has K columns from `p` on
+__device__ __forceinline__ void trailing_strip(float* As, int ti, int tj, int half, const float* p, int K, int lane) {
+    const int row = kSub * ti + 16 * half;
+    float* c = As + row * kPitch + kSub * tj;
+    floatx4 acc[2];
+    strip_load(c, kPitch, acc, lane);
+    strip_product<true>(p + row * kPitch, kPitch, p + kSub * tj * kPitch, kPitch, K, -1.0f, acc, lane);
+    strip_store(c, kPitch, acc, lane);
+}
+
+constexpr int kDiagLdsFloats = 2 * NB * kPitch + kSub * kTPitch;  // 147 968 bytes
 
 // `panel`, when not null, is the 128 x 128 block of the factor to the left of this diagonal block
 // (row pitch ldp) whose contribution has not been taken off W yet: the block that is factored is
@@ -179,138 +259,98 @@ __device__ __forceinline__ void diag_block(const float* __restrict__ W, uint64_t
                                            int32_t* __restrict__ status, const float* __restrict__ panel,
                                            uint64_t ldp, float* __restrict__ lds) {
     float* As = lds;                        // the block, overwritten by its factor
-    float* Xs = As + NB * kPitch;           // the inverse of the factor
-    float* Ts = Xs + NB * kPitch;           // B A^-1 of the halving steps
+    float* Xs = As + NB * kPitch;           // the inverse of the factor; before that, the panel block
+    float* Ts = Xs + NB * kPitch;           // T_j of the sub-block row at work
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;  // wave index in a scalar register
+    constexpr int kBlocks = NB / kSub, kRows = NB * (NB / 4) / kDiagThreads;
+    const int r0 = tid >> 5, c = 4 * (tid & 31);
 
-    // thread -> (row tid / 32 + 8 i, four columns from 4 (tid % 32)); all sixteen loads in flight at once
+    // thread -> (row tid / 32 + 16 i, four columns from 4 (tid % 32)); all loads in flight at once
     // (the block starts at a multiple of 128 floats of a 16-byte aligned matrix with ldw % 128 == 0)
     {
-        const int r0 = tid >> 5, c = 4 * (tid & 31);
-        float4 v[16];
+        floatx4 v[kRows], w[kRows];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const float4*>(W + (uint64_t)(r0 + 8 * i) * ldw + c);
+        for (int i = 0; i < kRows; ++i) v[i] = *reinterpret_cast<const floatx4*>(W + (uint64_t)(r0 + 16 * i) * ldw + c);
+        if (panel) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = r0 + 8 * i;
-            float* a = As + r * kPitch + c;
-            float* x = Xs + r * kPitch + c;
-            a[0] = (c + 0 <= r) ? v[i].x : 0.0f;
-            a[1] = (c + 1 <= r) ? v[i].y : 0.0f;
-            a[2] = (c + 2 <= r) ? v[i].z : 0.0f;
-            a[3] = (c + 3 <= r) ? v[i].w : 0.0f;
-            x[0] = x[1] = x[2] = x[3] = 0.0f;
+            for (int i = 0; i < kRows; ++i) w[i] = *reinterpret_cast<const floatx4*>(panel + (uint64_t)(r0 + 16 * i) * ldp + c);
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) *reinterpret_cast<floatx4*>(Xs + (r0 + 16 * i) * kPitch + c) = w[i];
         }
-    }
-    constexpr int kBlocks = NB / kSub;
-    if (panel) {
-        // Xs borrows the panel block; the ten 32 x 32 sub-blocks on or under the diagonal get
-        // A -= P P^T (what is left above the diagonal is never read); then Xs is cleared again
-        const int r0 = tid >> 5, c = 4 * (tid & 31);
-        float4 v[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const float4*>(panel + (uint64_t)(r0 + 8 * i) * ldp + c);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float* x = Xs + (r0 + 8 * i) * kPitch + c;
-            x[0] = v[i].x, x[1] = v[i].y, x[2] = v[i].z, x[3] = v[i].w;
-        }
-        __syncthreads();
-        for (int t = wave; t < kBlocks * (kBlocks + 1) / 2; t += 4) {
-            const int ti = t < 1 ? 0 : (t < 3 ? 1 : (t < 6 ? 2 : 3)), tj = t - ti * (ti + 1) / 2;
-            float* tile = As + kSub * ti * kPitch + kSub * tj;
-            const floatx16 acc = tile_product<true>(Xs + kSub * ti * kPitch, kPitch, Xs + kSub * tj * kPitch, kPitch, NB,
-                                                    -1.0f, tile_load(tile, kPitch, lane), lane);
-            tile_store(tile, kPitch, acc, lane);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float* x = Xs + (r0 + 8 * i) * kPitch + c;
-            x[0] = x[1] = x[2] = x[3] = 0.0f;
-        }
+        for (int i = 0; i < kRows; ++i) *reinterpret_cast<floatx4*>(As + (r0 + 16 * i) * kPitch + c) = v[i];
     }
     __syncthreads();
+    if (panel) {  // the ten sub-blocks on or under the diagonal (what is above it is never read)
+        for (int u = wave; u < kBlocks * (kBlocks + 1); u += kDiagWaves) {
+            const int t = u >> 1;
+            const int ti = t < 1 ? 0 : (t < 3 ? 1 : (t < 6 ? 2 : 3)), tj = t - ti * (ti + 1) / 2;
+            trailing_strip(As, ti, tj, u & 1, Xs, NB, lane);
+        }
+        __syncthreads();
+    }
 
     for (int p = 0; p < kBlocks; ++p) {
         const int base = kSub * p;
-        if (wave == 0) factor_sub_block(As, Xs, base, lane, block_index * NB + base, status);
+        if (wave == 0) {
+            factor_sub_block(As, Xs, base, lane, block_index * NB + base, status);
+        } else if (p > 0 && wave != 4) {  // (wave 4 shares wave 0's SIMD)
+            // trailing sub-blocks (ti, tj), p <= tj <= ti, except (p, p), by column p - 1; then T_j
+            const int q = kBlocks - p, trailing = q * (q + 1) - 2;
+            for (int u = wave < 4 ? wave - 1 : wave - 2; u < trailing + 2 * p; u += kDiagWaves - 2) {
+                if (u < trailing) {
+                    const int t = 1 + (u >> 1), ti = t < 3 ? 1 : 2, tj = t - ti * (ti + 1) / 2;
+                    trailing_strip(As, p + ti, p + tj, u & 1, As + base - kSub, kSub, lane);
+                } else {
+                    const int j = (u - trailing) >> 1, half = u & 1;
+                    floatx4 acc[2];
+                    strip_zero(acc);
+                    strip_product<false>(As + (base + 16 * half) * kPitch + kSub * j, kPitch,
+                                         Xs + kSub * j * kPitch + kSub * j, kPitch, base - kSub * j, 1.0f, acc, lane);
+                    strip_store(Ts + 16 * half * kTPitch + kSub * j, kTPitch, acc, lane);
+                }
+            }
+        }
         __syncthreads();
         const int below = kBlocks - 1 - p;  // sub-blocks under the diagonal one
+        for (int u = wave; u < 2 * (below + p); u += kDiagWaves) {
+            const int half = u & 1;
+            floatx4 acc[2];
+            strip_zero(acc);
+            if (u < 2 * below) {  // L[t][p], in place: a wave has read its rows before it writes them
+                float* rows = As + (base + kSub * (1 + (u >> 1)) + 16 * half) * kPitch + base;
+                strip_product<true>(rows, kPitch, Xs + base * kPitch + base, kPitch, kSub, 1.0f, acc, lane);
+                strip_store(rows, kPitch, acc, lane);
+            } else {  // X[p][j]
+                const int j = (u - 2 * below) >> 1;
+                float* rows = Xs + (base + 16 * half) * kPitch;
+                strip_product<false>(rows + base, kPitch, Ts + kSub * j, kTPitch, kSub, -1.0f, acc, lane);
+                strip_store(rows + kSub * j, kPitch, acc, lane);
+            }
+        }
+        __syncthreads();
         if (below == 0) break;
-        // L[t][p] = A[t][p] X_pp^T, one sub-block per wave (at most three)
-        if (wave < below) {
-            float* tile = As + (base + kSub * (1 + wave)) * kPitch + base;
-            const floatx16 acc = tile_product<true>(tile, kPitch, Xs + base * kPitch + base, kPitch, kSub, 1.0f,
-                                                    tile_zero(), lane);
-            tile_store(tile, kPitch, acc, lane);  // every read of the tile precedes this in the wave's LDS order
-        }
-        __syncthreads();
-        // A[ti][tj] -= L[ti][p] L[tj][p]^T for the sub-blocks tj <= ti below and right of (p, p)
-        const int tiles = below * (below + 1) / 2;
-        for (int t = wave; t < tiles; t += 4) {
-            const int ti = t < 1 ? 0 : (t < 3 ? 1 : 2), tj = t - ti * (ti + 1) / 2;
-            const int ri = base + kSub * (1 + ti), rj = base + kSub * (1 + tj);
-            float* tile = As + ri * kPitch + rj;
-            const floatx16 acc = tile_product<true>(As + ri * kPitch + base, kPitch, As + rj * kPitch + base, kPitch,
-                                                    kSub, -1.0f, tile_load(tile, kPitch, lane), lane);
-            tile_store(tile, kPitch, acc, lane);
-        }
+        if (wave < 2) trailing_strip(As, p + 1, p + 1, wave, As + base, kSub, lane);
         __syncthreads();
     }
 
-    // halving, level 1: sub-block pairs (0, 1) and (2, 3) on waves 0 and 1
-    if (wave < 2) {
-        const int lo = 2 * kSub * wave, mid = lo + kSub;
-        float* scratch = Ts + kSub * wave * kTPitch;
-        const floatx16 t = tile_product<false>(As + mid * kPitch + lo, kPitch, Xs + lo * kPitch + lo, kPitch, kSub, 1.0f,
-                                               tile_zero(), lane);
-        tile_store(scratch, kTPitch, t, lane);
-    }
-    __syncthreads();
-    if (wave < 2) {
-        const int lo = 2 * kSub * wave, mid = lo + kSub;
-        const float* scratch = Ts + kSub * wave * kTPitch;
-        const floatx16 r = tile_product<false>(Xs + mid * kPitch + mid, kPitch, scratch, kTPitch, kSub, -1.0f,
-                                               tile_zero(), lane);
-        tile_store(Xs + mid * kPitch + lo, kPitch, r, lane);
-    }
-    __syncthreads();
-    // level 2: the 64 x 64 block under the diagonal, one 32 x 32 tile per wave
-    {
-        const int ti = wave >> 1, tj = wave & 1, half = 2 * kSub;
-        const floatx16 t = tile_product<false>(As + (half + kSub * ti) * kPitch, kPitch, Xs + kSub * tj, kPitch, half,
-                                               1.0f, tile_zero(), lane);
-        tile_store(Ts + kSub * ti * kTPitch + kSub * tj, kTPitch, t, lane);
-        __syncthreads();
-        const floatx16 r = tile_product<false>(Xs + (half + kSub * ti) * kPitch + half, kPitch, Ts + kSub * tj, kTPitch,
-                                               half, -1.0f, tile_zero(), lane);
-        tile_store(Xs + (half + kSub * ti) * kPitch + kSub * tj, kPitch, r, lane);
-    }
-    __syncthreads();
-
-    {
-        const int r0 = tid >> 5, c = 4 * (tid & 31);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = r0 + 8 * i;
-            const float* a = As + r * kPitch + c;
-            const float* x = Xs + r * kPitch + c;
-            const float a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];  // read first, then select: no branches
-            const float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
-            float4 l, li;
-            l.x = (c + 0 <= r) ? a0 : 0.0f, li.x = (c + 0 <= r) ? x0 : 0.0f;
-            l.y = (c + 1 <= r) ? a1 : 0.0f, li.y = (c + 1 <= r) ? x1 : 0.0f;
-            l.z = (c + 2 <= r) ? a2 : 0.0f, li.z = (c + 2 <= r) ? x2 : 0.0f;
-            l.w = (c + 3 <= r) ? a3 : 0.0f, li.w = (c + 3 <= r) ? x3 : 0.0f;
-            *reinterpret_cast<float4*>(Lout + (uint64_t)r * ldl + c) = l;
-            *reinterpret_cast<float4*>(Linv_out + (uint64_t)r * ldl + c) = li;
+    for (int i = 0; i < kRows; ++i) {
+        const int r = r0 + 16 * i;
+        floatx4 l = *reinterpret_cast<const floatx4*>(As + r * kPitch + c);
+        floatx4 li = *reinterpret_cast<const floatx4*>(Xs + r * kPitch + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            l[e] = c + e <= r ? l[e] : 0.0f;
+            li[e] = c + e <= r ? li[e] : 0.0f;
         }
+        *reinterpret_cast<floatx4*>(Lout + (uint64_t)r * ldl + c) = l;
+        *reinterpret_cast<floatx4*>(Linv_out + (uint64_t)r * ldl + c) = li;
     }
 }
 
-__global__ __launch_bounds__(256) void spd_diag_kernel(const float* __restrict__ W, uint64_t ldw,
+__global__ __launch_bounds__(kDiagThreads, 2) void spd_diag_kernel(const float* __restrict__ W, uint64_t ldw,
                                                        float* __restrict__ Lout, float* __restrict__ Linv_out,
                                                        uint64_t ldl, int32_t block_index,
                                                        int32_t* __restrict__ status) {
@@ -322,10 +362,10 @@ __global__ __launch_bounds__(256) void spd_diag_kernel(const float* __restrict__
 // workgroup 0 takes the next diagonal block (j+1, j+1) - its own trailing update, then factor and
 // inverse - while workgroups 1 .. T-1 apply the trailing update W -= panel panel^T to the other
 // lower-triangle tiles (tile numbers in the triangle's row-by-row order; number 0 is that diagonal
-// block).  Nothing in the launch depends on anything else in it, and the 31 us of the sequential
+// block).  Nothing in the launch depends on anything else in it, and the 21-28 us of the sequential
 // diagonal work no longer sit between two launches but beside the trailing update.
 //   Wt    trailing matrix, block (j+1, j+1) at its origin;  panel  L[j+1:, j] (rows x 128, pitch np)
-__global__ __launch_bounds__(256, 1) void spd_step_kernel(float* __restrict__ Wt, const float* __restrict__ panel,
+__global__ __launch_bounds__(kDiagThreads, 2) void spd_step_kernel(float* __restrict__ Wt, const float* __restrict__ panel,
                                                           uint64_t np, uint64_t rows, float* __restrict__ Lout,
                                                           float* __restrict__ Linv_out, int32_t block_index,
                                                           int32_t* __restrict__ status) {
@@ -336,7 +376,7 @@ __global__ __launch_bounds__(256, 1) void spd_step_kernel(float* __restrict__ Wt
     } else {
         uint32_t tile_m, tile_n;
         short_k::triangle_tile(blockIdx.x, tile_m, tile_n);
-        short_k::tile<NB>(panel, np, panel, np, Wt, np, rows, rows, NB, -1.0f, 1.0f, tile_m, tile_n, lds);
+        short_k::tile<NB, kDiagThreads>(panel, np, panel, np, Wt, np, rows, rows, NB, -1.0f, 1.0f, tile_m, tile_n, lds);
     }
 }
 
@@ -413,8 +453,6 @@ constexpr int kColPitch = kTriTile + 8;   // k-row tile, 32 rows: the half-waves
 constexpr int kTriFloats = kTriTile * kRowPitch;
 static_assert(kTriStep * kColPitch == kTriFloats, "both operand layouts take the same room");
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
 template <bool KROW>
 __device__ __forceinline__ void tri_load(const float* __restrict__ p, uint64_t ld, uint32_t x0, uint32_t k0, int tid,
                                          floatx4 (&r)[2]) {
@@ -477,7 +515,9 @@ __global__ __launch_bounds__(256, 2) void tri_product_kernel(const float* __rest
         tri_load<kKrowA>(A, np, m0, k_begin + kTriStep * u, tid, ra[u]);
         tri_load<true>(B, np, n0, k_begin + kTriStep * u, tid, rb[u]);
     }
-    floatx16 acc[2] = {tile_zero(), tile_zero()};
+    floatx16 acc[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
     for (uint32_t k0 = k_begin; k0 < k_end; k0 += NB) {
         const bool more = k0 + NB < k_end;
 #pragma unroll
@@ -623,7 +663,7 @@ int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t
     // Diagonal block 0 alone; then per block column j: the panel below it, and one launch that holds both
     // the trailing update and the next diagonal block (spd_step_kernel).  Trailing updates of more than
     // 512 tiles (n > 4096) go through the general product, with the diagonal block in a launch of its own.
-    hipLaunchKernelGGL(spd_diag_kernel, dim3(1), dim3(256), 0, s, W, np, L, Li, np, 0, status);
+    hipLaunchKernelGGL(spd_diag_kernel, dim3(1), dim3(kDiagThreads), 0, s, W, np, L, Li, np, 0, status);
     if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
     for (uint64_t j = 0; j + 1 < nblk; ++j) {
         const uint64_t off = j * NB * np + j * NB;
@@ -635,7 +675,7 @@ int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t
         if (e) return e;
         const uint64_t tiles = blocks * (blocks + 1) / 2;
         if (tiles <= 512) {
-            hipLaunchKernelGGL(spd_step_kernel, dim3((uint32_t)tiles), dim3(256), 0, s, W + tr, L + below, np, rows,
+            hipLaunchKernelGGL(spd_step_kernel, dim3((uint32_t)tiles), dim3(kDiagThreads), 0, s, W + tr, L + below, np, rows,
                                L + tr, Li + tr, (int32_t)(j + 1), status);
             if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
             continue;
@@ -644,7 +684,7 @@ int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t
         e = gemm_nt(L + below, np, L + below, np, W + tr, np, rows, rows, NB, -1.0f, 1.0f, nullptr, s,
                     kGemmLowerTilesOnly);
         if (e) return e;
-        hipLaunchKernelGGL(spd_diag_kernel, dim3(1), dim3(256), 0, s, W + tr, np, L + tr, Li + tr, np,
+        hipLaunchKernelGGL(spd_diag_kernel, dim3(1), dim3(kDiagThreads), 0, s, W + tr, np, L + tr, Li + tr, np,
                            (int32_t)(j + 1), status);
         if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
     }
