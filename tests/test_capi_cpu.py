@@ -254,3 +254,16 @@ def test_split_gemm_entry_points_validate_before_touching_the_device():
     assert ws(4096, 256, F32, 0) == 0 and ws(4096, 1024, F16, 0) == 0      # too few k steps to share out
     assert ws(0, 5, F32, 0) == 0 and ws(5, 0, F32, 0) == 0 and ws(5, 5, 9, 0) == 0
     assert gr(K=4096, N=300, ws=p, wsb=1 << 30, ldc=299) == -2 and gr(K=4096, N=300, ws=p, wsb=1 << 30, c=None) == -5
+
+
+@pytest.mark.parametrize("N", [1 << 31, (1 << 31) - 1, 3 << 31, 1 << 32])
+@pytest.mark.parametrize("workspace", [0, 1 << 30])
+def test_gram_of_more_rows_than_fit_is_refused(N, workspace):
+    """N * N * 4 is a multiple of 2^64 for N a multiple of 2^31: a size that is refused, not divided by."""
+    lib = _lib.load()
+    p, ws = ctypes.c_void_p(4096), ctypes.c_void_p(4096 if workspace else None)
+    for dtype in (_lib.F16, _lib.BF16, _lib.F32):
+        assert lib.trakhip_gram_split(p, N, 4096, dtype, p, N, 1.0, 0.0, ws, workspace, None) == -2
+    assert lib.trakhip_gram_split2(p, p, N, 4096, p, N, 1.0, 0.0, ws, workspace, None) == -2
+    for size in (lib.trakhip_gram_split_workspace, lib.trakhip_gram_split_workspace_most):
+        assert size(N, 4096, _lib.F32, 0) == 0

@@ -901,8 +901,10 @@ int gram_impl(const void* A_planes, const float* a_scales, uint64_t N, uint64_t 
     if (N == 0) return TRAKHIP_OK;
     const bool two_planes = a_scales != nullptr;
     uint32_t parts = gram_parts(N, K, dtype, two_planes);
-    const size_t fit = ws_bytes / ((size_t)N * N * sizeof(float));  // a smaller scratch takes fewer shares
-    if (fit < parts) parts = (uint32_t)fit;
+    if (parts > 1) {  // (N is bounded then: N * N * 4 neither overflows nor is zero)
+        const size_t fit = ws_bytes / ((size_t)N * N * sizeof(float));  // a smaller scratch takes fewer shares
+        if (fit < parts) parts = (uint32_t)fit;
+    }
     if (parts > 1 && ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0) {
         if (!C) return TRAKHIP_ERR_NULL;
         if (ldc < N) return TRAKHIP_ERR_SHAPE;
