@@ -187,16 +187,15 @@ int trakhip_gemm_tn(const float* A_dev, uint64_t lda, const float* B_dev, uint64
  *                                  is overwritten with the mirror image, so C is exactly
  *                                  symmetric; with beta != 0, C must have been produced this way.
  *                                  workspace_dev (may be NULL): trakhip_gram_split_workspace bytes,
- *                                  16-byte aligned.  A product with few tiles (N up to 4608) leaves
- *                                  CUs idle; with the workspace its k range is shared out over as
- *                                  many sets of workgroups as the workspace has room for N x N
- *                                  matrices (at most as many as pay off), whose sums are added in a
- *                                  fixed order
+ *                                  16-byte aligned.  A product with few tiles (N up to 4352) leaves
+ *                                  CUs idle; with the workspace its k range is shared out over
+ *                                  several sets of workgroups, each with an N x N matrix of its own
+ *                                  there, whose sums are added in a fixed order: as many sets as are
+ *                                  fastest among those that the workspace holds (which may be one)
  *   trakhip_gram_split_workspace   bytes that trakhip_gram_split (two_planes == 0) or
- *                                  trakhip_gram_split2 (two_planes != 0) can use for these sizes; 0
- *                                  when they would not use any: room for three sets
- *   trakhip_gram_split_workspace_most  the same for the number of sets that is fastest (up to 16 sets,
- *                                  512 MB)
+ *                                  trakhip_gram_split2 (two_planes != 0) uses for these sizes with at
+ *                                  most three sets; 0 when it would not use any
+ *   trakhip_gram_split_workspace_most  the same with at most 16 sets and 512 MB
  * Stand in, like trakhip_gemm_nt / trakhip_gemm_tn, for trak/score_computers.py:153 (the Gram
  * product, A = the planes of block^T), :176 and trak/utils.py:131. */
 size_t trakhip_split_bytes(uint64_t rows, uint64_t K, int src_dtype);

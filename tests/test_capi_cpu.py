@@ -267,3 +267,30 @@ def test_gram_of_more_rows_than_fit_is_refused(N, workspace):
     assert lib.trakhip_gram_split2(p, p, N, 4096, p, N, 1.0, 0.0, ws, workspace, None) == -2
     for size in (lib.trakhip_gram_split_workspace, lib.trakhip_gram_split_workspace_most):
         assert size(N, 4096, _lib.F32, 0) == 0
+
+
+def test_gram_scratch_is_the_scratch_that_the_call_uses():
+    """Both workspace functions ask the rule that the call itself goes by: no scratch where it would use none, at
+    most three sets from one and sixteen sets or 512 MB from the other."""
+    lib = _lib.load()
+    few, most = lib.trakhip_gram_split_workspace, lib.trakhip_gram_split_workspace_most
+    F16, BF16, F32 = _lib.F16, _lib.BF16, _lib.F32
+
+    def sets(size, N, K, dtype, two=0):
+        n_bytes = size(N, K, dtype, two)
+        assert n_bytes % (4 * N * N) == 0
+        return n_bytes // (4 * N * N)
+
+    for dtype in (F16, BF16, F32):
+        assert sets(few, 2048, 50_000, dtype) == 3 and sets(most, 2048, 50_000, dtype) == 7
+    assert sets(few, 4096, 50_000, F32) == 3 and sets(most, 4096, 50_000, F32) == 7
+    assert sets(few, 512, 2000, F32) == 3 and sets(most, 512, 2000, F32) == 16
+    assert sets(few, 4096, 2000, F16) == 0 and sets(most, 4096, 2000, F16) == 0    # one launch of 136 tiles is faster
+    assert sets(few, 4096, 2000, F32, 1) == 3 and sets(most, 4096, 2000, F32, 1) == 3
+    assert sets(most, 4352, 50_000, F32) > 1 and sets(most, 4353, 50_000, F32) == 0    # 17 and 18 tiles a side
+    for N in range(64, 4400, 192):
+        for K in (100, 400, 1000, 3000, 20_000, 200_000):
+            for dtype, two in ((F16, 0), (F32, 0), (F32, 1)):
+                a, b = sets(few, N, K, dtype, two), sets(most, N, K, dtype, two)
+                assert a in (0, 2, 3) and b in (0, *range(2, 17)) and a <= b and 4 * N * N * b <= 512e6
+                assert (a == b) or b > 3

@@ -789,3 +789,33 @@ def test_gram_takes_the_shares_that_its_scratch_holds(gpu, fmt, N, K):
         assert rc == 0 and torch.equal(out, out.T)
         assert rel_max(out.cpu().numpy(), want) < gemm_tol(K)
         assert ws[size // 4:].isnan().all()                                   # nothing written behind the scratch
+
+
+@pytest.mark.parametrize("fmt,N,K", [("fp16", 4096, 2000), ("split2", 4096, 2000), ("fp32", 512, 2000), ("bf16", 1024, 9000)])
+@pytest.mark.parametrize("which", ["trakhip_gram_split_workspace", "trakhip_gram_split_workspace_most"])
+def test_gram_uses_all_of_the_scratch_it_asks_for(gpu, fmt, N, K, which):
+    import ctypes
+
+    from trak_amd import _lib
+
+    dtype = {"fp32": torch.float32, "split2": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}[fmt]
+    code = {"fp32": _lib.F32, "split2": _lib.F32, "fp16": _lib.F16, "bf16": _lib.BF16}[fmt]
+    x = torch.randn(K, N, generator=torch.Generator(device=gpu).manual_seed(N), device=gpu).to(dtype)
+    two = fmt == "split2"
+    operand = split2_rows(x, transposed=True) if two else split_rows(x, transposed=True)
+    lib = _lib.load()
+    size = getattr(lib, which)(N, K, code, int(two))
+    ws = torch.full((max(size // 4, 4),), float("nan"), device=gpu)
+    out = torch.zeros(N, N, device=gpu)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    tail = (N, K) + (() if two else (code,)) + (ptr(out), N, 1.0, 0.0, ptr(ws), size,
+                                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    if two:
+        rc = lib.trakhip_gram_split2(ptr(operand.planes), ptr(operand.scales), *tail)
+    else:
+        rc = lib.trakhip_gram_split(ptr(operand.planes), *tail)
+    assert rc == 0 and torch.equal(out, out.T)
+    for share in range(size // (4 * N * N)):   # the last row of every share's lower triangle is written
+        assert not ws[share * N * N :][(N - 1) * N : N * N].isnan().any()
+    want = (x.double().T @ x.double()).cpu().numpy()
+    assert rel_max(out.cpu().numpy(), want) < (2.0 ** -19 if two else 0.0) + gemm_tol(K)

@@ -871,26 +871,32 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
 }
 
 // A symmetric product has (tiles + 1) tiles / 2 workgroups' worth of work; up to 170 of them leave a third of the
-// CUs idle, and the k range is long enough to share out.  The number of shares is the one whose estimate is
-// smallest: rounds of workgroups over the 256 CUs times the steps of a share (1.7 us each, whatever the operand
-// format; 5 us for a workgroup's first loads and its stores), plus the pass that adds the shares up (its reads at about
-// 3 TB/s).  N = 2048 takes seven (36 tiles: 252 workgroups; three gave 108), N = 512 at 2000 values of k fifteen,
-// N = 4096 seven (952 workgroups, 3.7 rounds; three leave the second of two rounds 60 % full).  A share has at
-// least eight steps, and the shares together at most 512 MB.  Measured against three shares, X^T X of [50 000, 2048]
-// fp16: 438 -> 228 us, of [2000, 512] fp32: 80 -> 25 us.
+// CUs idle, and the k range is long enough to share out.  The number of shares, up to `most` and to what `room` bytes hold,
+// is the one whose estimate is smallest: rounds of workgroups over the 256 CUs times the steps of a share (1.6 us each,
+// 1.8 for two planes; 6 us for a workgroup's first loads and its stores), plus 0.2 us per MB that the pass behind the product
+// goes over: the shares it adds up or, for one share, the matrix it mirrors.  Fitted to the times of all numbers of shares at
+// N = 512 .. 4352, K = 500 .. 50 000 in the three formats: the choice is 0.13 % above the fastest number on average and
+// 11 % at worst ([8300, 1536] fp16: 58 us with the ten it takes, 52 with eight), never more than 4 % above three shares.
+// N = 2048 takes seven (36 tiles: 252 workgroups; three gave 108), N = 512 at 2000 values of k sixteen, N = 4096 seven at
+// 50 000 values of k (952 workgroups, 3.7 rounds; three leave the second of two rounds 60 % full) and one at 2000 of 16 bits
+// (89 us; three 97).  A share has at least eight steps, and the shares together at most 512 MB.  Product and
+// sum against three shares, X^T X of [50 000, 2048] fp16: 445 -> 248 us, of [50 000, 512]: 371 -> 87 us.
 constexpr uint32_t kGramPartsMax = 16, kGramPartsFew = 3, kGramTilesMax = 170;
-uint32_t gram_parts(uint64_t N, uint64_t K, int dtype, bool two_planes) {
+uint32_t gram_parts(uint64_t N, uint64_t K, int dtype, bool two_planes, uint32_t most, size_t room = SIZE_MAX) {
     const uint64_t tiles = (N + BM - 1) / BM, lower = tiles * (tiles + 1) / 2;
     const uint64_t steps = octets(K) / (2 * sub_steps(dtype, two_planes));
     if (lower > kGramTilesMax || steps < 8 * kGramPartsFew) return 1;
+    // (N is bounded from here on: N * N * 4 neither overflows nor is zero)
+    const size_t fit = room / ((size_t)N * N * sizeof(float));
     constexpr uint64_t kCus = 256;
     const double share_mb = 4e-6 * (double)N * (double)N;
+    const double step_us = two_planes ? 1.8 : 1.6;
     uint32_t best = 1;
     double best_us = 0;
-    for (uint32_t p = 1; p <= kGramPartsMax; ++p) {
-        if (p > 1 && (steps < 8 * p || p * share_mb > 512.0)) break;
+    for (uint32_t p = 1; p <= most; ++p) {
+        if (p > 1 && (p > fit || steps < 8 * p || p * share_mb > 512.0)) break;
         const uint64_t rounds = (lower * p + kCus - 1) / kCus;
-        const double us = (double)rounds * (1.7 * (double)((steps + p - 1) / p) + 5.0) + (p > 1 ? 0.18 * p * share_mb : 0.0);
+        const double us = (double)rounds * (step_us * (double)((steps + p - 1) / p) + 6.0) + 0.2 * p * share_mb;
         if (p == 1 || us < best_us) best = p, best_us = us;
     }
     return best;
@@ -900,12 +906,10 @@ int gram_impl(const void* A_planes, const float* a_scales, uint64_t N, uint64_t 
               float alpha, float beta, void* ws, size_t ws_bytes, hipStream_t s) {
     if (N == 0) return TRAKHIP_OK;
     const bool two_planes = a_scales != nullptr;
-    uint32_t parts = gram_parts(N, K, dtype, two_planes);
-    if (parts > 1) {  // (N is bounded then: N * N * 4 neither overflows nor is zero)
-        const size_t fit = ws_bytes / ((size_t)N * N * sizeof(float));  // a smaller scratch takes fewer shares
-        if (fit < parts) parts = (uint32_t)fit;
-    }
-    if (parts > 1 && ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0) {
+    // a smaller scratch takes the number of shares that is fastest among those it holds
+    const bool usable = ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0;
+    const uint32_t parts = usable ? gram_parts(N, K, dtype, two_planes, kGramPartsMax, ws_bytes) : 1;
+    if (parts > 1) {
         if (!C) return TRAKHIP_ERR_NULL;
         if (ldc < N) return TRAKHIP_ERR_SHAPE;
         float* shares = static_cast<float*>(ws);
@@ -986,11 +990,7 @@ int gemm_nt_split2(const void* A_planes, const float* a_scales, uint64_t M, cons
 
 size_t gram_split_workspace_bytes(uint64_t N, uint64_t K, int dtype, int two_planes, bool most) {
     if (N == 0 || K == 0 || !known_dtype(dtype)) return 0;
-    uint32_t parts = gram_parts(N, K, dtype, two_planes != 0);
-    if (!most) {
-        const uint64_t tiles = (N + BM - 1) / BM, steps = octets(K) / (2 * sub_steps(dtype, two_planes != 0));
-        parts = (tiles * (tiles + 1) / 2 <= kGramTilesMax && steps >= 8 * kGramPartsFew) ? kGramPartsFew : 1;
-    }
+    const uint32_t parts = gram_parts(N, K, dtype, two_planes != 0, most ? kGramPartsMax : kGramPartsFew);
     return parts > 1 ? (size_t)parts * N * N * sizeof(float) : 0;
 }
 

@@ -63,7 +63,7 @@ int split_rows(const void* src, int dtype, uint64_t ld, uint64_t rows, uint64_t 
 int gemm_nt_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_t N, uint64_t K, int dtype, float* C,
                   uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags = 0);
 // ws (may be null): room for as many N x N matrices as a product with few tiles may share its k range out over
-// (gram_split_workspace_bytes: for three, or for the number that is fastest)
+// (gram_split_workspace_bytes: for the number that is fastest among up to three, or among all of them)
 size_t gram_split_workspace_bytes(uint64_t N, uint64_t K, int dtype, int two_planes, bool most);
 int gram_split(const void* A_planes, uint64_t N, uint64_t K, int dtype, float* C, uint64_t ldc, float alpha, float beta,
                void* ws, size_t ws_bytes, hipStream_t s);
