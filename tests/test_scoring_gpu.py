@@ -819,3 +819,26 @@ def test_gram_uses_all_of_the_scratch_it_asks_for(gpu, fmt, N, K, which):
         assert not ws[share * N * N :][(N - 1) * N : N * N].isnan().any()
     want = (x.double().T @ x.double()).cpu().numpy()
     assert rel_max(out.cpu().numpy(), want) < (2.0 ** -19 if two else 0.0) + gemm_tol(K)
+
+
+@pytest.mark.parametrize("room", [7, 6, 3, 2, 0])
+def test_gram_makes_do_with_the_memory_that_is_left(gpu, monkeypatch, room):
+    """The allocator has room for all seven shares, for three, or for none (the error it raises, forced here)."""
+    N, K = 2048, 9000
+    x = torch.randn(K, N, generator=torch.Generator(device=gpu).manual_seed(3), device=gpu).half()
+    operand = split_rows(x, transposed=True)
+    out = torch.empty(N, N, device=gpu)
+    share, asked, empty = 4 * N * N, [], torch.empty
+
+    def limited(size, **kw):
+        asked.append(size)
+        if size > room * share:
+            raise torch.OutOfMemoryError("no room")
+        return empty(size, **kw)
+
+    monkeypatch.setattr(torch, "empty", limited)
+    gram_split(operand, out=out)
+    monkeypatch.undo()
+    assert asked == ([7 * share] if room == 7 else [7 * share, 3 * share])
+    want = (x.double().T @ x.double()).cpu().numpy()
+    assert torch.equal(out, out.T) and rel_max(out.cpu().numpy(), want) < gemm_tol(K)

@@ -324,6 +324,19 @@ def matmul_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None, two_planes=Fa
     return gemm_nt_split(*split_pair(a, b), out=out, alpha=alpha, beta=beta, row_scale=row_scale)
 
 
+def _gram_scratch(lib, N, K, dtype, two, device):
+    """Scratch that lets a symmetric product with few tiles share its k range out over the idle CUs (None where
+    it would use none): up to 512 MB, or where that is not to be had, up to three N x N matrices, or none."""
+    for size in (lib.trakhip_gram_split_workspace_most, lib.trakhip_gram_split_workspace):
+        n_bytes = size(N, K, dtype, two)
+        if n_bytes:
+            try:
+                return torch.empty(n_bytes, dtype=torch.uint8, device=device)
+            except torch.OutOfMemoryError:
+                pass
+    return None
+
+
 def gram_split(a, out=None, alpha=1.0, beta=0.0):
     """out[N, N] = alpha * A @ A.T + beta * out for a SplitOperand A [N, K]: the lower-triangle tiles
     are computed and mirrored, so the result is exactly symmetric at about half the cost of
@@ -339,11 +352,9 @@ def gram_split(a, out=None, alpha=1.0, beta=0.0):
     lib = _lib.load()
     with torch.cuda.device(a.device):
         stream = torch.cuda.current_stream(a.device).cuda_stream
-        # scratch that lets a product with few tiles share its k range out over the idle CUs
         two = a.scales is not None
-        ws_bytes = lib.trakhip_gram_split_workspace_most(N, a.K, _STORE_DTYPES[a.dtype], int(two))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
-        ws_ptr = ctypes.c_void_p(ws.data_ptr()) if ws is not None else None
+        ws = _gram_scratch(lib, N, a.K, _STORE_DTYPES[a.dtype], int(two), a.device)
+        ws_ptr, ws_bytes = (ctypes.c_void_p(ws.data_ptr()), ws.numel()) if ws is not None else (None, 0)
         if two:
             code = lib.trakhip_gram_split2(
                 ctypes.c_void_p(a.planes.data_ptr()), ctypes.c_void_p(a.scales.data_ptr()), N, a.K,
