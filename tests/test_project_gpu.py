@@ -638,6 +638,22 @@ def test_passes_of_up_to_sixteen_rows(gpu, c_oracle, dtype, B, k, P, tiles):
         assert torch.equal(fn(R)(wide, k, seed, tiles)[:B], out)
 
 
+@pytest.mark.parametrize("proj_type", [R, G])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 7, 196, 255, 256, 257, 258, 259, 260])
+@pytest.mark.parametrize("B", [5, 17, 32])
+def test_fp32_chunks_at_the_ends_of_tiles(gpu, c_oracle, proj_type, tile, B):
+    """fp32 chunks that end 0 .. 3 values into a 16-byte piece, in tiles shorter than a chunk, of a chunk and a
+    little longer; what follows the gradient in memory is NaN."""
+    k, tiles, seed = 512, 3, 11
+    P = 3 * tile - (1 if tile > 3 else 0)   # the last tile one feature shorter
+    buffer = torch.full((B * P + 512,), float("nan"), device=gpu)
+    g = buffer[: B * P].view(B, P)
+    g.copy_(torch.randn(B, P, generator=torch.Generator().manual_seed(tile)))
+    want = g.double().cpu().numpy() @ c_oracle.materialize(seed, tiles, P, 0, P, 0, k, proj_type).astype(np.float64)
+    got = fn(proj_type)(g, k, seed, tiles)
+    assert rel_l2_rows(got.cpu().numpy(), want).max() < TOL[torch.float32]
+
+
 def test_many_rows_gather(gpu):
     from trak_amd import vectorize
 
