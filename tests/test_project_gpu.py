@@ -654,6 +654,24 @@ def test_fp32_chunks_at_the_ends_of_tiles(gpu, c_oracle, proj_type, tile, B):
     assert rel_l2_rows(got.cpu().numpy(), want).max() < TOL[torch.float32]
 
 
+@pytest.mark.parametrize("tile", [5, 196, 255, 257, 259, 510, 770])
+@pytest.mark.parametrize("B", [5, 17, 32])
+@pytest.mark.parametrize("cuts", [(), (0.31,), (1.0, 2.0), (0.3, 0.31, 0.99, 1.01, 2.5)])
+def test_gathered_fp32_chunks_at_the_ends_of_tiles(gpu, tile, B, cuts):
+    """The same through a list of tensors: tiles that end inside a tensor, at its end and beyond it have the bits of
+    the dense gradient; each tensor is followed by NaN."""
+    k, tiles, seed = 512, 3, 11
+    P = 3 * tile - 1
+    g = torch.randn(B, P, generator=torch.Generator().manual_seed(tile)).to(gpu)
+    edges = sorted({0, P, *(max(1, min(P - 1, int(c * tile))) for c in cuts)})
+    pieces = []
+    for lo, hi in zip(edges, edges[1:]):
+        buffer = torch.full((B * (hi - lo) + 512,), float("nan"), device=gpu)
+        pieces.append(buffer[: B * (hi - lo)].view(B, hi - lo).copy_(g[:, lo:hi]))
+    got = fast_jl.project_gather(pieces, k, seed, tiles, "rademacher")
+    assert torch.equal(got, fn(R)(g, k, seed, tiles))
+
+
 def test_many_rows_gather(gpu):
     from trak_amd import vectorize
 

@@ -222,10 +222,9 @@ struct Stage32 {
     // statement keeps them there).  With a branch per piece the compiler waited for a piece's load before it wrote the
     // zeros of the next: every chunk at a tile's end, and with less than 65 536 features every chunk is one, took four round
     // trips to memory ([64, 10 007] -> 2048 78.5 us, now 74.6; [20, 50 001] -> 1536 26.5 and 25.7).
-    __device__ __forceinline__ void load(const float* __restrict__ g, uint64_t ld, uint32_t rows,
-                                         uint64_t f_begin, uint64_t f_end, int tid) {
-        const uint64_t f = f_begin + 4u * (tid & 63);
-        const float* p = g + (uint64_t)(tid >> 6) * ld + f;
+    // (p: the thread's first piece, which starts at feature f)
+    __device__ __forceinline__ void load_end(const char* p, uint64_t piece_pitch, uint32_t rows, uint64_t f, uint64_t f_end,
+                                             int tid) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             v[i] = {0u, 0u, 0u, 0u};
@@ -235,19 +234,24 @@ struct Stage32 {
 #pragma unroll
             for (int i = 0; i < N; ++i)
                 if ((uint32_t)(tid >> 6) + W * i < rows) {
-                    const Raw16f r = gload<Raw16f>(p + (uint64_t)(W * i) * ld);
+                    const Raw16f r = gload<Raw16f>(p + i * piece_pitch);
                     v[i] = {r.x, r.y, r.z, r.w};
                 }
         } else if (f < f_end) {
 #pragma unroll
             for (int i = 0; i < N; ++i)
                 if ((uint32_t)(tid >> 6) + W * i < rows) {
-                    const float* q = p + (uint64_t)(W * i) * ld;
+                    const char* q = p + i * piece_pitch;
                     v[i].x = gload<uint32_t>(q);
-                    if (f + 1 < f_end) v[i].y = gload<uint32_t>(q + 1);
-                    if (f + 2 < f_end) v[i].z = gload<uint32_t>(q + 2);
+                    if (f + 1 < f_end) v[i].y = gload<uint32_t>(q + 4);
+                    if (f + 2 < f_end) v[i].z = gload<uint32_t>(q + 8);
                 }
         }
+    }
+    __device__ __forceinline__ void load(const float* __restrict__ g, uint64_t ld, uint32_t rows,
+                                         uint64_t f_begin, uint64_t f_end, int tid) {
+        const uint64_t f = f_begin + 4u * (tid & 63);
+        load_end(reinterpret_cast<const char*>(g + (uint64_t)(tid >> 6) * ld + f), (uint64_t)W * ld * 4, rows, f, f_end, tid);
     }
     __device__ __forceinline__ static void split(uint32_t xb, uint32_t& b1, uint32_t& b2, uint32_t& b3) {
         const float x = __uint_as_float(xb);
@@ -380,6 +384,17 @@ struct UniformSeg {
     __device__ __forceinline__ void advance(const trakhip_segment* segs, uint32_t n, uint32_t f, int tid, uint32_t row_step) {
         while (f >= end && idx + 1 < n) set(segs, idx + 1, tid, row_step);
     }
+    // a thread's cursor in this segment (nothing is read for it)
+    template <int PIECES>
+    __device__ __forceinline__ SegCursor<PIECES> cursor(int tid) const {
+        SegCursor<PIECES> c;
+        c.idx = idx;
+        c.first = first;
+        c.end = end;
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) c.base[i] = tbase - (uint32_t)(kElems * (tid % kLanes) * ESZ) + i * piece_pitch;
+        return c;
+    }
 };
 
 template <int W, int ROWS = 32>
@@ -403,12 +418,11 @@ struct Gather16 : Stage16<W, ROWS> {
     }
     // The same with a cursor that lives for this call only and starts at segment `start`, one that begins
     // at or before f_begin: for a caller that takes this path rarely and saves the registers.
-    __device__ __forceinline__ void load_from(const trakhip_segment* segs, uint32_t n, uint32_t start, uint32_t rows,
+    __device__ __forceinline__ void load_from(const trakhip_segment* segs, uint32_t n, const UniformSeg<2>& start, uint32_t rows,
                                               uint64_t f_begin, uint64_t f_end, int tid) {
         const uint64_t f64 = f_begin + 8u * (tid & 31);
         const bool live = f64 < f_end;
-        SegCursor<N> c;
-        c.set(segs, start, tid >> 5, 2 * W, 2);
+        SegCursor<N> c = start.template cursor<N>(tid);
         if (live) c.advance(segs, n, (uint32_t)f64, tid >> 5, 2 * W, 2);
         load_at(segs, n, c, rows, f64, f_end, live, tid);
     }
@@ -453,12 +467,11 @@ struct Gather32 : Stage32<W, ROWS> {
         load_at(segs, n, cur, rows, f64, f_end, live, tid);
     }
     // as Gather16::load_from
-    __device__ __forceinline__ void load_from(const trakhip_segment* segs, uint32_t n, uint32_t start, uint32_t rows,
+    __device__ __forceinline__ void load_from(const trakhip_segment* segs, uint32_t n, const UniformSeg<4>& start, uint32_t rows,
                                               uint64_t f_begin, uint64_t f_end, int tid) {
         const uint64_t f64 = f_begin + 4u * (tid & 63);
         const bool live = f64 < f_end;
-        SegCursor<N> c;
-        c.set(segs, start, tid >> 6, W, 4);
+        SegCursor<N> c = start.template cursor<N>(tid);
         if (live) c.advance(segs, n, (uint32_t)f64, tid >> 6, W, 4);
         load_at(segs, n, c, rows, f64, f_end, live, tid);
     }
@@ -751,9 +764,16 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
                     st.load_pieces(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch, rows, tid);
                 else
                     st.load_pieces(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch);
-            } else {  // chunks that cross a segment or tile end: per-thread cursors, set up for this chunk only
-                st.load_from(g, (uint32_t)ld, useg.idx, rows, c.f, c.hi, tid);
+                return;
             }
+            if constexpr (kPlanes == 3) {  // the end of a tile, inside the segment
+                if (c.hi > c.f && f32 >= useg.first && c.hi <= useg.end) {
+                    st.load_end(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch, rows, c.f + 4u * (tid & 63), c.hi, tid);
+                    return;
+                }
+            }
+            // chunks that cross a segment's end: per-thread cursors, set up for this chunk only
+            st.load_from(g, (uint32_t)ld, useg, rows, c.f, c.hi, tid);
         }
     };
     const uint32_t n_chunks = (uint32_t)(c_end - c_begin);
