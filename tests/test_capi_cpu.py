@@ -4,6 +4,7 @@ with the oracle bit for bit."""
 import ctypes
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -294,3 +295,23 @@ def test_gram_scratch_is_the_scratch_that_the_call_uses():
                 a, b = sets(few, N, K, dtype, two), sets(most, N, K, dtype, two)
                 assert a in (0, 2, 3) and b in (0, *range(2, 17)) and a <= b and 4 * N * N * b <= 512e6
                 assert (a == b) or b > 3
+
+
+def test_rademacher_kernels_keep_their_values_in_registers(tmp_path):
+    """A reload from scratch memory in the chunk loop waits for the gradient loads in flight: no instance of the kernel
+    may spill (read from the metadata of the built code objects)."""
+    llvm = "/opt/rocm/llvm/bin"
+    if not os.path.exists(f"{llvm}/llvm-objdump") or not os.path.exists(f"{llvm}/llvm-readelf"):
+        pytest.skip("no LLVM tools")
+    lib = tmp_path / "lib.so"
+    lib.symlink_to(_lib.LIB_PATH)
+    subprocess.run([f"{llvm}/llvm-objdump", "--offloading", str(lib)], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    seen = 0
+    for code in tmp_path.glob("*gfx950"):
+        notes = subprocess.run([f"{llvm}/llvm-readelf", "--notes", str(code)], check=True, capture_output=True, text=True).stdout
+        for kernel in notes.split("- .agpr_count:")[1:]:
+            name = re.search(r"\.name:\s+(\S+)", kernel).group(1)
+            if "jl_project_kernel" in name:
+                assert re.search(r"\.vgpr_spill_count:\s+0\b", kernel) and re.search(r"\.sgpr_spill_count:\s+0\b", kernel), name
+                seen += 1
+    assert seen == 3 * 2 * (3 * 3) - 2 * 3   # types x dense or gathered x columns x rows, no 64 rows of fp32

@@ -758,22 +758,27 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
             }
         } else {
             const uint32_t f32 = (uint32_t)c.f;  // P < 2^32 with segments; beyond P: c.whole is 0
-            useg.advance(g, (uint32_t)ld, f32, tid, kRowStep);
+            // 64 rows and 1024 columns leave no registers for what these paths derive from the thread's number: held across
+            // the chunk it went to scratch memory, and its reloads wait for the gradient loads in flight ([128, 703 386] fp16 -> 1024
+            // from 62 tensors: 278 us; worked out here, 271).  The other instances hold it.
+            int tid_here = tid;
+            if constexpr (RB == 2 && GPW == 4) asm volatile("" : "+v"(tid_here));
+            useg.advance(g, (uint32_t)ld, f32, tid_here, kRowStep);
             if (full_rows && c.s < c.whole && f32 >= useg.first && f32 + (uint32_t)kChunk <= useg.end) {
                 if constexpr (kSmall || kPlanes == 3)
-                    st.load_pieces(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch, rows, tid);
+                    st.load_pieces(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch, rows, tid_here);
                 else
                     st.load_pieces(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch);
                 return;
             }
             if constexpr (kPlanes == 3) {  // the end of a tile, inside the segment
                 if (c.hi > c.f && f32 >= useg.first && c.hi <= useg.end) {
-                    st.load_end(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch, rows, c.f + 4u * (tid & 63), c.hi, tid);
+                    st.load_end(useg.tbase + kEsz * (uint64_t)f32, useg.piece_pitch, rows, c.f + 4u * (tid_here & 63), c.hi, tid_here);
                     return;
                 }
             }
             // chunks that cross a segment's end: per-thread cursors, set up for this chunk only
-            st.load_from(g, (uint32_t)ld, useg, rows, c.f, c.hi, tid);
+            st.load_from(g, (uint32_t)ld, useg, rows, c.f, c.hi, tid_here);
         }
     };
     const uint32_t n_chunks = (uint32_t)(c_end - c_begin);
