@@ -19,7 +19,7 @@ sustained = the same calls back to back for --sustain seconds (default 2).
 other_configs = whole calls (Python wrapper included) of the other benchmark configurations: c1 (fp32
             [16, 1_048_576] -> 512), c2 (ResNet-9-sized), c4 (BERT-sized chunked normal), the headline shape as
             a gradient dict, and projection dimensions 3072 and 15 360.
-`--only NAME` runs one workload alone (for profiler runs): c1 | c2 | c3_b40 | c3_b48 | c3_b64 | c3_k1536 | c3_k3072 |
+`--only NAME` runs one workload alone (for profiler runs): c1 | c2 | c3_b8 | c3_b16 | c3_b40 | c3_b48 | c3_b64 | c3_k1536 | c3_k3072 |
             c3_k15360 | c3_k40960 | c3_normal_b32 | c3_normal_b64 | c3_dict | c4 | c4_rademacher | vendor_gemm | scoring |
             general_inverse | mfma_rate.
 """
@@ -271,9 +271,10 @@ def _config_calls(torch, dev, name):
         g = (torch.randn(64, P, generator=gen, device=dev) * 1e-3).half()
         p = CudaProjector(P, 4096, 7, ProjectionType.rademacher, dev, 32)
         return (lambda: p.project(g, 0)), 2.0 * 64 * P * 4096, "fp16 rademacher [64,11689512] -> 4096 (one pass of 64 rows)"
-    if name in ("c3_k1536", "c3_k3072", "c3_k15360", "c3_k40960", "c3_b40", "c3_b48"):
+    if name in ("c3_k1536", "c3_k3072", "c3_k15360", "c3_k40960", "c3_b8", "c3_b16", "c3_b40", "c3_b48"):
         # the benchmark shape at other projection dimensions (the reference's tests use 15 360, its
-        # documentation recommends 1 000 - 40 000) and at batch sizes between one and two 32-row blocks
+        # documentation recommends 1 000 - 40 000) and at batch sizes of half a 32-row block and less and between one
+        # and two of them
         P = sum(math.prod(sh) for sh in resnet18_param_shapes())
         k = int(name[4:]) if name[3] == "k" else 4096
         B = int(name[4:]) if name[3] == "b" else 32
@@ -692,7 +693,7 @@ def main():
                     help="also time the featurize / store paths and batch scaling and print them to stderr")
     ap.add_argument("--only", default=None, metavar="NAME",
                     help="run just one workload for --steps calls and print its timing (for profiler runs): "
-                         "c1 | c2 | c3_b40 | c3_b48 | c3_b64 | c3_k1536 | c3_k3072 | c3_k15360 | c3_k40960 | c3_normal_b32 | "
+                         "c1 | c2 | c3_b8 | c3_b16 | c3_b40 | c3_b48 | c3_b64 | c3_k1536 | c3_k3072 | c3_k15360 | c3_k40960 | c3_normal_b32 | "
                          "c3_normal_b64 | c3_dict | c4 | c4_rademacher | scoring | general_inverse | mfma_rate | vendor_gemm "
                          "(torch.mm on the scoring operands, for comparison)")
     ap.add_argument("--steady", action="store_true",

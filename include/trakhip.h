@@ -267,7 +267,7 @@ size_t trakhip_spd_inverse_workspace(uint64_t n);
  * receives that mean.  Stands in for torch.linalg.inv + `xtx_inv /= xtx_inv.abs().mean()` of
  * trak/score_computers.py:160-166.  A_dev is not modified; inv_dev may not alias it.
  * status_dev (device, 1 int32, may be NULL) is set to 0, or to 1 + the index of the first
- * non-positive pivot. */
+ * non-positive pivot (the result is then not finite). */
 int trakhip_spd_inverse(const float* A_dev, uint64_t lda, float lambda, float* inv_dev, uint64_t ldi,
                         uint64_t n, int normalize, float* mean_abs_dev, int32_t* status_dev,
                         void* workspace_dev, size_t workspace_bytes, void* stream);

@@ -875,11 +875,11 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
 // is the one whose estimate is smallest: rounds of workgroups over the 256 CUs times the steps of a share (1.6 us each,
 // 1.8 for two planes; 6 us for a workgroup's first loads and its stores), plus 0.2 us per MB that the pass behind the product
 // goes over: the shares it adds up or, for one share, the matrix it mirrors.  Fitted to the times of all numbers of shares at
-// N = 512 .. 4352, K = 500 .. 50 000 in the three formats: the choice is 0.13 % above the fastest number on average and
+// N = 512 .. 4352, K = 500 .. 50 000 in the three formats: the choice is 0.3 % above the fastest number on average and
 // 11 % at worst ([8300, 1536] fp16: 58 us with the ten it takes, 52 with eight), never more than 4 % above three shares.
 // N = 2048 takes seven (36 tiles: 252 workgroups; three gave 108), N = 512 at 2000 values of k sixteen, N = 4096 seven at
 // 50 000 values of k (952 workgroups, 3.7 rounds; three leave the second of two rounds 60 % full) and one at 2000 of 16 bits
-// (89 us; three 97).  A share has at least eight steps, and the shares together at most 512 MB.  Product and
+// (80 us; three 95).  A share has at least eight steps, and the shares together at most 512 MB.  Product and
 // sum against three shares, X^T X of [50 000, 2048] fp16: 445 -> 248 us, of [50 000, 512]: 371 -> 87 us.
 constexpr uint32_t kGramPartsMax = 16, kGramPartsFew = 3, kGramTilesMax = 170;
 uint32_t gram_parts(uint64_t N, uint64_t K, int dtype, bool two_planes, uint32_t most, size_t room = SIZE_MAX) {

@@ -8,18 +8,21 @@
 // the workgroup staged in LDS.
 //
 // Work decomposition
-//   workgroup = 8 waves = 1024 JL columns (512 columns when the projection
+//   workgroup = 8 waves = 1024 JL columns (768 or 512 when the projection
 //               dimension is an odd multiple of 512) x a run of consecutive
 //               256-feature chunks of the reference's feature tiles
 //               (fts = ceil(P / T) consecutive features each);
-//   wave      = 4 (or 2) groups of 32 columns, one 32x32 fp32 accumulator each;
+//   wave      = 4 (3, 2) groups of 32 columns, one 32x32 fp32 accumulator each
+//               (two for passes of more than 32 rows);
 //   lane      = (n = lane % 32, h = lane / 32): column n of each group, and the
 //               k-slots 8h..8h+7 of every MFMA.
 // The tile is walked in chunks of 256 features.  Lane half h owns features
 // [128h, 128h+128) of a chunk: MFMA number q (0..15) of the chunk contracts
 // features 128h + 8q + i (i = 0..7), so the 8 Rademacher signs a lane needs for it
 // are byte q of ONE Philox block per column per chunk, and the A operand is 16
-// contiguous bytes of a gradient row.
+// contiguous bytes of a gradient row.  Passes of up to 16 rows contract the same
+// features two q at a time on v_mfma_f32_16x16x32_{f16,bf16}, two 16x16
+// accumulators per group (see jl_project_kernel).
 //
 // A workgroup walks a run of consecutive chunks (across tile boundaries, adding the
 // products up in its accumulators) and writes one partial [B, 1024] block; a second
@@ -625,8 +628,10 @@ __device__ __forceinline__ void for_each_step(F& f, std::integer_sequence<int, S
 //       generator behind it) feeds two MFMAs;
 //   16  batches of up to 16 rows, for which half or more of a 32-row MFMA multiplies zero rows: MFMA 16x16x32 in
 //       half the time.  Step = (p, j, side), columns 32 j + 16 side ..+15, k slots 0..15 = the features of q = 2p and
-//       16..31 those of q = 2p + 1 of the 32-row step: the matrix pipe adds the two halves one after the other, so a row's
-//       result has the bits that it has in a 32-row pass.  A lane generates the block of (column 32 j + lane % 16 +
+//       16..31 those of q = 2p + 1 of the 32-row step: the matrix pipe adds the two halves one after the other, so a row of
+//       16-bit gradients has the bits that it has in a 32-row pass.  (Of fp32 gradients it has not: there a step adds
+//       the first terms of both q, then the second and the third ones, the 32-row step all three of q = 2p before those of 2p + 1.)
+//       A lane generates the block of (column 32 j + lane % 16 +
 //       16 (lane / 32), half (lane / 16) % 2), as in the 32-row kernel; a step needs bytes 2p of a block in the lower lanes
 //       and bytes 2p + 1 of the same block in the upper ones, so once per block and chunk the two half-waves trade
 //       odd bytes for even ones (pack_sides: six instructions for sixteen steps).
@@ -1011,9 +1016,9 @@ __global__ __launch_bounds__(512) void jl_project_kernel(
 //
 // Same decomposition as the Rademacher kernel (8 waves, 32-column groups, 256-feature chunks,
 // lane half h owns features [128h, 128h + 128) of a chunk), but the cost sits elsewhere: a matrix
-// entry is used for 32 multiply-adds only, and making one costs about ten vector instructions
-// (Philox4x32-10: one block per eight entries) against 1.5 for a sign, so the kernel is bound by
-// the vector ALU, not by the matrix pipe.  What keeps the count that low:
+// entry is used for 32 multiply-adds only, and making one costs about six vector instructions
+// (Philox4x32-10: one block per eight entries; eight issue slots) against 1.5 for a sign, so the kernel is
+// bound by the vector ALU (95 % of its issue slots), not by the matrix pipe (12 %).  What keeps the count that low:
 //   * one random word makes a whole Box-Muller pair: the radius R[x] and the signed pair
 //     (C[a], S[a]) come out of two LDS tables (32 KB + 64 KB, filled at kernel start from the
 //     binary32 sequences of jl_stream.h), each addressed by ONE instruction (the fields of the
@@ -1318,9 +1323,10 @@ __global__ __launch_bounds__(64 * W) void jl_project_normal_kernel(
             // Philox block of (column, offset o): o / 8 with o = 256 s + 128 h + 8 q.  What its first rounds make of the
             // block's number is the same for all columns: lane 16 x + q of a half-wave works it out for q, once per
             // chunk, and step q reads it from there through DPP (row_newbcast, an operand modifier of the xors that
-            // use it).  Issue slots per MFMA 68 -> 62; the LDS, 88 % busy with the look-ups, is what binds then:
-            // [32, 109 482 240] bf16 in chunks -> 4096 99.5 -> 98.7 ms, [64, 3 000 000] bf16 -> 4096 3.24 -> 3.10 ms,
-            // [8, 3 000 000] fp16 -> 512 0.362 -> 0.344 ms.  (The same values through an LDS table: 103 ms.)
+            // use it).  Issue slots per MFMA 68 -> 65, vector issue 99 -> 95 % busy, conflicts 59 % of the LDS cycles either way:
+            // [64, 3 000 000] bf16 -> 4096 3.24 -> 3.10 ms, [8, 3 000 000] fp16 -> 512 0.362 -> 0.344 ms, the BERT-sized
+            // [32, 109 482 240] bf16 in chunks -> 4096 as before (98.6 ms, 0.5 % less, within its noise).  (The same values through an
+            // LDS table: 103 ms.)
             const jl::BlockRounds mine = jl::block_rounds(seed, 32u * s + 16u * h + (lane & 15u));
             auto do_step = [&](auto q_c) __attribute__((always_inline)) {
                 constexpr int q = decltype(q_c)::value;
