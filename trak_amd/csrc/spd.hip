@@ -54,19 +54,22 @@ __global__ __launch_bounds__(256) void spd_init_kernel(const float* __restrict__
 // L block to Lout (upper part zero), its inverse to Linv_out.
 //
 // The block is handled as 4 x 4 sub-blocks of 32 in LDS.  ONE WAVE factors a 32 x 32 diagonal sub-block and inverts
-// the factor, registers only, values of other lanes through DPP: no barriers and no LDS round trips inside this
-// strictly sequential part (see factor_sub_block).  Everything else is products of 16 x 32 strips on
-// v_mfma_f32_16x16x4_f32, and what the next factorization does not wait for runs on waves of the other SIMDs beside it:
+// the factor, without barriers inside this strictly sequential part (see factor_sub_block).  Everything else is products of
+// 16 x 32 strips on v_mfma_f32_16x16x4_f32, and what the next factorization does not wait for runs on waves of the other
+// SIMDs beside it:
 //
-//   phase p   wave 0: factor and invert (p, p)         six waves: the other trailing updates by column p - 1, and
+//   before    all waves: the panel's share of (0, 0) and (1, 1)
+//   phase p   wave 0: factor and invert (p, p)         six waves: (t, p) for t > p and (p + 1, p + 1) less the panel's share
+//                                                      and columns 0 .. p - 1 of the factor, and
 //                                                      T_j = sum over m of L[p][m] X[m][j], j < p
 //             L[t][p] = A[t][p] X_pp^T for t > p, X[p][j] = -X_pp T_j for j < p            (six strips)
 //             A[p+1][p+1] -= L[p+1][p] L[p+1][p]^T                                        (two strips)
 //
-// so the inverse of the factor grows row by row with the factorization and is complete one product after the last
-// sub-block.  Bound: the four sub-blocks in sequence (32 000 of 51 000 cycles, the loads 4 300, a block's own
-// trailing update 13 700 more).  With four waves, one 32 x 32 tile at a time and the inverse behind the factorization a
-// step of the factorization (this beside the trailing update) took 43 us, now 30.
+// so every sub-block is brought up to date in one pass just before it is needed, and the inverse of the factor grows row by
+// row with the factorization and is complete one product after the last sub-block.  Bound: the four sub-blocks in
+// sequence, 28 000 of 47 500 cycles; loads 4400, the first two sub-blocks' share of the panel 3300, strips 6800, their
+// update 2700, stores 2300.  With the panel's share of the whole block taken off before the first sub-block (13 700
+// cycles on all waves) and 7950 cycles per sub-block it took 64 700: a step of the factorization 28 us, now 22.
 constexpr int kSub = 32;
 constexpr int kPitch = NB + 4;            // 528-byte rows: 16-byte reads, conflict free over 16 rows
 constexpr int kTPitch = 3 * kSub + 4;
@@ -82,124 +85,130 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 // Row 8*(r/4) + 4*(lane/32) + r%4 of a 32x32 MFMA result is in register r; its column is lane % 32.
 __device__ __forceinline__ int mfma_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
 
-// Factor and invert the 32 x 32 sub-block at (base, base) of As with one wave.  Lane x of the lower
-// half-wave holds row x of A in v[0..31]; lane 32 + c of the upper half holds column c of X, which
-// starts as the identity (v[j] = X[j][c]).  Step k scales v[k] by s = 1 / sqrt(A[k][k]) in every lane
-// (lower half: column k of L; upper half: the finished row k of X = L^-1), then for j > k every lane
-// does v[j] -= v[k] L[j][k] with L[j][k] read from lane j: the trailing update of A in the lower half,
-// forward elimination of the identity in the upper half.  What a lane holds right of its own row (x < j) is never
-// used.
+// Factor and invert the 32 x 32 sub-block at (base, base) of As with one wave: L over As, X = L^-1 to Dx (32 rows of
+// kDxPitch floats).  A and X (initially the identity) sit in the result layout of a 32x32 MFMA: lane = column x, register
+// r = row 8 (r / 4) + 4 (lane / 32) + r % 4, so that rows 4m .. 4m + 3 are four registers of one half-wave - and, A being
+// symmetric, those four registers of lane x are also the four entries of row x in columns 4m .. 4m + 3.  Eight panels of
+// four columns, then: the panel's columns are eliminated one by one inside these four registers (lanes of other columns
+// through v_readlane), the same four eliminations go through rows 4m .. 4m + 3 of X, and everything behind the panel gets
+// its four columns at once, A -= L4 L4^T and X -= L4 X4, two 32x32x2 MFMAs each whose operands are one
+// v_permlane32_swap away.  Rows and columns that are finished go on being updated and are not looked at again.
 //
-// L[j][k] sits in lane j of t.  Two copies of t are made per step, one with lanes 0-15 and one with lanes 16-31 in every
-// row of 16 lanes (v_permlane16_swap, v_permlane32_swap); a multiply-add then takes lane j of its row as a DPP operand
-// (row_newbcast), one instruction per (k, j).  Bound: the chain from pivot to pivot (scale, lane read, multiply-add,
-// reciprocal root, Newton step, lane read), 250 cycles per step; the other multiply-adds pass beside it.  7950 cycles per
-// sub-block; with a v_readlane into a scalar register per (k, j) in front of the multiply-add, and the test of each
-// pivot inside the chain, 8900.
-// (As assembly: the compiler folds a DPP move into v_fmac_f32 only where it had made one of the fma before, which it
-// does too late.  A register written by a vector instruction may be read through DPP two wait states later: s_nop 1.)
-template <int LANE>
-__device__ __forceinline__ void multiply_add_row(float& v, float bcast, float m) {  // v += (lane LANE of bcast's row) * m
-    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-        : "+v"(v)
-        : "v"(bcast), "v"(m), "i"(LANE));
-}
-
-template <int LANE>
-__device__ __forceinline__ void multiply_add_rows4(float* v, float bcast, float m) {  // four lanes and values in a row
-    asm("s_nop 1\n\t"
-        "v_fmac_f32_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f32_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f32_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f32_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
-        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])
-        : "v"(bcast), "v"(m), "i"(LANE), "i"(LANE + 1), "i"(LANE + 2), "i"(LANE + 3));
-}
+// Bound: the chain of one wave from pivot to pivot (reciprocal root, Newton step, lane read, scale, lane read,
+// multiply-add), 700 cycles per panel; the last of X's two products waits until the next panel's first pivot is
+// through.  6200 cycles per sub-block; a column at a time with every multiply-add on the vector unit took 7950.  The 4 x 4
+// block's factor worked out in all lanes without lane reads in the chain: 6400; X's rows a panel late between the
+// pivots: 7300.
+constexpr int kDxPitch = kSub + 4;
 
 template <class F, int... S>
 __device__ __forceinline__ void for_each_index(F& f, std::integer_sequence<int, S...>) {
     (f(std::integral_constant<int, S>{}), ...);
 }
 
-__device__ __forceinline__ void factor_sub_block(float* As, float* Xs, int base, int lane, int32_t first_index,
+__device__ __forceinline__ void factor_sub_block(float* As, float* Dx, int base, int lane, int32_t first_index,
                                                  int32_t* status) {
-    const int x = lane & 31;
-    const bool lower = lane < kSub;
-    float v[kSub];
-    // every lane reads its row (the upper half-wave the same one again): eight 16-byte loads in flight, no
-    // branch per element around them
-    floatx4 row[kSub / 4];
+    const int x = lane & 31, h = lane >> 5;
+    floatx16 a, xi;  // both with their signs turned: the products below only add
+    {
+        // lower triangle only: row x left of the diagonal, column x below it
+        floatx4 row[4];
+        float col[16];
 #pragma unroll
-    for (int j = 0; j < kSub / 4; ++j) row[j] = *reinterpret_cast<const floatx4*>(As + (base + x) * kPitch + base + 4 * j);
+        for (int j = 0; j < 4; ++j) row[j] = *reinterpret_cast<const floatx4*>(As + (base + x) * kPitch + base + 8 * j + 4 * h);
 #pragma unroll
-    for (int j = 0; j < kSub; ++j) v[j] = lower ? row[j / 4][j % 4] : (j == x ? 1.0f : 0.0f);
-    // 1 / sqrt of pivot k, which lane k holds: every lane works on its own value (one Newton step on the 1 ulp hardware
-    // value) and lane k's result is the one that counts.  The pivots are kept, lane k's in lane k, and looked at once at
-    // the end: one that is not positive makes everything behind it NaN.
+        for (int r = 0; r < 16; ++r) col[r] = As[(base + mfma_row(r, h)) * kPitch + base + x];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            a[r] = mfma_row(r, h) >= x ? -col[r] : -row[r >> 2][r & 3];
+            xi[r] = mfma_row(r, h) == x ? -1.0f : 0.0f;
+        }
+    }
+    // The pivots are kept, pivot k's in lane k of its half-wave, and looked at once at the end: one that is not positive
+    // makes everything behind it NaN.
     float pivots = 1.0f;
-    auto pivot_scale = [&](int k) __attribute__((always_inline)) {
-        const float d = v[k], r = __builtin_amdgcn_rsqf(d);
-        pivots = lane == k ? d : pivots;
-        return lane_value(r * __builtin_fmaf(-0.5f * d * r, r, 1.5f), k);
-    };
-    float s = pivot_scale(0);
-    // (written out through compile-time sequences: DPP controls are immediates)
-    auto step_k = [&](auto k_const) __attribute__((always_inline)) {
-        constexpr int k = decltype(k_const)::value;
-        const float t = v[k] * s;
-        v[k] = t;
-        if constexpr (k + 1 < kSub) {
-            const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
-            const float lo = __uint_as_float(__builtin_amdgcn_permlane32_swap(rows[0], rows[0], false, false)[0]);
-            const float hi = __uint_as_float(__builtin_amdgcn_permlane32_swap(rows[1], rows[1], false, false)[0]);
-            const float minus_t = -t;
-            // The next pivot needs only the first multiply-add: its chain (lane read, reciprocal root, Newton
-            // step) passes under the others, single ones up to a multiple of four, then four at a time.  The empty
-            // volatile statement and the fence pin each step between its neighbours.
-            constexpr int j1 = k + 1, j4 = (k + 5) / 4 * 4;
-            v[j1] = __builtin_fmaf(lane_value(t, j1), minus_t, v[j1]);  // (a scalar operand: sooner there than lo and hi)
-            s = pivot_scale(j1);
-            auto single = [&](auto i_const) __attribute__((always_inline)) {
-                constexpr int j = j1 + 1 + decltype(i_const)::value;
-                multiply_add_row<j % 16>(v[j], j < 16 ? lo : hi, minus_t);
-            };
-            for_each_index(single, std::make_integer_sequence<int, j4 - j1 - 1>{});
-            auto four = [&](auto i_const) __attribute__((always_inline)) {
-                constexpr int j = j4 + 4 * decltype(i_const)::value;
-                multiply_add_rows4<j % 16>(v + j, j < 16 ? lo : hi, minus_t);
-            };
-            for_each_index(four, std::make_integer_sequence<int, (kSub - j4) / 4>{});
-            asm volatile("" : "+v"(v[k + 1]));
+    const bool first_of_four = (lane & 3) == 0, second_of_four = (lane & 3) == 1, third_of_four = (lane & 3) == 2;
+    float l_late = 0.0f, y_late = 0.0f;  // operands of the product that a panel leaves to the next one
+    auto panel = [&](auto m_const) __attribute__((always_inline)) {
+        constexpr int m = decltype(m_const)::value, kHalf = m & 1, kReg = 4 * (m >> 1), kLane = 32 * kHalf + 4 * m;
+        float l[4], y[4], d[4], s[4], b[4][4], l_pair[2];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) l[t] = -a[kReg + t];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            // 1 / sqrt of the pivot (one Newton step on the 1 ulp hardware value): every lane works on its own value and
+            // the pivot's lane is the one that counts
+            d[t] = l[t];
+            const float r = __builtin_amdgcn_rsqf(d[t]);
+            s[t] = lane_value(r * __builtin_fmaf(-0.5f * d[t] * r, r, 1.5f), kLane + t);
+            l[t] *= s[t];
+#pragma unroll
+            for (int u = t + 1; u < 4; ++u) {
+                b[u][t] = lane_value(l[t], kLane + u);
+                l[u] = __builtin_fmaf(-b[u][t], l[t], l[u]);
+            }
+            if constexpr (m > 0) {
+                if (t == 1) xi = __builtin_amdgcn_mfma_f32_32x32x2f32(l_late, y_late, xi, 0, 0, 0);
+            }
+            if constexpr (m < 7) {
+                if (t & 1) {  // lower half-wave: first column of a pair, upper half-wave: the second one
+                    const auto pair =
+                        __builtin_amdgcn_permlane32_swap(__float_as_uint(l[t - 1]), __float_as_uint(l[t]), false, false);
+                    l_pair[t >> 1] = __uint_as_float(pair[kHalf]);
+                    a = __builtin_amdgcn_mfma_f32_32x32x2f32(l_pair[t >> 1], l_pair[t >> 1], a, 0, 0, 0);
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    for_each_index(step_k, std::make_integer_sequence<int, kSub>{});
-    const uint64_t bad = __builtin_amdgcn_ballot_w64(!(pivots > 0.0f));
-    if (bad != 0 && lane == 0 && status && *status == 0) *status = 1 + first_index + __builtin_ctzll(bad);
-    // lower half: row x of L (zero above the diagonal); upper half: X[j][x], zero above the diagonal by
-    // construction.  One store per j for the whole wave.
-    float* dst = lower ? As + (base + x) * kPitch + base : Xs + base * kPitch + base + x;
-    const int step = lower ? 1 : kPitch;
 #pragma unroll
-    for (int j = 0; j < kSub; ++j) dst[j * step] = (lower && j > x) ? 0.0f : v[j];
+        for (int t = 0; t < 4; ++t) {
+            y[t] = -xi[kReg + t];
+#pragma unroll
+            for (int u = 0; u < t; ++u) y[t] = __builtin_fmaf(-b[t][u], y[u], y[t]);
+            y[t] *= s[t];
+        }
+        {
+            int four = lane >> 2;
+            asm volatile("" : "+v"(four));  // (compared here: held across the eight panels, the masks go to spilled registers)
+            const float mine = first_of_four ? d[0] : second_of_four ? d[1] : third_of_four ? d[2] : d[3];
+            pivots = four == kLane / 4 ? mine : pivots;
+        }
+        if (h == kHalf) {
+            // (L is not read above its diagonal; X is zero there by construction)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) Dx[(4 * m + t) * kDxPitch + x] = y[t];
+            *reinterpret_cast<floatx4*>(As + (base + x) * kPitch + base + 4 * m) = floatx4{l[0], l[1], l[2], l[3]};
+        }
+        if constexpr (m < 7) {
+            const auto q0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[0]), __float_as_uint(y[1]), false, false);
+            const auto q1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[2]), __float_as_uint(y[3]), false, false);
+            xi = __builtin_amdgcn_mfma_f32_32x32x2f32(l_pair[0], __uint_as_float(q0[kHalf]), xi, 0, 0, 0);
+            l_late = l_pair[1], y_late = __uint_as_float(q1[kHalf]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for_each_index(panel, std::make_integer_sequence<int, 8>{});
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(!(pivots > 0.0f));
+    const uint32_t which = (uint32_t)bad | (uint32_t)(bad >> 32);
+    if (which != 0 && lane == 0 && status && *status == 0) *status = 1 + first_index + __builtin_ctz(which);
 }
 
-// acc[q] += sign * A[16 x K] * op(B)[:, 16 q .. 16 q + 15], q = 0, 1: a strip of 16 rows and 32 columns.  A rows at `a`
-// (pitch pa, k contiguous); B^T rows at `b` (B_T: pitch pb, k contiguous) or B rows at `b` (k down the rows).  K a
-// multiple of 32.  Quarter g of the wave (lane / 16) takes k = 16 s + 4 g + t for the t-th MFMA of sub-step s, so that
-// an operand whose k is contiguous is one 16-byte LDS read per four MFMAs.
-template <bool B_T>
-__device__ __forceinline__ void strip_product(const float* a, int pa, const float* b, int pb, int K, float sign,
-                                              floatx4 (&acc)[2], int lane) {
-    const int x = lane & 15, g = lane >> 4;
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        floatx4 fa[2], fb[2][2];
+// acc[q] += A[16 x K] * op(B)[:, 16 q .. 16 q + 15], q = 0, 1: a strip of 16 rows and 32 columns (ONE: only its first
+// 16 columns, acc[1] takes the odd steps).  A rows at `a` (pitch pa, k contiguous); B^T rows at `b` (B_T: pitch pb, k
+// contiguous) or B rows at `b` (k down the rows).  Quarter g of the wave (lane / 16) takes k = 16 s + 4 g + t for the
+// t-th MFMA of sub-step s, so that an operand whose k is contiguous is one 16-byte LDS read per four MFMAs.
+template <bool B_T, bool ONE>
+struct StripStep {
+    static constexpr int kQ = ONE ? 1 : 2;
+    floatx4 fa[2], fb[2][kQ];
+    __device__ __forceinline__ void fetch(const float* a, int pa, const float* b, int pb, int k0, int lane) {
+        const int x = lane & 15, g = lane >> 4;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int k = k0 + 16 * s + 4 * g;
             fa[s] = *reinterpret_cast<const floatx4*>(a + x * pa + k);
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
+            for (int q = 0; q < kQ; ++q) {
                 if (B_T) {
                     fb[s][q] = *reinterpret_cast<const floatx4*>(b + (16 * q + x) * pb + k);
                 } else {
@@ -208,14 +217,42 @@ __device__ __forceinline__ void strip_product(const float* a, int pa, const floa
                 }
             }
         }
+    }
+    __device__ __forceinline__ void multiply(floatx4 (&acc)[2]) const {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(sign * fa[s][t], fb[s][q][t], acc[q], 0, 0, 0);
+                for (int q = 0; q < kQ; ++q) {
+                    floatx4& c = acc[ONE ? t & 1 : q];
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[s][t], fb[s][q][t], c, 0, 0, 0);
+                }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
+
+// K a multiple of 32
+template <bool B_T, bool ONE = false>
+__device__ __forceinline__ void strip_product(const float* a, int pa, const float* b, int pb, int K, floatx4 (&acc)[2],
+                                              int lane) {
+    for (int k0 = 0; k0 < K; k0 += 32) {
+        StripStep<B_T, ONE> step;
+        step.fetch(a, pa, b, pb, k0, lane);
+        step.multiply(acc);
+    }
+}
+
+// K = 32 STEPS, B^T rows: the reads of a step on their way under the MFMAs of the one before
+template <int STEPS, bool ONE = false>
+__device__ __forceinline__ void strip_product_fixed(const float* a, const float* b, floatx4 (&acc)[2], int lane) {
+    StripStep<true, ONE> step[2];
+    step[0].fetch(a, kPitch, b, kPitch, 0, lane);
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+        if (i + 1 < STEPS) step[(i + 1) & 1].fetch(a, kPitch, b, kPitch, 32 * (i + 1), lane);
+        step[i & 1].multiply(acc);
     }
 }
 
@@ -227,11 +264,14 @@ __device__ __forceinline__ void strip_load(const float* c, int pc, floatx4 (&acc
         for (int r = 0; r < 4; ++r) acc[q][r] = c[(4 * (lane >> 4) + r) * pc + 16 * q + (lane & 15)];
 }
 
+// (SIGN: -1 where the sum was kept with its sign turned)
+template <int SIGN = 1>
 __device__ __forceinline__ void strip_store(float* c, int pc, const floatx4 (&acc)[2], int lane) {
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) c[(4 * (lane >> 4) + r) * pc + 16 * q + (lane & 15)] = acc[q][r];
+        for (int r = 0; r < 4; ++r)
+            c[(4 * (lane >> 4) + r) * pc + 16 * q + (lane & 15)] = SIGN < 0 ? -acc[q][r] : acc[q][r];
 }
 
 __device__ __forceinline__ void strip_zero(floatx4 (&acc)[2]) {
@@ -239,17 +279,36 @@ __device__ __forceinline__ void strip_zero(floatx4 (&acc)[2]) {
     acc[1] = acc[0];
 }
 
-// A[ti][tj] -= P[ti] P[tj]^T, rows 16 half .. 16 half + 15 of the sub-block; P has K columns from `p` on
-__device__ __forceinline__ void trailing_strip(float* As, int ti, int tj, int half, const float* p, int K, int lane) {
-    const int row = kSub * ti + 16 * half;
-    float* c = As + row * kPitch + kSub * tj;
-    floatx4 acc[2];
-    strip_load(c, kPitch, acc, lane);
-    strip_product<true>(p + row * kPitch, kPitch, p + kSub * tj * kPitch, kPitch, K, -1.0f, acc, lane);
-    strip_store(c, kPitch, acc, lane);
+// Rows 16 half .. 16 half + 15 of A[ti][tj] -= P[ti] P[tj]^T (P: the panel block, 128 columns, or null) and
+// -= L[ti][c] L[tj][c]^T, columns c = c0 .. c0 + K - 1 of the factor (K may be 0).  Of a sub-block on the diagonal the upper
+// rows need their first 16 columns only.
+template <bool ONE>
+__device__ __forceinline__ void update_strip_part(float* As, int ti, int tj, int row, const float* P, int c0, int K, int lane) {
+    float* c = As + row * kPitch + kSub * tj + 4 * (lane >> 4) * kPitch + (lane & 15);
+    floatx4 acc[2], old[2];  // (the sum with its sign turned, from zero: A is read under the products)
+    strip_zero(acc);
+#pragma unroll
+    for (int q = 0; q < (ONE ? 1 : 2); ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[q][r] = c[r * kPitch + 16 * q];
+    if (P) strip_product_fixed<NB / 32, ONE>(P + row * kPitch, P + kSub * tj * kPitch, acc, lane);
+    strip_product<true, ONE>(As + row * kPitch + c0, kPitch, As + kSub * tj * kPitch + c0, kPitch, K, acc, lane);
+    if constexpr (ONE) acc[0] += acc[1];
+#pragma unroll
+    for (int q = 0; q < (ONE ? 1 : 2); ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[r * kPitch + 16 * q] = old[q][r] - acc[q][r];
 }
 
-constexpr int kDiagLdsFloats = 2 * NB * kPitch + kSub * kTPitch;  // 147 968 bytes
+__device__ __forceinline__ void update_strip(float* As, int ti, int tj, int half, const float* P, int c0, int K, int lane) {
+    const int row = kSub * ti + 16 * half;
+    if (ti == tj && half == 0)
+        update_strip_part<true>(As, ti, tj, row, P, c0, K, lane);
+    else
+        update_strip_part<false>(As, ti, tj, row, P, c0, K, lane);
+}
+
+constexpr int kDiagLdsFloats = 2 * NB * kPitch + kSub * kTPitch + kSub * kDxPitch;  // 152 576 bytes
 
 // `panel`, when not null, is the 128 x 128 block of the factor to the left of this diagonal block
 // (row pitch ldp) whose contribution has not been taken off W yet: the block that is factored is
@@ -259,8 +318,9 @@ __device__ __forceinline__ void diag_block(const float* __restrict__ W, uint64_t
                                            int32_t* __restrict__ status, const float* __restrict__ panel,
                                            uint64_t ldp, float* __restrict__ lds) {
     float* As = lds;                        // the block, overwritten by its factor
-    float* Xs = As + NB * kPitch;           // the inverse of the factor; before that, the panel block
+    float* Xs = As + NB * kPitch;           // the panel block; row by row of sub-blocks, the inverse of the factor
     float* Ts = Xs + NB * kPitch;           // T_j of the sub-block row at work
+    float* Dx = Ts + kSub * kTPitch;        // the inverse of the sub-block at work
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;  // wave index in a scalar register
     constexpr int kBlocks = NB / kSub, kRows = NB * (NB / 4) / kDiagThreads;
@@ -282,56 +342,80 @@ __device__ __forceinline__ void diag_block(const float* __restrict__ W, uint64_t
         for (int i = 0; i < kRows; ++i) *reinterpret_cast<floatx4*>(As + (r0 + 16 * i) * kPitch + c) = v[i];
     }
     __syncthreads();
-    if (panel) {  // the ten sub-blocks on or under the diagonal (what is above it is never read)
-        for (int u = wave; u < kBlocks * (kBlocks + 1); u += kDiagWaves) {
-            const int t = u >> 1;
-            const int ti = t < 1 ? 0 : (t < 3 ? 1 : (t < 6 ? 2 : 3)), tj = t - ti * (ti + 1) / 2;
-            trailing_strip(As, ti, tj, u & 1, Xs, NB, lane);
+    if (panel) {
+        // the panel's share of (0, 0) and (1, 1): waves 0-3 a strip each, waves 4-7 the second half of its columns
+        const int sub = (wave >> 1) & 1, half = wave & 1, row = kSub * sub + 16 * half, k0 = wave < 4 ? 0 : NB / 2;
+        float* c_strip = As + row * kPitch + kSub * sub;
+        float* other = Ts + (wave & 3) * 512 + 4 * lane;
+        floatx4 acc[2];
+        strip_zero(acc);
+        strip_product_fixed<NB / 64>(Xs + row * kPitch + k0, Xs + kSub * sub * kPitch + k0, acc, lane);
+        if (wave >= 4) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) *reinterpret_cast<floatx4*>(other + 256 * q) = acc[q];
+        }
+        __syncthreads();
+        if (wave < 4) {
+            floatx4 old[2];
+            strip_load(c_strip, kPitch, old, lane);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) acc[q] = old[q] - (acc[q] + *reinterpret_cast<const floatx4*>(other + 256 * q));
+            strip_store(c_strip, kPitch, acc, lane);
         }
         __syncthreads();
     }
 
     for (int p = 0; p < kBlocks; ++p) {
-        const int base = kSub * p;
+        const int base = kSub * p, below = kBlocks - 1 - p;  // sub-blocks under the diagonal one
         if (wave == 0) {
-            factor_sub_block(As, Xs, base, lane, block_index * NB + base, status);
-        } else if (p > 0 && wave != 4) {  // (wave 4 shares wave 0's SIMD)
-            // trailing sub-blocks (ti, tj), p <= tj <= ti, except (p, p), by column p - 1; then T_j
-            const int q = kBlocks - p, trailing = q * (q + 1) - 2;
-            for (int u = wave < 4 ? wave - 1 : wave - 2; u < trailing + 2 * p; u += kDiagWaves - 2) {
-                if (u < trailing) {
-                    const int t = 1 + (u >> 1), ti = t < 3 ? 1 : 2, tj = t - ti * (ti + 1) / 2;
-                    trailing_strip(As, p + ti, p + tj, u & 1, As + base - kSub, kSub, lane);
+            factor_sub_block(As, Dx, base, lane, block_index * NB + base, status);
+        } else if (wave != 4) {  // (wave 4 shares wave 0's SIMD)
+            // Everything that the sub-blocks below (p, p), and (p + 1, p + 1), lack up to column p - 1; then T_j.  Dealt so
+            // that the three SIMDs get equal shares (waves 1 and 5, 2 and 6, 3 and 7): p = 1, eight units, the short ones
+            // to wave 7; p = 2, eight units, to waves 6 and 7 the four T.
+            const int strips = p == 0 ? (panel ? 2 * below : 0) : (below ? 2 * below + 2 : 0), units = strips + 2 * p;
+            const int v = wave < 4 ? wave - 1 : wave - 2, several = p == 1 ? 5 : p == 2 ? 4 : 0;
+            const int end = v < several ? v + 1 : units;
+            for (int u = v; u < end; u += kDiagWaves - 2 - several) {
+                const int i = u >> 1;
+                if (u < strips) {  // of (p + 1, p + 1) the longer strip first
+                    update_strip(As, i < below ? p + 1 + i : p + 1, i < below ? p : p + 1, i < below ? u & 1 : ~u & 1,
+                                 panel ? Xs : nullptr, 0, base, lane);
                 } else {
-                    const int j = (u - trailing) >> 1, half = u & 1;
+                    const int j = i - (strips >> 1), half = u & 1;
                     floatx4 acc[2];
                     strip_zero(acc);
                     strip_product<false>(As + (base + 16 * half) * kPitch + kSub * j, kPitch,
-                                         Xs + kSub * j * kPitch + kSub * j, kPitch, base - kSub * j, 1.0f, acc, lane);
+                                         Xs + kSub * j * kPitch + kSub * j, kPitch, base - kSub * j, acc, lane);
                     strip_store(Ts + 16 * half * kTPitch + kSub * j, kTPitch, acc, lane);
                 }
             }
         }
         __syncthreads();
-        const int below = kBlocks - 1 - p;  // sub-blocks under the diagonal one
-        for (int u = wave; u < 2 * (below + p); u += kDiagWaves) {
-            const int half = u & 1;
+        {
+            // six strips for waves 0-5, X_pp into its place by waves 6 and 7 (row p of the panel block is done with)
+            const int half = wave & 1;
             floatx4 acc[2];
             strip_zero(acc);
-            if (u < 2 * below) {  // L[t][p], in place: a wave has read its rows before it writes them
-                float* rows = As + (base + kSub * (1 + (u >> 1)) + 16 * half) * kPitch + base;
-                strip_product<true>(rows, kPitch, Xs + base * kPitch + base, kPitch, kSub, 1.0f, acc, lane);
+            if (wave < 2 * below) {  // L[t][p], in place: a wave has read its rows before it writes them
+                float* rows = As + (base + kSub * (1 + (wave >> 1)) + 16 * half) * kPitch + base;
+                strip_product<true>(rows, kPitch, Dx, kDxPitch, kSub, acc, lane);
                 strip_store(rows, kPitch, acc, lane);
-            } else {  // X[p][j]
-                const int j = (u - 2 * below) >> 1;
-                float* rows = Xs + (base + 16 * half) * kPitch;
-                strip_product<false>(rows + base, kPitch, Ts + kSub * j, kTPitch, kSub, -1.0f, acc, lane);
-                strip_store(rows + kSub * j, kPitch, acc, lane);
+            } else if (wave < 2 * (kBlocks - 1)) {  // X[p][j]
+                const int j = (wave >> 1) - below;
+                strip_product<false>(Dx + 16 * half * kDxPitch, kDxPitch, Ts + kSub * j, kTPitch, kSub, acc, lane);
+                strip_store<-1>(Xs + (base + 16 * half) * kPitch + kSub * j, kPitch, acc, lane);
+            } else {
+                const int row = 16 * half + (lane >> 2), col = 8 * (lane & 3);
+#pragma unroll
+                for (int e = 0; e < 8; e += 4)
+                    *reinterpret_cast<floatx4*>(Xs + (base + row) * kPitch + base + col + e) =
+                        *reinterpret_cast<const floatx4*>(Dx + row * kDxPitch + col + e);
             }
         }
         __syncthreads();
         if (below == 0) break;
-        if (wave < 2) trailing_strip(As, p + 1, p + 1, wave, As + base, kSub, lane);
+        if (wave < 2) update_strip(As, p + 1, p + 1, wave, nullptr, base, kSub, lane);
         __syncthreads();
     }
 
