@@ -127,6 +127,18 @@ def test_gemm_argument_validation_needs_no_device():
     assert lib.trakhip_gemm_nt(p, 8, p, 8, p, 4, 4, 4, 16, 1.0, 0.0, None, None) == -2   # lda < K
     assert lib.trakhip_gemm_nt(None, 16, p, 16, p, 4, 4, 4, 16, 1.0, 0.0, None, None) == -5
     assert lib.trakhip_gemm_nt(p, 16, p, 16, p, 4, 0, 4, 16, 1.0, 0.0, None, None) == 0  # empty
+    # the product on smaller tiles: k in rounds of 256, rows 16-byte aligned, pitches below 2^23
+    small = lib.trakhip_gemm_nt_in_place
+    assert small(p, 264, p, 264, p, 4, 4, 4, 264, 1.0, 0.0, None, None) == -2
+    assert small(p, 252, p, 256, p, 4, 4, 4, 256, 1.0, 0.0, None, None) == -2
+    assert small(p, 256, p, 1 << 23, p, 4, 4, 4, 256, 1.0, 0.0, None, None) == -2
+    assert small(p, 257, p, 256, p, 4, 4, 4, 256, 1.0, 0.0, None, None) == -7
+    assert small(ctypes.c_void_p(4100), 256, p, 256, p, 4, 4, 4, 256, 1.0, 0.0, None, None) == -7
+    assert small(None, 256, p, 256, p, 4, 4, 4, 256, 1.0, 0.0, None, None) == -5
+    assert small(p, 256, p, 256, p, 4, 4, 0, 256, 1.0, 0.0, None, None) == 0
+    pays = lib.trakhip_gemm_nt_in_place_pays
+    assert pays(2000, 512, 512) == 1 and pays(50_000, 100, 2048) == 1 and pays(50_000, 10_000, 4096) == 0
+    assert pays(2000, 512, 500) == 0 and pays(0, 5, 512) == 0 and pays(1 << 40, 1 << 40, 512) == 0
     assert lib.trakhip_gemm_tn(p, 2, p, 8, p, 8, 4, 4, 16, 1.0, 0.0, None) == -2          # lda < M
     assert lib.trakhip_spd_inverse(p, 2, 0.0, p, 4, 4, 0, None, None, p, 1 << 30, None) == -2
     assert lib.trakhip_spd_inverse(p, 4, 0.0, p, 4, 4, 0, None, None, p, 16, None) == -6

@@ -72,6 +72,50 @@ def test_gemm_nt_short_contraction(gpu, M, N, K):
     assert rel_max(wide[:, :N].cpu().numpy(), want) < gemm_tol(K) and bool((wide[:, N:] == 7.0).all())
 
 
+# tiles of 32 x 32 (four waves share the k range) and, from (1100, 1090, 256) on, of 64 x 64
+@pytest.mark.parametrize("M,N,K", [(1, 1, 256), (31, 33, 256), (32, 32, 512), (65, 100, 768), (2000, 1, 512), (300, 64, 4096),
+                                   (1100, 1090, 256), (1984, 1025, 1024), (4159, 640, 512)])
+def test_products_of_few_tiles_read_their_operands_in_place(gpu, M, N, K):
+    from trak_amd.utils import in_place_pays
+
+    gen = torch.Generator(device="cpu").manual_seed(M + N + K)
+    wide_a, wide_b = torch.randn(M, K + 20, generator=gen), torch.randn(N, K + 4, generator=gen)
+    a, b = wide_a.to(gpu)[:, 8:8 + K], wide_b.to(gpu)[:, :K]         # pitches above K, rows 16-byte aligned
+    rs, c0 = torch.rand(M, generator=gen), torch.randn(M, N, generator=gen)
+    assert in_place_pays(a, b)
+    a64, b64 = a.cpu().double().numpy(), b.cpu().double().numpy()
+    want = a64 @ b64.T
+    # at most K / 2 + 8 roundings of partial sums between an entry's first product and its last sum
+    bound = (K / 2 + 8) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64).T)
+    out = torch.full((M, N + 3), 7.0, device=gpu)
+    got = matmul_nt(a, b, out=out[:, :N]).cpu().double().numpy()
+    assert (np.abs(got - want) <= bound).all()
+    assert (out[:, N:] == 7.0).all()                                  # nothing beside the result is written
+    got = matmul_nt(a, b, out=c0.to(gpu), alpha=0.5, beta=-2.0, row_scale=rs.to(gpu)).cpu().double().numpy()
+    rows = rs.double().numpy()[:, None]
+    want = (0.5 * want - 2.0 * c0.double().numpy()) * rows
+    assert (np.abs(got - want) <= rows * (0.5 * bound + 2.0 ** -21 * (np.abs(c0.numpy()) + np.abs(a64 @ b64.T)))).all()
+
+
+def test_products_that_are_split_and_products_that_are_not(gpu):
+    from trak_amd.utils import in_place_pays
+
+    a, b = torch.randn(2000, 516, device=gpu), torch.randn(100, 516, device=gpu)
+    assert in_place_pays(a[:, :512], b[:, :512]) and not in_place_pays(a[:, :500], b[:, :500])      # k in rounds of 256
+    assert not in_place_pays(a[:, 1:513], b[:, :512])                                                # rows not aligned
+    assert not in_place_pays(a[:512].T, b[:, :512]) and not in_place_pays(a[:, :512].half(), b[:, :512].half())
+    assert not in_place_pays(torch.empty(8192, 4096, device=gpu), torch.empty(4096, 4096, device=gpu))   # the split pays
+    assert not in_place_pays(a[:0, :512], b[:, :512])
+    # whatever the route: strides, offsets and types give the same product
+    a64, b64 = a.cpu().double().numpy(), b.cpu().double().numpy()
+    for x, y, x64, y64 in ((a[:, 1:513], b[:, 2:514], a64[:, 1:513], b64[:, 2:514]),
+                           (a[::2, 4:516], b[::3, :512], a64[::2, 4:516], b64[::3, :512]),
+                           (a[:512].T, b[:, :512], a64[:512].T, b64[:, :512]),
+                           (a[:, :512].half(), b[:, :512], a[:, :512].half().cpu().double().numpy(), b64[:, :512])):
+        got = matmul_nt(x, y).cpu().numpy()
+        assert rel_max(got, x64 @ y64.T) < 2e-6
+
+
 @pytest.mark.parametrize("M,N,K", [(128, 128, 16), (96, 200, 1000), (33, 17, 5), (512, 512, 2050)])
 def test_gemm_tn(gpu, M, N, K):
     gen = torch.Generator(device="cpu").manual_seed(M + N + K)

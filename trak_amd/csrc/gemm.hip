@@ -256,6 +256,185 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_nt_short_k_kernel(const floa
     short_k::tile<ROWS>(A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, tile_m, tile_n, lds);
 }
 
+// NT products of few tiles or few columns: C[M, N] = alpha * A[M, K] * B[N, K]^T + beta * C (row i *= row_scale[i]).
+//
+// WM x WN x WK = 4 waves; the tile has 32 WM x 32 WN entries, a stage 32 WK values of k, of which wave (.., wk) takes 32,
+// and DEPTH stages are in flight in registers (the general kernel above goes to memory once per 16 values of k, and with a
+// tile or less per CU nothing hides that).  WK > 1 shares one tile's k range out over the waves (their sums are
+// added up in LDS at the end, in order), so a tile's chain of MFMAs is a quarter as long and a product of
+// [2000 x 512] by [100 x 512] has 252 workgroups where 128 x 128 tiles give 16.  Every wave keeps two sums, of the
+// even and the odd groups of eight k.  16-byte aligned rows, K a multiple of 32 WK DEPTH; rows past M or N are read from the last
+// row and not stored.  Measured (general kernel; three-plane product, splits included; now; call to call):
+// [2000 x 512][100 x 512]^T 55, 79, 14 us; [2000 x 512][512 x 512]^T 55, 72, 17 us; [8000 x 4096][40 x 4096]^T 348, 490, 54 us;
+// [50 000 x 2048][100 x 2048]^T 305, 441, 253 us; [50 000 x 4096][20 x 4096]^T 574, 904, 184 us (4.5 TB/s of A).  Error against
+// 64 bits 0.4 (32 x 32) and 0.8 (64 x 64) of the three-plane product's.
+constexpr int kSmallPitchPad = 4;
+
+template <int WM, int WN, int WK, int DEPTH>
+__global__ __launch_bounds__(kThreads, 2) void gemm_nt_small_kernel(const float* __restrict__ A, uint64_t lda,
+                                                                    const float* __restrict__ B, uint64_t ldb,
+                                                                    float* __restrict__ C, uint64_t ldc, uint64_t M,
+                                                                    uint64_t N, uint64_t K, float alpha, float beta,
+                                                                    const float* __restrict__ row_scale, uint32_t tiles_n,
+                                                                    uint32_t tiles) {
+    static_assert(WM * WN * WK == 4 && DEPTH % 2 == 0, "four waves, two LDS buffers");
+    constexpr int TM = 32 * WM, TN = 32 * WN, KS = 32 * WK;   // a stage: KS values of k
+    constexpr int kPitch = KS + kSmallPitchPad;                // 16-byte reads of sixteen rows: conflict free
+    constexpr int kPerRow = KS / 4;                            // 16-byte pieces of a row
+    constexpr int kA = TM * kPerRow / kThreads, kB = TN * kPerRow / kThreads;
+    constexpr int kFloats = (TM + TN) * kPitch;
+    static_assert(2 * kFloats >= 4 * 16 * 64 || WK == 1, "the sums of four waves fit into the buffers");
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    __shared__ __attribute__((aligned(16))) float lds[2][kFloats];
+
+    // the column tiles of a row of tiles go to one XCD, one after another: its rows of A come from memory once
+    const uint32_t xcd = blockIdx.x & 7u, lo = (uint32_t)((uint64_t)xcd * tiles / 8u), hi = (uint32_t)((xcd + 1ull) * tiles / 8u);
+    const uint32_t tile = lo + (blockIdx.x >> 3);
+    if (tile >= hi) return;
+    const uint64_t m0 = (uint64_t)(tile / tiles_n) * TM, n0 = (uint64_t)(tile % tiles_n) * TN;
+
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wk = wave % WK, wn = wave / WK % WN, wm = wave / WK / WN;
+    const int x = lane & 31, h = lane >> 5;
+
+    // this thread's pieces: byte offsets from the tile's first row (pitches below 2^23 elements)
+    const char* a_tile = reinterpret_cast<const char*>(A + m0 * lda);
+    const char* b_tile = reinterpret_cast<const char*>(B + n0 * ldb);
+    uint32_t at[kA], bt[kB];
+#pragma unroll
+    for (int i = 0; i < kA; ++i) {
+        const uint32_t id = tid + kThreads * i, row = id / kPerRow;
+        const uint64_t last = M - 1 - m0;
+        at[i] = (uint32_t)((row < last ? row : last) * lda + 4 * (id % kPerRow)) * 4u;
+    }
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+        const uint32_t id = tid + kThreads * i, row = id / kPerRow;
+        const uint64_t last = N - 1 - n0;
+        bt[i] = (uint32_t)((row < last ? row : last) * ldb + 4 * (id % kPerRow)) * 4u;
+    }
+    floatx4 ra[DEPTH][kA], rb[DEPTH][kB];
+    auto load = [&](int u, uint64_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kA; ++i) ra[u][i] = *reinterpret_cast<const floatx4*>(a_tile + k0 * 4 + at[i]);
+#pragma unroll
+        for (int i = 0; i < kB; ++i) rb[u][i] = *reinterpret_cast<const floatx4*>(b_tile + k0 * 4 + bt[i]);
+    };
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) load(u, KS * u);
+
+    floatx16 acc[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
+    for (uint64_t k0 = 0; k0 < K; k0 += KS * DEPTH) {
+        const bool more = k0 + KS * DEPTH < K;
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u) {
+            // a buffer is written again two stages later, behind the barrier that follows its reads
+            float* buf = lds[u & 1];
+#pragma unroll
+            for (int i = 0; i < kA; ++i) {
+                const int id = tid + kThreads * i;
+                *reinterpret_cast<floatx4*>(buf + (id / kPerRow) * kPitch + 4 * (id % kPerRow)) = ra[u][i];
+            }
+#pragma unroll
+            for (int i = 0; i < kB; ++i) {
+                const int id = tid + kThreads * i;
+                *reinterpret_cast<floatx4*>(buf + (TM + id / kPerRow) * kPitch + 4 * (id % kPerRow)) = rb[u][i];
+            }
+            if (more) load(u, k0 + KS * (DEPTH + u));
+            __syncthreads();
+            floatx4 fa[4], fb[4];
+            const float* as = buf + (32 * wm + x) * kPitch + 32 * wk + 4 * h;
+            const float* bs = buf + (TM + 32 * wn + x) * kPitch + 32 * wk + 4 * h;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                fa[q] = *reinterpret_cast<const floatx4*>(as + 8 * q);
+                fb[q] = *reinterpret_cast<const floatx4*>(bs + 8 * q);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // all reads of the stage in flight before its first MFMA waits
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][t], fb[q][t], acc[q & 1], 0, 0, 0);
+        }
+    }
+    floatx16 sum = acc[0] + acc[1];
+    // WK waves hold a share of the same entries: registers [first, first + kMine) of the sum are this wave's to store
+    constexpr int kMine = 16 / WK;
+    const int first = kMine * wk;
+    float out[kMine];
+    if constexpr (WK > 1) {
+        float* shares = &lds[0][0];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) shares[(wave * 16 + r) * 64 + lane] = sum[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kMine; ++r) {
+            out[r] = 0.0f;
+#pragma unroll
+            for (int w = 0; w < WK; ++w) out[r] += shares[((wave - wk + w) * 16 + first + r) * 64 + lane];
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) out[r] = sum[r];
+    }
+    const uint64_t col = n0 + 32 * wn + x;
+    if (col >= N) return;
+    const uint64_t row0 = m0 + 32 * wm + 4 * h;
+    float prev[kMine];
+#pragma unroll
+    for (int r = 0; r < kMine; ++r) {
+        const uint64_t row = row0 + 8 * ((first + r) >> 2) + ((first + r) & 3);
+        prev[r] = beta != 0.0f && row < M ? C[row * ldc + col] : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < kMine; ++r) {
+        const uint64_t row = row0 + 8 * ((first + r) >> 2) + ((first + r) & 3);
+        if (row >= M) continue;
+        float v = alpha * out[r];
+        if (beta != 0.0f) v += beta * prev[r];
+        C[row * ldc + col] = v * (row_scale ? row_scale[row] : 1.0f);
+    }
+}
+
+// What an NT product takes, in microseconds, fitted to 200 products of M = 1000 .. 50 000, N = 1 .. 2048 and K = 512 .. 4096:
+// rounds of tiles over the 256 CUs times the time of one, which goes with K.  A tile of 32 x 32 entries shared by four
+// waves takes 6.0 ns per value of k whether one or two of them share a CU (bound by what 256 CUs read from L2: 10.7 TB/s);
+// a 64 x 64 tile 17.6 ns where two or more share a CU, 19.8 alone (120 TFLOP/s).  (The general kernel: 128 x 128 tiles 83 ns,
+// 128 x 256 tiles, from 256 of them on, 134 ns.)
+double tiles_of(uint64_t M, uint64_t N, uint64_t rows, uint64_t cols) {
+    return (double)((M + rows - 1) / rows) * (double)((N + cols - 1) / cols);
+}
+double rounds_of(double tiles) { return tiles <= 256.0 ? 1.0 : tiles / 256.0; }
+double one_tile_us(uint64_t M, uint64_t N, uint64_t K) {
+    return 5.0 + 6.0e-3 * (double)K * rounds_of(tiles_of(M, N, 32, 32));
+}
+double four_tiles_us(uint64_t M, uint64_t N, uint64_t K) {
+    const double rounds = tiles_of(M, N, 64, 64) / 256.0;
+    return 5.0 + 17.6e-3 * (double)K * (rounds < 1.12 ? 1.12 : rounds);
+}
+// Both operands split into planes (10 bytes of traffic per value) and their product (gemm_split.hip): 256 x 256 tiles,
+// per 16 values of k 2.1 us for a round on all CUs and 1.7 us for one that leaves some idle (the clock is higher then).
+double split_us(uint64_t M, uint64_t N, uint64_t K) {
+    const double tiles = tiles_of(M, N, 256, 256);
+    const double full = (double)(uint64_t)(tiles / 256.0);
+    return 25.0 + 2.0e-6 * ((double)M + (double)N) * (double)K +
+           (double)K / 16.0 * (2.1 * full + (tiles > 256.0 * full ? 1.7 : 0.0));
+}
+
+template <int WM, int WN, int WK, int DEPTH>
+int launch_small(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M, uint64_t N,
+                 uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s) {
+    const uint64_t tn = (N + 32 * WN - 1) / (32 * WN), tiles = (M + 32 * WM - 1) / (32 * WM) * tn;
+    if (tiles > 0x7FFFFFF0ull) return TRAKHIP_ERR_SHAPE;
+    hipLaunchKernelGGL((gemm_nt_small_kernel<WM, WN, WK, DEPTH>), dim3((uint32_t)((tiles + 7) / 8 * 8)), dim3(kThreads), 0, s,
+                       A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, row_scale, (uint32_t)tn, (uint32_t)tiles);
+    return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+}
+
 template <bool AK, bool BK, int WN>
 int launch_tiles(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
                  uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, bool aligned,
@@ -321,6 +500,26 @@ int gemm_nt(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C
         }
     }
     return launch<false, false>(A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, row_scale, flags, s);
+}
+
+bool gemm_nt_in_place_pays(uint64_t M, uint64_t N, uint64_t K) {
+    if (M == 0 || N == 0 || K == 0 || K % 256) return false;
+    const double one = one_tile_us(M, N, K), four = four_tiles_us(M, N, K);
+    return (one < four ? one : four) < split_us(M, N, K);
+}
+
+int gemm_nt_in_place(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
+                     uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s) {
+    if (M == 0 || N == 0) return TRAKHIP_OK;
+    // (a lane's byte offset inside the rows of a tile is kept in 32 bits)
+    if (K == 0 || K % 256 || lda < K || ldb < K || ldc < N || lda >= (1ull << 23) || ldb >= (1ull << 23)) return TRAKHIP_ERR_SHAPE;
+    if (!A || !B || !C) return TRAKHIP_ERR_NULL;
+    if ((reinterpret_cast<uintptr_t>(A) % 16) || (reinterpret_cast<uintptr_t>(B) % 16) || (lda % 4) || (ldb % 4) ||
+        (reinterpret_cast<uintptr_t>(C) % 4) || (reinterpret_cast<uintptr_t>(row_scale) % 4))
+        return TRAKHIP_ERR_ALIGN;
+    if (one_tile_us(M, N, K) < four_tiles_us(M, N, K))
+        return launch_small<1, 1, 4, 2>(A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, row_scale, s);
+    return launch_small<2, 2, 1, 4>(A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, row_scale, s);
 }
 
 int gemm_tn(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,

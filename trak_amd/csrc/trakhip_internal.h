@@ -52,6 +52,11 @@ int gemm_nn_batched(const float* A, uint64_t lda, const float* B, uint64_t ldb, 
 int gemm_nt(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
             uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s,
             uint32_t flags = 0);
+// the same product, 16-byte aligned rows and K % 256 == 0, on smaller tiles; whether it is expected to take less time than
+// splitting both operands for gemm_nt_split
+int gemm_nt_in_place(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
+                     uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s);
+bool gemm_nt_in_place_pays(uint64_t M, uint64_t N, uint64_t K);
 int gemm_tn(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
             uint64_t N, uint64_t K, float alpha, float beta, hipStream_t s, uint32_t flags = 0);
 int gemm_nn(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,

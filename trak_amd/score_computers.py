@@ -18,6 +18,7 @@ from .utils import (
     gemm_tn,
     get_matrix_mult_blockwise,
     gram_split,
+    in_place_pays,
     matmul_nt,
     nt16_ok,
     output_fits_on_device,
@@ -160,6 +161,8 @@ class BasicScoreComputer(AbstractScoreComputer):
                 block = block.to(self._dev)
                 if half and nt16_ok(block, xtx_inv):
                     gemm_nt16(block, xtx_inv, out=result[start:end])
+                elif self.gemm == "split" and not half and in_place_pays(block, xtx_inv):
+                    gemm_nt(block, xtx_inv, out=result[start:end], in_place=True)
                 else:
                     if inv_split is None:
                         inv_split = self._split(xtx_inv if half else xtx_inv.float())

@@ -74,9 +74,10 @@ def _ld(t):
     return t.stride(0) if t.shape[0] > 1 else max(t.shape[1], 1)
 
 
-def gemm_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
+def gemm_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None, in_place=False):
     """out[M, N] = alpha * a[M, K] @ b[N, K].T + beta * out (fp32 on the GPU), rows optionally
-    scaled by row_scale[M]."""
+    scaled by row_scale[M].  in_place: on the smaller tiles for few rows or columns, operands as
+    `in_place_pays` asks for them."""
     a = _as_f32_rows(a, "a")
     b = _as_f32_rows(b, "b")
     if not a.is_cuda or b.device != a.device:
@@ -98,7 +99,7 @@ def gemm_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
     lib = _lib.load()
     with torch.cuda.device(a.device):
         stream = torch.cuda.current_stream(a.device).cuda_stream
-        code = lib.trakhip_gemm_nt(
+        code = (lib.trakhip_gemm_nt_in_place if in_place else lib.trakhip_gemm_nt)(
             ctypes.c_void_p(a.data_ptr()),
             _ld(a),
             ctypes.c_void_p(b.data_ptr()),
@@ -115,6 +116,22 @@ def gemm_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
         )
     _lib.check(code)
     return out
+
+
+def in_place_pays(a, b):
+    """Whether a @ b.T of two matrices that are multiplied from fp32 values is faster with `gemm_nt(in_place=True)`,
+    which reads them where they are (16-byte aligned rows, K % 256 == 0), than from splits: products of few rows or columns, for which the passes
+    that split the operands and 256 x 256 tiles cost more than the slower instruction."""
+    if a.dtype != torch.float32 or b.dtype != torch.float32 or not a.is_cuda or a.device != b.device:
+        return False
+    if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[1] or a.numel() == 0 or b.numel() == 0:
+        return False
+    for t in (a, b):
+        if t.stride(1) != 1 or t.data_ptr() % 16 or (t.shape[0] > 1 and (t.stride(0) % 4 or t.stride(0) < t.shape[1])):
+            return False
+        if max(t.stride(0), t.shape[1]) >= 1 << 23:  # a lane's offset inside a tile is kept in 32 bits
+            return False
+    return bool(_lib.load().trakhip_gemm_nt_in_place_pays(a.shape[0], b.shape[0], a.shape[1]))
 
 
 def gemm_tn(a, b, out=None, alpha=1.0, beta=0.0):
@@ -315,12 +332,17 @@ def gemm_nt16(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
 def matmul_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None, two_planes=False):
     """alpha * a @ b.T + beta * out with fp32 accuracy on the 16-bit matrix cores, whatever the operand
     types: two fp16 or two bf16 matrices that qualify are multiplied where they are (`gemm_nt16`),
-    other 16-bit pairs as single planes, anything else from fp32 splits (`gemm_nt_split`; the exact
-    three-plane split, or the two-plane one of `split2_rows` when `two_planes` is set)."""
+    other 16-bit pairs as single planes, anything else from fp32 values: where they are, on the fp32 instruction,
+    when that is faster (`in_place_pays`), else from splits (`gemm_nt_split`; the exact three-plane split, or the
+    two-plane one of `split2_rows` when `two_planes` is set)."""
     if nt16_ok(a, b):
         return gemm_nt16(a, b, out=out, alpha=alpha, beta=beta, row_scale=row_scale)
-    if two_planes and not (a.dtype == b.dtype and a.dtype in (torch.float16, torch.bfloat16)):
-        return gemm_nt_split(split2_rows(a), split2_rows(b), out=out, alpha=alpha, beta=beta, row_scale=row_scale)
+    if not (a.dtype == b.dtype and a.dtype in (torch.float16, torch.bfloat16)):
+        if two_planes:
+            return gemm_nt_split(split2_rows(a), split2_rows(b), out=out, alpha=alpha, beta=beta, row_scale=row_scale)
+        a, b = a.float(), b.float()
+        if in_place_pays(a, b):
+            return gemm_nt(a, b, out=out, alpha=alpha, beta=beta, row_scale=row_scale, in_place=True)
     return gemm_nt_split(*split_pair(a, b), out=out, alpha=alpha, beta=beta, row_scale=row_scale)
 
 
