@@ -218,6 +218,15 @@ size_t trakhip_gram_split_workspace_most(uint64_t N, uint64_t K, int src_dtype, 
 int trakhip_gram_split(const void* A_planes_dev, uint64_t N, uint64_t K, int src_dtype, float* C_dev, uint64_t ldc,
                        float alpha, float beta, void* workspace_dev, size_t workspace_bytes, void* stream);
 
+/* C[N, N] = alpha * X^T X + beta * C for an fp16 or bf16 matrix X_dev[K, N] read where it is (row pitch ld): the product
+ * of trakhip_gram_split without the pass that lays X^T out as a plane, bit for bit.  N and ld multiples of 8,
+ * ld < 2^23, X_dev 16-byte aligned.  out_dtype: element type of C; a 16-bit C (beta = 0, 8-byte aligned, ldc a
+ * multiple of 4) is rounded from the sums, which then have to be in the workspace.  workspace_dev:
+ * trakhip_gram_split_workspace(_most)(N, K, dtype, 0) bytes as for trakhip_gram_split, at least one N x N
+ * matrix of fp32 for a 16-bit C, 16-byte aligned. */
+int trakhip_gram16(const void* X_dev, int dtype, uint64_t ld, uint64_t K, uint64_t N, int out_dtype, void* C_dev,
+                   uint64_t ldc, float alpha, float beta, void* workspace_dev, size_t workspace_bytes, void* stream);
+
 /* An opt-in cheaper form of the split products for fp32 operands: two fp16 planes per operand and
  * three fp16 MFMAs per k step instead of three bf16 planes and six MFMAs (about 1.75 times the speed).
  * trakhip_split2_rows multiplies every operand row by the power of two that brings its largest

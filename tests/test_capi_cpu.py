@@ -136,6 +136,18 @@ def test_gemm_argument_validation_needs_no_device():
     assert small(ctypes.c_void_p(4100), 256, p, 256, p, 4, 4, 4, 256, 1.0, 0.0, None, None) == -7
     assert small(None, 256, p, 256, p, 4, 4, 4, 256, 1.0, 0.0, None, None) == -5
     assert small(p, 256, p, 256, p, 4, 4, 0, 256, 1.0, 0.0, None, None) == 0
+    # the Gram product of 16-bit rows in place: columns and pitch in multiples of 8; a 16-bit result needs scratch
+    gram = lib.trakhip_gram16
+    assert gram(p, 2, 256, 64, 256, 2, p, 256, 1.0, 0.0, None, 0, None) == -3
+    assert gram(p, 0, 252, 64, 252, 2, p, 256, 1.0, 0.0, None, 0, None) == -2
+    assert gram(p, 0, 256, 0, 256, 2, p, 256, 1.0, 0.0, None, 0, None) == -2
+    assert gram(p, 0, 1 << 23, 64, 256, 2, p, 256, 1.0, 0.0, None, 0, None) == -2
+    assert gram(ctypes.c_void_p(4104), 0, 256, 64, 256, 2, p, 256, 1.0, 0.0, None, 0, None) == -7
+    assert gram(None, 0, 256, 64, 256, 2, p, 256, 1.0, 0.0, None, 0, None) == -5
+    assert gram(p, 0, 256, 64, 256, 0, p, 256, 1.0, 0.0, None, 0, None) == -6
+    assert gram(p, 0, 256, 64, 256, 0, p, 256, 1.0, 0.0, p, 4 * 256 * 256 - 4, None) == -6
+    assert gram(p, 0, 256, 64, 256, 0, p, 256, 1.0, 0.5, p, 4 * 256 * 256, None) == -2
+    assert gram(p, 0, 256, 64, 0, 0, p, 256, 1.0, 0.0, None, 0, None) == 0
     pays = lib.trakhip_gemm_nt_in_place_pays
     assert pays(2000, 512, 512) == 1 and pays(50_000, 100, 2048) == 1 and pays(50_000, 10_000, 4096) == 0
     assert pays(2000, 512, 500) == 0 and pays(0, 5, 512) == 0 and pays(1 << 40, 1 << 40, 512) == 0

@@ -861,6 +861,51 @@ def test_gram_uses_all_of_the_scratch_it_asks_for(gpu, fmt, N, K, which):
     assert rel_max(out.cpu().numpy(), (x.double().T @ x.double()).cpu().numpy()) < tol
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,N,pad", [(1, 8, 0), (63, 248, 8), (64, 256, 0), (65, 264, 0), (127, 520, 24), (5000, 512, 0),
+                                     (4099, 1000, 8), (6001, 2048, 0), (700, 4104, 0), (130, 4616, 0)])
+def test_gram_of_16_bit_rows_in_place(gpu, dtype, K, N, pad):
+    """The product that reads X where it is has the bits of the one through a plane of X^T: tile and step edges, row
+    pitches, with and without shares of the k range, accumulation, results rounded to 16 bits."""
+    from trak_amd.utils import gram16, gram16_ok
+
+    store = torch.full((K, N + pad), float("nan"), dtype=dtype, device=gpu)
+    x = store[:, :N]
+    x.copy_(torch.randn(K, N, generator=torch.Generator(device=gpu).manual_seed(K + N), device=gpu))
+    assert gram16_ok(x)
+    want = gram_split(split_rows(x, transposed=True))
+    got = gram16(x)
+    assert torch.equal(got, want) and torch.equal(got, got.T)
+    wide = torch.full((N, N + 3), 7.0, device=gpu)
+    gram16(x, out=wide[:, :N])
+    assert torch.equal(wide[:, :N], want) and bool((wide[:, N:] == 7.0).all())
+    acc, same = want.clone(), want.clone()
+    gram16(x, out=acc, alpha=0.5, beta=2.0)
+    gram_split(split_rows(x, transposed=True), out=same, alpha=0.5, beta=2.0)
+    assert torch.equal(acc, same)
+    assert torch.equal(gram16(x, out_dtype=dtype), want.to(dtype))
+    sc = BasicScoreComputer(dtype=dtype, device=gpu)
+    assert torch.equal(sc.get_xtx(x), want.to(dtype))
+    assert torch.equal(sc.get_xtx(x.cpu()), want.to(dtype))                     # from the host, one block
+
+
+def test_gram_of_16_bit_rows_that_cannot_be_read_in_place(gpu):
+    from trak_amd.utils import gram16, gram16_ok
+
+    x = torch.randn(300, 520, device=gpu).half()
+    inf = x.clone()
+    inf[7, 5] = float("inf")
+    assert torch.equal(torch.isfinite(gram16(inf)), torch.isfinite(gram_split(split_rows(inf, transposed=True))))
+    for bad in (x[:, :516], x[:, 4:516], x.float(), x.T, x[:0], x.cpu(), torch.empty(4, 517, device=gpu).half()[:, :512]):
+        assert not gram16_ok(bad)
+        with pytest.raises(RuntimeError):
+            gram16(bad)
+    sc = BasicScoreComputer(dtype=torch.float16, device=gpu)
+    for view in (x[:, :516], x[:, 4:516], x[::2, :512], x[:200].T):               # whatever the route, the same product
+        got, want = sc.get_xtx(view), gram_split(split_rows(view, transposed=True)).half()
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("room", [7, 6, 3, 2, 0])
 def test_gram_makes_do_with_the_memory_that_is_left(gpu, monkeypatch, room):
     """The allocator has room for all seven shares, for three, or for none (the error it raises, forced here)."""

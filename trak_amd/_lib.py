@@ -81,6 +81,8 @@ def load():
         workspace.restype = sz
     lib.trakhip_gram_split.argtypes = [vp, u64, u64, i32, vp, u64, f32, f32, vp, sz, vp]
     lib.trakhip_gram_split.restype = i32
+    lib.trakhip_gram16.argtypes = [vp, i32, u64, u64, u64, i32, vp, u64, f32, f32, vp, sz, vp]
+    lib.trakhip_gram16.restype = i32
     lib.trakhip_split2_bytes.argtypes = [u64, u64]
     lib.trakhip_split2_bytes.restype = sz
     lib.trakhip_split2_rows.argtypes = [vp, u64, u64, u64, i32, vp, sz, vp, vp]

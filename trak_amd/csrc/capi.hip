@@ -146,6 +146,12 @@ size_t trakhip_gram_split_workspace_most(uint64_t N, uint64_t K, int dtype, int 
     return trakhip::gram_split_workspace_bytes(N, K, dtype, two_planes, true);
 }
 
+int trakhip_gram16(const void* X_dev, int dtype, uint64_t ld, uint64_t K, uint64_t N, int out_dtype, void* C_dev,
+                   uint64_t ldc, float alpha, float beta, void* workspace_dev, size_t workspace_bytes, void* stream) {
+    return trakhip::gram16(X_dev, dtype, ld, K, N, out_dtype, C_dev, ldc, alpha, beta, workspace_dev, workspace_bytes,
+                           static_cast<hipStream_t>(stream));
+}
+
 int trakhip_gram_split(const void* A_planes_dev, uint64_t N, uint64_t K, int dtype, float* C_dev, uint64_t ldc,
                        float alpha, float beta, void* workspace_dev, size_t workspace_bytes, void* stream) {
     return trakhip::gram_split(A_planes_dev, N, K, dtype, C_dev, ldc, alpha, beta, workspace_dev, workspace_bytes,

@@ -36,6 +36,7 @@
 #include <stdint.h>
 
 #include "short_k_tile.h"
+#include "store_cast.h"
 #include "trakhip_internal.h"
 
 namespace {
@@ -430,6 +431,18 @@ struct StepMover {
     }
 };
 
+// Workgroup -> unit of a symmetric product (share of the k range, tile): the shares' lists of tiles one after another, of
+// which each of the eight XCDs, which are handed the workgroups round-robin, takes a contiguous eighth.  The tiles of a
+// share read the same rows of X at about the same time, so an XCD then fetches its share's rows once; with the tiles
+// dealt out over all XCDs each of them fetched every row of X ([50 000, 2048] fp16: 1.6 GB; 285 us, now 249; the
+// three-plane product of [4100, 2048] fp32 138 -> 126, of [50 000, 4096] 4.41 -> 4.33 ms).  The grid has a multiple of
+// eight workgroups; false: one without a unit.
+__device__ __forceinline__ bool gram_unit(uint32_t units, uint32_t& unit) {
+    const uint32_t xcd = blockIdx.x & 7u;
+    unit = (uint32_t)((uint64_t)xcd * units / 8u) + (blockIdx.x >> 3);
+    return unit < (uint32_t)((xcd + 1ull) * units / 8u);
+}
+
 // P planes per operand (3: split fp32, 1: a 16-bit type), F16 selects the fp16 MFMA, S sub-steps
 // per barrier.
 template <int P, bool F16, int S, bool ACCUM>
@@ -444,17 +457,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_split_kernel(
     constexpr int kBufPieces = S * kSubPieces;
     __shared__ piece lds[2][kBufPieces];
 
-    // parts > 1: the grid is `parts` copies of the tile list; copy p multiplies the p-th share of the k
-    // steps and writes its sums to the p-th matrix at C (a later pass adds the shares in order)
-    uint32_t tile_id = blockIdx.x, part = 0;
-    if (parts > 1) {
-        const uint32_t per_part = gridDim.x / parts;
-        part = blockIdx.x / per_part;
-        tile_id = blockIdx.x % per_part;
+    uint32_t tile_id = blockIdx.x, part = 0, tile_m, tile_n;
+    if (flags & kGemmTriangleGrid) {
+        // the tile list is the lower triangle, row by row; `parts` copies of it: copy p multiplies the p-th share of the k
+        // steps and writes its sums to the p-th matrix at C (a later pass adds the shares in order)
+        const uint32_t lower = tiles_n * (tiles_n + 1) / 2;
+        uint32_t unit;
+        if (!gram_unit(lower * parts, unit)) return;
+        part = unit / lower;
+        tile_id = unit % lower;
         C += (uint64_t)part * part_stride;
-    }
-    uint32_t tile_m, tile_n;
-    if (flags & kGemmTriangleGrid) {  // the tile list is the lower triangle, row by row
         short_k::triangle_tile(tile_id, tile_m, tile_n);
     } else {
         tile_m = tile_id / tiles_n;
@@ -677,6 +689,144 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
     }
 }
 
+// ---- Gram product of 16-bit rows read in place -------------------------------------------------
+//
+// C = alpha X^T X + beta C for a row-major fp16 / bf16 matrix X[K, N]: the contraction runs down the rows, an MFMA
+// operand is eight values of one column.  A step is 64 rows of the tile's 256 columns (32 KB per operand); gfx950's
+// transposing LDS read (ds_read_b64_tr_b16) hands sixteen lanes, which name four rows of sixteen columns, four rows of a
+// column each, so that two of them make an operand and X needs no transposing pass (94 us and 410 MB of traffic for
+// [50 000, 2048] fp16).  X^T X with the result rounded: [50 000, 2048] 349 -> 249 us, [8200, 4096] 274 -> 200,
+// [2000, 512] 39 -> 25; bound by the MFMAs' power and, per step, the 64 LDS-direct loads of a CU.
+// LDS holds a row as 32 pieces of 16 bytes; the 64-byte units of row k are permuted, unit u in place u ^ (k % 4): the
+// four rows that 32 lanes read at a time then lie in different quarters of the 64 banks.  A wave's LDS-direct load
+// brings two rows' 512 bytes, whole lines.  Rows past K (in the last step) are written to LDS as zeros; columns past N
+// are read from the last eight and not stored.  MFMAs, their order and with it every bit are those of the one-plane
+// product; the fragment pipeline is gemm_nt16_kernel's.  The grid lists the lower-triangle tiles, `parts` copies of them as
+// in gemm_split_kernel.
+typedef short short4v __attribute__((ext_vector_type(4)));
+
+// rows 4 r + i / 4 of the lane's operand, r = 0, 1 (i = lane % 16)
+__device__ __forceinline__ piece read_transposed(const char* at) {
+    typedef __attribute__((address_space(3))) short4v* lds_ptr;
+    typedef uint32_t pair __attribute__((ext_vector_type(2)));
+    constexpr int kRowBytes = 2 * BM;
+    const pair a = __builtin_bit_cast(pair, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at)));
+    const pair b = __builtin_bit_cast(pair, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at + 4 * kRowBytes)));
+    return piece{a[0], a[1], b[0], b[1]};
+}
+
+template <bool F16, bool ACCUM>
+__global__ __launch_bounds__(64 * kWaves, 2) void gram16_kernel(const char* __restrict__ X, uint64_t ld, uint64_t K,
+                                                                uint64_t N, float* __restrict__ C, uint64_t ldc, float alpha,
+                                                                float beta, uint32_t parts, uint64_t part_stride) {
+    constexpr int JT = BN / kWavesN / 32;
+    constexpr int kStep = 64, kRowBytes = 2 * BM, kOperandBytes = kStep * kRowBytes;  // 32 KB
+    static_assert(BM == BN, "both operands are columns of X");
+    constexpr int kMoves = kOperandBytes / 1024 / kWaves;  // loads of two rows per wave, step and operand
+    __shared__ __attribute__((aligned(16))) char lds[2][2 * kOperandBytes];
+
+    const uint32_t tiles = (uint32_t)((N + BM - 1) / BM), lower = tiles * (tiles + 1) / 2;
+    uint32_t unit, tile_m, tile_n;
+    if (!gram_unit(lower * parts, unit)) return;
+    const uint32_t part = unit / lower;
+    C += (uint64_t)part * part_stride;
+    short_k::triangle_tile(unit % lower, tile_m, tile_n);
+    const uint64_t m0 = (uint64_t)tile_m * BM, n0 = (uint64_t)tile_n * BN;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;  // the wave number as a scalar
+    const int wm = wave / kWavesN, wn = wave % kWavesN;
+    const int x = lane & 31, h = lane >> 5;
+
+    floatx16 acc[2][JT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < JT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    const uint64_t all_steps = (K + kStep - 1) / kStep;
+    const uint64_t first = all_steps * part / parts, steps = all_steps * (part + 1) / parts;  // [first, steps)
+
+    // load i of a wave: rows 16 i + 2 wave + lane / 32 of the step; the lane's slot holds piece `from` of its row
+    const int row = 2 * wave + h, slot = lane & 31;
+    const uint32_t from = 8u * (uint32_t)(4 * ((slot >> 2) ^ (row & 3)) + (slot & 3));  // first column of the piece
+    const uint64_t last_m = N - 8 - m0, last_n = N - 8 - n0;
+    const uint32_t a_from = from < last_m ? from : (uint32_t)last_m, b_from = from < last_n ? from : (uint32_t)last_n;
+    const uint32_t a_off = (uint32_t)(row * ld + a_from) * 2u, b_off = (uint32_t)(row * ld + b_from) * 2u;
+    const char* a_tile = X + 2 * m0;
+    const char* b_tile = X + 2 * n0;
+    auto dma = [&](uint64_t s, char* buf) {
+        if ((s + 1) * kStep <= K) {
+#pragma unroll
+            for (int i = 0; i < 2 * kMoves; ++i) {
+                const uint64_t at = (s * kStep + 16 * (i % kMoves)) * ld * 2;  // scalar
+                const char* base = (i < kMoves ? a_tile : b_tile) + at;
+                char* to = buf + (i < kMoves ? 0 : kOperandBytes) + 1024 * (wave + kWaves * (i % kMoves));
+                __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(base + (i < kMoves ? a_off : b_off)),
+                                                 (void __attribute__((address_space(3)))*)to, 16, 0, 0);
+            }
+        } else {
+            for (int i = 0; i < 2 * kMoves; ++i) {
+                const uint64_t k = s * kStep + 16 * (i % kMoves);
+                piece v = {0u, 0u, 0u, 0u};
+                if (k + row < K)
+                    v = *reinterpret_cast<const piece*>((i < kMoves ? a_tile : b_tile) + k * ld * 2 + (i < kMoves ? a_off : b_off));
+                *reinterpret_cast<piece*>(buf + (i < kMoves ? 0 : kOperandBytes) + 1024 * (wave + kWaves * (i % kMoves)) + 16 * lane) = v;
+            }
+        }
+    };
+
+    // this lane's part of an operand's address: row 8 h + i / 4 of a sub-step's sixteen, columns 16 (lane / 16 % 2) + 4 (i % 4)
+    const int i16 = lane & 15, quarter = i16 >> 2;
+    const int lane_at = (8 * h + quarter) * kRowBytes + 32 * ((lane >> 4) & 1) + 8 * (i16 & 3);
+    int a_at[2], b_at[JT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) a_at[i] = lane_at + 64 * ((2 * wm + i) ^ quarter);
+#pragma unroll
+    for (int j = 0; j < JT; ++j) b_at[j] = kOperandBytes + lane_at + 64 * ((JT * wn + j) ^ quarter);
+
+    piece fa[2][2], fb[2][JT];
+    auto fetch = [&](int buf, int u, int set) {
+        const char* l = lds[buf] + 16 * u * kRowBytes;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) fa[set][i] = read_transposed(l + a_at[i]);
+#pragma unroll
+        for (int j = 0; j < JT; ++j) fb[set][j] = read_transposed(l + b_at[j]);
+    };
+
+    dma(first, lds[0]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    fetch(0, 0, 0);
+    for (uint64_t s = first; s < steps; ++s) {
+        const int cur = (int)((s - first) & 1);
+        const bool last_step = s + 1 == steps;
+        if (!last_step) dma(s + 1, lds[cur ^ 1]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int set = u & 1;
+            // the fragments of this sub-step are waited for here, before the next ones are requested (see gemm_nt16_kernel)
+            asm volatile("" ::"v"(fa[set][0]), "v"(fa[set][1]), "v"(fb[set][0]), "v"(fb[set][1]), "v"(fb[set][2]), "v"(fb[set][3]));
+            __builtin_amdgcn_sched_barrier(0);
+            if (u < 3) {
+                fetch(cur, u + 1, set ^ 1);
+            } else {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+                if (!last_step) fetch(cur ^ 1, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < JT; ++j)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc[i][j] = mfma16<F16>(fa[set][i], fb[set][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    store_c<ACCUM, JT>(acc, C, ldc, N, N, m0 + wm * 64, n0 + wn * (32 * JT) + x, h, alpha, beta, nullptr);
+}
+
 // C[i][j] = C[j][i] for j > i: completes a symmetric matrix whose lower triangle was computed.
 __global__ __launch_bounds__(256) void mirror_lower_kernel(float* __restrict__ C, uint64_t ldc, uint64_t n) {
     __shared__ float t[32][33];
@@ -698,9 +848,26 @@ __global__ __launch_bounds__(256) void mirror_lower_kernel(float* __restrict__ C
 }
 
 // C = alpha * (P_0 + P_1 + ... in this order) + beta * C on the lower triangle, mirrored into the upper
-// one: closes a symmetric product whose k range was shared out over `parts` matrices at P.
+// one: closes a symmetric product whose k range was shared out over `parts` matrices at P.  OUT: element type of C; 16-bit
+// results are rounded here (beta = 0; C 8-byte aligned, ldc a multiple of 4) instead of in a pass of their own.
+template <int OUT>
+__device__ __forceinline__ void store_quad(char* C, uint64_t at, const float (&v)[4]) {
+    if constexpr (OUT == TRAKHIP_F32)
+        *reinterpret_cast<float4u*>(C + 4 * at) = float4u{v[0], v[1], v[2], v[3]};  // 4-byte aligned
+    else
+        trakhip::store4<OUT>(C + 2 * at, make_float4(v[0], v[1], v[2], v[3]));
+}
+template <int OUT>
+__device__ __forceinline__ void store_one(char* C, uint64_t at, float v) {
+    if constexpr (OUT == TRAKHIP_F32)
+        reinterpret_cast<float*>(C)[at] = v;
+    else
+        reinterpret_cast<uint16_t*>(C)[at] = OUT == TRAKHIP_F16 ? trakhip::cast_f16_bits(v) : trakhip::cast_bf16_bits(v);
+}
+
+template <int OUT>
 __global__ __launch_bounds__(256) void gram_combine_kernel(const float* __restrict__ P, uint64_t part_stride,
-                                                           uint32_t parts, float* __restrict__ C, uint64_t ldc,
+                                                           uint32_t parts, char* __restrict__ C, uint64_t ldc,
                                                            uint64_t n, float alpha, float beta) {
     __shared__ float t[32][33];
     const uint32_t bi = blockIdx.y, bj = blockIdx.x;  // 32 x 32 block (bi, bj) on or under the diagonal
@@ -730,39 +897,36 @@ __global__ __launch_bounds__(256) void gram_combine_kernel(const float* __restri
             for (int e = 0; e < 4; ++e)
                 if (col + e < n) v[e] += P[(uint64_t)p * part_stride + row * n + col + e];
     }
-    float* out = C + row * ldc + col;
+    const uint64_t at = row * ldc + col;
+    const float* old = reinterpret_cast<const float*>(C) + at;  // (32-bit results only)
     if (whole && bj < bi) {
-        float4u old = {0.0f, 0.0f, 0.0f, 0.0f}, sum;
-        if (beta != 0.0f) old = *reinterpret_cast<const float4u*>(out);
+        float4u prev = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (OUT == TRAKHIP_F32 && beta != 0.0f) prev = *reinterpret_cast<const float4u*>(old);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             v[e] = alpha * v[e];
-            if (beta != 0.0f) v[e] += beta * old[e];
-            sum[e] = v[e];
+            if (OUT == TRAKHIP_F32 && beta != 0.0f) v[e] += beta * prev[e];
         }
-        *reinterpret_cast<float4u*>(out) = sum;
+        store_quad<OUT>(C, at, v);
     } else if (row < n) {
         for (int e = 0; e < 4; ++e) {
             if (col + e > row || col + e >= n) continue;
             v[e] = alpha * v[e];
-            if (beta != 0.0f) v[e] += beta * out[e];
-            out[e] = v[e];
+            if (OUT == TRAKHIP_F32 && beta != 0.0f) v[e] += beta * old[e];
+            store_one<OUT>(C, at + e, v[e]);
         }
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) t[r][c + e] = v[e];
     __syncthreads();
     // the mirror image: four columns of row 32 bj + r, from column c .. c + 3 of the transpose
-    const uint64_t mrow = (uint64_t)bj * 32 + r, mcol = (uint64_t)bi * 32 + c;
-    float* mirror = C + mrow * ldc + mcol;
+    const uint64_t mrow = (uint64_t)bj * 32 + r, mcol = (uint64_t)bi * 32 + c, mirror = mrow * ldc + mcol;
     if (bj < bi && mcol + 4 <= n) {  // (mrow < mcol then)
-        float4u o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = t[c + e][r];
-        *reinterpret_cast<float4u*>(mirror) = o;
+        const float o[4] = {t[c][r], t[c + 1][r], t[c + 2][r], t[c + 3][r]};
+        store_quad<OUT>(C, mirror, o);
     } else {
         for (int e = 0; e < 4; ++e)
-            if (mrow < n && mcol + e < n && mcol + e > mrow) mirror[e] = t[c + e][r];
+            if (mrow < n && mcol + e < n && mcol + e > mrow) store_one<OUT>(C, mirror + e, t[c + e][r]);
     }
 }
 
@@ -847,7 +1011,7 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
     uint64_t workgroups = tiles_m * tiles_n;
     if (parts > 1) {
         flags = kGemmTriangleGrid;
-        workgroups = tiles_m * (tiles_m + 1) / 2 * parts;
+        workgroups = (tiles_m * (tiles_m + 1) / 2 * parts + 7) / 8 * 8;
     }
     const dim3 grid((uint32_t)workgroups), block(64 * kWaves);
     const piece* a = static_cast<const piece*>(A_planes);
@@ -902,6 +1066,20 @@ uint32_t gram_parts(uint64_t N, uint64_t K, int dtype, bool two_planes, uint32_t
     return best;
 }
 
+// adds up the shares at P and mirrors the sum
+int combine_shares(const float* P, uint32_t parts, int out_dtype, void* C, uint64_t ldc, uint64_t N, float alpha, float beta,
+                   hipStream_t s) {
+    const uint64_t blocks = (N + 31) / 32;
+    if (blocks > 65535) return TRAKHIP_ERR_SHAPE;
+    const dim3 grid((uint32_t)blocks, (uint32_t)blocks);
+    char* out = static_cast<char*>(C);
+    auto kernel = out_dtype == TRAKHIP_F32   ? gram_combine_kernel<TRAKHIP_F32>
+                  : out_dtype == TRAKHIP_F16 ? gram_combine_kernel<TRAKHIP_F16>
+                                             : gram_combine_kernel<TRAKHIP_BF16>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, P, (uint64_t)N * N, parts, out, ldc, N, alpha, beta);
+    return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+}
+
 int gram_impl(const void* A_planes, const float* a_scales, uint64_t N, uint64_t K, int dtype, float* C, uint64_t ldc,
               float alpha, float beta, void* ws, size_t ws_bytes, hipStream_t s) {
     if (N == 0) return TRAKHIP_OK;
@@ -916,11 +1094,7 @@ int gram_impl(const void* A_planes, const float* a_scales, uint64_t N, uint64_t 
         const int e = launch_split(A_planes, N, A_planes, N, K, dtype, shares, N, 1.0f, 0.0f, nullptr, s, 0u, a_scales,
                                    a_scales, parts);
         if (e) return e;
-        const uint64_t blocks = (N + 31) / 32;
-        if (blocks > 65535) return TRAKHIP_ERR_SHAPE;
-        hipLaunchKernelGGL(gram_combine_kernel, dim3((uint32_t)blocks, (uint32_t)blocks), dim3(256), 0, s, shares,
-                           (uint64_t)N * N, parts, C, ldc, N, alpha, beta);
-        return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+        return combine_shares(shares, parts, TRAKHIP_F32, C, ldc, N, alpha, beta, s);
     }
     const int e = launch_split(A_planes, N, A_planes, N, K, dtype, C, ldc, alpha, beta, nullptr, s, trakhip::kGemmLowerTilesOnly,
                                a_scales, a_scales);
@@ -1030,6 +1204,34 @@ int gemm_nt16(const void* A, uint64_t lda, const void* B, uint64_t ldb, int dtyp
                        static_cast<const piece*>(A), lda / 8, static_cast<const piece*>(B), ldb / 8, K / 64, C, ldc, M, N,
                        alpha, beta, row_scale, (uint32_t)tiles_n, tiles);
     return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+}
+
+int gram16(const void* X, int dtype, uint64_t ld, uint64_t K, uint64_t N, int out_dtype, void* C, uint64_t ldc, float alpha,
+           float beta, void* ws, size_t ws_bytes, hipStream_t s) {
+    if (dtype != TRAKHIP_F16 && dtype != TRAKHIP_BF16) return TRAKHIP_ERR_DTYPE;
+    if (!known_dtype(out_dtype)) return TRAKHIP_ERR_DTYPE;
+    if (N == 0) return TRAKHIP_OK;
+    // (a lane's byte offset inside sixteen rows is kept in 32 bits)
+    if (K == 0 || N % 8 || ld % 8 || ld < N || ld >= (1ull << 23) || ldc < N) return TRAKHIP_ERR_SHAPE;
+    if (!X || !C) return TRAKHIP_ERR_NULL;
+    const bool wide = out_dtype == TRAKHIP_F32;
+    if ((reinterpret_cast<uintptr_t>(X) % 16) || (reinterpret_cast<uintptr_t>(C) % (wide ? 4 : 8))) return TRAKHIP_ERR_ALIGN;
+    if (!wide && (ldc % 4 || beta != 0.0f)) return TRAKHIP_ERR_SHAPE;
+    const uint64_t tiles = (N + BM - 1) / BM, lower = tiles * (tiles + 1) / 2;
+    const bool usable = ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0;
+    const uint32_t parts = usable ? gram_parts(N, K, dtype, false, kGramPartsMax, ws_bytes) : 1;
+    // a 16-bit result is rounded by the pass behind the product, which needs the sums in scratch
+    const bool scratch = parts > 1 || !wide;
+    if (scratch && !(usable && ws_bytes / sizeof(float) / N >= N * parts)) return TRAKHIP_ERR_WORKSPACE;
+    if (lower * parts > 0x7FFFFFF0ull) return TRAKHIP_ERR_SHAPE;
+    float* sums = scratch ? static_cast<float*>(ws) : static_cast<float*>(C);
+    const bool accum = !scratch && beta != 0.0f;
+    auto kernel = dtype == TRAKHIP_F16 ? (accum ? gram16_kernel<true, true> : gram16_kernel<true, false>)
+                                       : (accum ? gram16_kernel<false, true> : gram16_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)((lower * parts + 7) / 8 * 8)), dim3(64 * kWaves), 0, s, static_cast<const char*>(X), ld, K, N,
+                       sums, scratch ? N : ldc, scratch ? 1.0f : alpha, scratch ? 0.0f : beta, parts, (uint64_t)N * N);
+    if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
+    return scratch ? combine_shares(sums, parts, out_dtype, C, ldc, N, alpha, beta, s) : mirror_lower(sums, ldc, N, s);
 }
 
 int gram_split(const void* A_planes, uint64_t N, uint64_t K, int dtype, float* C, uint64_t ldc, float alpha, float beta,

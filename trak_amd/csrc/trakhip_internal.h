@@ -72,6 +72,9 @@ int gemm_nt_split(const void* A_planes, uint64_t M, const void* B_planes, uint64
 size_t gram_split_workspace_bytes(uint64_t N, uint64_t K, int dtype, int two_planes, bool most);
 int gram_split(const void* A_planes, uint64_t N, uint64_t K, int dtype, float* C, uint64_t ldc, float alpha, float beta,
                void* ws, size_t ws_bytes, hipStream_t s);
+// X^T X of 16-bit rows where they are (N, ld multiples of 8, 16-byte aligned); ws as for gram_split, needed for a 16-bit result
+int gram16(const void* X, int dtype, uint64_t ld, uint64_t K, uint64_t N, int out_dtype, void* C, uint64_t ldc, float alpha,
+           float beta, void* ws, size_t ws_bytes, hipStream_t s);
 size_t split2_bytes(uint64_t rows, uint64_t K);
 int split2_rows(const float* src, uint64_t ld, uint64_t rows, uint64_t K, int transposed, void* planes,
                 size_t planes_bytes, float* scales, hipStream_t s);

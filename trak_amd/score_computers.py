@@ -17,6 +17,8 @@ from .utils import (
     gemm_nt_split,
     gemm_tn,
     get_matrix_mult_blockwise,
+    gram16,
+    gram16_ok,
     gram_split,
     in_place_pays,
     matmul_nt,
@@ -115,7 +117,9 @@ class BasicScoreComputer(AbstractScoreComputer):
         return ch.split(grads, split_size_or_sections=self.CUDA_MAX_DIM_SIZE, dim=0)
 
     def _gram(self, block, out, beta):
-        if self.gemm != "fp32":
+        if self.gemm != "fp32" and gram16_ok(block):
+            gram16(block, out=out, alpha=1.0, beta=beta)
+        elif self.gemm != "fp32":
             # the operand is block^T, read in place; lower-triangle tiles + mirror image
             gram_split(self._split(block, transposed=True), out=out, alpha=1.0, beta=beta)
         else:
@@ -132,9 +136,14 @@ class BasicScoreComputer(AbstractScoreComputer):
                 self._gram(block.to(self._dev), product, 0.0)
                 result += product.to(block.dtype)  # the block product in the gradients' type, as `block.T @ block` returns it
             return result
-        result = ch.zeros(self.proj_dim, self.proj_dim, dtype=ch.float32, device=self._dev)
-        for block in self._blocks(grads):
-            self._gram(block.to(self._dev), result, 1.0)
+        blocks = self._blocks(grads)
+        if len(blocks) == 1 and self.gemm != "fp32" and self.dtype in (ch.float16, ch.bfloat16):
+            block = blocks[0].to(self._dev)
+            if gram16_ok(block):
+                return gram16(block, out_dtype=self.dtype)
+        result = ch.empty(self.proj_dim, self.proj_dim, dtype=ch.float32, device=self._dev)
+        for i, block in enumerate(blocks):
+            self._gram(block.to(self._dev), result, 0.0 if i == 0 else 1.0)
         return result.to(self.dtype)
 
     def get_x_xtx_inv(self, grads: Tensor, xtx: Tensor) -> Tensor:

@@ -392,6 +392,41 @@ def gram_split(a, out=None, alpha=1.0, beta=0.0):
     return out
 
 
+def gram16_ok(x):
+    """Whether `gram16` can read this matrix where it is."""
+    return (x.dtype in (torch.float16, torch.bfloat16) and x.dim() == 2 and x.is_cuda and x.numel() > 0
+            and x.stride(1) == 1 and x.shape[1] % 8 == 0 and x.data_ptr() % 16 == 0
+            and (x.shape[0] == 1 or (x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1]))
+            and max(x.stride(0), x.shape[1]) < 1 << 23)  # a lane's offset is kept in 32 bits
+
+
+def gram16(x, out=None, alpha=1.0, beta=0.0, out_dtype=torch.float32):
+    """out[N, N] = alpha * x.T @ x + beta * out for an fp16 or bf16 CUDA matrix x [K, N] read in place (N % 8 == 0, rows
+    16-byte aligned): the result of `gram_split(split_rows(x, transposed=True))`, bit for bit, exactly symmetric.
+    Without `out`, an fp32 matrix or, with out_dtype, that result rounded to 16 bits."""
+    if not gram16_ok(x):
+        raise RuntimeError("gram16 needs an fp16 or bf16 CUDA matrix with N % 8 == 0 and 16-byte aligned rows")
+    K, N = x.shape
+    lib = _lib.load()
+    ws = _gram_scratch(lib, N, K, _STORE_DTYPES[x.dtype], 0, x.device)
+    rounded = None
+    if out is None:
+        if out_dtype != torch.float32 and ws is None:  # no scratch that the sums would pass through
+            rounded, out_dtype = out_dtype, torch.float32
+        out, beta = torch.empty((N, N), dtype=out_dtype, device=x.device), 0.0
+    elif out.dtype != torch.float32 or tuple(out.shape) != (N, N) or (N > 1 and out.stride(1) != 1) or out.device != x.device:
+        raise RuntimeError("out must be an fp32 [N, N] tensor with unit column stride on the operand's device")
+    with torch.cuda.device(x.device):
+        stream = torch.cuda.current_stream(x.device).cuda_stream
+        ws_ptr, ws_bytes = (ctypes.c_void_p(ws.data_ptr()), ws.numel()) if ws is not None else (None, 0)
+        code = lib.trakhip_gram16(
+            ctypes.c_void_p(x.data_ptr()), _STORE_DTYPES[x.dtype], _ld(x), K, N, _STORE_DTYPES[out.dtype],
+            ctypes.c_void_p(out.data_ptr()), _ld(out), float(alpha), float(beta), ws_ptr, ws_bytes, ctypes.c_void_p(stream),
+        )
+    _lib.check(code)
+    return out if rounded is None else out.to(rounded)
+
+
 def _inverse_call(a, lambda_reg, normalize, general):
     """One call of trakhip_spd_inverse (Cholesky) or trakhip_general_inverse (pivoted elimination):
     (inverse, mean_abs, status word)."""
