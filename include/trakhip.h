@@ -266,6 +266,12 @@ int trakhip_gemm_nt16(const void* A_dev, uint64_t lda, const void* B_dev, uint64
                       uint64_t ldc, uint64_t M, uint64_t N, uint64_t K, float alpha, float beta,
                       const float* row_scale_dev, void* stream);
 
+/* The same with beta = 0 and C of element type out_dtype: every fp32 sum rounded to it once, the values that
+ * trakhip_gemm_nt16 and a cast of its result give. */
+int trakhip_gemm_nt16_rounded(const void* A_dev, uint64_t lda, const void* B_dev, uint64_t ldb, int dtype, int out_dtype,
+                              void* C_dev, uint64_t ldc, uint64_t M, uint64_t N, uint64_t K, float alpha,
+                              const float* row_scale_dev, void* stream);
+
 /* out[i, j] = cast((acc[i, j] / divisor) * row_factor[i]) for the [N, M] fp32 score sums that
  * trakhip_gemm_nt accumulated over checkpoints (beta = 1): the closing expression of
  * TRAKer.finalize_scores, `(_scores / n) * (_avg_out_to_losses / n)` (trak/traker.py:670-678), with

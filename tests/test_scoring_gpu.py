@@ -478,6 +478,50 @@ def test_gemm_nt16_reads_operands_in_place(gpu, dtype, M, N, K):
     assert torch.equal(wide[:, :N], gemm_nt16(ag, bg)) and bool((wide[:, N:] == -1.0).all())
 
 
+# columns of tiles: one, two, eight (one band), nine and twelve (two bands), thirteen (row by row)
+@pytest.mark.parametrize("M,N", [(2100, 256), (1300, 300), (700, 2048), (1300, 2309), (520, 3072), (600, 3100), (20, 2500), (5000, 1)])
+def test_products_in_every_order_of_their_tiles(gpu, M, N):
+    gen = torch.Generator(device=gpu).manual_seed(M + N)
+    for dtype, K in ((torch.float16, 128), (torch.float32, 32)):
+        a, b = (torch.randn(r, K, generator=gen, device=gpu).to(dtype) for r in (M, N))
+        want = (a.double() @ b.double().T).cpu().numpy()
+        out = torch.full((M, N), float("nan"), device=gpu)
+        got = gemm_nt16(a, b, out=out) if dtype == torch.float16 else gemm_nt_split(split_rows(a), split_rows(b), out=out)
+        assert rel_max(got.cpu().numpy(), want) < gemm_tol(K)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,pad,shift", [(1, 1, 64, 0, 0), (64, 128, 64, 0, 0), (257, 255, 128, 0, 0), (300, 700, 4096, 4, 0),
+                                             (513, 1024, 192, 3, 0), (256, 512, 64, 8, 2), (256, 512, 64, 8, 1)])
+def test_gemm_nt16_rounds_its_result(gpu, dtype, M, N, K, pad, shift):
+    gen = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a, b = (torch.randn(r, K, generator=gen, device=gpu).to(dtype) for r in (M, N))
+    rs = torch.rand(M, generator=gen, device=gpu)
+    for out_dtype in (torch.float16, torch.bfloat16):
+        wide = torch.full((M, N + pad + shift), 7.0, dtype=out_dtype, device=gpu)      # pitches and starts of every alignment
+        out = wide[:, shift:N + shift]
+        assert torch.equal(gemm_nt16(a, b, out=out), gemm_nt16(a, b).to(out_dtype))
+        assert bool((wide[:, :shift] == 7.0).all()) and bool((wide[:, N + shift:] == 7.0).all())
+        gemm_nt16(a, b, out=out, alpha=0.25, row_scale=rs)
+        assert torch.equal(out, gemm_nt16(a, b, alpha=0.25, row_scale=rs).to(out_dtype))
+        with pytest.raises(RuntimeError):
+            gemm_nt16(a, b, out=out, beta=1.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_features_are_the_rounded_product_whatever_the_route(gpu, dtype):
+    k = 520
+    x = (torch.randn(1100, k, generator=torch.Generator(device=gpu).manual_seed(5), device=gpu) / k ** 0.5).to(dtype)
+    for cols in (512, 520, 500):                                    # read in place; through planes; rows not aligned
+        block = x[:, :cols]
+        sc = BasicScoreComputer(dtype=dtype, device=gpu, lambda_reg=1e-2, CUDA_MAX_DIM_SIZE=400)
+        xtx = sc.get_xtx(block)
+        inv = spd_inverse(xtx, lambda_reg=1e-2, normalize=True, general_fallback=True)[0].to(dtype)
+        want = gemm_nt_split(split_rows(block), split_rows(inv)).to(dtype)
+        assert torch.equal(sc.get_x_xtx_inv(block, xtx), want)
+        assert torch.equal(sc.get_x_xtx_inv(block.cpu(), xtx), want)               # from the host, block by block
+
+
 def test_gemm_nt16_refuses_what_it_cannot_read_in_place(gpu):
     a = torch.randn(64, 128, device=gpu).half()
     b = torch.randn(32, 128, device=gpu).half()

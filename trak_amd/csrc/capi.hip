@@ -183,7 +183,14 @@ int trakhip_gram_split2(const void* A_planes_dev, const float* A_scales_dev, uin
 int trakhip_gemm_nt16(const void* A_dev, uint64_t lda, const void* B_dev, uint64_t ldb, int dtype, float* C_dev,
                       uint64_t ldc, uint64_t M, uint64_t N, uint64_t K, float alpha, float beta,
                       const float* row_scale_dev, void* stream) {
-    return trakhip::gemm_nt16(A_dev, lda, B_dev, ldb, dtype, C_dev, ldc, M, N, K, alpha, beta, row_scale_dev,
+    return trakhip::gemm_nt16(A_dev, lda, B_dev, ldb, dtype, TRAKHIP_F32, C_dev, ldc, M, N, K, alpha, beta, row_scale_dev,
+                              static_cast<hipStream_t>(stream));
+}
+
+int trakhip_gemm_nt16_rounded(const void* A_dev, uint64_t lda, const void* B_dev, uint64_t ldb, int dtype, int out_dtype,
+                              void* C_dev, uint64_t ldc, uint64_t M, uint64_t N, uint64_t K, float alpha,
+                              const float* row_scale_dev, void* stream) {
+    return trakhip::gemm_nt16(A_dev, lda, B_dev, ldb, dtype, out_dtype, C_dev, ldc, M, N, K, alpha, 0.0f, row_scale_dev,
                               static_cast<hipStream_t>(stream));
 }
 

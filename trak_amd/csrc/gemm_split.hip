@@ -49,6 +49,7 @@ typedef uint32_t piece __attribute__((ext_vector_type(4)));  // 16 bytes = 8 x 1
 constexpr int kWavesM = 4, kWavesN = 2;            // 4 x 2 waves, each owns 64 x 128 of C
 constexpr int BM = 64 * kWavesM, BN = 128 * kWavesN;
 constexpr int kWaves = kWavesM * kWavesN;
+constexpr uint32_t kGemmBandedGrid = 4u;            // kernel flag: the grid is numbered as banded_tile says
 constexpr uint32_t kGemmTriangleGrid = 2u;          // kernel flag: the grid lists the lower-triangle tiles only
 constexpr int kRowPad = 256;                       // rows of an operand are padded to this
 constexpr int kOctetPad = 8;                       // octets (64 values of k) are padded to this
@@ -372,6 +373,47 @@ __device__ __forceinline__ void store_c(const floatx16 (&acc)[2][JT], float* __r
     }
 }
 
+// The same for a 16-bit C (OUT: its element type; beta = 0): rounded from the accumulators instead of by a pass over an
+// fp32 result (94 us for [50 000, 2048]).  vec: C 8-byte aligned, ldc a multiple of 4.
+template <int OUT, int JT>
+__device__ __forceinline__ void store_c16(const floatx16 (&acc)[2][JT], uint16_t* __restrict__ C, uint64_t ldc, uint64_t M,
+                                          uint64_t N, uint64_t row_base, uint64_t col0, int h, float alpha,
+                                          const float* __restrict__ row_scale, bool vec) {
+    const int lane = threadIdx.x & 63, q = lane & 3;
+    if (vec && row_base + 64 <= M && col0 - (lane & 31) + 32 * JT <= N) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {  // as in store_c: four columns of one row per lane
+                const uint64_t row = row_base + 32 * i + 8 * g + 4 * h + q;
+                const float rs = row_scale ? row_scale[row] : 1.0f;
+                uint16_t* p = C + row * ldc + (col0 - q);
+#pragma unroll
+                for (int j = 0; j < JT; ++j) {
+                    float v[4] = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+                    quad_transpose(v, lane);
+                    trakhip::store4<OUT>(p + 32 * j, make_float4(alpha * v[0] * rs, alpha * v[1] * rs, alpha * v[2] * rs,
+                                                                 alpha * v[3] * rs));
+                }
+            }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint64_t row = row_base + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (row >= M) continue;
+            const float rs = row_scale ? row_scale[row] : 1.0f;
+#pragma unroll
+            for (int j = 0; j < JT; ++j) {
+                const float v = alpha * acc[i][j][r] * rs;
+                if (col0 + 32 * j < N)
+                    C[row * ldc + col0 + 32 * j] = OUT == TRAKHIP_F16 ? trakhip::cast_f16_bits(v) : trakhip::cast_bf16_bits(v);
+            }
+        }
+}
+
 // A step of a tile is S sub-steps (two octets = one MFMA depth each); sub-step u holds
 // [A: plane][half][256 rows] followed by [B: plane][half][256 rows].  The pieces are moved in chunks
 // of 64 consecutive ones by the load unit straight into LDS (global_load_lds_dwordx4): the 64
@@ -437,11 +479,30 @@ struct StepMover {
 // dealt out over all XCDs each of them fetched every row of X ([50 000, 2048] fp16: 1.6 GB; 285 us, now 249; the
 // three-plane product of [4100, 2048] fp32 138 -> 126, of [50 000, 4096] 4.41 -> 4.33 ms).  The grid has a multiple of
 // eight workgroups; false: one without a unit.
-__device__ __forceinline__ bool gram_unit(uint32_t units, uint32_t& unit) {
+__device__ __forceinline__ bool xcd_unit(uint32_t units, uint32_t& unit) {
     const uint32_t xcd = blockIdx.x & 7u;
     unit = (uint32_t)((uint64_t)xcd * units / 8u) + (blockIdx.x >> 3);
     return unit < (uint32_t)((xcd + 1ull) * units / 8u);
 }
+
+// The same for the grid of tiles of a product with up to kBandedTiles columns of tiles: number `position` of an order in which
+// neighbours share operands.  Up to eight columns are walked row by row, more of them in two bands, and each XCD takes a
+// contiguous eighth of the walk, so that the 32 tiles that an XCD works on at a time are some four rows of eight columns.
+// (Row by row over all XCDs, eight columns give each XCD one column of 32 rows: 33 operand panels where 12 would do.)
+// [50 000, 2048] by 2048 columns fp16 441 -> 432 us, 1536 257 -> 245; fp32 2048 1.93 -> 1.89 ms, 2560 2.83 -> 2.71.  With
+// 16 columns the same time, from 24 on 2-9 % slower: row by row, an XCD then has five or more columns of six or fewer rows.
+constexpr uint32_t kBandedTiles = 12;
+__device__ __forceinline__ void banded_tile(uint32_t position, uint32_t tiles_m, uint32_t tiles_n, uint32_t& tile_m,
+                                            uint32_t& tile_n) {
+    uint32_t first = 0, width = tiles_n;
+    if (tiles_n > 8) {
+        width = tiles_n / 2;
+        if (position >= width * tiles_m) position -= width * tiles_m, first = width, width = tiles_n - width;
+    }
+    tile_m = position / width;
+    tile_n = first + position % width;
+}
+bool banded(uint64_t tiles_n) { return tiles_n > 1 && tiles_n <= kBandedTiles; }
 
 // P planes per operand (3: split fp32, 1: a 16-bit type), F16 selects the fp16 MFMA, S sub-steps
 // per barrier.
@@ -463,11 +524,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_split_kernel(
         // steps and writes its sums to the p-th matrix at C (a later pass adds the shares in order)
         const uint32_t lower = tiles_n * (tiles_n + 1) / 2;
         uint32_t unit;
-        if (!gram_unit(lower * parts, unit)) return;
+        if (!xcd_unit(lower * parts, unit)) return;
         part = unit / lower;
         tile_id = unit % lower;
         C += (uint64_t)part * part_stride;
         short_k::triangle_tile(tile_id, tile_m, tile_n);
+    } else if (flags & kGemmBandedGrid) {
+        const uint32_t tiles_m = (uint32_t)((M + BM - 1) / BM);
+        if (!xcd_unit(tiles_m * tiles_n, tile_id)) return;
+        banded_tile(tile_id, tiles_m, tiles_n, tile_m, tile_n);
     } else {
         tile_m = tile_id / tiles_n;
         tile_n = tile_id % tiles_n;
@@ -562,11 +627,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_split_kernel(
 // of those 256 bytes - rows of equal parity share a 128-byte half and differ in r / 2.  Linear global
 // reads, conflict-free LDS reads (XOR with r % 8 instead leaves a two-way conflict), and the same MFMA loop as
 // the one-plane kernel.  Rows past M or N are fetched from the last row (their results are not stored).
-template <bool F16, bool ACCUM>
+template <bool F16, bool ACCUM, int OUT = TRAKHIP_F32>
 __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
     const piece* __restrict__ A, uint64_t lda8, const piece* __restrict__ B, uint64_t ldb8, uint64_t steps,
-    float* __restrict__ C, uint64_t ldc, uint64_t M, uint64_t N, float alpha, float beta,
-    const float* __restrict__ row_scale, uint32_t tiles_n, uint32_t tiles) {
+    void* __restrict__ C_any, uint64_t ldc, uint64_t M, uint64_t N, float alpha, float beta,
+    const float* __restrict__ row_scale, uint32_t tiles_n, uint32_t tiles, uint32_t in_bands, bool vec16) {
     constexpr int JT = BN / kWavesN / 32;
     constexpr int kBufPieces = 8 * (BM + BN);  // 64 KB
     constexpr int kMoves = (BM + BN) / 8 / kWaves, kMovesA = BM / 8 / kWaves;  // chunks per wave and step
@@ -578,14 +643,25 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
     const int x = lane & 31, h = lane >> 5;
     const int a_row = (wm * 64 + x) * 8, b_row = (BM + wn * (32 * JT) + x) * 8;  // first piece of the lane's rows
 
-    // The workgroups are persistent: workgroup w computes tiles w, w + gridDim.x, ...  A load's address is a
+    // The workgroups are persistent: those of an XCD go through its eighth of the tiles side by side.  A load's address is a
     // scalar base (first row of the tile, advanced by one 128-byte line per step) plus this lane's byte offset
     // inside the tile's rows.
     const char* a_tile;
     const char* b_tile;
     uint32_t voff[kMoves];
+    const uint32_t tiles_m = tiles / tiles_n;
+    auto place = [&](uint32_t t, uint32_t& tm, uint32_t& tn) {
+        if (in_bands) {
+            banded_tile(t, tiles_m, tiles_n, tm, tn);
+        } else {
+            tm = t / tiles_n;
+            tn = t % tiles_n;
+        }
+    };
     auto set_tile = [&](uint32_t t) {
-        const uint64_t m0 = (uint64_t)(t / tiles_n) * BM, n0 = (uint64_t)(t % tiles_n) * BN;
+        uint32_t tm, tn;
+        place(t, tm, tn);
+        const uint64_t m0 = (uint64_t)tm * BM, n0 = (uint64_t)tn * BN;
         a_tile = reinterpret_cast<const char*>(A + m0 * lda8);
         b_tile = reinterpret_cast<const char*>(B + n0 * ldb8);
         // rows 8c + sub of chunk c = wave + 8 i': (row >> 1) % 8 = 4 (wave % 2) + sub / 2
@@ -625,8 +701,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
         for (int j = 0; j < JT; ++j) fb[set][j] = l[b_row + 256 * j];
     };
 
-    uint32_t tile = blockIdx.x;
-    if (tile >= tiles) return;
+    uint32_t tile, end = tiles, stride = gridDim.x;
+    if (in_bands) {
+        const uint32_t xcd = blockIdx.x & 7u;
+        tile = (uint32_t)((uint64_t)xcd * tiles / 8u) + (blockIdx.x >> 3);
+        end = (uint32_t)((xcd + 1ull) * tiles / 8u);
+        stride = gridDim.x >> 3;
+    } else {
+        tile = blockIdx.x;
+    }
+    if (tile >= end) return;
     set_tile(tile);
     int first = 0;  // buffer that holds step 0 of the current tile
     dma(0, lds[0]);
@@ -641,8 +725,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
             for (int j = 0; j < JT; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-        const uint64_t m0 = (uint64_t)(tile / tiles_n) * BM, n0 = (uint64_t)(tile % tiles_n) * BN;
-        const uint32_t next = tile + gridDim.x;
+        uint32_t tile_m, tile_n;
+        place(tile, tile_m, tile_n);
+        const uint64_t m0 = (uint64_t)tile_m * BM, n0 = (uint64_t)tile_n * BN;
+        const uint32_t next = tile + stride;
 
         fetch(first, 0, 0);
         for (uint64_t s = 0; s < steps; ++s) {
@@ -650,7 +736,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
             const bool last_step = s + 1 == steps;
             if (!last_step) {
                 dma(s + 1, lds[cur ^ 1]);
-            } else if (next < tiles) {
+            } else if (next < end) {
                 // step 0 of the next tile arrives under the last MFMAs and the stores of this one
                 set_tile(next);
                 dma(0, lds[cur ^ 1]);
@@ -682,8 +768,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        store_c<ACCUM, JT>(acc, C, ldc, M, N, m0 + wm * 64, n0 + wn * (32 * JT) + x, h, alpha, beta, row_scale);
-        if (next >= tiles) break;
+        if constexpr (OUT == TRAKHIP_F32)
+            store_c<ACCUM, JT>(acc, static_cast<float*>(C_any), ldc, M, N, m0 + wm * 64, n0 + wn * (32 * JT) + x, h, alpha, beta,
+                               row_scale);
+        else
+            store_c16<OUT, JT>(acc, static_cast<uint16_t*>(C_any), ldc, M, N, m0 + wm * 64, n0 + wn * (32 * JT) + x, h, alpha,
+                               row_scale, vec16);
+        if (next >= end) break;
         first = (int)((steps + first) & 1);
         tile = next;
     }
@@ -727,7 +818,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gram16_kernel(const char* __re
 
     const uint32_t tiles = (uint32_t)((N + BM - 1) / BM), lower = tiles * (tiles + 1) / 2;
     uint32_t unit, tile_m, tile_n;
-    if (!gram_unit(lower * parts, unit)) return;
+    if (!xcd_unit(lower * parts, unit)) return;
     const uint32_t part = unit / lower;
     C += (uint64_t)part * part_stride;
     short_k::triangle_tile(unit % lower, tile_m, tile_n);
@@ -1013,6 +1104,10 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
         flags = kGemmTriangleGrid;
         workgroups = (tiles_m * (tiles_m + 1) / 2 * parts + 7) / 8 * 8;
     }
+    if (parts == 1 && !flags && banded(tiles_n)) {
+        flags = kGemmBandedGrid;
+        workgroups = (workgroups + 7) / 8 * 8;
+    }
     const dim3 grid((uint32_t)workgroups), block(64 * kWaves);
     const piece* a = static_cast<const piece*>(A_planes);
     const piece* b = static_cast<const piece*>(B_planes);
@@ -1174,35 +1269,46 @@ int gram_split2(const void* A_planes, const float* a_scales, uint64_t N, uint64_
     return gram_impl(A_planes, a_scales, N, K, TRAKHIP_F32, C, ldc, alpha, beta, ws, ws_bytes, s);
 }
 
-int gemm_nt16(const void* A, uint64_t lda, const void* B, uint64_t ldb, int dtype, float* C, uint64_t ldc, uint64_t M,
-              uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s) {
+int gemm_nt16(const void* A, uint64_t lda, const void* B, uint64_t ldb, int dtype, int out_dtype, void* C, uint64_t ldc,
+              uint64_t M, uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s) {
     if (dtype != TRAKHIP_F16 && dtype != TRAKHIP_BF16) return TRAKHIP_ERR_DTYPE;
+    if (!known_dtype(out_dtype)) return TRAKHIP_ERR_DTYPE;
     if (M == 0 || N == 0) return TRAKHIP_OK;
     if (K == 0 || K % 64 || lda < K || ldb < K || ldc < N) return TRAKHIP_ERR_SHAPE;
     // a lane's byte offset inside the 256 rows of a tile is kept in 32 bits
     if (lda >= (1ull << 23) || ldb >= (1ull << 23)) return TRAKHIP_ERR_SHAPE;
     if (!A || !B || !C) return TRAKHIP_ERR_NULL;
     if ((reinterpret_cast<uintptr_t>(A) % 16) || (reinterpret_cast<uintptr_t>(B) % 16) || (lda % 8) || (ldb % 8) ||
-        (reinterpret_cast<uintptr_t>(C) % 4))
+        (reinterpret_cast<uintptr_t>(C) % (out_dtype == TRAKHIP_F32 ? 4 : 2)))
         return TRAKHIP_ERR_ALIGN;
+    if (out_dtype != TRAKHIP_F32 && beta != 0.0f) return TRAKHIP_ERR_SHAPE;
     const uint64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     if (tiles_m * tiles_n > 0x7FFFFFFFull) return TRAKHIP_ERR_SHAPE;
-    void (*kernel)(const piece*, uint64_t, const piece*, uint64_t, uint64_t, float*, uint64_t, uint64_t, uint64_t, float,
-                   float, const float*, uint32_t, uint32_t);
+    void (*kernel)(const piece*, uint64_t, const piece*, uint64_t, uint64_t, void*, uint64_t, uint64_t, uint64_t, float,
+                   float, const float*, uint32_t, uint32_t, uint32_t, bool);
     const bool accum = beta != 0.0f;
-    if (dtype == TRAKHIP_F16)
+    const bool f16 = dtype == TRAKHIP_F16;
+    if (out_dtype == TRAKHIP_F16)
+        kernel = f16 ? gemm_nt16_kernel<true, false, TRAKHIP_F16> : gemm_nt16_kernel<false, false, TRAKHIP_F16>;
+    else if (out_dtype == TRAKHIP_BF16)
+        kernel = f16 ? gemm_nt16_kernel<true, false, TRAKHIP_BF16> : gemm_nt16_kernel<false, false, TRAKHIP_BF16>;
+    else if (f16)
         kernel = accum ? gemm_nt16_kernel<true, true> : gemm_nt16_kernel<true, false>;
     else
         kernel = accum ? gemm_nt16_kernel<false, true> : gemm_nt16_kernel<false, false>;
+    const bool vec16 = reinterpret_cast<uintptr_t>(C) % 8 == 0 && ldc % 4 == 0;  // 8-byte stores of a 16-bit result
     const uint32_t tiles = (uint32_t)(tiles_m * tiles_n);
     // persistent workgroups, one per CU (128 KB of LDS each)
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
-    hipLaunchKernelGGL(kernel, dim3(tiles < (uint32_t)cus ? tiles : (uint32_t)cus), dim3(64 * kWaves), 0, s,
-                       static_cast<const piece*>(A), lda / 8, static_cast<const piece*>(B), ldb / 8, K / 64, C, ldc, M, N,
-                       alpha, beta, row_scale, (uint32_t)tiles_n, tiles);
+    const bool in_bands = banded(tiles_n) && cus >= 8;
+    uint32_t workgroups = tiles < (uint32_t)cus ? tiles : (uint32_t)cus;
+    if (in_bands) workgroups = tiles < (uint32_t)cus ? (tiles + 7) / 8 * 8 : (uint32_t)cus / 8 * 8;
+    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(64 * kWaves), 0, s, static_cast<const piece*>(A), lda / 8,
+                       static_cast<const piece*>(B), ldb / 8, K / 64, C, ldc, M, N, alpha, beta, row_scale, (uint32_t)tiles_n,
+                       tiles, in_bands ? 1u : 0u, vec16);
     return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
 }
 

@@ -83,8 +83,8 @@ int gemm_nt_split2(const void* A_planes, const float* a_scales, uint64_t M, cons
                    hipStream_t s, uint32_t flags = 0);
 int gram_split2(const void* A_planes, const float* a_scales, uint64_t N, uint64_t K, float* C, uint64_t ldc, float alpha,
                 float beta, void* ws, size_t ws_bytes, hipStream_t s);
-int gemm_nt16(const void* A, uint64_t lda, const void* B, uint64_t ldb, int dtype, float* C, uint64_t ldc, uint64_t M,
-              uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s);
+int gemm_nt16(const void* A, uint64_t lda, const void* B, uint64_t ldb, int dtype, int out_dtype, void* C, uint64_t ldc,
+              uint64_t M, uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s);
 size_t spd_inverse_workspace_bytes(uint64_t n);
 int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t ldi, uint64_t n,
                 int normalize, float* mean_abs, int32_t* status, void* ws, size_t ws_bytes, hipStream_t s);

@@ -158,9 +158,11 @@ class BasicScoreComputer(AbstractScoreComputer):
             xtx_inv, _ = spd_inverse(xtx, lambda_reg=self.lambda_reg, normalize=True, general_fallback=True)
         xtx_inv = xtx_inv.to(self.dtype)
 
-        result = ch.empty(grads.shape[0], xtx_inv.shape[1], dtype=ch.float32, device=self._dev)
         # 16-bit gradients meet the inverse cast to their type (as in the reference) as single planes
         half = grads.dtype == xtx_inv.dtype and grads.dtype in (ch.float16, ch.bfloat16)
+        # the sums of a product that reads both in place are rounded as they are stored
+        result = ch.empty(grads.shape[0], xtx_inv.shape[1], dtype=self.dtype if half and self.gemm != "fp32" else ch.float32,
+                          device=self._dev)
         inv_split = None  # planes of the inverse, made when the first block needs them
         start = 0
         for block in self._blocks(grads):
@@ -175,7 +177,10 @@ class BasicScoreComputer(AbstractScoreComputer):
                 else:
                     if inv_split is None:
                         inv_split = self._split(xtx_inv if half else xtx_inv.float())
-                    gemm_nt_split(self._split(block if half else block.float()), inv_split, out=result[start:end])
+                    if half:
+                        result[start:end] = gemm_nt_split(self._split(block), inv_split)
+                    else:
+                        gemm_nt_split(self._split(block.float()), inv_split, out=result[start:end])
             else:
                 gemm_nt(block.to(self._dev), xtx_inv, out=result[start:end])
             start = end

@@ -301,17 +301,19 @@ def nt16_ok(a, b):
 
 
 def gemm_nt16(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
-    """out[M, N] (fp32) = alpha * a @ b.T + beta * out (rows optionally scaled) for fp16 or bf16 CUDA
+    """out[M, N] = alpha * a @ b.T + beta * out (rows optionally scaled) for fp16 or bf16 CUDA
     matrices a [M, K], b [N, K] read in place: K a multiple of 64, rows 16-byte aligned (see
-    `matmul_nt` for the general case).  Exact products, fp32 accumulation."""
+    `matmul_nt` for the general case).  Exact products, fp32 accumulation.  `out` is fp32, or (beta = 0)
+    fp16 or bf16: every sum rounded once."""
     if not nt16_ok(a, b):
         raise RuntimeError("gemm_nt16 needs two fp16 or two bf16 CUDA matrices with K % 64 == 0 and 16-byte aligned rows")
     M, N, K = a.shape[0], b.shape[0], a.shape[1]
     if out is None:
         out = torch.empty((M, N), dtype=torch.float32, device=a.device)
         beta = 0.0
-    if out.dtype != torch.float32 or tuple(out.shape) != (M, N) or (N > 1 and out.stride(1) != 1) or out.device != a.device:
-        raise RuntimeError("out must be an fp32 [M, N] tensor with unit column stride on the operands' device")
+    rounded = out.dtype in (torch.float16, torch.bfloat16) and beta == 0.0
+    if (out.dtype != torch.float32 and not rounded) or tuple(out.shape) != (M, N) or (N > 1 and out.stride(1) != 1) or out.device != a.device:
+        raise RuntimeError("out must be an fp32 [M, N] tensor (fp16 or bf16 with beta = 0) with unit column stride on the operands' device")
     rs = None
     if row_scale is not None:
         rs = row_scale.to(device=a.device, dtype=torch.float32).contiguous().reshape(-1)
@@ -320,11 +322,13 @@ def gemm_nt16(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
     lib = _lib.load()
     with torch.cuda.device(a.device):
         stream = torch.cuda.current_stream(a.device).cuda_stream
-        code = lib.trakhip_gemm_nt16(
-            ctypes.c_void_p(a.data_ptr()), _ld(a), ctypes.c_void_p(b.data_ptr()), _ld(b), _STORE_DTYPES[a.dtype],
-            ctypes.c_void_p(out.data_ptr()), _ld(out), M, N, K, float(alpha), float(beta),
-            ctypes.c_void_p(rs.data_ptr()) if rs is not None else None, ctypes.c_void_p(stream),
-        )
+        operands = (ctypes.c_void_p(a.data_ptr()), _ld(a), ctypes.c_void_p(b.data_ptr()), _ld(b), _STORE_DTYPES[a.dtype])
+        result = (ctypes.c_void_p(out.data_ptr()), _ld(out), M, N, K, float(alpha))
+        tail = (ctypes.c_void_p(rs.data_ptr()) if rs is not None else None, ctypes.c_void_p(stream))
+        if rounded:
+            code = lib.trakhip_gemm_nt16_rounded(*operands, _STORE_DTYPES[out.dtype], *result, *tail)
+        else:
+            code = lib.trakhip_gemm_nt16(*operands, *result, float(beta), *tail)
     _lib.check(code)
     return out
 
@@ -440,8 +444,10 @@ def _inverse_call(a, lambda_reg, normalize, general):
             raise torch.linalg.LinAlgError(
                 f"the matrix is not positive definite and too large (n = {n}) for the general inverse of this library")
         inv = torch.empty((n, n), dtype=torch.float32, device=a.device)
-        mean_abs = torch.zeros(1, dtype=torch.float32, device=a.device)
-        status = torch.zeros(1, dtype=torch.int32, device=a.device)
+        # (the call writes both, except for the empty matrix)
+        new = torch.empty if n else torch.zeros
+        mean_abs = new(1, dtype=torch.float32, device=a.device)
+        status = new(1, dtype=torch.int32, device=a.device)
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=a.device)
         stream = torch.cuda.current_stream(a.device).cuda_stream
         code = run(
