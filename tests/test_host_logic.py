@@ -1,4 +1,5 @@
 """Host-side mirror of the reference's projector helpers (no GPU needed)."""
+import numpy as np
 import pytest
 import torch
 
@@ -95,3 +96,35 @@ def test_chunked_projector_bookkeeping_with_a_fake_chunk_projector():
     assert torch.allclose(out, torch.full((2, 4), 2 * 11.0 + 10 * 2 * 20.0))
     proj.free_memory()
     assert not proj.input_allocated
+
+
+def test_out_to_loss_sums_in_half_precision_are_numpys():
+    import warnings
+
+    from trak_amd.score_computers import _add_half, _row_factors, _store_rows
+
+    every = np.arange(1 << 16, dtype=np.uint32).astype(np.uint16).view(np.float16)      # subnormals, infinities, NaN
+    rng = np.random.default_rng(0)
+    same = lambda a, b: np.array_equal(a, b, equal_nan=True) and np.array_equal(np.signbit(a[a == 0]), np.signbit(b[b == 0]))
+    with warnings.catch_warnings(), np.errstate(all="ignore"):
+        warnings.simplefilter("ignore")
+        for values in (rng.permutation(every), (rng.standard_normal(1 << 16) * 1e-3).astype(np.float32),
+                       (10.0 ** rng.uniform(-9, 6, 1 << 16)).astype(np.float32)):
+            got, want = every.copy().reshape(-1, 1), every.copy().reshape(-1, 1)
+            values = values.reshape(-1, 1)
+            values.flags.writeable = False                                                # as a store opened for reading gives them
+            _add_half(got, values)
+            want += values
+            assert got.dtype == np.float16 and same(got, want)
+        for n in (1.0, 2.0, 3.0, 7.0, 50.0, 2049.0, 65504.0, 70000.0):
+            for sums in (every.reshape(-1, 1), rng.standard_normal((1000, 1)).astype(np.float32)):
+                got = _row_factors(sums.copy(), n)
+                assert got.dtype == np.float32 and same(got, (sums / n).astype(np.float32))
+    src = torch.arange(12.0).reshape(3, 4)
+    for out in (np.zeros((5, 4), np.float32), np.zeros((5, 8), np.float32)[:, ::2], np.zeros((5, 4), np.float32)[:, ::-1]):
+        _store_rows(out, 1, 4, src)
+        assert np.array_equal(out[1:4], src.numpy()) and not out[[0, 4]].any()
+    fixed = np.zeros((5, 4), np.float32)
+    fixed.flags.writeable = False
+    with pytest.raises(ValueError):
+        _store_rows(fixed, 1, 4, src)

@@ -8,6 +8,7 @@ running the three GEMMs and the regularized inverse on the GPU through libtrakhi
 import logging
 from abc import ABC, abstractmethod
 
+import numpy as np
 import torch
 from torch import Tensor
 
@@ -234,17 +235,35 @@ class BasicScoreComputer(AbstractScoreComputer):
         return gemm_nt(a, b, out=out, alpha=alpha, beta=beta, row_scale=row_scale)
 
 
-_COPY_THREADS = 4
-_pool = None
+# The out_to_loss sums in half precision, in the arithmetic of numpy (values widened to fp32, one operation, rounded back),
+# by torch: its conversions are vectorized and threaded (50 000 values: 124 -> 24 us the sum, 206 -> 38 us the quotient,
+# both between a user's call and the launch that needs them).
 
 
-def _copy_pool():
-    global _pool
-    if _pool is None:
-        from concurrent.futures import ThreadPoolExecutor
+def _add_half(sums, values):
+    """sums += values for a float16 array and one of float16 or float32 of its shape."""
+    if not values.flags.writeable:
+        values = values.copy()  # (torch wants to be able to write)
+    t = ch.from_numpy(sums)
+    t.copy_(t.float().add_(ch.from_numpy(np.ascontiguousarray(values))))
 
-        _pool = ThreadPoolExecutor(_COPY_THREADS)
-    return _pool
+
+def _row_factors(sums, n):
+    """(sums / n).astype(np.float32) for a contiguous array of float16 or float32."""
+    if sums.dtype != np.float16:
+        return (sums / n).astype(np.float32)
+    with np.errstate(over="ignore"):
+        divisor = float(np.float16(n))  # a Python number meets an array in the array's type
+    return (ch.from_numpy(sums).float() / divisor).half().float().numpy()
+
+
+def _store_rows(out, r0, r1, src):
+    """out[r0:r1] = src (a CPU tensor): by torch's threads, one thread copies less than half of what PCIe delivers."""
+    dst = out[r0:r1]
+    if dst.flags.writeable and all(s >= 0 for s in dst.strides):
+        ch.from_numpy(dst).copy_(src)
+    else:
+        dst[...] = src.numpy()
 
 
 class ScoreAccumulator:
@@ -267,9 +286,6 @@ class ScoreAccumulator:
     """
 
     def __init__(self, score_computer, train_set_size, num_targets, dtype=ch.float32):
-        import numpy as np
-
-        self._np = np
         self.score_computer = score_computer
         self.shape = (int(train_set_size), int(num_targets))
         self.dtype = dtype
@@ -283,20 +299,23 @@ class ScoreAccumulator:
         """One checkpoint: sums += features @ target_grads^T (trak/traker.py:667) and
         out_to_loss sums += out_to_loss (trak/traker.py:670)."""
         self.score_computer.get_scores(features, target_grads, accumulator=self._acc)
-        o = out_to_loss.detach().cpu().numpy() if isinstance(out_to_loss, Tensor) else self._np.asarray(out_to_loss)
-        self._out_to_loss += o.reshape(self.shape[0], 1)
+        o = out_to_loss.detach().cpu().numpy() if isinstance(out_to_loss, Tensor) else np.asarray(out_to_loss)
+        o = o.reshape(self.shape[0], 1)
+        if self._out_to_loss.dtype == np.float16 and o.dtype in (np.float16, np.float32):
+            _add_half(self._out_to_loss, o)
+        else:
+            self._out_to_loss += o
         self.num_models += 1
 
     def finalize(self, out, chunk_bytes: int = 256 << 20):
         """Writes `(sums / n) * (out_to_loss sums / n)` (trak/traker.py:674-676) into `out`, the
         [N, M] array behind the saver's `<exp>_scores` store (numpy array or memmap of float16 or
         float32) or a tensor (CUDA, or page-locked CPU).  Returns `out`."""
-        np = self._np
         if self.num_models == 0:
             raise ValueError("no checkpoint was added")
         n = float(self.num_models)
         # the second factor exactly as numpy computes it in the reference, then widened (exact)
-        row_factor = (self._out_to_loss / n).astype(np.float32).reshape(-1)
+        row_factor = _row_factors(self._out_to_loss, n).reshape(-1)
         row_factor = ch.from_numpy(row_factor).to(self._acc.device)
         N, M = self.shape
         if isinstance(out, Tensor):
@@ -307,8 +326,10 @@ class ScoreAccumulator:
         if tuple(out.shape) != (N, M) or out.dtype not in (np.float16, np.float32):
             raise ValueError(f"out must be a [{N}, {M}] array of float16 or float32")
         tdtype = ch.float16 if out.dtype == np.float16 else ch.float32
-        rows = max(1, min(N, int(chunk_bytes) // max(1, M * out.dtype.itemsize)))
-        stage = [ch.empty((rows, M), dtype=tdtype).pin_memory() for _ in range(2 if rows < N else 1)]
+        row_bytes = max(1, M * out.dtype.itemsize)
+        # four chunks of at least 1 MB or more of them: the copy of one into the store passes under the next one's crossing
+        rows = max(1, min(N, int(chunk_bytes) // row_bytes, max(-(-N // 4), (1 << 20) // row_bytes)))
+        stage = [ch.empty((rows, M), dtype=tdtype, pin_memory=True) for _ in range(2 if rows < N else 1)]
         pending = [None] * len(stage)
         stream = ch.cuda.current_stream(self._acc.device)
 
@@ -317,12 +338,7 @@ class ScoreAccumulator:
                 return
             event, r0, r1 = pending[i]
             event.synchronize()
-            # one thread copies about 30 GB/s, less than the 55 GB/s the kernel delivers over PCIe:
-            # the copy into the store is spread over a few threads (numpy releases the GIL in it)
-            src = stage[i][: r1 - r0].numpy()
-            step = -(-(r1 - r0) // _COPY_THREADS)
-            parts = [(a, min(r1 - r0, a + step)) for a in range(0, r1 - r0, step)]
-            list(_copy_pool().map(lambda ab: out.__setitem__(slice(r0 + ab[0], r0 + ab[1]), src[ab[0] : ab[1]]), parts))
+            _store_rows(out, r0, r1, stage[i][: r1 - r0])
             pending[i] = None
 
         for index, r0 in enumerate(range(0, N, rows)):
