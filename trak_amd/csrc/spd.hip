@@ -10,8 +10,8 @@
 //      (L_jj) and inverts it; the panel below it is  W[j+1:, j] * L_jj^-T  and the trailing
 //      matrix gets  W -= panel * panel^T   (MFMA products; the trailing update and the next
 //      diagonal block share one launch, see spd_step_kernel);
-//   3. L^-1 by recursive halving: inv([[A,0],[B,C]]) = [[A^-1,0],[-C^-1 B A^-1, C^-1]]
-//      (two products per node of the recursion tree);
+//   3. L^-1 by rows of blocks beside the factorization (n <= 4096; see sum_tile), or afterwards by recursive halving:
+//      inv([[A,0],[B,C]]) = [[A^-1,0],[-C^-1 B A^-1, C^-1]] (two products per node of the recursion tree);
 //   4. inverse = L^-T L^-1 (one product), then the mean of |.| by a two-stage reduction in a
 //      fixed order and a scaling pass (the products of 3 and 4: tri_product_kernel).
 #include <hip/hip_runtime.h>
@@ -27,6 +27,8 @@
 namespace {
 
 constexpr int NB = 128;
+constexpr uint64_t kStepTiles = 512;  // tiles of a trailing update that share a launch with the next diagonal block
+constexpr uint64_t kStepBlocks = 32;  // n = 4096: blocks a side up to which every step's update has at most that many
 constexpr int kSumBlocks = 1024;
 
 // W = A + lambda I padded with an identity block, the 128-blocks on and below the diagonal only: nothing above them
@@ -442,25 +444,189 @@ __global__ __launch_bounds__(kDiagThreads, 2) void spd_diag_kernel(const float* 
     diag_block(W, ldw, Lout, Linv_out, ldl, block_index, status, nullptr, 0, lds);
 }
 
+// ---- the inverse of the factor, a row of blocks per step ------------------------------------------------------
+//
+// X = L^-1 grows with the factorization: row p is  X[p][c] = -X_pp T_c,  T_c = sum over m = c .. p - 1 of L[p][m] X[m][c].  The
+// sums need rows of X and L that are there before block (p, p) is factored, so they run in the same launch as it, on CUs
+// that the trailing update leaves idle (its tiles get fewer as the sums get longer); the product with X_pp runs beside the
+// next panel.  Against L^-1 by recursive halving behind the factorization (two launches per depth, 27 us at n = 512, 104 at
+// 2048, 346 at 4096) one launch of 6 us is left and the steps are as long as before up to n = 2048 (22 us).  Whole call: 256
+// 122 -> 93 us, 512 220 -> 153, 2048 804 -> 534, 4096 1910 -> 1562, of which the panels of the diagonal block gave two fifths.
+
+// T tile: 32 rows x 64 columns, tile number = 4 (column group) + row group; eight waves = two 32 x 32 parts x four
+// quarters of every 128 values of k, whose sums are added up at the end.  Two chunks of 128 k in flight in registers.
+constexpr int kSumRows = 32, kSumCols = 64;
+constexpr int kSumPitchA = NB + 4, kSumPitchB = kSumCols + 8;  // conflict-free 16-byte reads; half-waves in other banks
+constexpr int kSumFloats = kSumRows * kSumPitchA + NB * kSumPitchB;
+
+__device__ __forceinline__ void sum_tile(const float* __restrict__ L, const float* __restrict__ Li, float* __restrict__ T,
+                                         uint64_t np, uint32_t p, uint32_t tile, float* __restrict__ lds) {
+    const uint32_t row0 = p * NB + kSumRows * (tile & 3), col0 = kSumCols * (tile >> 2), c = col0 / NB;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, x = lane & 31, h = lane >> 5;
+    const int wk = wave >> 1, wn = wave & 1;
+    constexpr int kA = kSumRows * (NB / 4) / kDiagThreads, kB = NB * (kSumCols / 4) / kDiagThreads;
+    const float* a0 = L + (uint64_t)row0 * np + (uint64_t)c * NB;
+    const float* b0 = Li + (uint64_t)c * NB * np + col0;
+    const uint32_t count = p - c;
+    floatx4 ra[2][kA], rb[2][kB];
+    auto load = [&](uint32_t i, int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < kA; ++e) {
+            const int id = tid + kDiagThreads * e;
+            ra[u][e] = *reinterpret_cast<const floatx4*>(a0 + (uint64_t)(id >> 5) * np + i * NB + 4 * (id & 31));
+        }
+#pragma unroll
+        for (int e = 0; e < kB; ++e) {
+            const int id = tid + kDiagThreads * e;
+            rb[u][e] = *reinterpret_cast<const floatx4*>(b0 + ((uint64_t)i * NB + (id >> 4)) * np + 4 * (id & 15));
+        }
+    };
+    load(0, 0);
+    if (count > 1) load(1, 1);
+    floatx16 acc[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
+    auto chunk = [&](uint32_t i, auto u_const) __attribute__((always_inline)) {
+        constexpr int u = decltype(u_const)::value;
+        // a buffer is written again two chunks later, behind the barrier that follows its reads
+        float* as = lds + u * kSumFloats;
+        float* bs = as + kSumRows * kSumPitchA;
+#pragma unroll
+        for (int e = 0; e < kA; ++e) {
+            const int id = tid + kDiagThreads * e;
+            *reinterpret_cast<floatx4*>(as + (id >> 5) * kSumPitchA + 4 * (id & 31)) = ra[u][e];
+        }
+#pragma unroll
+        for (int e = 0; e < kB; ++e) {
+            const int id = tid + kDiagThreads * e;
+            *reinterpret_cast<floatx4*>(bs + (id >> 4) * kSumPitchB + 4 * (id & 15)) = rb[u][e];
+        }
+        if (i + 2 < count) load(i + 2, u);
+        __syncthreads();
+        floatx4 fa[4], fb[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = 32 * wk + 8 * q + 4 * h;
+            fa[q] = *reinterpret_cast<const floatx4*>(as + x * kSumPitchA + k);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) fb[q][t] = bs[(k + t) * kSumPitchB + 32 * wn + x];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all reads of the chunk in flight before its first MFMA waits
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                acc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][t], fb[q][t], acc[q & 1], 0, 0, 0);
+    };
+    for (uint32_t i = 0; i < count; i += 2) {
+        chunk(i, std::integral_constant<int, 0>{});
+        if (i + 1 < count) chunk(i + 1, std::integral_constant<int, 1>{});
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) lds[(wave * 16 + r) * 64 + lane] = acc[0][r] + acc[1][r];
+    __syncthreads();
+    float* out = T + (uint64_t)row0 * np + col0 + 32 * wn + x;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {  // registers 4 wk .. 4 wk + 3 of the four quarters' sums
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) v += lds[((2 * w + wn) * 16 + 4 * wk + r) * 64 + lane];
+        out[(uint64_t)(8 * wk + 4 * h + r) * np] = v;
+    }
+}
+
+// Launch between two steps: workgroups 0 .. panel_tiles - 1 the panel below diagonal block j, 32 rows each,
+// L[j+1:, j] = W[j+1:, j] X_jj^T; the others row j of X, 32 columns each, X[j][c] = -X_jj T_c.
+constexpr int kXPitchB = 32 + 8;
+constexpr int kXFloats = NB * (NB + 4) + NB * kXPitchB;
+constexpr int kPanelLdsFloats = kXFloats > short_k::lds_floats<32>() ? kXFloats : short_k::lds_floats<32>();
+
+__global__ __launch_bounds__(256, 1) void spd_panel_kernel(const float* __restrict__ W, float* __restrict__ L,
+                                                           float* __restrict__ Li, uint64_t np, uint32_t j,
+                                                           uint32_t panel_tiles) {
+    __shared__ __attribute__((aligned(16))) float lds[kPanelLdsFloats];
+    const uint64_t diag = (uint64_t)j * NB * np + (uint64_t)j * NB;
+    if (blockIdx.x < panel_tiles) {
+        const uint64_t below = diag + NB * np;
+        short_k::tile<32>(W + below, np, Li + diag, np, L + below, np, np - (j + 1) * NB, NB, NB, 1.0f, 0.0f, blockIdx.x, 0,
+                          lds);
+        return;
+    }
+    const uint32_t col0 = 32 * (blockIdx.x - panel_tiles);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, x = lane & 31, h = lane >> 5;
+    const float* A = Li + diag;                              // X_jj, zero above its diagonal
+    const float* B = W + (uint64_t)j * NB * np + col0;       // T
+    floatx4 ra[16], rb[4];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int id = tid + 256 * i;
+        ra[i] = *reinterpret_cast<const floatx4*>(A + (uint64_t)(id >> 5) * np + 4 * (id & 31));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int id = tid + 256 * i;
+        rb[i] = *reinterpret_cast<const floatx4*>(B + (uint64_t)(id >> 3) * np + 4 * (id & 7));
+    }
+    float* as = lds;
+    float* bs = lds + NB * (NB + 4);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int id = tid + 256 * i;
+        *reinterpret_cast<floatx4*>(as + (id >> 5) * (NB + 4) + 4 * (id & 31)) = ra[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int id = tid + 256 * i;
+        *reinterpret_cast<floatx4*>(bs + (id >> 3) * kXPitchB + 4 * (id & 7)) = rb[i];
+    }
+    __syncthreads();
+    floatx16 acc[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
+    for (int k0 = 0; k0 <= 32 * wave; k0 += 32) {  // rows 32 wave .. + 31 of a lower triangular operand
+        floatx4 fa[4], fb[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = k0 + 8 * q + 4 * h;
+            fa[q] = *reinterpret_cast<const floatx4*>(as + (32 * wave + x) * (NB + 4) + k);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) fb[q][t] = bs[(k + t) * kXPitchB + x];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                acc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][t], fb[q][t], acc[q & 1], 0, 0, 0);
+    }
+    float* out = Li + ((uint64_t)j * NB + 32 * wave) * np + col0 + x;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) out[(uint64_t)mfma_row(r, h) * np] = -(acc[0][r] + acc[1][r]);
+}
+
 // One step of the factorization in one launch, after the panel below diagonal block j is known:
 // workgroup 0 takes the next diagonal block (j+1, j+1) - its own trailing update, then factor and
-// inverse - while workgroups 1 .. T-1 apply the trailing update W -= panel panel^T to the other
-// lower-triangle tiles (tile numbers in the triangle's row-by-row order; number 0 is that diagonal
-// block).  Nothing in the launch depends on anything else in it, and the 21-28 us of the sequential
-// diagonal work no longer sit between two launches but beside the trailing update.
-//   Wt    trailing matrix, block (j+1, j+1) at its origin;  panel  L[j+1:, j] (rows x 128, pitch np)
-__global__ __launch_bounds__(kDiagThreads, 2) void spd_step_kernel(float* __restrict__ Wt, const float* __restrict__ panel,
-                                                          uint64_t np, uint64_t rows, float* __restrict__ Lout,
-                                                          float* __restrict__ Linv_out, int32_t block_index,
-                                                          int32_t* __restrict__ status) {
+// inverse - the next 8 (j+1) the sums T for row j+1 of X, and the others apply the trailing update W -= panel panel^T to
+// the other lower-triangle tiles (tile numbers in the triangle's row-by-row order; number 0 is that diagonal
+// block).  Nothing in the launch depends on anything else in it: the sequential diagonal work does not sit between two
+// launches but beside the trailing update and the sums.  T takes the place of W[j+1][0 .. j], which the panels have read.
+__global__ __launch_bounds__(kDiagThreads, 2) void spd_step_kernel(float* __restrict__ W, float* __restrict__ L,
+                                                                   float* __restrict__ Li, uint64_t np, uint32_t j,
+                                                                   uint32_t sum_tiles, int32_t* __restrict__ status) {
     constexpr int kLds = kDiagLdsFloats > short_k::lds_floats<NB>() ? kDiagLdsFloats : short_k::lds_floats<NB>();
+    static_assert(2 * kSumFloats <= kLds && 8 * 16 * 64 <= kLds, "the sums' buffers");
     __shared__ __attribute__((aligned(16))) float lds[kLds];
+    const uint64_t tr = (uint64_t)(j + 1) * NB * np + (uint64_t)(j + 1) * NB, rows = np - (uint64_t)(j + 1) * NB;
+    const float* panel = L + tr - NB;  // L[j+1:, j]
     if (blockIdx.x == 0) {
-        diag_block(Wt, np, Lout, Linv_out, np, block_index, status, panel, np, lds);
+        diag_block(W + tr, np, L + tr, Li + tr, np, (int32_t)(j + 1), status, panel, np, lds);
+    } else if (blockIdx.x <= sum_tiles) {
+        sum_tile(L, Li, W, np, j + 1, blockIdx.x - 1, lds);
     } else {
         uint32_t tile_m, tile_n;
-        short_k::triangle_tile(blockIdx.x, tile_m, tile_n);
-        short_k::tile<NB, kDiagThreads>(panel, np, panel, np, Wt, np, rows, rows, NB, -1.0f, 1.0f, tile_m, tile_n, lds);
+        short_k::triangle_tile(blockIdx.x - sum_tiles, tile_m, tile_n);
+        short_k::tile<NB, kDiagThreads>(panel, np, panel, np, W + tr, np, rows, rows, NB, -1.0f, 1.0f, tile_m, tile_n, lds);
     }
 }
 
@@ -745,38 +911,52 @@ int spd_inverse(const float* A, uint64_t lda, float lambda, float* inv, uint64_t
                        (uint32_t)np, segments, W, status);
     if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
 
-    // Diagonal block 0 alone; then per block column j: the panel below it, and one launch that holds both
-    // the trailing update and the next diagonal block (spd_step_kernel).  Trailing updates of more than
-    // 512 tiles (n > 4096) go through the general product, with the diagonal block in a launch of its own.
+    // Diagonal block 0 alone; then per block column j: the panel below it with row j of L^-1, and one launch that holds
+    // the trailing update, the next diagonal block and the sums for the next row of L^-1 (spd_step_kernel).  Where there are
+    // more blocks (n > 4096): trailing updates of more than 512 tiles by the general product, with the diagonal block in a
+    // launch of its own, and L^-1 by recursive halving afterwards (the sums would lengthen the steps).
     hipLaunchKernelGGL(spd_diag_kernel, dim3(1), dim3(kDiagThreads), 0, s, W, np, L, Li, np, 0, status);
     if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
-    for (uint64_t j = 0; j + 1 < nblk; ++j) {
-        const uint64_t off = j * NB * np + j * NB;
-        const uint64_t rows = np - (j + 1) * NB, blocks = rows / NB;
-        const uint64_t below = (j + 1) * NB * np + j * NB;
-        const uint64_t tr = (j + 1) * NB * np + (j + 1) * NB;
-        // panel = W[j+1:, j] * (L_jj^-1)^T
-        int e = gemm_nt(W + below, np, Li + off, np, L + below, np, rows, NB, NB, 1.0f, 0.0f, nullptr, s);
-        if (e) return e;
-        const uint64_t tiles = blocks * (blocks + 1) / 2;
-        if (tiles <= 512) {
-            hipLaunchKernelGGL(spd_step_kernel, dim3((uint32_t)tiles), dim3(kDiagThreads), 0, s, W + tr, L + below, np, rows,
-                               L + tr, Li + tr, (int32_t)(j + 1), status);
+    if (nblk <= kStepBlocks) {
+        for (uint32_t j = 0; j + 1 < nblk; ++j) {
+            const uint32_t blocks = (uint32_t)nblk - j - 1, tiles = blocks * (blocks + 1) / 2, sums = 8 * (j + 1);
+            hipLaunchKernelGGL(spd_panel_kernel, dim3(4 * blocks + 4 * j), dim3(256), 0, s, W, L, Li, np, j, 4 * blocks);
+            hipLaunchKernelGGL(spd_step_kernel, dim3(tiles + sums), dim3(kDiagThreads), 0, s, W, L, Li, np, j, sums, status);
             if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
-            continue;
         }
-        // trailing matrix -= panel * panel^T (only the lower triangle of W is ever read)
-        e = gemm_nt(L + below, np, L + below, np, W + tr, np, rows, rows, NB, -1.0f, 1.0f, nullptr, s,
-                    kGemmLowerTilesOnly);
+        if (nblk > 1) {
+            const uint32_t j = (uint32_t)nblk - 1;
+            hipLaunchKernelGGL(spd_panel_kernel, dim3(4 * j), dim3(256), 0, s, W, L, Li, np, j, 0u);
+            if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
+        }
+    } else {
+        for (uint64_t j = 0; j + 1 < nblk; ++j) {
+            const uint64_t off = j * NB * np + j * NB;
+            const uint64_t rows = np - (j + 1) * NB;
+            const uint64_t below = (j + 1) * NB * np + j * NB;
+            const uint64_t tr = (j + 1) * NB * np + (j + 1) * NB;
+            // panel = W[j+1:, j] * (L_jj^-1)^T
+            int e = gemm_nt(W + below, np, Li + off, np, L + below, np, rows, NB, NB, 1.0f, 0.0f, nullptr, s);
+            if (e) return e;
+            const uint64_t blocks = rows / NB, tiles = blocks * (blocks + 1) / 2;
+            if (tiles <= kStepTiles) {
+                hipLaunchKernelGGL(spd_step_kernel, dim3((uint32_t)tiles), dim3(kDiagThreads), 0, s, W, L, Li, np, (uint32_t)j,
+                                   0u, status);
+                if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
+                continue;
+            }
+            // trailing matrix -= panel * panel^T (only the lower triangle of W is ever read)
+            e = gemm_nt(L + below, np, L + below, np, W + tr, np, rows, rows, NB, -1.0f, 1.0f, nullptr, s,
+                        kGemmLowerTilesOnly);
+            if (e) return e;
+            hipLaunchKernelGGL(spd_diag_kernel, dim3(1), dim3(kDiagThreads), 0, s, W + tr, np, L + tr, Li + tr, np,
+                               (int32_t)(j + 1), status);
+            if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
+        }
+        Ctx c = {W, L, Li, np, s};
+        const int e = tri_inverse(c, nblk);
         if (e) return e;
-        hipLaunchKernelGGL(spd_diag_kernel, dim3(1), dim3(kDiagThreads), 0, s, W + tr, np, L + tr, Li + tr, np,
-                           (int32_t)(j + 1), status);
-        if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
     }
-
-    Ctx c = {W, L, Li, np, s};
-    int e = tri_inverse(c, nblk);
-    if (e) return e;
 
     // inverse = Li^T * Li: lower-triangle tiles and their mirror image, so the result is exactly symmetric
     const uint64_t tiles = (n + kTriTile - 1) / kTriTile;
