@@ -478,6 +478,24 @@ def test_gemm_nt16_reads_operands_in_place(gpu, dtype, M, N, K):
     assert torch.equal(wide[:, :N], gemm_nt16(ag, bg)) and bool((wide[:, N:] == -1.0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(100, 127, 64), (129, 130, 192), (1000, 1100, 128),      # 128 x 128 tiles
+                                   (8200, 2100, 2048),                                       # whole rounds of 256 x 256, the rest
+                                   (8192, 2048, 1024), (4100, 4000, 2048)])                  # 256 x 256
+def test_gemm_nt16_has_the_same_bits_on_every_shape_of_tiles(gpu, dtype, M, N, K):
+    gen = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a, b = (torch.randn(r, K, generator=gen, device=gpu).to(dtype) for r in (M, N))
+    rs, c0 = torch.rand(M, generator=gen, device=gpu), torch.randn(M, N, generator=gen, device=gpu)
+    planes = split_rows(a), split_rows(b)                      # the one-plane product: 256 x 256 tiles
+    wide = torch.full((M, N + 5), 7.0, device=gpu)
+    assert torch.equal(gemm_nt16(a, b, out=wide[:, :N]), gemm_nt_split(*planes))
+    assert bool((wide[:, N:] == 7.0).all())
+    got = gemm_nt16(a, b, out=c0.clone(), alpha=0.5, beta=-2.0, row_scale=rs)
+    assert torch.equal(got, gemm_nt_split(*planes, out=c0.clone(), alpha=0.5, beta=-2.0, row_scale=rs))
+    half = torch.empty(M, N, dtype=dtype, device=gpu)
+    assert torch.equal(gemm_nt16(a, b, out=half, row_scale=rs), gemm_nt_split(*planes, row_scale=rs).to(dtype))
+
+
 # columns of tiles: one, two, eight (one band), nine and twelve (two bands), thirteen (row by row)
 @pytest.mark.parametrize("M,N", [(2100, 256), (1300, 300), (700, 2048), (1300, 2309), (520, 3072), (600, 3100), (20, 2500), (5000, 1)])
 def test_products_in_every_order_of_their_tiles(gpu, M, N):

@@ -485,19 +485,29 @@ __device__ __forceinline__ bool xcd_unit(uint32_t units, uint32_t& unit) {
     return unit < (uint32_t)((xcd + 1ull) * units / 8u);
 }
 
-// The same for the grid of tiles of a product with up to kBandedTiles columns of tiles: number `position` of an order in which
-// neighbours share operands.  Up to eight columns are walked row by row, more of them in two bands, and each XCD takes a
-// contiguous eighth of the walk, so that the 32 tiles that an XCD works on at a time are some four rows of eight columns.
+// The same for the grid of tiles of a product: number `position` of an order in which neighbours share operands.  Up to eight
+// columns are walked row by row, more of them in bands of at most eight, and each XCD takes a contiguous eighth of the walk,
+// so that the 32 tiles of 256 x 256 that an XCD works on at a time are some four rows of eight columns.
 // (Row by row over all XCDs, eight columns give each XCD one column of 32 rows: 33 operand panels where 12 would do.)
 // [50 000, 2048] by 2048 columns fp16 441 -> 432 us, 1536 257 -> 245; fp32 2048 1.93 -> 1.89 ms, 2560 2.83 -> 2.71.  With
-// 16 columns the same time, from 24 on 2-9 % slower: row by row, an XCD then has five or more columns of six or fewer rows.
+// 16 columns of 256 the same time, from 24 on 2-9 % slower: row by row, an XCD then has five or more columns of six or fewer rows.
 constexpr uint32_t kBandedTiles = 12;
 __device__ __forceinline__ void banded_tile(uint32_t position, uint32_t tiles_m, uint32_t tiles_n, uint32_t& tile_m,
                                             uint32_t& tile_n) {
     uint32_t first = 0, width = tiles_n;
-    if (tiles_n > 8) {
-        width = tiles_n / 2;
-        if (position >= width * tiles_m) position -= width * tiles_m, first = width, width = tiles_n - width;
+    if (tiles_n > 8) {  // the first `wider` bands have a column more than the others
+        const uint32_t bands = (tiles_n + 7) / 8, wider = tiles_n % bands;
+        uint32_t band;
+        width = tiles_n / bands;
+        if (position < wider * (width + 1) * tiles_m) {
+            ++width;
+            band = position / (width * tiles_m);
+            first = band * width;
+        } else {
+            band = (position - wider * tiles_m) / (width * tiles_m);
+            first = band * width + wider;
+        }
+        position -= first * tiles_m;
     }
     tile_m = position / width;
     tile_n = first + position % width;
@@ -627,13 +637,22 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_split_kernel(
 // of those 256 bytes - rows of equal parity share a 128-byte half and differ in r / 2.  Linear global
 // reads, conflict-free LDS reads (XOR with r % 8 instead leaves a two-way conflict), and the same MFMA loop as
 // the one-plane kernel.  Rows past M or N are fetched from the last row (their results are not stored).
-template <bool F16, bool ACCUM, int OUT = TRAKHIP_F32>
-__global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
+//
+// SmallTile: the same on 128 x 128 tiles of four waves, 64 KB of LDS and two workgroups per CU, for products that leave CUs
+// idle with 256 x 256 tiles and for the rows of one that are left behind whole rounds of tiles over the CUs.
+struct BigTile {
+    static constexpr int kWavesM = 4, kWavesN = 2, JT = 4, BM = 64 * kWavesM, BN = 32 * JT * kWavesN, kWaves = kWavesM * kWavesN;
+};
+struct SmallTile {
+    static constexpr int kWavesM = 2, kWavesN = 2, JT = 2, BM = 64 * kWavesM, BN = 32 * JT * kWavesN, kWaves = kWavesM * kWavesN;
+};
+template <class Shape, bool F16, bool ACCUM, int OUT = TRAKHIP_F32>
+__global__ __launch_bounds__(64 * Shape::kWaves, 2) void gemm_nt16_kernel(
     const piece* __restrict__ A, uint64_t lda8, const piece* __restrict__ B, uint64_t ldb8, uint64_t steps,
     void* __restrict__ C_any, uint64_t ldc, uint64_t M, uint64_t N, float alpha, float beta,
     const float* __restrict__ row_scale, uint32_t tiles_n, uint32_t tiles, uint32_t in_bands, bool vec16) {
-    constexpr int JT = BN / kWavesN / 32;
-    constexpr int kBufPieces = 8 * (BM + BN);  // 64 KB
+    constexpr int BM = Shape::BM, BN = Shape::BN, JT = Shape::JT, kWaves = Shape::kWaves, kWavesN = Shape::kWavesN;
+    constexpr int kBufPieces = 8 * (BM + BN);  // 64 KB, or 32
     constexpr int kMoves = (BM + BN) / 8 / kWaves, kMovesA = BM / 8 / kWaves;  // chunks per wave and step
     __shared__ piece lds[2][kBufPieces];
 
@@ -748,8 +767,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt16_kernel(
                 // compiler waits for all outstanding LDS reads at once (it cannot order them against the
                 // LDS-direct loads), so the next reads are issued after this point and stay in flight under
                 // the MFMAs.
-                asm volatile("" ::"v"(fa[set][0]), "v"(fa[set][1]), "v"(fb[set][0]), "v"(fb[set][1]), "v"(fb[set][2]),
-                             "v"(fb[set][3]));
+                asm volatile("" ::"v"(fa[set][0]), "v"(fa[set][1]), "v"(fb[set][0]), "v"(fb[set][1]));
+                if constexpr (JT == 4) asm volatile("" ::"v"(fb[set][JT - 2]), "v"(fb[set][JT - 1]));
                 __builtin_amdgcn_sched_barrier(0);
                 if (u < 3) {
                     fetch(cur, u + 1, set ^ 1);
@@ -1129,6 +1148,64 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
     return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
 }
 
+// C = alpha A B^T + beta C of 16-bit operands in place on one shape of tiles; `slots` workgroups at a time
+template <class Shape>
+int launch_nt16(const char* A, uint64_t lda, const void* B, uint64_t ldb, int dtype, int out_dtype, char* C, uint64_t ldc,
+                uint64_t M, uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, int slots, hipStream_t s) {
+    const uint64_t tiles_m = (M + Shape::BM - 1) / Shape::BM, tiles_n = (N + Shape::BN - 1) / Shape::BN;
+    void (*kernel)(const piece*, uint64_t, const piece*, uint64_t, uint64_t, void*, uint64_t, uint64_t, uint64_t, float,
+                   float, const float*, uint32_t, uint32_t, uint32_t, bool);
+    const bool accum = beta != 0.0f, f16 = dtype == TRAKHIP_F16;
+    if (out_dtype == TRAKHIP_F16)
+        kernel = f16 ? gemm_nt16_kernel<Shape, true, false, TRAKHIP_F16> : gemm_nt16_kernel<Shape, false, false, TRAKHIP_F16>;
+    else if (out_dtype == TRAKHIP_BF16)
+        kernel = f16 ? gemm_nt16_kernel<Shape, true, false, TRAKHIP_BF16> : gemm_nt16_kernel<Shape, false, false, TRAKHIP_BF16>;
+    else if (f16)
+        kernel = accum ? gemm_nt16_kernel<Shape, true, true> : gemm_nt16_kernel<Shape, true, false>;
+    else
+        kernel = accum ? gemm_nt16_kernel<Shape, false, true> : gemm_nt16_kernel<Shape, false, false>;
+    const bool vec16 = reinterpret_cast<uintptr_t>(C) % 8 == 0 && ldc % 4 == 0;  // 8-byte stores of a 16-bit result
+    const uint32_t tiles = (uint32_t)(tiles_m * tiles_n);
+    // (tiles of 128 x 128: twice as many columns, and 64 tiles of an XCD at a time)
+    const bool in_bands = (Shape::BN < 256 ? tiles_n > 1 && tiles_n <= 2 * kBandedTiles : banded(tiles_n)) && slots >= 8;
+    uint32_t workgroups = tiles < (uint32_t)slots ? tiles : (uint32_t)slots;
+    if (in_bands) workgroups = tiles < (uint32_t)slots ? (tiles + 7) / 8 * 8 : (uint32_t)slots / 8 * 8;
+    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(64 * Shape::kWaves), 0, s, reinterpret_cast<const piece*>(A), lda / 8,
+                       static_cast<const piece*>(B), ldb / 8, K / 64, C, ldc, M, N, alpha, beta, row_scale, (uint32_t)tiles_n,
+                       tiles, in_bands ? 1u : 0u, vec16);
+    return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+}
+
+// Rows of a 16-bit product in place that go to 256 x 256 tiles; the others go to 128 x 128: none, all, or those behind as many
+// rows of tiles as make whole rounds over the CUs, whichever estimate is smallest.  Microseconds, per 64 values of k and
+// round of tiles over the CUs: 256 x 256 1.75 and 8.5 for the stores of C (a last round that leaves CUs idle 1.33, up to
+// 1.73 as it fills: the clock), 128 x 128, two per CU, 1.03 and 4.5 (a last round 0.5 to 1.1).  Fitted to 237 products of
+// M = 1000 .. 50 000, N = 1 .. 8000, K = 512 .. 4096: on average 0.2 % above the fastest of the three, at worst 13 %, never
+// more than 2 % slower than 256 x 256 tiles alone and two thirds of their time on average: [50 000 x 2048] by 100 rows
+// 64 -> 43 us, by 2048 427 -> 410, [2000 x 512] by 512 21 -> 13, [4000 x 2048] by 1024 55 -> 28.
+double big_tiles_us(uint64_t M, uint64_t N, uint64_t K, int cus) {
+    if (M == 0) return 0.0;
+    const uint64_t tiles = (M + 255) / 256 * ((N + 255) / 256), full = tiles / cus;
+    const double rest = (double)tiles / cus - (double)full, k = (double)K / 64.0;
+    const double last = 8.0 + k * (1.33 + (rest > 0.5 ? 0.8 * (rest - 0.5) : 0.0));
+    return (double)full * (8.5 + 1.75 * k) + (rest > 0.0 ? last : 0.0);
+}
+double small_tiles_us(uint64_t M, uint64_t N, uint64_t K, int cus) {
+    if (M == 0) return 0.0;
+    const uint64_t tiles = (M + 127) / 128 * ((N + 127) / 128), full = tiles / (2 * cus);
+    const double rest = (double)tiles / (2 * cus) - (double)full, k = (double)K / 64.0;
+    return (double)full * (4.5 + 1.03 * k) + (rest > 0.0 ? 5.0 + k * (0.5 + 0.6 * rest) : 0.0);
+}
+uint64_t big_tile_rows(uint64_t M, uint64_t N, uint64_t K, int cus) {
+    const uint64_t tiles_n = (N + 255) / 256, tiles = (M + 255) / 256 * tiles_n;
+    uint64_t whole = tiles / cus * cus / tiles_n * 256;
+    if (whole > M) whole = M;
+    const double big = big_tiles_us(M, N, K, cus), small = small_tiles_us(M, N, K, cus);
+    const double both = big_tiles_us(whole, N, K, cus) + small_tiles_us(M - whole, N, K, cus) + 1.0;
+    if (whole > 0 && whole < M && both < big && both < small) return whole;
+    return small < big ? 0 : M;
+}
+
 // A symmetric product has (tiles + 1) tiles / 2 workgroups' worth of work; up to 170 of them leave a third of the
 // CUs idle, and the k range is long enough to share out.  The number of shares, up to `most` and to what `room` bytes hold,
 // is the one whose estimate is smallest: rounds of workgroups over the 256 CUs times the steps of a share (1.6 us each,
@@ -1282,34 +1359,21 @@ int gemm_nt16(const void* A, uint64_t lda, const void* B, uint64_t ldb, int dtyp
         (reinterpret_cast<uintptr_t>(C) % (out_dtype == TRAKHIP_F32 ? 4 : 2)))
         return TRAKHIP_ERR_ALIGN;
     if (out_dtype != TRAKHIP_F32 && beta != 0.0f) return TRAKHIP_ERR_SHAPE;
-    const uint64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    if (tiles_m * tiles_n > 0x7FFFFFFFull) return TRAKHIP_ERR_SHAPE;
-    void (*kernel)(const piece*, uint64_t, const piece*, uint64_t, uint64_t, void*, uint64_t, uint64_t, uint64_t, float,
-                   float, const float*, uint32_t, uint32_t, uint32_t, bool);
-    const bool accum = beta != 0.0f;
-    const bool f16 = dtype == TRAKHIP_F16;
-    if (out_dtype == TRAKHIP_F16)
-        kernel = f16 ? gemm_nt16_kernel<true, false, TRAKHIP_F16> : gemm_nt16_kernel<false, false, TRAKHIP_F16>;
-    else if (out_dtype == TRAKHIP_BF16)
-        kernel = f16 ? gemm_nt16_kernel<true, false, TRAKHIP_BF16> : gemm_nt16_kernel<false, false, TRAKHIP_BF16>;
-    else if (f16)
-        kernel = accum ? gemm_nt16_kernel<true, true> : gemm_nt16_kernel<true, false>;
-    else
-        kernel = accum ? gemm_nt16_kernel<false, true> : gemm_nt16_kernel<false, false>;
-    const bool vec16 = reinterpret_cast<uintptr_t>(C) % 8 == 0 && ldc % 4 == 0;  // 8-byte stores of a 16-bit result
-    const uint32_t tiles = (uint32_t)(tiles_m * tiles_n);
-    // persistent workgroups, one per CU (128 KB of LDS each)
+    if (((M + 127) / 128) * ((N + 127) / 128) > 0x7FFFFFF0ull) return TRAKHIP_ERR_SHAPE;
+    // persistent workgroups: one per CU with 256 x 256 tiles (128 KB of LDS each), two with 128 x 128
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
-    const bool in_bands = banded(tiles_n) && cus >= 8;
-    uint32_t workgroups = tiles < (uint32_t)cus ? tiles : (uint32_t)cus;
-    if (in_bands) workgroups = tiles < (uint32_t)cus ? (tiles + 7) / 8 * 8 : (uint32_t)cus / 8 * 8;
-    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(64 * kWaves), 0, s, static_cast<const piece*>(A), lda / 8,
-                       static_cast<const piece*>(B), ldb / 8, K / 64, C, ldc, M, N, alpha, beta, row_scale, (uint32_t)tiles_n,
-                       tiles, in_bands ? 1u : 0u, vec16);
-    return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+    const char* a = static_cast<const char*>(A);
+    char* c = static_cast<char*>(C);
+    const uint64_t big = big_tile_rows(M, N, K, cus);
+    if (big) {
+        const int e = launch_nt16<BigTile>(a, lda, B, ldb, dtype, out_dtype, c, ldc, big, N, K, alpha, beta, row_scale, cus, s);
+        if (e || big == M) return e;
+    }
+    return launch_nt16<SmallTile>(a + 2 * big * lda, lda, B, ldb, dtype, out_dtype, c + big * ldc * (out_dtype == TRAKHIP_F32 ? 4 : 2),
+                                  ldc, M - big, N, K, alpha, beta, row_scale ? row_scale + big : nullptr, 2 * cus, s);
 }
 
 int gram16(const void* X, int dtype, uint64_t ld, uint64_t K, uint64_t N, int out_dtype, void* C, uint64_t ldc, float alpha,
