@@ -496,6 +496,27 @@ def test_gemm_nt16_has_the_same_bits_on_every_shape_of_tiles(gpu, dtype, M, N, K
     assert torch.equal(gemm_nt16(a, b, out=half, row_scale=rs), gemm_nt_split(*planes, row_scale=rs).to(dtype))
 
 
+@pytest.mark.parametrize("M,N,K", [(100, 127, 16), (129, 130, 40), (1000, 1100, 64),       # 128 x 128 tiles
+                                   (8200, 2100, 2048),                                       # whole rounds of 256 x 256, the rest
+                                   (8192, 2048, 256), (4100, 4000, 512)])                    # 256 x 256
+def test_gemm_nt_split_on_every_shape_of_tiles(gpu, M, N, K):
+    gen = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a, b = (torch.randn(r, K, generator=gen, device=gpu) for r in (M, N))
+    rs, c0 = torch.rand(M, generator=gen, device=gpu), torch.randn(M, N, generator=gen, device=gpu)
+    sa, sb = split_rows(a), split_rows(b)
+    want = (a.double() @ b.double().T).cpu()
+    wide = torch.full((M, N + 5), 7.0, device=gpu)
+    assert rel_max(gemm_nt_split(sa, sb, out=wide[:, :N]).cpu().numpy(), want.numpy()) < gemm_tol(K)
+    assert bool((wide[:, N:] == 7.0).all())
+    got = gemm_nt_split(sa, sb, out=c0.clone(), alpha=0.5, beta=-2.0, row_scale=rs)
+    want = (0.5 * want - 2.0 * c0.double().cpu()) * rs.double().cpu()[:, None]
+    assert rel_max(got.cpu().numpy(), want.numpy()) < gemm_tol(K)
+    # a row's sums do not depend on the tiles that hold it
+    few = min(M, 300)
+    assert torch.equal(wide[:few, :N], gemm_nt_split(split_rows(a[:few]), sb))
+    assert torch.equal(wide[M - few:, :N], gemm_nt_split(split_rows(a[M - few:]), sb))
+
+
 # columns of tiles: one, two, eight (one band), nine and twelve (two bands), thirteen (row by row)
 @pytest.mark.parametrize("M,N", [(2100, 256), (1300, 300), (700, 2048), (1300, 2309), (520, 3072), (600, 3100), (20, 2500), (5000, 1)])
 def test_products_in_every_order_of_their_tiles(gpu, M, N):

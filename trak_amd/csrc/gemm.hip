@@ -413,16 +413,13 @@ double one_tile_us(uint64_t M, uint64_t N, uint64_t K) {
     return 5.0 + 6.0e-3 * (double)K * rounds_of(tiles_of(M, N, 32, 32));
 }
 double four_tiles_us(uint64_t M, uint64_t N, uint64_t K) {
-    const double rounds = tiles_of(M, N, 64, 64) / 256.0;
-    return 5.0 + 17.6e-3 * (double)K * (rounds < 1.12 ? 1.12 : rounds);
+    const double tiles = tiles_of(M, N, 64, 64);
+    const double rounds = tiles <= 256.0 ? 1.12 : tiles < 1e15 ? (double)(uint64_t)((tiles + 255.0) / 256.0) : tiles / 256.0;
+    return 5.0 + 17.6e-3 * (double)K * rounds;
 }
-// Both operands split into planes (10 bytes of traffic per value) and their product (gemm_split.hip): 256 x 256 tiles,
-// per 16 values of k 2.1 us for a round on all CUs and 1.7 us for one that leaves some idle (the clock is higher then).
+// Both operands split into planes (10 bytes of traffic per value) and their product (gemm_split.hip).
 double split_us(uint64_t M, uint64_t N, uint64_t K) {
-    const double tiles = tiles_of(M, N, 256, 256);
-    const double full = (double)(uint64_t)(tiles / 256.0);
-    return 25.0 + 2.0e-6 * ((double)M + (double)N) * (double)K +
-           (double)K / 16.0 * (2.1 * full + (tiles > 256.0 * full ? 1.7 : 0.0));
+    return 18.0 + 2.0e-6 * ((double)M + (double)N) * (double)K + trakhip::split_product_us(M, N, K);
 }
 
 template <int WM, int WN, int WK, int DEPTH>

@@ -46,9 +46,20 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef uint32_t piece __attribute__((ext_vector_type(4)));  // 16 bytes = 8 x 16 bit = one lane's MFMA operand
 
-constexpr int kWavesM = 4, kWavesN = 2;            // 4 x 2 waves, each owns 64 x 128 of C
-constexpr int BM = 64 * kWavesM, BN = 128 * kWavesN;
-constexpr int kWaves = kWavesM * kWavesN;
+// Shapes of a workgroup's tile.  BigTile: 4 x 2 waves, each owns 64 x 128 of C.  SmallTile: 2 x 2 waves of 64 x 64, for products
+// that leave CUs idle with the big one and for the rows of a product that are left behind whole rounds of tiles over the CUs;
+// the same MFMAs in the same order, two (16-bit operands in place) or three (three planes) workgroups per CU.
+struct BigTile {
+    static constexpr int kWavesM = 4, kWavesN = 2, JT = 4, BM = 64 * kWavesM, BN = 32 * JT * kWavesN, kWaves = kWavesM * kWavesN;
+    static constexpr int kPerSimd = 2;
+};
+struct SmallTile {
+    static constexpr int kWavesM = 2, kWavesN = 2, JT = 2, BM = 64 * kWavesM, BN = 32 * JT * kWavesN, kWaves = kWavesM * kWavesN;
+    static constexpr int kPerSimd = 3;
+};
+constexpr int kWavesM = BigTile::kWavesM, kWavesN = BigTile::kWavesN;
+constexpr int BM = BigTile::BM, BN = BigTile::BN;
+constexpr int kWaves = BigTile::kWaves;
 constexpr uint32_t kGemmBandedGrid = 4u;            // kernel flag: the grid is numbered as banded_tile says
 constexpr uint32_t kGemmTriangleGrid = 2u;          // kernel flag: the grid lists the lower-triangle tiles only
 constexpr int kRowPad = 256;                       // rows of an operand are padded to this
@@ -426,8 +437,9 @@ __device__ __forceinline__ void store_c16(const floatx16 (&acc)[2][JT], uint16_t
 // to step: the bases live in scalar registers and a load costs two scalar additions.  (Computing the
 // piece address per lane from plane, octet and row took about thirty instructions per load, in front of
 // the MFMAs of every step.)
-template <int P, int S>
+template <int P, int S, class Shape>
 struct StepMover {
+    static constexpr int BM = Shape::BM, BN = Shape::BN, kWaves = Shape::kWaves;
     static constexpr int kAChunks = P * 2 * BM / 64, kBChunks = P * 2 * BN / 64;
     static constexpr int kSubChunks = kAChunks + kBChunks, kChunks = S * kSubChunks;
     // the first kLoaders waves move the chunks: wave w chunks w, w + kLoaders, ...  (all eight: leaving the loads
@@ -516,13 +528,14 @@ bool banded(uint64_t tiles_n) { return tiles_n > 1 && tiles_n <= kBandedTiles; }
 
 // P planes per operand (3: split fp32, 1: a 16-bit type), F16 selects the fp16 MFMA, S sub-steps
 // per barrier.
-template <int P, bool F16, int S, bool ACCUM>
-__global__ __launch_bounds__(64 * kWaves, 2) void gemm_split_kernel(
+template <int P, bool F16, int S, bool ACCUM, class Shape = BigTile>
+__global__ __launch_bounds__(64 * Shape::kWaves, Shape::kPerSimd) void gemm_split_kernel(
     const piece* __restrict__ A, uint64_t Rpa, const piece* __restrict__ B, uint64_t Rpb, uint64_t K8,
     float* __restrict__ C, uint64_t ldc, uint64_t M, uint64_t N, float alpha, float beta,
     const float* __restrict__ row_scale, uint32_t tiles_n, uint32_t flags, const float* __restrict__ a_unscale,
     const float* __restrict__ b_unscale, uint32_t parts, uint64_t part_stride) {
-    constexpr int JT = BN / kWavesN / 32;            // 32-column MFMA tiles per wave
+    constexpr int BM = Shape::BM, BN = Shape::BN, kWavesN = Shape::kWavesN;
+    constexpr int JT = Shape::JT;                    // 32-column MFMA tiles per wave
     constexpr int kAPieces = P * 2 * BM;             // [plane][half][row]
     constexpr int kSubPieces = P * 2 * (BM + BN);    // three planes: 3072 pieces = 48 KB
     constexpr int kBufPieces = S * kSubPieces;
@@ -565,7 +578,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_split_kernel(
 
     const uint64_t all_steps = K8 / (2 * S);
     const uint64_t first = all_steps * part / parts, steps = all_steps * (part + 1) / parts;  // [first, steps)
-    StepMover<P, S> mover;
+    StepMover<P, S, Shape> mover;
     mover.init(A, Rpa, B, Rpb, K8, m0, n0, first, wave);
     const uint32_t lane_bytes = (uint32_t)lane * (uint32_t)sizeof(piece);
     mover.move_all(wave, lane_bytes, lds[0]);
@@ -637,15 +650,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_split_kernel(
 // of those 256 bytes - rows of equal parity share a 128-byte half and differ in r / 2.  Linear global
 // reads, conflict-free LDS reads (XOR with r % 8 instead leaves a two-way conflict), and the same MFMA loop as
 // the one-plane kernel.  Rows past M or N are fetched from the last row (their results are not stored).
-//
-// SmallTile: the same on 128 x 128 tiles of four waves, 64 KB of LDS and two workgroups per CU, for products that leave CUs
-// idle with 256 x 256 tiles and for the rows of one that are left behind whole rounds of tiles over the CUs.
-struct BigTile {
-    static constexpr int kWavesM = 4, kWavesN = 2, JT = 4, BM = 64 * kWavesM, BN = 32 * JT * kWavesN, kWaves = kWavesM * kWavesN;
-};
-struct SmallTile {
-    static constexpr int kWavesM = 2, kWavesN = 2, JT = 2, BM = 64 * kWavesM, BN = 32 * JT * kWavesN, kWaves = kWavesM * kWavesN;
-};
 template <class Shape, bool F16, bool ACCUM, int OUT = TRAKHIP_F32>
 __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gemm_nt16_kernel(
     const piece* __restrict__ A, uint64_t lda8, const piece* __restrict__ B, uint64_t ldb8, uint64_t steps,
@@ -1107,35 +1111,32 @@ int sub_steps(int dtype, bool two_planes) { return two_planes ? 2 : (dtype == TR
 
 // parts > 1 (symmetric products only): the k steps are shared out over `parts` launches' worth of
 // workgroups that write plain sums into `parts` N x N matrices at C; see gram_combine_kernel.
-int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_t N, uint64_t K, int dtype, float* C,
-                 uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags,
-                 const float* a_unscale, const float* b_unscale, uint32_t parts = 1) {
-    if (M == 0 || N == 0) return TRAKHIP_OK;
-    if (K == 0 || ldc < N) return TRAKHIP_ERR_SHAPE;
-    if (!A_planes || !B_planes || !C) return TRAKHIP_ERR_NULL;
-    if ((reinterpret_cast<uintptr_t>(A_planes) % 16) || (reinterpret_cast<uintptr_t>(B_planes) % 16) ||
-        (reinterpret_cast<uintptr_t>(C) % 4))
-        return TRAKHIP_ERR_ALIGN;
-    const uint64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    if (tiles_m * tiles_n > 0x7FFFFFFFull) return TRAKHIP_ERR_SHAPE;
+// Rpa: rows that A's planes are laid out with (M and more, where A is the rest of a taller operand).
+template <class Shape>
+int launch_split_tiles(const piece* a, uint64_t Rpa, uint64_t M, const piece* b, uint64_t N, uint64_t K, int dtype, float* C,
+                       uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags,
+                       const float* a_unscale, const float* b_unscale, uint32_t parts) {
+    const uint64_t tiles_m = (M + Shape::BM - 1) / Shape::BM, tiles_n = (N + Shape::BN - 1) / Shape::BN;
+    if (tiles_m * tiles_n > 0x7FFFFFF0ull) return TRAKHIP_ERR_SHAPE;
     uint64_t workgroups = tiles_m * tiles_n;
     if (parts > 1) {
         flags = kGemmTriangleGrid;
         workgroups = (tiles_m * (tiles_m + 1) / 2 * parts + 7) / 8 * 8;
     }
-    if (parts == 1 && !flags && banded(tiles_n)) {
+    constexpr bool kBig = Shape::BN == BN;
+    if (parts == 1 && !flags && (kBig ? banded(tiles_n) : tiles_n > 1 && tiles_n <= 2 * kBandedTiles)) {
         flags = kGemmBandedGrid;
         workgroups = (workgroups + 7) / 8 * 8;
     }
-    const dim3 grid((uint32_t)workgroups), block(64 * kWaves);
-    const piece* a = static_cast<const piece*>(A_planes);
-    const piece* b = static_cast<const piece*>(B_planes);
-    const uint64_t Rpa = padded_rows(M), Rpb = padded_rows(N), K8 = octets(K);
+    const dim3 grid((uint32_t)workgroups), block(64 * Shape::kWaves);
+    const uint64_t Rpb = padded_rows(N), K8 = octets(K);
     // ACCUM (beta != 0) fetches the old C in the epilogue; kept out of the plain kernel
     void (*kernel)(const piece*, uint64_t, const piece*, uint64_t, uint64_t, float*, uint64_t, uint64_t, uint64_t, float,
                    float, const float*, uint32_t, uint32_t, const float*, const float*, uint32_t, uint64_t);
     const bool accum = beta != 0.0f;
-    if (a_unscale)
+    if constexpr (!kBig)  // three planes only
+        kernel = accum ? gemm_split_kernel<3, false, 1, true, Shape> : gemm_split_kernel<3, false, 1, false, Shape>;
+    else if (a_unscale)
         kernel = accum ? gemm_split_kernel<2, true, 2, true> : gemm_split_kernel<2, true, 2, false>;
     else if (dtype == TRAKHIP_F32)
         kernel = accum ? gemm_split_kernel<3, false, 1, true> : gemm_split_kernel<3, false, 1, false>;
@@ -1146,6 +1147,59 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
     hipLaunchKernelGGL(kernel, grid, block, 0, s, a, Rpa, b, Rpb, K8, C, ldc, M, N, alpha, beta, row_scale,
                        (uint32_t)tiles_n, flags, a_unscale, b_unscale, parts, (uint64_t)N * N);
     return hipGetLastError() == hipSuccess ? TRAKHIP_OK : TRAKHIP_ERR_LAUNCH;
+}
+
+// Rows of a three-plane product that go to 256 x 256 tiles (the others to 128 x 128): as big_tile_rows, microseconds per 16 values
+// of k: 256 x 256 2.12 a round (a last one that leaves CUs idle 1.64, up to 2.1 as it fills), 128 x 128 tiles 0.82 for one on
+// a CU, 1.34 for two side by side, 1.8 for three.  158 products of M = 1000 .. 50 000, N = 100 .. 8000, K = 512 .. 4096: 0.1 %
+// above the fastest of the three on average, 2 % at worst, 28 % below 256 x 256 tiles alone: [4000 x 4096] by 1024 rows 427 ->
+// 210 us, [16 000 x 1024] by 300 117 -> 81, [50 000 x 2048] by 1024 1036 -> 975, [25 000 x 2048] by 4096 1851 -> 1790.
+constexpr uint64_t kPlanCus = 256;
+double big_planes_us(uint64_t M, uint64_t N, uint64_t K) {
+    if (M == 0) return 0.0;
+    const uint64_t tiles = (M + 255) / 256 * ((N + 255) / 256), full = tiles / kPlanCus;
+    const double rest = (double)(tiles % kPlanCus) / (double)kPlanCus, k = (double)K / 16.0;
+    return (double)full * (5.0 + 2.12 * k) + (rest > 0.0 ? 8.0 + k * (1.64 + (rest > 0.5 ? 0.9 * (rest - 0.5) : 0.0)) : 0.0);
+}
+double small_planes_us(uint64_t M, uint64_t N, uint64_t K) {
+    if (M == 0) return 0.0;
+    const uint64_t tiles = (M + 127) / 128 * ((N + 127) / 128), per_cu = (tiles + kPlanCus - 1) / kPlanCus;
+    const double last[3] = {0.0, 0.82, 1.34};
+    return 5.0 + (double)K / 16.0 * (1.8 * (double)(per_cu / 3) + last[per_cu % 3]);
+}
+uint64_t big_plane_rows(uint64_t M, uint64_t N, uint64_t K, double& us) {
+    const uint64_t tiles_n = (N + 255) / 256, tiles = (M + 255) / 256 * tiles_n;
+    uint64_t whole = tiles / kPlanCus * kPlanCus / tiles_n * 256;
+    if (whole > M) whole = M;
+    const double big = big_planes_us(M, N, K), small = small_planes_us(M, N, K);
+    const double both = big_planes_us(whole, N, K) + small_planes_us(M - whole, N, K) + 1.0;
+    if (whole > 0 && whole < M && both < 0.99 * big && both < small) return us = both, whole;
+    return small < big ? (us = small, 0) : (us = big, M);
+}
+
+int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_t N, uint64_t K, int dtype, float* C,
+                 uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags,
+                 const float* a_unscale, const float* b_unscale, uint32_t parts = 1) {
+    if (M == 0 || N == 0) return TRAKHIP_OK;
+    if (K == 0 || ldc < N) return TRAKHIP_ERR_SHAPE;
+    if (!A_planes || !B_planes || !C) return TRAKHIP_ERR_NULL;
+    if ((reinterpret_cast<uintptr_t>(A_planes) % 16) || (reinterpret_cast<uintptr_t>(B_planes) % 16) ||
+        (reinterpret_cast<uintptr_t>(C) % 4))
+        return TRAKHIP_ERR_ALIGN;
+    const piece* a = static_cast<const piece*>(A_planes);
+    const piece* b = static_cast<const piece*>(B_planes);
+    const uint64_t Rpa = padded_rows(M);
+    if (((M + 127) / 128) * ((N + 127) / 128) > 0x7FFFFFF0ull) return TRAKHIP_ERR_SHAPE;
+    const bool three = dtype == TRAKHIP_F32 && !a_unscale && parts == 1 && !flags;
+    double us;
+    const uint64_t big = three ? big_plane_rows(M, N, K, us) : M;
+    if (big) {
+        const int e = launch_split_tiles<BigTile>(a, Rpa, big, b, N, K, dtype, C, ldc, alpha, beta, row_scale, s, flags, a_unscale,
+                                                  b_unscale, parts);
+        if (e || big == M) return e;
+    }
+    return launch_split_tiles<SmallTile>(a + big, Rpa, M - big, b, N, K, dtype, C + big * ldc, ldc, alpha, beta,
+                                         row_scale ? row_scale + big : nullptr, s, 0u, nullptr, nullptr, 1);
 }
 
 // C = alpha A B^T + beta C of 16-bit operands in place on one shape of tiles; `slots` workgroups at a time
@@ -1277,6 +1331,12 @@ int gram_impl(const void* A_planes, const float* a_scales, uint64_t N, uint64_t 
 }  // namespace
 
 namespace trakhip {
+
+double split_product_us(uint64_t M, uint64_t N, uint64_t K) {
+    double us;
+    big_plane_rows(M, N, K, us);
+    return us;
+}
 
 int gemm_nt_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_t N, uint64_t K, int dtype, float* C,
                   uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags) {
