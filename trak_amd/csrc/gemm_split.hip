@@ -865,23 +865,25 @@ __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gemm_nt16_kernel(
 typedef short short4v __attribute__((ext_vector_type(4)));
 
 // rows 4 r + i / 4 of the lane's operand, r = 0, 1 (i = lane % 16)
+template <int kRowBytes>
 __device__ __forceinline__ piece read_transposed(const char* at) {
     typedef __attribute__((address_space(3))) short4v* lds_ptr;
     typedef uint32_t pair __attribute__((ext_vector_type(2)));
-    constexpr int kRowBytes = 2 * BM;
     const pair a = __builtin_bit_cast(pair, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at)));
     const pair b = __builtin_bit_cast(pair, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(at + 4 * kRowBytes)));
     return piece{a[0], a[1], b[0], b[1]};
 }
 
-template <bool F16, bool ACCUM>
-__global__ __launch_bounds__(64 * kWaves, 2) void gram16_kernel(const char* __restrict__ X, uint64_t ld, uint64_t K,
+template <class Shape, bool F16, bool ACCUM>
+__global__ __launch_bounds__(64 * Shape::kWaves, 2) void gram16_kernel(const char* __restrict__ X, uint64_t ld, uint64_t K,
                                                                 uint64_t N, float* __restrict__ C, uint64_t ldc, float alpha,
                                                                 float beta, uint32_t parts, uint64_t part_stride) {
-    constexpr int JT = BN / kWavesN / 32;
-    constexpr int kStep = 64, kRowBytes = 2 * BM, kOperandBytes = kStep * kRowBytes;  // 32 KB
+    constexpr int BM = Shape::BM, BN = Shape::BN, JT = Shape::JT, kWaves = Shape::kWaves, kWavesN = Shape::kWavesN;
+    constexpr int kStep = 64, kRowBytes = 2 * BM, kOperandBytes = kStep * kRowBytes;  // 32 KB, or 16
     static_assert(BM == BN, "both operands are columns of X");
-    constexpr int kMoves = kOperandBytes / 1024 / kWaves;  // loads of two rows per wave, step and operand
+    constexpr int kMoves = kOperandBytes / 1024 / kWaves;    // loads per wave, step and operand
+    constexpr int kLoadRows = 1024 / kRowBytes, kRowSlots = 64 / kLoadRows;  // rows of a load, 16-byte pieces of a row
+    static_assert(kLoadRows * kWaves == 16 && kMoves == 4, "load i of a wave: 16 i rows further down");
     __shared__ __attribute__((aligned(16))) char lds[2][2 * kOperandBytes];
 
     const uint32_t tiles = (uint32_t)((N + BM - 1) / BM), lower = tiles * (tiles + 1) / 2;
@@ -907,8 +909,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gram16_kernel(const char* __re
     const uint64_t all_steps = (K + kStep - 1) / kStep;
     const uint64_t first = all_steps * part / parts, steps = all_steps * (part + 1) / parts;  // [first, steps)
 
-    // load i of a wave: rows 16 i + 2 wave + lane / 32 of the step; the lane's slot holds piece `from` of its row
-    const int row = 2 * wave + h, slot = lane & 31;
+    // load i of a wave: rows 16 i + kLoadRows wave .. of the step; the lane's slot holds piece `from` of its row
+    const int row = kLoadRows * wave + lane / kRowSlots, slot = lane % kRowSlots;
     const uint32_t from = 8u * (uint32_t)(4 * ((slot >> 2) ^ (row & 3)) + (slot & 3));  // first column of the piece
     const uint64_t last_m = N - 8 - m0, last_n = N - 8 - n0;
     const uint32_t a_from = from < last_m ? from : (uint32_t)last_m, b_from = from < last_n ? from : (uint32_t)last_n;
@@ -949,9 +951,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gram16_kernel(const char* __re
     auto fetch = [&](int buf, int u, int set) {
         const char* l = lds[buf] + 16 * u * kRowBytes;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) fa[set][i] = read_transposed(l + a_at[i]);
+        for (int i = 0; i < 2; ++i) fa[set][i] = read_transposed<kRowBytes>(l + a_at[i]);
 #pragma unroll
-        for (int j = 0; j < JT; ++j) fb[set][j] = read_transposed(l + b_at[j]);
+        for (int j = 0; j < JT; ++j) fb[set][j] = read_transposed<kRowBytes>(l + b_at[j]);
     };
 
     dma(first, lds[0]);
@@ -966,7 +968,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gram16_kernel(const char* __re
         for (int u = 0; u < 4; ++u) {
             const int set = u & 1;
             // the fragments of this sub-step are waited for here, before the next ones are requested (see gemm_nt16_kernel)
-            asm volatile("" ::"v"(fa[set][0]), "v"(fa[set][1]), "v"(fb[set][0]), "v"(fb[set][1]), "v"(fb[set][2]), "v"(fb[set][3]));
+            asm volatile("" ::"v"(fa[set][0]), "v"(fa[set][1]), "v"(fb[set][0]), "v"(fb[set][1]));
+            if constexpr (JT == 4) asm volatile("" ::"v"(fb[set][JT - 2]), "v"(fb[set][JT - 1]));
             __builtin_amdgcn_sched_barrier(0);
             if (u < 3) {
                 fetch(cur, u + 1, set ^ 1);
@@ -1223,6 +1226,21 @@ uint64_t big_plane_rows(uint64_t M, uint64_t N, uint64_t K, double& us) {
     return small < big ? (us = small, 0) : (us = big, M);
 }
 
+// Whether a symmetric product in `parts` shares takes 128 x 128 tiles: with N <= 768 the lower tiles of 256 x 256 are three or six
+// a share, and sixteen shares leave most CUs idle.  Three planes: the estimate of big_plane_rows per share; 16-bit rows in place
+// 0.9 us a step for a small tile on a CU and 1.3 for two (they bring twice the rows per entry).  [50 000, 512] fp32 372 -> 206 us
+// and fp16 89 -> 54, [2000, 512] 36 -> 30 and 25 -> 20; [50 000, 1024] fp16 stays at 103 (121 on 128 x 128).
+bool gram_small_tiles(uint64_t N, uint64_t K, int dtype, uint32_t parts) {
+    const uint64_t big = (N + 255) / 256, small = (N + 127) / 128;
+    const uint64_t big_tiles = big * (big + 1) / 2 * parts, small_tiles = small * (small + 1) / 2 * parts;
+    const uint64_t rounds = (big_tiles + kPlanCus - 1) / kPlanCus, per_cu = (small_tiles + kPlanCus - 1) / kPlanCus;
+    const double three[3] = {0.0, 0.82, 1.34}, two[2] = {0.0, 0.9};
+    const double steps = (double)K / (dtype == TRAKHIP_F32 ? 16.0 : 64.0) / (double)parts;
+    const double per_step = dtype == TRAKHIP_F32 ? 1.8 * (double)(per_cu / 3) + three[per_cu % 3]
+                                                 : 1.3 * (double)(per_cu / 2) + two[per_cu % 2];
+    return 5.0 + steps * per_step < (double)rounds * (6.0 + 1.6 * steps);
+}
+
 int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_t N, uint64_t K, int dtype, float* C,
                  uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags,
                  const float* a_unscale, const float* b_unscale, uint32_t parts = 1) {
@@ -1236,6 +1254,8 @@ int launch_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_
     const piece* b = static_cast<const piece*>(B_planes);
     const uint64_t Rpa = padded_rows(M);
     if (((M + 127) / 128) * ((N + 127) / 128) > 0x7FFFFFF0ull) return TRAKHIP_ERR_SHAPE;
+    if (parts > 1 && dtype == TRAKHIP_F32 && !a_unscale && gram_small_tiles(N, K, dtype, parts))
+        return launch_split_tiles<SmallTile>(a, Rpa, M, b, N, K, dtype, C, ldc, alpha, beta, row_scale, s, 0u, nullptr, nullptr, parts);
     const bool three = dtype == TRAKHIP_F32 && !a_unscale && parts == 1 && !flags;
     double us;
     const uint64_t big = three ? big_plane_rows(M, N, K, us) : M;
@@ -1493,19 +1513,26 @@ int gram16(const void* X, int dtype, uint64_t ld, uint64_t K, uint64_t N, int ou
     const bool wide = out_dtype == TRAKHIP_F32;
     if ((reinterpret_cast<uintptr_t>(X) % 16) || (reinterpret_cast<uintptr_t>(C) % (wide ? 4 : 8))) return TRAKHIP_ERR_ALIGN;
     if (!wide && (ldc % 4 || beta != 0.0f)) return TRAKHIP_ERR_SHAPE;
-    const uint64_t tiles = (N + BM - 1) / BM, lower = tiles * (tiles + 1) / 2;
     const bool usable = ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0;
     const uint32_t parts = usable ? gram_parts(N, K, dtype, false, kGramPartsMax, ws_bytes) : 1;
     // a 16-bit result is rounded by the pass behind the product, which needs the sums in scratch
     const bool scratch = parts > 1 || !wide;
     if (scratch && !(usable && ws_bytes / sizeof(float) / N >= N * parts)) return TRAKHIP_ERR_WORKSPACE;
+    const bool small = gram_small_tiles(N, K, dtype, parts);
+    const uint64_t tiles = small ? (N + SmallTile::BM - 1) / SmallTile::BM : (N + BM - 1) / BM, lower = tiles * (tiles + 1) / 2;
     if (lower * parts > 0x7FFFFFF0ull) return TRAKHIP_ERR_SHAPE;
     float* sums = scratch ? static_cast<float*>(ws) : static_cast<float*>(C);
-    const bool accum = !scratch && beta != 0.0f;
-    auto kernel = dtype == TRAKHIP_F16 ? (accum ? gram16_kernel<true, true> : gram16_kernel<true, false>)
-                                       : (accum ? gram16_kernel<false, true> : gram16_kernel<false, false>);
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)((lower * parts + 7) / 8 * 8)), dim3(64 * kWaves), 0, s, static_cast<const char*>(X), ld, K, N,
-                       sums, scratch ? N : ldc, scratch ? 1.0f : alpha, scratch ? 0.0f : beta, parts, (uint64_t)N * N);
+    const bool accum = !scratch && beta != 0.0f, f16 = dtype == TRAKHIP_F16;
+    void (*kernel)(const char*, uint64_t, uint64_t, uint64_t, float*, uint64_t, float, float, uint32_t, uint64_t);
+    if (small)
+        kernel = f16 ? (accum ? gram16_kernel<SmallTile, true, true> : gram16_kernel<SmallTile, true, false>)
+                     : (accum ? gram16_kernel<SmallTile, false, true> : gram16_kernel<SmallTile, false, false>);
+    else
+        kernel = f16 ? (accum ? gram16_kernel<BigTile, true, true> : gram16_kernel<BigTile, true, false>)
+                     : (accum ? gram16_kernel<BigTile, false, true> : gram16_kernel<BigTile, false, false>);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)((lower * parts + 7) / 8 * 8)), dim3(64 * (small ? SmallTile::kWaves : kWaves)), 0, s,
+                       static_cast<const char*>(X), ld, K, N, sums, scratch ? N : ldc, scratch ? 1.0f : alpha,
+                       scratch ? 0.0f : beta, parts, (uint64_t)N * N);
     if (hipGetLastError() != hipSuccess) return TRAKHIP_ERR_LAUNCH;
     return scratch ? combine_shares(sums, parts, out_dtype, C, ldc, N, alpha, beta, s) : mirror_lower(sums, ldc, N, s);
 }
