@@ -26,7 +26,7 @@ from .utils import (
     nt16_ok,
     output_fits_on_device,
     scores_finalize,
-    spd_inverse,
+    spd_inverse_unchecked,
     split2_rows,
     split_rows,
 )
@@ -154,11 +154,14 @@ class BasicScoreComputer(AbstractScoreComputer):
         if self.accumulate_in_dtype:
             # lambda is added in the dtype of xtx (trak/score_computers.py:160-162), then fp32
             xtx_reg = xtx + self.lambda_reg * ch.eye(xtx.size(dim=0), device=xtx.device, dtype=xtx.dtype)
-            xtx_inv, _ = spd_inverse(xtx_reg, lambda_reg=0.0, normalize=True, general_fallback=True)
+            xtx_inv, _, checked = spd_inverse_unchecked(xtx_reg, lambda_reg=0.0, normalize=True, general_fallback=True)
         else:
-            xtx_inv, _ = spd_inverse(xtx, lambda_reg=self.lambda_reg, normalize=True, general_fallback=True)
-        xtx_inv = xtx_inv.to(self.dtype)
+            xtx_inv, _, checked = spd_inverse_unchecked(xtx, lambda_reg=self.lambda_reg, normalize=True, general_fallback=True)
+        return self._times_inverse(grads, xtx_inv.to(self.dtype), checked)
 
+    def _times_inverse(self, grads, xtx_inv, checked):
+        """grads @ xtx_inv in `dtype`.  `checked` (see `spd_inverse_unchecked`) is asked behind the first block's product,
+        which runs while the host waits for the answer; a matrix that was not positive definite starts again."""
         # 16-bit gradients meet the inverse cast to their type (as in the reference) as single planes
         half = grads.dtype == xtx_inv.dtype and grads.dtype in (ch.float16, ch.bfloat16)
         # the sums of a product that reads both in place are rounded as they are stored
@@ -185,6 +188,11 @@ class BasicScoreComputer(AbstractScoreComputer):
             else:
                 gemm_nt(block.to(self._dev), xtx_inv, out=result[start:end])
             start = end
+            if checked is not None:
+                replaced = checked()
+                if replaced is not None:
+                    return self._times_inverse(grads, replaced[0].to(self.dtype), None)
+                checked = None
         return result.to(self.dtype)
 
     def get_scores(self, features: Tensor, target_grads: Tensor, accumulator: Tensor) -> None:

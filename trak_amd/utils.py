@@ -432,8 +432,8 @@ def gram16(x, out=None, alpha=1.0, beta=0.0, out_dtype=torch.float32):
 
 
 def _inverse_call(a, lambda_reg, normalize, general):
-    """One call of trakhip_spd_inverse (Cholesky) or trakhip_general_inverse (pivoted elimination):
-    (inverse, mean_abs, status word)."""
+    """One call of trakhip_spd_inverse (Cholesky) or trakhip_general_inverse (pivoted elimination), enqueued:
+    (inverse, mean_abs, status word on the device)."""
     n = a.shape[0]
     lib = _lib.load()
     size, run = ((lib.trakhip_general_inverse_workspace, lib.trakhip_general_inverse) if general
@@ -465,8 +465,7 @@ def _inverse_call(a, lambda_reg, normalize, general):
             ctypes.c_void_p(stream),
         )
         _lib.check(code)
-        bad = int(status.item())  # also orders the workspace's lifetime after the kernels
-    return inv, mean_abs, bad
+    return inv, mean_abs, status
 
 
 def general_inverse(a, lambda_reg=0.0, normalize=False):
@@ -480,7 +479,8 @@ def general_inverse(a, lambda_reg=0.0, normalize=False):
     a = _as_f32_rows(a, "a")
     if not a.is_cuda:
         raise RuntimeError("general_inverse needs a GPU tensor")
-    inv, mean_abs, bad = _inverse_call(a, lambda_reg, normalize, general=True)
+    inv, mean_abs, status = _inverse_call(a, lambda_reg, normalize, general=True)
+    bad = int(status.item())
     if bad != 0:
         raise torch.linalg.LinAlgError(f"general_inverse: the matrix is singular (pivot {bad - 1} is zero)")
     return inv, mean_abs
@@ -497,13 +497,33 @@ def spd_inverse(a, lambda_reg=0.0, normalize=False, general_fallback=False):
     trak/score_computers.py:163), which returns something for every matrix that is not exactly
     singular (a Gram matrix rounded to fp16, or one of deficient rank, is symmetric but need not
     be positive definite)."""
+    inv, mean_abs, checked = spd_inverse_unchecked(a, lambda_reg, normalize, general_fallback)
+    return checked() or (inv, mean_abs)
+
+
+def spd_inverse_unchecked(a, lambda_reg=0.0, normalize=False, general_fallback=False):
+    """`spd_inverse` without its wait for the factorization's verdict: (inverse, mean_abs, checked), the call enqueued.
+    checked() waits for it and does what `spd_inverse` does about a matrix that is not positive definite - it
+    raises, or returns the pair that stands in for the first two -, and returns None for one that is.  A caller
+    enqueues what uses the inverse before it asks, so that the device does not stand still meanwhile."""
     if a.dim() != 2 or a.shape[0] != a.shape[1]:
         raise RuntimeError("spd_inverse needs a square matrix")
     a = _as_f32_rows(a, "a")
     if not a.is_cuda:
         raise RuntimeError("spd_inverse needs a GPU tensor")
-    inv, mean_abs, bad = _inverse_call(a, lambda_reg, normalize, general=False)
-    if bad != 0:
+    inv, mean_abs, status = _inverse_call(a, lambda_reg, normalize, general=False)
+    # the verdict crosses to the host in front of what the caller enqueues next, and only its crossing is waited for
+    verdict = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    with torch.cuda.device(a.device):
+        verdict.copy_(status, non_blocking=True)
+        crossed = torch.cuda.Event()
+        crossed.record(torch.cuda.current_stream(a.device))
+
+    def checked():
+        crossed.synchronize()
+        bad = int(verdict[0])
+        if bad == 0:
+            return None
         if not general_fallback:
             raise torch.linalg.LinAlgError(
                 f"spd_inverse: the matrix is not positive definite (pivot {bad - 1} is not positive)"
@@ -513,7 +533,8 @@ def spd_inverse(a, lambda_reg=0.0, normalize=False, general_fallback=False):
             "reference's LU does", bad - 1
         )
         return general_inverse(a, lambda_reg, normalize)
-    return inv, mean_abs
+
+    return inv, mean_abs, checked
 
 
 _STORE_DTYPES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
