@@ -917,10 +917,10 @@ __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gram16_kernel(const cha
     const uint32_t a_off = (uint32_t)(row * ld + a_from) * 2u, b_off = (uint32_t)(row * ld + b_from) * 2u;
     const char* a_tile = X + 2 * m0;
     const char* b_tile = X + 2 * n0;
-    auto dma = [&](uint64_t s, char* buf) {
+    auto dma = [&](uint64_t s, char* buf, int lo, int hi) {  // loads [lo, hi) of the wave
         if ((s + 1) * kStep <= K) {
 #pragma unroll
-            for (int i = 0; i < 2 * kMoves; ++i) {
+            for (int i = lo; i < hi; ++i) {
                 const uint64_t at = (s * kStep + 16 * (i % kMoves)) * ld * 2;  // scalar
                 const char* base = (i < kMoves ? a_tile : b_tile) + at;
                 char* to = buf + (i < kMoves ? 0 : kOperandBytes) + 1024 * (wave + kWaves * (i % kMoves));
@@ -928,7 +928,7 @@ __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gram16_kernel(const cha
                                                  (void __attribute__((address_space(3)))*)to, 16, 0, 0);
             }
         } else {
-            for (int i = 0; i < 2 * kMoves; ++i) {
+            for (int i = lo; i < hi; ++i) {
                 const uint64_t k = s * kStep + 16 * (i % kMoves);
                 piece v = {0u, 0u, 0u, 0u};
                 if (k + row < K)
@@ -956,14 +956,13 @@ __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gram16_kernel(const cha
         for (int j = 0; j < JT; ++j) fb[set][j] = read_transposed<kRowBytes>(l + b_at[j]);
     };
 
-    dma(first, lds[0]);
+    dma(first, lds[0], 0, 2 * kMoves);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     fetch(0, 0, 0);
     for (uint64_t s = first; s < steps; ++s) {
         const int cur = (int)((s - first) & 1);
         const bool last_step = s + 1 == steps;
-        if (!last_step) dma(s + 1, lds[cur ^ 1]);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int set = u & 1;
@@ -973,6 +972,11 @@ __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gram16_kernel(const cha
             __builtin_amdgcn_sched_barrier(0);
             if (u < 3) {
                 fetch(cur, u + 1, set ^ 1);
+                // One operand's loads of the next step under each of the first two sub-steps: all eight of a wave at once
+                // fill LDS's write side while every wave waits for its fragments (50 000 rows, 1024 / 2048 / 3072 columns:
+                // 102 -> 95, 249 -> 242, 551 -> 521 us; no size slower).  gemm_nt16_kernel gains 0-2 % from it at 2048
+                // columns and loses 2 % at 128, so it keeps its loads together.
+                if (u < 2 && !last_step) dma(s + 1, lds[cur ^ 1], u * kMoves, (u + 1) * kMoves);
             } else {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
