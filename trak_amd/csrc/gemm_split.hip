@@ -854,7 +854,7 @@ __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gemm_nt16_kernel(
 // operand is eight values of one column.  A step is 64 rows of the tile's 256 columns (32 KB per operand); gfx950's
 // transposing LDS read (ds_read_b64_tr_b16) hands sixteen lanes, which name four rows of sixteen columns, four rows of a
 // column each, so that two of them make an operand and X needs no transposing pass (94 us and 410 MB of traffic for
-// [50 000, 2048] fp16).  X^T X with the result rounded: [50 000, 2048] 349 -> 249 us, [8200, 4096] 274 -> 200,
+// [50 000, 2048] fp16).  X^T X with the result rounded: [50 000, 2048] 349 -> 242 us, [8200, 4096] 274 -> 196,
 // [2000, 512] 39 -> 25; bound by the MFMAs' power and, per step, the 64 LDS-direct loads of a CU.
 // LDS holds a row as 32 pieces of 16 bytes; the 64-byte units of row k are permuted, unit u in place u ^ (k % 4): the
 // four rows that 32 lanes read at a time then lie in different quarters of the 64 banks.  A wave's LDS-direct load
@@ -1340,7 +1340,8 @@ uint64_t big_tile_rows(uint64_t M, uint64_t N, uint64_t K, int cus) {
 // N = 2048 takes seven (36 tiles: 252 workgroups; three gave 108), N = 512 at 2000 values of k sixteen, N = 4096 seven at
 // 50 000 values of k (952 workgroups, 3.7 rounds; three leave the second of two rounds 60 % full) and one at 2000 of 16 bits
 // (80 us; three 95).  A share has at least eight steps, and the shares together at most 512 MB.  Product and
-// sum against three shares, X^T X of [50 000, 2048] fp16: 445 -> 248 us, of [50 000, 512]: 371 -> 87 us.
+// sum against three shares, X^T X of [50 000, 2048] fp16 from its planes: 445 -> 248 us, of [50 000, 512] 371 -> 87.
+// (gram16_kernel takes the same numbers; where the tiles of the chosen shares leave CUs idle, see gram_small_tiles.)
 constexpr uint32_t kGramPartsMax = 16, kGramPartsFew = 3, kGramTilesMax = 170;
 uint32_t gram_parts(uint64_t N, uint64_t K, int dtype, bool two_planes, uint32_t most, size_t room = SIZE_MAX) {
     const uint64_t tiles = (N + BM - 1) / BM, lower = tiles * (tiles + 1) / 2;

@@ -686,9 +686,9 @@ int divide_by_mean(float* M, uint64_t ld, uint64_t n, int normalize, float* part
 
 // ---- products with a triangular operand ---------------------------------------------------------------------
 //
-// fp32 MFMA products of the triangular inverse and the final L^-T L^-1.  Bound: the latency of the global loads at
-// the sizes of the recursion (a [1024 x 1024] node has 2 GFLOP for the whole chip); L^-T L^-1 at n = 4096 runs at 86 TFLOP/s of
-// the 124 that the general fp32 MFMA product reaches (64 x 64 tiles, the mirror image stored a row apart per lane).
+// fp32 MFMA products of the triangular inverse by recursion (n > 4096) and the final L^-T L^-1 (n > 2048; below, see
+// tri_gram_small_kernel).  Bound: the latency of the global loads in the recursion's small nodes (a [1024 x 1024] one has
+// 2 GFLOP for the whole chip); L^-T L^-1 at n = 4096 runs at 86 TFLOP/s of the 124 that the general fp32 MFMA product reaches (64 x 64 tiles, the mirror image stored a row apart per lane).
 // So: 64 x 64 tiles (256 workgroups where 128 x 128 tiles gave 64), four k steps of 32 in flight in registers while
 // one is multiplied from LDS, and k ranges cut to the part where the triangular operand is not zero (rounded to
 // 128, so a range is whole chunks of four steps), tiles with the longest range first.
@@ -698,8 +698,8 @@ enum class Tri { kLowerB, kLowerA, kGram };
 //   kGram    C = A^T A        A lower triangular, lower tiles + mirror image: k from the tile's rows on; n x n stored
 // Operands have whole 128-blocks (row pitch np).  A wave owns one 32 x 32 tile, two accumulators (even and odd
 // sub-steps) that are added at the end: error of the inverse against 64 bits 9.4e-7 at n = 2048, 1.26e-6 with one
-// accumulator over the whole range in the earlier kernels.  Measured: the recursion 415 -> 112 us at n = 2048 and
-// 824 -> 350 us at 4096 (128 x 128 tiles over the full k range), L^-T L^-1 240 -> 66 us and 516 -> 277 us (256 x 256 tiles of the
+// accumulator over the whole range in the earlier kernels.  Measured: a whole recursion of n = 4096
+// 824 -> 350 us (128 x 128 tiles over the full k range), L^-T L^-1 516 -> 277 us (256 x 256 tiles of the
 // six-term bf16 product, planes included).  The staging registers are vector types (arrays of HIP's float4 stayed in
 // scratch) and all fragment reads of a step stand before its first MFMA: without these two the same products took
 // twice as long.
