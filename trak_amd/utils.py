@@ -311,7 +311,7 @@ def gemm_nt16(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
     if out is None:
         out = torch.empty((M, N), dtype=torch.float32, device=a.device)
         beta = 0.0
-    rounded = out.dtype in (torch.float16, torch.bfloat16) and beta == 0.0
+    rounded = out.dtype != torch.float32 and out.dtype in (torch.float16, torch.bfloat16) and beta == 0.0
     if (out.dtype != torch.float32 and not rounded) or tuple(out.shape) != (M, N) or (N > 1 and out.stride(1) != 1) or out.device != a.device:
         raise RuntimeError("out must be an fp32 [M, N] tensor (fp16 or bf16 with beta = 0) with unit column stride on the operands' device")
     rs = None
@@ -322,13 +322,18 @@ def gemm_nt16(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None):
     lib = _lib.load()
     with torch.cuda.device(a.device):
         stream = torch.cuda.current_stream(a.device).cuda_stream
-        operands = (ctypes.c_void_p(a.data_ptr()), _ld(a), ctypes.c_void_p(b.data_ptr()), _ld(b), _STORE_DTYPES[a.dtype])
-        result = (ctypes.c_void_p(out.data_ptr()), _ld(out), M, N, K, float(alpha))
-        tail = (ctypes.c_void_p(rs.data_ptr()) if rs is not None else None, ctypes.c_void_p(stream))
         if rounded:
-            code = lib.trakhip_gemm_nt16_rounded(*operands, _STORE_DTYPES[out.dtype], *result, *tail)
+            code = lib.trakhip_gemm_nt16_rounded(
+                ctypes.c_void_p(a.data_ptr()), _ld(a), ctypes.c_void_p(b.data_ptr()), _ld(b), _STORE_DTYPES[a.dtype],
+                _STORE_DTYPES[out.dtype], ctypes.c_void_p(out.data_ptr()), _ld(out), M, N, K, float(alpha),
+                ctypes.c_void_p(rs.data_ptr()) if rs is not None else None, ctypes.c_void_p(stream),
+            )
         else:
-            code = lib.trakhip_gemm_nt16(*operands, *result, float(beta), *tail)
+            code = lib.trakhip_gemm_nt16(
+                ctypes.c_void_p(a.data_ptr()), _ld(a), ctypes.c_void_p(b.data_ptr()), _ld(b), _STORE_DTYPES[a.dtype],
+                ctypes.c_void_p(out.data_ptr()), _ld(out), M, N, K, float(alpha), float(beta),
+                ctypes.c_void_p(rs.data_ptr()) if rs is not None else None, ctypes.c_void_p(stream),
+            )
     _lib.check(code)
     return out
 
