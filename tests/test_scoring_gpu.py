@@ -12,7 +12,7 @@ from oracle import score_oracle as so
 import trak_amd.score_computers as score_computers_module
 from trak_amd import _lib
 import trak_amd.utils as utils_module
-from trak_amd import BasicScoreComputer, get_matrix_mult
+from trak_amd import BasicScoreComputer, ScoreAccumulator, get_matrix_mult
 from trak_amd.utils import (
     gemm_nt,
     gemm_nt16,
@@ -188,6 +188,20 @@ def test_spd_inverse_names_the_first_bad_pivot(gpu, first, value):
         a[first + 9, first + 9] = -3.0
     with pytest.raises(torch.linalg.LinAlgError, match=rf"pivot {first} "):
         spd_inverse(a.to(gpu))
+
+
+def test_scoring_under_a_default_device(gpu):
+    # page-locked buffers are host memory whatever device new tensors go to by default
+    x = torch.randn(300, 64, generator=torch.Generator(device=gpu).manual_seed(2), device=gpu)
+    sc = BasicScoreComputer(dtype=torch.float32, device=gpu, lambda_reg=1e-2)
+    xtx = sc.get_xtx(x)
+    want = sc.get_x_xtx_inv(x, xtx)
+    acc = ScoreAccumulator(sc, 300, 7)
+    acc.add(want, x[:7], torch.ones(300, 1))
+    scores = acc.finalize(np.zeros((300, 7), np.float32))
+    with torch.device(gpu):
+        assert torch.equal(sc.get_x_xtx_inv(x, xtx), want)
+        assert np.array_equal(acc.finalize(np.zeros((300, 7), np.float32)), scores)
 
 
 def test_spd_inverse_many_blocks(gpu):

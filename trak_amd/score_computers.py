@@ -337,7 +337,7 @@ class ScoreAccumulator:
         row_bytes = max(1, M * out.dtype.itemsize)
         # four chunks of at least 1 MB or more of them: the copy of one into the store passes under the next one's crossing
         rows = max(1, min(N, int(chunk_bytes) // row_bytes, max(-(-N // 4), (1 << 20) // row_bytes)))
-        stage = [ch.empty((rows, M), dtype=tdtype, pin_memory=True) for _ in range(2 if rows < N else 1)]
+        stage = [ch.empty((rows, M), dtype=tdtype, device="cpu", pin_memory=True) for _ in range(2 if rows < N else 1)]
         pending = [None] * len(stage)
         stream = ch.cuda.current_stream(self._acc.device)
 

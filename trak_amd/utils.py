@@ -518,7 +518,7 @@ def spd_inverse_unchecked(a, lambda_reg=0.0, normalize=False, general_fallback=F
         raise RuntimeError("spd_inverse needs a GPU tensor")
     inv, mean_abs, status = _inverse_call(a, lambda_reg, normalize, general=False)
     # the verdict crosses to the host in front of what the caller enqueues next, and only its crossing is waited for
-    verdict = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    verdict = torch.empty(1, dtype=torch.int32, device="cpu", pin_memory=True)  # (the default device may be another)
     with torch.cuda.device(a.device):
         verdict.copy_(status, non_blocking=True)
         crossed = torch.cuda.Event()
