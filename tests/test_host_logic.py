@@ -128,3 +128,16 @@ def test_out_to_loss_sums_in_half_precision_are_numpys():
     fixed.flags.writeable = False
     with pytest.raises(ValueError):
         _store_rows(fixed, 1, 4, src)
+
+
+@pytest.mark.parametrize("kind", [[("score", "f2"), ("flag", "u1")], [("flag", "u1"), ("score", "f4")], [("flag", "u1"), ("score", "f2"), ("pad", "u1")]])
+def test_scores_into_a_field_of_records(kind, tmp_path):
+    from trak_amd.score_computers import _store_rows
+
+    # steps of 3, 5 and 4 bytes; an aligned start and two that are not
+    src = torch.arange(12.0).reshape(3, 4)
+    mapped = np.memmap(tmp_path / "records", mode="w+", dtype=kind, shape=(5, 4))
+    for records in (np.zeros((5, 4), kind), mapped):
+        out = records["score"]
+        _store_rows(out, 1, 4, src.to(torch.float16 if out.dtype == np.float16 else torch.float32))
+        assert np.array_equal(out[1:4], src.numpy()) and not out[[0, 4]].any() and not records["flag"].any()

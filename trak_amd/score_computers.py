@@ -268,7 +268,8 @@ def _row_factors(sums, n):
 def _store_rows(out, r0, r1, src):
     """out[r0:r1] = src (a CPU tensor): by torch's threads, one thread copies less than half of what PCIe delivers."""
     dst = out[r0:r1]
-    if dst.flags.writeable and all(s >= 0 for s in dst.strides):
+    # (torch takes no steps backwards or by parts of an element, as a field of records has them)
+    if dst.flags.behaved and all(s >= 0 and s % dst.itemsize == 0 for s in dst.strides):
         ch.from_numpy(dst).copy_(src)
     else:
         dst[...] = src.numpy()
