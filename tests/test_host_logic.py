@@ -141,3 +141,25 @@ def test_scores_into_a_field_of_records(kind, tmp_path):
         out = records["score"]
         _store_rows(out, 1, 4, src.to(torch.float16 if out.dtype == np.float16 else torch.float32))
         assert np.array_equal(out[1:4], src.numpy()) and not out[[0, 4]].any() and not records["flag"].any()
+
+
+def test_scores_into_arrays_whose_slices_are_copies():
+    from trak_amd.score_computers import _store_rows
+
+    class Stored:  # as an array in a file: reading gives a copy, assignment writes
+        def __init__(self, shape, dtype):
+            self.data, self.shape, self.dtype = np.zeros(shape, dtype), shape, np.dtype(dtype)
+
+        def __getitem__(self, at):
+            return self.data[at].copy()
+
+        def __setitem__(self, at, value):
+            self.data[at] = value
+
+    src = torch.arange(12.0).reshape(3, 4)
+    stored = Stored((5, 4), np.float32)
+    _store_rows(stored, 1, 4, src)
+    assert np.array_equal(stored.data[1:4], src.numpy()) and not stored.data[[0, 4]].any()
+    masked = np.ma.masked_all((5, 4), np.float32)
+    _store_rows(masked, 1, 4, src)
+    assert np.array_equal(masked[1:4].filled(-1.0), src.numpy()) and masked[[0, 4]].mask.all()

@@ -267,12 +267,12 @@ def _row_factors(sums, n):
 
 def _store_rows(out, r0, r1, src):
     """out[r0:r1] = src (a CPU tensor): by torch's threads, one thread copies less than half of what PCIe delivers."""
-    dst = out[r0:r1]
-    # (torch takes no steps backwards or by parts of an element, as a field of records has them)
-    if dst.flags.behaved and all(s >= 0 and s % dst.itemsize == 0 for s in dst.strides):
-        ch.from_numpy(dst).copy_(src)
+    # Only what is known to be memory: the slices of another array (of a file, masked, ...) may be copies, and what is
+    # written to them lost.  (torch takes no steps backwards or by parts of an element, as a field of records has them.)
+    if type(out) in (np.ndarray, np.memmap) and out.flags.behaved and all(s >= 0 and s % out.itemsize == 0 for s in out.strides):
+        ch.from_numpy(out[r0:r1]).copy_(src)
     else:
-        dst[...] = src.numpy()
+        out[r0:r1] = src.numpy()
 
 
 class ScoreAccumulator:
