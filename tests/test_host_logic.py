@@ -163,3 +163,27 @@ def test_scores_into_arrays_whose_slices_are_copies():
     masked = np.ma.masked_all((5, 4), np.float32)
     _store_rows(masked, 1, 4, src)
     assert np.array_equal(masked[1:4].filled(-1.0), src.numpy()) and masked[[0, 4]].mask.all()
+
+
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 9])
+def test_scores_into_memory_by_our_own_threads_and_into_files_by_one(rows, tmp_path, monkeypatch):
+    from concurrent.futures import ThreadPoolExecutor
+
+    from trak_amd import score_computers as m
+
+    src = torch.arange(4.0 * rows).reshape(rows, 4)
+    memory = np.zeros((rows + 2, 4), np.float32)
+    mapped = np.lib.format.open_memmap(tmp_path / "scores.npy", mode="w+", dtype=np.float32, shape=(rows + 2, 4))
+    monkeypatch.setattr(m.ch, "get_num_threads", lambda: 1)
+    assert m._own_threads(memory, m._COPY_BYTES) and not m._own_threads(memory, m._COPY_BYTES - 1)
+    for out in (mapped, np.asarray(mapped), mapped[:, ::2]):
+        assert not m._in_memory(out) and not m._own_threads(out, m._COPY_BYTES)
+    monkeypatch.setattr(m.ch, "get_num_threads", lambda: m._COPY_THREADS)
+    assert not m._own_threads(memory, m._COPY_BYTES)
+    with ThreadPoolExecutor(m._COPY_THREADS) as pool:
+        for out, p in ((memory, pool), (mapped, None)):
+            m._store_rows(out, 1, rows + 1, src, p)
+            assert np.array_equal(out[1:-1], src.numpy()) and not out[[0, -1]].any()
+        memory.flags.writeable = False
+        with pytest.raises(ValueError):                                                  # what a thread raises is raised
+            m._store_rows(memory, 1, rows + 1, src, pool)

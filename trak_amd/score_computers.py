@@ -7,6 +7,7 @@ running the three GEMMs and the regularized inverse on the GPU through libtrakhi
 """
 import logging
 from abc import ABC, abstractmethod
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import torch
@@ -265,11 +266,41 @@ def _row_factors(sums, n):
     return (ch.from_numpy(sums).float() / divisor).half().float().numpy()
 
 
-def _store_rows(out, r0, r1, src):
-    """out[r0:r1] = src (a CPU tensor): by torch's threads, one thread copies less than half of what PCIe delivers."""
-    # Only what is known to be memory: the slices of another array (of a file, masked, ...) may be copies, and what is
-    # written to them lost.  (torch takes no steps backwards or by parts of an element, as a field of records has them.)
-    if type(out) in (np.ndarray, np.memmap) and out.flags.behaved and all(s >= 0 and s % out.itemsize == 0 for s in out.strides):
+# Who copies a block of scores into the store, by the time of a whole `finalize` on the GPU's host (16 CPUs; 10 MB, 260 MB and
+# 1 GB of fp16 scores).  Memory: torch's threads where there are as many as _COPY_THREADS or the block is small (16: 0.34, 5.4, 20.6 ms;
+# four: 0.33, 5.9, 21.8; one: 0.44, 12.3, 47.5), else as many of our own (under OMP_NUM_THREADS=1: 6.0 and 21.6 ms).  A mapped file: one
+# thread.  Its pages are new when scores are written, and threads that ask for them wait for one another (one: 3.1, 31, 114 ms; four
+# of our own 4-10, 75-100, 200-300; torch's sixteen 9-10, 151-156, 445-466; written a second time: 0.6, 11, 40-48 ms).
+_COPY_THREADS = 4
+_COPY_BYTES = 16 << 20
+
+
+def _in_memory(out):
+    """Whether this is an array in memory.  A mapped file is not; and the slices of other kinds of array (in a file, masked, ...) may
+    be copies, in which what is written is lost."""
+    if type(out) is not np.ndarray:
+        return False
+    base = out.base
+    while isinstance(base, np.ndarray) and not isinstance(base, np.memmap):
+        base = base.base
+    return not isinstance(base, np.memmap)
+
+
+def _own_threads(out, block_bytes):
+    return block_bytes >= _COPY_BYTES and ch.get_num_threads() < _COPY_THREADS and _in_memory(out)
+
+
+def _store_rows(out, r0, r1, src, pool=None):
+    """out[r0:r1] = src (a CPU tensor), by the _COPY_THREADS threads of `pool` if it is given."""
+    if pool is not None:
+        values, step = src.numpy(), -(-(r1 - r0) // _COPY_THREADS)
+
+        def assign(at):
+            out[r0 + at : min(r1, r0 + at + step)] = values[at : at + step]
+
+        list(pool.map(assign, range(0, r1 - r0, step)))
+    # (torch takes no steps backwards or by parts of an element, as a field of records has them)
+    elif _in_memory(out) and out.flags.behaved and all(s >= 0 and s % out.itemsize == 0 for s in out.strides):
         ch.from_numpy(out[r0:r1]).copy_(src)
     else:
         out[r0:r1] = src.numpy()
@@ -340,6 +371,7 @@ class ScoreAccumulator:
         rows = max(1, min(N, int(chunk_bytes) // row_bytes, max(-(-N // 4), (1 << 20) // row_bytes)))
         stage = [ch.empty((rows, M), dtype=tdtype, device="cpu", pin_memory=True) for _ in range(2 if rows < N else 1)]
         pending = [None] * len(stage)
+        pool = ThreadPoolExecutor(_COPY_THREADS) if _own_threads(out, rows * row_bytes) else None
         stream = ch.cuda.current_stream(self._acc.device)
 
         def retire(i):
@@ -347,17 +379,21 @@ class ScoreAccumulator:
                 return
             event, r0, r1 = pending[i]
             event.synchronize()
-            _store_rows(out, r0, r1, stage[i][: r1 - r0])
+            _store_rows(out, r0, r1, stage[i][: r1 - r0], pool)
             pending[i] = None
 
-        for index, r0 in enumerate(range(0, N, rows)):
-            i = index % len(stage)
-            retire(i)
-            r1 = min(N, r0 + rows)
-            scores_finalize(self._acc[r0:r1], n, row_factor[r0:r1], stage[i][: r1 - r0])
-            event = ch.cuda.Event()
-            event.record(stream)
-            pending[i] = (event, r0, r1)
-        for i in range(len(stage)):
-            retire((index + 1 + i) % len(stage))
+        try:
+            for index, r0 in enumerate(range(0, N, rows)):
+                i = index % len(stage)
+                retire(i)
+                r1 = min(N, r0 + rows)
+                scores_finalize(self._acc[r0:r1], n, row_factor[r0:r1], stage[i][: r1 - r0])
+                event = ch.cuda.Event()
+                event.record(stream)
+                pending[i] = (event, r0, r1)
+            for i in range(len(stage)):
+                retire((index + 1 + i) % len(stage))
+        finally:
+            if pool is not None:
+                pool.shutdown()
         return out
