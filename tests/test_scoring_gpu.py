@@ -18,6 +18,7 @@ from trak_amd.utils import (
     gemm_nt16,
     gemm_nt_split,
     gemm_tn,
+    general_inverse,
     gram_split,
     matmul_nt,
     spd_inverse,
@@ -188,6 +189,36 @@ def test_spd_inverse_names_the_first_bad_pivot(gpu, first, value):
         a[first + 9, first + 9] = -3.0
     with pytest.raises(torch.linalg.LinAlgError, match=rf"pivot {first} "):
         spd_inverse(a.to(gpu))
+
+
+@pytest.mark.parametrize("dtype,gemm", [(torch.float16, "split"), (torch.float32, "split"), (torch.float32, "split2"), (torch.float32, "fp32")])
+@pytest.mark.parametrize("where", ["cuda", "cpu"])
+def test_features_of_a_matrix_that_is_not_positive_definite(gpu, dtype, gemm, where):
+    # the verdict arrives behind a product with a matrix of no use: nothing of it is in the result or kept in memory
+    n, k = 70_000, 256
+    gen = torch.Generator(device=gpu).manual_seed(9)
+    x = torch.randn(n, k, generator=gen, device=gpu).to(dtype)
+    d = torch.ones(k, device=gpu)
+    d[::3] = -2.0
+    q = torch.linalg.qr(torch.randn(k, k, generator=gen, device=gpu))[0]
+    xtx = ((q * d) @ q.T).to(dtype)
+    want = general_inverse(xtx, normalize=True)[0].to(dtype).double()
+    x = x.to(where)
+    sc = BasicScoreComputer(dtype=dtype, device=gpu, gemm=gemm, CUDA_MAX_DIM_SIZE=20_000)
+    got = sc.get_x_xtx_inv(x, xtx)
+    want = x.to(gpu).double() @ want
+    assert rel_max(got.cpu().numpy(), want.cpu().numpy()) < (2.0**-10 if dtype == torch.float16 else gemm_tol(k))
+    del got, want
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats(gpu)
+    before = torch.cuda.memory_allocated(gpu)
+    sc.get_x_xtx_inv(x, xtx)
+    # one result, in fp32 where it is not rounded by the product; of the gradients, resident ones as planes ("split": 6, "split2": 4
+    # bytes a value) or a block of host ones with its planes; matrices of k x k
+    rows = 20_000 if where == "cpu" else n
+    planes = {"split": 6, "split2": 4, "fp32": 0}[gemm] if dtype == torch.float32 else 0
+    block = rows * k * (planes + (x.element_size() if where == "cpu" else 0))
+    assert torch.cuda.max_memory_allocated(gpu) - before <= 1.05 * (n * k * x.element_size() + block) + 64 * k * k
 
 
 def test_scoring_under_a_default_device(gpu):

@@ -23,6 +23,7 @@ from .utils import (
     gram16_ok,
     gram_split,
     in_place_pays,
+    inverse_of_rejected,
     matmul_nt,
     nt16_ok,
     output_fits_on_device,
@@ -151,18 +152,22 @@ class BasicScoreComputer(AbstractScoreComputer):
     def get_x_xtx_inv(self, grads: Tensor, xtx: Tensor) -> Tensor:
         # (xtx + lambda I)^-1 in fp32, divided by the mean absolute entry
         # (trak/score_computers.py:160-166)
-        xtx = xtx.to(self._dev)
+        xtx, lambda_reg = xtx.to(self._dev), self.lambda_reg
         if self.accumulate_in_dtype:
             # lambda is added in the dtype of xtx (trak/score_computers.py:160-162), then fp32
-            xtx_reg = xtx + self.lambda_reg * ch.eye(xtx.size(dim=0), device=xtx.device, dtype=xtx.dtype)
-            xtx_inv, _, checked = spd_inverse_unchecked(xtx_reg, lambda_reg=0.0, normalize=True, general_fallback=True)
-        else:
-            xtx_inv, _, checked = spd_inverse_unchecked(xtx, lambda_reg=self.lambda_reg, normalize=True, general_fallback=True)
-        return self._times_inverse(grads, xtx_inv.to(self.dtype), checked)
+            xtx = xtx + lambda_reg * ch.eye(xtx.size(dim=0), device=xtx.device, dtype=xtx.dtype)
+            lambda_reg = 0.0
+        inverse, _, verdict = spd_inverse_unchecked(xtx, lambda_reg, normalize=True)
+        result, pivot = self._times_inverse(grads, inverse.to(self.dtype), verdict)
+        if pivot is not None:
+            del inverse  # (what the first attempt held is given back before the elimination asks for its workspace)
+            inverse, _ = inverse_of_rejected(xtx, pivot, lambda_reg, normalize=True)
+            result, _ = self._times_inverse(grads, inverse.to(self.dtype))
+        return result
 
-    def _times_inverse(self, grads, xtx_inv, checked):
-        """grads @ xtx_inv in `dtype`.  `checked` (see `spd_inverse_unchecked`) is asked behind the first block's product,
-        which runs while the host waits for the answer; a matrix that was not positive definite starts again."""
+    def _times_inverse(self, grads, xtx_inv, verdict=None):
+        """(grads @ xtx_inv in `dtype`, None).  `verdict` (see `spd_inverse_unchecked`) is asked behind the first block's product,
+        which runs while the host waits for the answer; a matrix that was not positive definite gives (None, pivot)."""
         # 16-bit gradients meet the inverse cast to their type (as in the reference) as single planes
         half = grads.dtype == xtx_inv.dtype and grads.dtype in (ch.float16, ch.bfloat16)
         # the sums of a product that reads both in place are rounded as they are stored
@@ -189,12 +194,11 @@ class BasicScoreComputer(AbstractScoreComputer):
             else:
                 gemm_nt(block.to(self._dev), xtx_inv, out=result[start:end])
             start = end
-            if checked is not None:
-                replaced = checked()
-                if replaced is not None:
-                    return self._times_inverse(grads, replaced[0].to(self.dtype), None)
-                checked = None
-        return result.to(self.dtype)
+            if verdict is not None:
+                pivot, verdict = verdict(), None
+                if pivot is not None:
+                    return None, pivot
+        return result.to(self.dtype), None
 
     def get_scores(self, features: Tensor, target_grads: Tensor, accumulator: Tensor) -> None:
         train_dim = features.shape[0]

@@ -502,14 +502,19 @@ def spd_inverse(a, lambda_reg=0.0, normalize=False, general_fallback=False):
     trak/score_computers.py:163), which returns something for every matrix that is not exactly
     singular (a Gram matrix rounded to fp16, or one of deficient rank, is symmetric but need not
     be positive definite)."""
-    inv, mean_abs, checked = spd_inverse_unchecked(a, lambda_reg, normalize, general_fallback)
-    return checked() or (inv, mean_abs)
+    inv, mean_abs, verdict = spd_inverse_unchecked(a, lambda_reg, normalize)
+    pivot = verdict()
+    if pivot is None:
+        return inv, mean_abs
+    if not general_fallback:
+        raise torch.linalg.LinAlgError(f"spd_inverse: the matrix is not positive definite (pivot {pivot} is not positive)")
+    del inv
+    return inverse_of_rejected(a, pivot, lambda_reg, normalize)
 
 
-def spd_inverse_unchecked(a, lambda_reg=0.0, normalize=False, general_fallback=False):
-    """`spd_inverse` without its wait for the factorization's verdict: (inverse, mean_abs, checked), the call enqueued.
-    checked() waits for it and does what `spd_inverse` does about a matrix that is not positive definite - it
-    raises, or returns the pair that stands in for the first two -, and returns None for one that is.  A caller
+def spd_inverse_unchecked(a, lambda_reg=0.0, normalize=False):
+    """`spd_inverse` without its wait for the factorization's verdict: (inverse, mean_abs, verdict), the call enqueued.
+    verdict() waits for it: None, or the first pivot that is not positive, and then the first two hold nothing of use.  A caller
     enqueues what uses the inverse before it asks, so that the device does not stand still meanwhile."""
     if a.dim() != 2 or a.shape[0] != a.shape[1]:
         raise RuntimeError("spd_inverse needs a square matrix")
@@ -517,29 +522,28 @@ def spd_inverse_unchecked(a, lambda_reg=0.0, normalize=False, general_fallback=F
     if not a.is_cuda:
         raise RuntimeError("spd_inverse needs a GPU tensor")
     inv, mean_abs, status = _inverse_call(a, lambda_reg, normalize, general=False)
-    # the verdict crosses to the host in front of what the caller enqueues next, and only its crossing is waited for
-    verdict = torch.empty(1, dtype=torch.int32, device="cpu", pin_memory=True)  # (the default device may be another)
+    # the status word crosses to the host in front of what the caller enqueues next, and only its crossing is waited for
+    word = torch.empty(1, dtype=torch.int32, device="cpu", pin_memory=True)  # (the default device may be another)
     with torch.cuda.device(a.device):
-        verdict.copy_(status, non_blocking=True)
+        word.copy_(status, non_blocking=True)
         crossed = torch.cuda.Event()
         crossed.record(torch.cuda.current_stream(a.device))
 
-    def checked():
+    def verdict():
         crossed.synchronize()
-        bad = int(verdict[0])
-        if bad == 0:
-            return None
-        if not general_fallback:
-            raise torch.linalg.LinAlgError(
-                f"spd_inverse: the matrix is not positive definite (pivot {bad - 1} is not positive)"
-            )
-        logging.getLogger("ScoreComputer").warning(
-            "X^T X + lambda I is not positive definite (pivot %d): inverting it with partial pivoting, as the "
-            "reference's LU does", bad - 1
-        )
-        return general_inverse(a, lambda_reg, normalize)
+        bad = int(word[0])
+        return bad - 1 if bad else None
 
-    return inv, mean_abs, checked
+    return inv, mean_abs, verdict
+
+
+def inverse_of_rejected(a, pivot, lambda_reg=0.0, normalize=False):
+    """`general_inverse` of a matrix whose factorization stopped at `pivot`, with a warning."""
+    logging.getLogger("ScoreComputer").warning(
+        "X^T X + lambda I is not positive definite (pivot %d): inverting it with partial pivoting, as the "
+        "reference's LU does", pivot
+    )
+    return general_inverse(a, lambda_reg, normalize)
 
 
 _STORE_DTYPES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
