@@ -221,6 +221,31 @@ def test_features_of_a_matrix_that_is_not_positive_definite(gpu, dtype, gemm, wh
     assert torch.cuda.max_memory_allocated(gpu) - before <= 1.05 * (n * k * x.element_size() + block) + 64 * k * k
 
 
+@pytest.mark.parametrize("where", ["cuda", "cpu"])
+def test_little_is_multiplied_by_an_inverse_that_is_rejected(gpu, monkeypatch, where):
+    k, n = 1024, 140_000
+    x = (torch.randn(n, k, generator=torch.Generator(device=gpu).manual_seed(4), device=gpu) / 32).half()
+    xtx = torch.eye(k, device=gpu).half()
+    xtx[5, 5] = -0.5
+    calls = []
+    product, elimination = score_computers_module.gemm_nt16, utils_module.general_inverse
+    monkeypatch.setattr(score_computers_module, "gemm_nt16", lambda a, b, out: (calls.append(a.shape[0]), product(a, b, out=out)))
+    monkeypatch.setattr(utils_module, "general_inverse", lambda *args: (calls.append("elimination"), elimination(*args))[1])
+    sc = BasicScoreComputer(dtype=torch.float16, device=gpu)
+    got = sc.get_x_xtx_inv(x.to(where), xtx)
+    at = calls.index("elimination")
+    assert sum(calls[:at]) == (16_384 if where == "cuda" else 0)      # four columns of 256 x 256 tiles by 64 rows of them
+    assert sum(calls[at + 1:]) == n
+    want = torch.ones(k, device=gpu)
+    want[5] = -2.0
+    assert torch.equal(got, x * (want / ((k + 1) / k**2)).half())     # one product per entry
+    # and of one that is not, everything once, in two pieces
+    calls.clear()
+    xtx[5, 5] = 0.5
+    sc.get_x_xtx_inv(x.to(where), xtx)
+    assert calls == ([16_384, n - 16_384] if where == "cuda" else [20_000] * 7)
+
+
 def test_scoring_under_a_default_device(gpu):
     # page-locked buffers are host memory whatever device new tensors go to by default
     x = torch.randn(300, 64, generator=torch.Generator(device=gpu).manual_seed(2), device=gpu)
