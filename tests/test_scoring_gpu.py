@@ -98,6 +98,21 @@ def test_products_of_few_tiles_read_their_operands_in_place(gpu, M, N, K):
     assert (np.abs(got - want) <= rows * (0.5 * bound + 2.0 ** -21 * (np.abs(c0.numpy()) + np.abs(a64 @ b64.T)))).all()
 
 
+@pytest.mark.parametrize("K", [300, 1024])
+def test_products_of_mixed_types_keep_no_copy_of_their_operands(gpu, K):
+    M, N = 20_000, 3000
+    a, b = torch.randn(M, K, device=gpu).half(), torch.randn(N, K, device=gpu)
+    matmul_nt(a[:100], b[:100])
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats(gpu)
+    before = torch.cuda.memory_allocated(gpu)
+    out = matmul_nt(a, b)
+    # planes (rows to 256, k to 64: 6 bytes a value) and the result, not the fp32 copy that a's planes are made from
+    planes = 6 * (20_224 + 3072) * -(-K // 64) * 64
+    # (an allocation may keep up to 1 MB behind it)
+    assert torch.cuda.max_memory_allocated(gpu) - before <= planes + out.numel() * 4 + (3 << 20)
+
+
 def test_products_that_are_split_and_products_that_are_not(gpu):
     from trak_amd.utils import in_place_pays
 

@@ -118,20 +118,29 @@ def gemm_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None, in_place=False)
     return out
 
 
-def in_place_pays(a, b):
-    """Whether a @ b.T of two matrices that are multiplied from fp32 values is faster with `gemm_nt(in_place=True)`,
-    which reads them where they are (16-byte aligned rows, K % 256 == 0), than from splits: products of few rows or columns, for which the passes
-    that split the operands and 256 x 256 tiles cost more than the slower instruction."""
-    if a.dtype != torch.float32 or b.dtype != torch.float32 or not a.is_cuda or a.device != b.device:
+def _few_tiles(a, b):
+    """Whether a product of these shapes is faster from fp32 values where they are than from splits (`in_place_pays`)."""
+    if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[1] or a.shape[1] % 256 or a.numel() == 0 or b.numel() == 0:
         return False
-    if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[1] or a.numel() == 0 or b.numel() == 0:
+    return bool(_lib.load().trakhip_gemm_nt_in_place_pays(a.shape[0], b.shape[0], a.shape[1]))
+
+
+def _readable_in_place(a, b):
+    if a.dtype != torch.float32 or b.dtype != torch.float32 or not a.is_cuda or a.device != b.device:
         return False
     for t in (a, b):
         if t.stride(1) != 1 or t.data_ptr() % 16 or (t.shape[0] > 1 and (t.stride(0) % 4 or t.stride(0) < t.shape[1])):
             return False
         if max(t.stride(0), t.shape[1]) >= 1 << 23:  # a lane's offset inside a tile is kept in 32 bits
             return False
-    return bool(_lib.load().trakhip_gemm_nt_in_place_pays(a.shape[0], b.shape[0], a.shape[1]))
+    return True
+
+
+def in_place_pays(a, b):
+    """Whether a @ b.T of two matrices that are multiplied from fp32 values is faster with `gemm_nt(in_place=True)`,
+    which reads them where they are (16-byte aligned rows, K % 256 == 0), than from splits: products of few rows or columns, for which the passes
+    that split the operands and 256 x 256 tiles cost more than the slower instruction."""
+    return _few_tiles(a, b) and _readable_in_place(a, b)
 
 
 def gemm_tn(a, b, out=None, alpha=1.0, beta=0.0):
@@ -349,9 +358,11 @@ def matmul_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None, two_planes=Fa
     if not (a.dtype == b.dtype and a.dtype in (torch.float16, torch.bfloat16)):
         if two_planes:
             return gemm_nt_split(split2_rows(a), split2_rows(b), out=out, alpha=alpha, beta=beta, row_scale=row_scale)
-        a, b = a.float(), b.float()
-        if in_place_pays(a, b):
-            return gemm_nt(a, b, out=out, alpha=alpha, beta=beta, row_scale=row_scale, in_place=True)
+        if _few_tiles(a, b):
+            fa, fb = a.float(), b.float()
+            if _readable_in_place(fa, fb):
+                return gemm_nt(fa, fb, out=out, alpha=alpha, beta=beta, row_scale=row_scale, in_place=True)
+            del fa, fb
     return gemm_nt_split(*split_pair(a, b), out=out, alpha=alpha, beta=beta, row_scale=row_scale)
 
 
