@@ -152,6 +152,8 @@ def test_gemm_argument_validation_needs_no_device():
     assert rounded(p, 64, p, 64, 0, 3, p, 4, 4, 4, 64, 1.0, None, None) == -3
     assert rounded(p, 64, p, 64, 0, 0, ctypes.c_void_p(4097), 4, 4, 4, 64, 1.0, None, None) == -7
     assert rounded(p, 64, p, 64, 0, 0, p, 3, 4, 4, 64, 1.0, None, None) == -2
+    tile = lib.trakhip_gemm_nt_in_place_tile
+    assert [tile(*s) for s in ((1, 1, 256), (4159, 640, 512), (0, 1, 256), (1, 0, 256), (1, 1, 0), (1, 1, 255))] == [32, 64, 0, 0, 0, 0]
     pays = lib.trakhip_gemm_nt_in_place_pays
     assert pays(2000, 512, 512) == 1 and pays(50_000, 100, 2048) == 1 and pays(50_000, 10_000, 4096) == 0
     assert pays(2000, 512, 500) == 0 and pays(0, 5, 512) == 0 and pays(1 << 40, 1 << 40, 512) == 0

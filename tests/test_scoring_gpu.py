@@ -261,6 +261,22 @@ def test_little_is_multiplied_by_an_inverse_that_is_rejected(gpu, monkeypatch, w
     assert calls == ([16_384, n - 16_384] if where == "cuda" else [20_000] * 7)
 
 
+@pytest.mark.parametrize("k,block,rows", [(512, 2000, 2100), (512, 2000, 2001), (256, 20_000, 20_001), (1024, 700, 1450)])
+def test_a_row_has_the_same_features_in_every_block(gpu, k, block, rows):
+    lib = _lib.load()
+    assert 1 == lib.trakhip_gemm_nt_in_place_pays(rows % block, k, k) and lib.trakhip_gemm_nt_in_place_tile(rows % block, k, k) == 32
+    gen = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, k, generator=gen)
+    last = rows - rows // block * block
+    x[-last:] = x[:last]
+    r = torch.randn(k, k, generator=gen) / k**0.5
+    xtx = (r.T @ r).to(gpu)
+    got = BasicScoreComputer(dtype=torch.float32, device=gpu, lambda_reg=0.5, CUDA_MAX_DIM_SIZE=block).get_x_xtx_inv(x, xtx)
+    assert torch.equal(got[-last:], got[:last])
+    want = x.to(gpu).double() @ spd_inverse(xtx, lambda_reg=0.5, normalize=True)[0].double()
+    assert rel_max(got.cpu().numpy(), want.cpu().numpy()) < gemm_tol(k)
+
+
 def test_scoring_under_a_default_device(gpu):
     # page-locked buffers are host memory whatever device new tensors go to by default
     x = torch.randn(300, 64, generator=torch.Generator(device=gpu).manual_seed(2), device=gpu)

@@ -68,6 +68,8 @@ def load():
     lib.trakhip_gemm_nt_in_place.restype = i32
     lib.trakhip_gemm_nt_in_place_pays.argtypes = [u64, u64, u64]
     lib.trakhip_gemm_nt_in_place_pays.restype = i32
+    lib.trakhip_gemm_nt_in_place_tile.argtypes = [u64, u64, u64]
+    lib.trakhip_gemm_nt_in_place_tile.restype = i32
     lib.trakhip_gemm_tn.argtypes = [vp, u64, vp, u64, vp, u64, u64, u64, u64, f32, f32, vp]
     lib.trakhip_gemm_tn.restype = i32
     lib.trakhip_split_bytes.argtypes = [u64, u64, i32]

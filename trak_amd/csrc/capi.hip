@@ -117,6 +117,8 @@ int trakhip_gemm_nt_in_place_pays(uint64_t M, uint64_t N, uint64_t K) {
     return trakhip::gemm_nt_in_place_pays(M, N, K) ? 1 : 0;
 }
 
+int trakhip_gemm_nt_in_place_tile(uint64_t M, uint64_t N, uint64_t K) { return trakhip::gemm_nt_in_place_tile(M, N, K); }
+
 int trakhip_gemm_tn(const float* A_dev, uint64_t lda, const float* B_dev, uint64_t ldb, float* C_dev,
                     uint64_t ldc, uint64_t M, uint64_t N, uint64_t K, float alpha, float beta, void* stream) {
     return trakhip::gemm_tn(A_dev, lda, B_dev, ldb, C_dev, ldc, M, N, K, alpha, beta,

@@ -505,6 +505,11 @@ bool gemm_nt_in_place_pays(uint64_t M, uint64_t N, uint64_t K) {
     return (one < four ? one : four) < split_us(M, N, K);
 }
 
+int gemm_nt_in_place_tile(uint64_t M, uint64_t N, uint64_t K) {
+    if (M == 0 || N == 0 || K == 0 || K % 256) return 0;
+    return one_tile_us(M, N, K) < four_tiles_us(M, N, K) ? 32 : 64;
+}
+
 int gemm_nt_in_place(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
                      uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s) {
     if (M == 0 || N == 0) return TRAKHIP_OK;
@@ -514,7 +519,7 @@ int gemm_nt_in_place(const float* A, uint64_t lda, const float* B, uint64_t ldb,
     if ((reinterpret_cast<uintptr_t>(A) % 16) || (reinterpret_cast<uintptr_t>(B) % 16) || (lda % 4) || (ldb % 4) ||
         (reinterpret_cast<uintptr_t>(C) % 4) || (reinterpret_cast<uintptr_t>(row_scale) % 4))
         return TRAKHIP_ERR_ALIGN;
-    if (one_tile_us(M, N, K) < four_tiles_us(M, N, K))
+    if (gemm_nt_in_place_tile(M, N, K) == 32)
         return launch_small<1, 1, 4, 2>(A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, row_scale, s);
     return launch_small<2, 2, 1, 4>(A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, row_scale, s);
 }

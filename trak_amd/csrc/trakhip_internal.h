@@ -57,6 +57,7 @@ int gemm_nt(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C
 int gemm_nt_in_place(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
                      uint64_t N, uint64_t K, float alpha, float beta, const float* row_scale, hipStream_t s);
 bool gemm_nt_in_place_pays(uint64_t M, uint64_t N, uint64_t K);
+int gemm_nt_in_place_tile(uint64_t M, uint64_t N, uint64_t K);  // side of its tiles
 int gemm_tn(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,
             uint64_t N, uint64_t K, float alpha, float beta, hipStream_t s, uint32_t flags = 0);
 int gemm_nn(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C, uint64_t ldc, uint64_t M,

@@ -22,6 +22,7 @@ from .utils import (
     gram16,
     gram16_ok,
     gram_split,
+    in_place_alike,
     in_place_pays,
     inverse_of_rejected,
     matmul_nt,
@@ -174,6 +175,7 @@ class BasicScoreComputer(AbstractScoreComputer):
         result = ch.empty(grads.shape[0], xtx_inv.shape[1], dtype=self.dtype if half and self.gemm != "fp32" else ch.float32,
                           device=self._dev)
         inv_split = None  # planes of the inverse, made when the first block needs them
+        in_place = None  # one route for all blocks of fp32 values: a row's sums do not depend on the block that holds it
         start = 0
         blocks = self._blocks(grads)
         resident = blocks[0] is grads
@@ -193,9 +195,12 @@ class BasicScoreComputer(AbstractScoreComputer):
                     return None, pivot
             # the inverse is symmetric, so block @ inv == block @ inv^T
             if self.gemm != "fp32":
+                if in_place is None:
+                    in_place = (self.gemm == "split" and not half and in_place_pays(block, xtx_inv)
+                                and (len(blocks) == 1 or in_place_alike({b.shape[0] for b in blocks}, *xtx_inv.shape)))
                 if half and nt16_ok(block, xtx_inv):
                     gemm_nt16(block, xtx_inv, out=result[start:end])
-                elif self.gemm == "split" and not half and in_place_pays(block, xtx_inv):
+                elif in_place:
                     gemm_nt(block, xtx_inv, out=result[start:end], in_place=True)
                 else:
                     if inv_split is None:

@@ -143,6 +143,13 @@ def in_place_pays(a, b):
     return _few_tiles(a, b) and _readable_in_place(a, b)
 
 
+def in_place_alike(row_counts, columns, K):
+    """Whether products of these numbers of rows, blocks of one result, all pay in place and add up k in one order."""
+    lib = _lib.load()
+    return (all(lib.trakhip_gemm_nt_in_place_pays(rows, columns, K) for rows in row_counts)
+            and len({lib.trakhip_gemm_nt_in_place_tile(rows, columns, K) for rows in row_counts}) == 1)
+
+
 def gemm_tn(a, b, out=None, alpha=1.0, beta=0.0):
     """out[M, N] = alpha * a[K, M].T @ b[K, N] + beta * out (fp32 on the GPU)."""
     a = _as_f32_rows(a, "a")
@@ -352,7 +359,8 @@ def matmul_nt(a, b, out=None, alpha=1.0, beta=0.0, row_scale=None, two_planes=Fa
     types: two fp16 or two bf16 matrices that qualify are multiplied where they are (`gemm_nt16`),
     other 16-bit pairs as single planes, anything else from fp32 values: where they are, on the fp32 instruction,
     when that is faster (`in_place_pays`), else from splits (`gemm_nt_split`; the exact three-plane split, or the
-    two-plane one of `split2_rows` when `two_planes` is set)."""
+    two-plane one of `split2_rows` when `two_planes` is set).  Products of fp32 values add up k in an order that goes with the
+    number of rows and columns: the same row may differ in its last bits between calls of other sizes."""
     if nt16_ok(a, b):
         return gemm_nt16(a, b, out=out, alpha=alpha, beta=beta, row_scale=row_scale)
     if not (a.dtype == b.dtype and a.dtype in (torch.float16, torch.bfloat16)):
