@@ -634,6 +634,10 @@ __global__ __launch_bounds__(64 * Shape::kWaves, Shape::kPerSimd) void gemm_spli
     const int a_lane = h * BM + wm * 64 + x;
     const int b_lane = kAPieces + h * BN + wn * (32 * JT) + x;
 
+    // Fetching its code is part of a step of the one-plane product: [5000 x 4096] by 20 rows takes 94 us where the loop begins
+    // with a 64-byte line, 96 from word 9 of a line on and 102 from word 2, so one word of a line is left to what the compiler
+    // puts in front of the loop.  (Three planes differ by 1 %, two by up to 6 %; both lie well, and no time of theirs depends on this.)
+    if constexpr (P == 1) asm volatile(".p2align 6\n\t.fill 15, 4, 0xbf800000");  // s_nop 0
     for (uint64_t s = first; s < steps; ++s) {
         const int cur = (int)((s - first) & 1);
         // the other buffer was last read before the barrier that ended the previous step
