@@ -73,12 +73,16 @@ def test_gemm_nt_short_contraction(gpu, M, N, K):
     assert rel_max(wide[:, :N].cpu().numpy(), want) < gemm_tol(K) and bool((wide[:, N:] == 7.0).all())
 
 
-# tiles of 32 x 32 (four waves share the k range) and, from (1100, 1090, 256) on, of 64 x 64
-@pytest.mark.parametrize("M,N,K", [(1, 1, 256), (31, 33, 256), (32, 32, 512), (65, 100, 768), (2000, 1, 512), (300, 64, 4096),
-                                   (1100, 1090, 256), (1984, 1025, 1024), (4159, 640, 512)])
-def test_products_of_few_tiles_read_their_operands_in_place(gpu, M, N, K):
+# tiles of 32 x 32 (four waves share the k range) and of 64 x 64: whole ones, and with rows and columns left over on either side of half a
+# tile; the shortest k and many rounds of it
+@pytest.mark.parametrize("side,M,N,K", [(32, 1, 1, 256), (32, 31, 33, 256), (32, 32, 32, 512), (32, 65, 100, 768), (32, 2000, 1, 512),
+                                        (32, 300, 64, 4096), (32, 1100, 1090, 256), (32, 1984, 1025, 1024), (64, 4159, 640, 512),
+                                        (64, 4097, 600, 256), (64, 4111, 550, 256), (64, 2305, 1100, 512), (64, 5000, 340, 2048),
+                                        (64, 16_001, 117, 2048)])
+def test_products_of_few_tiles_read_their_operands_in_place(gpu, side, M, N, K):
     from trak_amd.utils import in_place_pays
 
+    assert _lib.load().trakhip_gemm_nt_in_place_tile(M, N, K) == side
     gen = torch.Generator(device="cpu").manual_seed(M + N + K)
     wide_a, wide_b = torch.randn(M, K + 20, generator=gen), torch.randn(N, K + 4, generator=gen)
     a, b = wide_a.to(gpu)[:, 8:8 + K], wide_b.to(gpu)[:, :K]         # pitches above K, rows 16-byte aligned
@@ -174,7 +178,7 @@ def test_spd_inverse(gpu, n, lam):
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 127, 129, 191, 256, 320, 641, 1100, 2048])
 def test_spd_inverse_at_the_edges_of_its_tiles(gpu, n):
-    # 64 x 64 tiles, k ranges cut to whole 128-blocks of the triangular factor, rows of a larger matrix
+    # the last product on 32 x 32 tiles, k ranges cut to whole 128-blocks of the triangular factor; rows of a larger matrix
     gen = torch.Generator(device="cpu").manual_seed(n)
     x = torch.randn(4 * n + 8, n, generator=gen) / math.sqrt(4 * n)
     full = torch.full((n, n + 5), float("nan"))
@@ -189,7 +193,7 @@ def test_spd_inverse_at_the_edges_of_its_tiles(gpu, n):
     ev = np.linalg.eigvalsh((a64 + a64.T) / 2)
     bound = 4 * 2.0**-24 * ev[-1] / ev[0] * np.linalg.norm(want)
     assert np.linalg.norm(inv.double().cpu().numpy() - want) <= bound
-    # n^2 terms added in fp32, 1024 partial sums of rows
+    # n^2 terms added in fp32: a sum per tile, then those
     assert abs(mean_abs.item() / inv.double().abs().mean().item() - 1) <= 64 * 2.0**-24
     scaled, _ = spd_inverse(a, lambda_reg=0.125, normalize=True)
     assert (scaled.double() * mean_abs.double() - inv.double()).abs().max() <= 4 * 2.0**-24 * inv.abs().max()
@@ -289,6 +293,33 @@ def test_scoring_under_a_default_device(gpu):
     with torch.device(gpu):
         assert torch.equal(sc.get_x_xtx_inv(x, xtx), want)
         assert np.array_equal(acc.finalize(np.zeros((300, 7), np.float32)), scores)
+
+
+@pytest.mark.parametrize("n", [2049, 2500, 3072, 4095, 4097])
+def test_spd_inverse_of_many_rows_of_blocks(gpu, n):
+    # 17 to 32 blocks: the last product on 64 x 64 tiles, whole and ragged, that add up magnitudes; above 4096 the recursion and a pass for the sums
+    gen = torch.Generator(device=gpu).manual_seed(n)
+    x = torch.randn(4 * n + 8, n, generator=gen, device=gpu) / math.sqrt(4 * n)
+    full = torch.full((n, n + 5), float("nan"), device=gpu)
+    full[:, :n] = (x.double().T @ x.double()).float()
+    a = full[:, :n]
+    a64 = a.double() + 0.125 * torch.eye(n, device=gpu, dtype=torch.float64)
+    want = torch.linalg.inv(a64.cpu()).to(gpu)
+    inv, mean_abs = spd_inverse(a, lambda_reg=0.125)
+    assert torch.equal(inv, inv.T)
+
+    def largest_eigenvalue(m):  # from below, by 40 steps of the power method: a stricter bound
+        v = torch.ones(n, device=gpu, dtype=torch.float64)
+        for _ in range(40):
+            v = m @ (v / v.norm())
+        return float(v.norm())
+
+    # the bound of the smaller sizes: a backward error of four times 2^-24
+    bound = 4 * 2.0**-24 * largest_eigenvalue(a64) * largest_eigenvalue(want) * float(want.norm())
+    assert float((inv.double() - want).norm()) <= bound
+    assert abs(mean_abs.item() / inv.double().abs().mean().item() - 1) <= 64 * 2.0**-24
+    scaled, _ = spd_inverse(a, lambda_reg=0.125, normalize=True)
+    assert (scaled.double() * mean_abs.double() - inv.double()).abs().max() <= 4 * 2.0**-24 * inv.abs().max()
 
 
 def test_spd_inverse_many_blocks(gpu):
@@ -618,11 +649,13 @@ def test_gemm_nt_split_on_every_shape_of_tiles(gpu, M, N, K):
     assert torch.equal(wide[M - few:, :N], gemm_nt_split(split_rows(a[M - few:]), sb))
 
 
-# columns of tiles: one, two, eight (one band), nine and twelve (two bands), thirteen (row by row)
-@pytest.mark.parametrize("M,N", [(2100, 256), (1300, 300), (700, 2048), (1300, 2309), (520, 3072), (600, 3100), (20, 2500), (5000, 1)])
+# columns of 128 x 128 tiles: two, three (one band), 16 (two bands), 19 (three, one of them wider), 24 (three), 25 (row by row), 20 (three,
+# two wider), one; of 256 x 256 tiles: ten and twelve (two bands), 13 (row by row), each in products of 16-bit values and of three planes
+@pytest.mark.parametrize("M,N", [(2100, 256), (1300, 300), (700, 2048), (1300, 2309), (520, 3072), (600, 3100), (20, 2500), (5000, 1),
+                                 (6395, 2500), (5300, 3072), (4860, 3280)])
 def test_products_in_every_order_of_their_tiles(gpu, M, N):
     gen = torch.Generator(device=gpu).manual_seed(M + N)
-    for dtype, K in ((torch.float16, 128), (torch.float32, 32)):
+    for dtype, K in ((torch.float16, 128), (torch.float32, 256 if M > 4000 and N > 2000 else 32)):
         a, b = (torch.randn(r, K, generator=gen, device=gpu).to(dtype) for r in (M, N))
         want = (a.double() @ b.double().T).cpu().numpy()
         out = torch.full((M, N), float("nan"), device=gpu)
