@@ -156,6 +156,10 @@ def test_gemm_argument_validation_needs_no_device():
     assert [tile(*s) for s in ((1, 1, 256), (4159, 640, 512), (0, 1, 256), (1, 0, 256), (1, 1, 0), (1, 1, 255))] == [32, 64, 0, 0, 0, 0]
     pays = lib.trakhip_gemm_nt_in_place_pays
     assert pays(2000, 512, 512) == 1 and pays(50_000, 100, 2048) == 1 and pays(50_000, 10_000, 4096) == 0
+    # us in place 68, 82, 98, 141, 245, split 52, 65, 84, 118, 228; and the other way round 43, 147, 79, split 77, 249, 92
+    split = ((16_000, 768, 256), (30_000, 512, 256), (20_000, 512, 512), (20_000, 512, 768), (20_000, 400, 1536))
+    assert [pays(*s) for s in split] == [0] * 5
+    assert [pays(*s) for s in ((8000, 512, 512), (8000, 512, 2048), (30_000, 256, 512))] == [1] * 3
     assert pays(2000, 512, 500) == 0 and pays(0, 5, 512) == 0 and pays(1 << 40, 1 << 40, 512) == 0
     assert lib.trakhip_gemm_tn(p, 2, p, 8, p, 8, 4, 4, 16, 1.0, 0.0, None) == -2          # lda < M
     assert lib.trakhip_spd_inverse(p, 2, 0.0, p, 4, 4, 0, None, None, p, 1 << 30, None) == -2

@@ -400,9 +400,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_small_kernel(const float*
     }
 }
 
-// What an NT product takes, in microseconds, fitted to 200 products of M = 1000 .. 50 000, N = 1 .. 2048 and K = 512 .. 4096:
-// rounds of tiles over the 256 CUs times the time of one, which goes with K.  A tile of 32 x 32 entries shared by four
-// waves takes 6.0 ns per value of k whether one or two of them share a CU (bound by what 256 CUs read from L2: 10.7 TB/s);
+// What an NT product takes, in microseconds: rounds of tiles over the 256 CUs times the time of one, which goes with K.  A tile
+// of 32 x 32 entries shared by four waves takes 6.0 ns per value of k whether one or two of them share a CU (bound by what 256 CUs read from L2: 10.7 TB/s);
 // a 64 x 64 tile 17.6 ns where two or more share a CU, 19.8 alone (120 TFLOP/s).  (The general kernel: 128 x 128 tiles 83 ns,
 // 128 x 256 tiles, from 256 of them on, 134 ns.)
 double tiles_of(uint64_t M, uint64_t N, uint64_t rows, uint64_t cols) {
@@ -420,6 +419,23 @@ double four_tiles_us(uint64_t M, uint64_t N, uint64_t K) {
 // Both operands split into planes (10 bytes of traffic per value) and their product (gemm_split.hip).
 double split_us(uint64_t M, uint64_t N, uint64_t K) {
     return 18.0 + 2.0e-6 * ((double)M + (double)N) * (double)K + trakhip::split_product_us(M, N, K);
+}
+// Where the two are close these tell them apart: a round of tiles has its stores of C to make besides (0.3 and 0.8 us, which
+// count where K is 256), and the planes of up to 15 million values are still in the 256 MB cache when the product reads them, 0.9
+// us a million instead of 2.2.  They price the split with its product on 256 x 256 tiles only: its 128 x 128 ones are up to 20 %
+// faster, but a product in place has the smaller error, and keeps what it does not do slower than that.  Call to call, 814
+// products within a factor of 1.8 (M = 300 .. 50 000, N = 64 .. 3000, K = 256 .. 4096): none is more than 2.4 % above the split on 256 x 256
+// tiles; by the estimates above alone 28 are, up to 30 % ([16 000 x 256] by 768 in place 68 us, split 52; [20 000 x 512] by 512 97, 84).
+double close_in_place_us(uint64_t M, uint64_t N, uint64_t K) {
+    const double k = (double)K, four = tiles_of(M, N, 64, 64);
+    const double one_us = (0.3 + 6.0e-3 * k) * rounds_of(tiles_of(M, N, 32, 32));
+    const double four_us = (0.8 + 17.0e-3 * k) * (four <= 256.0 ? 1.12 : __builtin_ceil(four / 256.0));
+    return 5.0 + (one_us < four_us ? one_us : four_us);
+}
+double close_split_us(uint64_t M, uint64_t N, uint64_t K) {
+    const double millions = 1e-6 * ((double)M + (double)N) * (double)K;
+    const double passes = millions <= 15.0 ? 0.9 * millions : 0.9 * 15.0 + 2.2 * (millions - 15.0);
+    return 15.0 + passes + trakhip::split_product_big_us(M, N, K);
 }
 
 template <int WM, int WN, int WK, int DEPTH>
@@ -502,7 +518,7 @@ int gemm_nt(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C
 bool gemm_nt_in_place_pays(uint64_t M, uint64_t N, uint64_t K) {
     if (M == 0 || N == 0 || K == 0 || K % 256) return false;
     const double one = one_tile_us(M, N, K), four = four_tiles_us(M, N, K);
-    return (one < four ? one : four) < split_us(M, N, K);
+    return (one < four ? one : four) < split_us(M, N, K) && close_in_place_us(M, N, K) < close_split_us(M, N, K);
 }
 
 int gemm_nt_in_place_tile(uint64_t M, uint64_t N, uint64_t K) {

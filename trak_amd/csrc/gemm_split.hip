@@ -1416,6 +1416,8 @@ double split_product_us(uint64_t M, uint64_t N, uint64_t K) {
     return us;
 }
 
+double split_product_big_us(uint64_t M, uint64_t N, uint64_t K) { return big_planes_us(M, N, K); }
+
 int gemm_nt_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_t N, uint64_t K, int dtype, float* C,
                   uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags) {
     if (!known_dtype(dtype)) return TRAKHIP_ERR_DTYPE;

@@ -66,8 +66,9 @@ int gemm_nn(const float* A, uint64_t lda, const float* B, uint64_t ldb, float* C
 size_t split_bytes(uint64_t rows, uint64_t K, int dtype);
 int split_rows(const void* src, int dtype, uint64_t ld, uint64_t rows, uint64_t K, int transposed, void* planes,
                size_t planes_bytes, hipStream_t s);
-// what gemm_nt_split of fp32 operands (three planes) is expected to take, in microseconds
+// what gemm_nt_split of fp32 operands (three planes) is expected to take, in microseconds; and on 256 x 256 tiles alone
 double split_product_us(uint64_t M, uint64_t N, uint64_t K);
+double split_product_big_us(uint64_t M, uint64_t N, uint64_t K);
 int gemm_nt_split(const void* A_planes, uint64_t M, const void* B_planes, uint64_t N, uint64_t K, int dtype, float* C,
                   uint64_t ldc, float alpha, float beta, const float* row_scale, hipStream_t s, uint32_t flags = 0);
 // ws (may be null): room for as many N x N matrices as a product with few tiles may share its k range out over
