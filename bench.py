@@ -548,7 +548,8 @@ def bench_scoring(torch, dev, reps=3):
             best = ms if best is None else min(best, ms)
         return r, best
 
-    from trak_amd.utils import gemm_nt, gemm_nt16, gemm_nt_split, gemm_tn, gram_split, spd_inverse, split2_rows, split_rows
+    from trak_amd.utils import (gemm_nt, gemm_nt16, gemm_nt_split, gemm_tn, gram16, gram_split, matmul_nt, spd_inverse,
+                                split2_rows, split_rows)
 
     # the fp32 MFMA instruction (v_mfma_f32_32x32x2_f32): priced against the 157.3 TFLOP/s fp32 peak
     xtx, t_xtx = timed(lambda: gemm_tn(X, X))
@@ -571,13 +572,15 @@ def bench_scoring(torch, dev, reps=3):
     _, q_feat = timed(lambda: gemm_nt_split(split2_rows(X), split2_rows(inv)))
     _, q_sc = timed(lambda: gemm_nt_split(split2_rows(feats), split2_rows(Xt), row_scale=otl))
     split2_ms = q_xtx + q_feat + q_sc
-    # TRAKer's default stores gradients and features as fp16 (use_half_precision): the same products
-    # with one MFMA per k step and exact products; X^T X from one fp16 plane (the transposed operand
-    # needs the re-layout), the two row-major products read in place (what BasicScoreComputer runs)
+    # TRAKer's default stores gradients and features as fp16 (use_half_precision): the same products with one MFMA
+    # per k step and exact products, all three operands read in place and X^T X and the features rounded to fp16 by their
+    # kernels (what BasicScoreComputer runs)
     Xh, invh, fh, Xth = X.half(), inv.half(), feats.half(), Xt.half()
-    _, h_xtx = timed(lambda: gram_split(split_rows(Xh, transposed=True)))
-    _, h_feat = timed(lambda: gemm_nt16(Xh, invh))
+    _, h_xtx = timed(lambda: gram16(Xh, out_dtype=torch.float16))
+    _, h_feat = timed(lambda: gemm_nt16(Xh, invh, out=fh))
     _, h_sc = timed(lambda: gemm_nt16(fh, Xth, row_scale=otl))
+    # a handful of targets in fp32: both operands read in place on the fp32 instruction
+    _, f_sc = timed(lambda: matmul_nt(feats, Xt[:20], row_scale=otl))
     del Xh, fh, Xth
     # X^T X is computed on the tiles that touch the lower triangle only (256 x 256 tiles) and mirrored:
     # its flops are counted as computed, not as 2*N*k*k
@@ -608,6 +611,7 @@ def bench_scoring(torch, dev, reps=3):
             "gemm_tflops": split_flop / ((h_xtx + h_feat + h_sc) * 1e-3) / 1e12,
             "frac_fp16_mfma_peak": split_flop / ((h_xtx + h_feat + h_sc) * 1e-3) / 1e12 / PEAK_FP16_TFLOPS,
         },
+        "fp32_scores_of_20_targets_ms": f_sc,
         "inverse_flop": float(k) ** 3,
         "scores_orientation": "[N_train, M_targets]",
     }
