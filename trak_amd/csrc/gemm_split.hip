@@ -533,7 +533,7 @@ struct StepMover {
 // Workgroup -> unit of a symmetric product (share of the k range, tile): the shares' lists of tiles one after another, of
 // which each of the eight XCDs, which are handed the workgroups round-robin, takes a contiguous eighth.  The tiles of a
 // share read the same rows of X at about the same time, so an XCD then fetches its share's rows once; with the tiles
-// dealt out over all XCDs each of them fetched every row of X ([50 000, 2048] fp16: 1.6 GB; 285 us, now 249; the
+// dealt out over all XCDs each of them fetched every row of X ([50 000, 2048] fp16: 1.6 GB; 285 us, 249 this way; the
 // three-plane product of [4100, 2048] fp32 138 -> 126, of [50 000, 4096] 4.41 -> 4.33 ms).  The grid has a multiple of
 // eight workgroups; false: one without a unit.
 __device__ __forceinline__ bool xcd_unit(uint32_t units, uint32_t& unit) {
@@ -861,7 +861,7 @@ __global__ __launch_bounds__(64 * Shape::kWaves, 2) void gemm_nt16_kernel(
 // operand is eight values of one column.  A step is 64 rows of the tile's 256 columns (32 KB per operand); gfx950's
 // transposing LDS read (ds_read_b64_tr_b16) hands sixteen lanes, which name four rows of sixteen columns, four rows of a
 // column each, so that two of them make an operand and X needs no transposing pass (94 us and 410 MB of traffic for
-// [50 000, 2048] fp16).  X^T X with the result rounded: [50 000, 2048] 349 -> 242 us, [8200, 4096] 274 -> 196,
+// [50 000, 2048] fp16).  X^T X with the result rounded: [50 000, 2048] 349 -> 242 us (to 260 on other cards), [8200, 4096] 274 -> 196,
 // [2000, 512] 39 -> 25; bound by the MFMAs' power and, per step, the 64 LDS-direct loads of a CU.
 // LDS holds a row as 32 pieces of 16 bytes; the 64-byte units of row k are permuted, unit u in place u ^ (k % 4): the
 // four rows that 32 lanes read at a time then lie in different quarters of the 64 banks.  A wave's LDS-direct load
@@ -1211,8 +1211,8 @@ int launch_split_tiles(const piece* a, uint64_t Rpa, uint64_t M, const piece* b,
 
 // Rows of a three-plane product that go to 256 x 256 tiles (the others to 128 x 128): as big_tile_rows, microseconds per 16 values
 // of k: 256 x 256 2.12 a round (a last one that leaves CUs idle 1.64, up to 2.1 as it fills), 128 x 128 tiles 0.82 for one on
-// a CU, 1.34 for two side by side, 1.8 for three.  158 products of M = 1000 .. 50 000, N = 100 .. 8000, K = 512 .. 4096: 0.1 %
-// above the fastest of the three on average, 2 % at worst, 28 % below 256 x 256 tiles alone: [4000 x 4096] by 1024 rows 427 ->
+// a CU, 1.34 for two side by side, 1.8 for three.  196 products of M = 1000 .. 50 000, N = 100 .. 8000, K = 512 .. 4096: 0.2 %
+// above the fastest of the three on average, 5 % at worst, 27 % below 256 x 256 tiles alone and nowhere more than 3 % above: [4000 x 4096] by 1024 rows 427 ->
 // 210 us, [16 000 x 1024] by 300 117 -> 81, [50 000 x 2048] by 1024 1036 -> 975, [25 000 x 2048] by 4096 1851 -> 1790.
 constexpr uint64_t kPlanCus = 256;
 double big_planes_us(uint64_t M, uint64_t N, uint64_t K) {
@@ -1310,9 +1310,9 @@ int launch_nt16(const char* A, uint64_t lda, const void* B, uint64_t ldb, int dt
 // Rows of a 16-bit product in place that go to 256 x 256 tiles; the others go to 128 x 128: none, all, or those behind as many
 // rows of tiles as make whole rounds over the CUs, whichever estimate is smallest.  Microseconds, per 64 values of k and
 // round of tiles over the CUs: 256 x 256 1.75 and 8.5 for the stores of C (a last round that leaves CUs idle 1.33, up to
-// 1.73 as it fills: the clock), 128 x 128, two per CU, 1.03 and 4.5 (a last round 0.5 to 1.1).  Fitted to 237 products of
-// M = 1000 .. 50 000, N = 1 .. 8000, K = 512 .. 4096: on average 0.2 % above the fastest of the three, at worst 13 %, never
-// more than 2 % slower than 256 x 256 tiles alone and two thirds of their time on average: [50 000 x 2048] by 100 rows
+// 1.73 as it fills: the clock), 128 x 128, two per CU, 1.03 and 4.5 (a last round 0.5 to 1.1).  196 products of
+// M = 1000 .. 50 000, N = 100 .. 8000, K = 512 .. 4096: on average 0.3 % above the fastest of the three, at worst 9 %, never
+// more than 2 % slower than 256 x 256 tiles alone and three quarters of their time on average: [50 000 x 2048] by 100 rows
 // 64 -> 43 us, by 2048 427 -> 410, [2000 x 512] by 512 21 -> 13, [4000 x 2048] by 1024 55 -> 28.
 double big_tiles_us(uint64_t M, uint64_t N, uint64_t K, int cus) {
     if (M == 0) return 0.0;
@@ -1341,14 +1341,15 @@ uint64_t big_tile_rows(uint64_t M, uint64_t N, uint64_t K, int cus) {
 // CUs idle, and the k range is long enough to share out.  The number of shares, up to `most` and to what `room` bytes hold,
 // is the one whose estimate is smallest: rounds of workgroups over the 256 CUs times the steps of a share (1.6 us each,
 // 1.8 for two planes; 6 us for a workgroup's first loads and its stores), plus 0.2 us per MB that the pass behind the product
-// goes over: the shares it adds up or, for one share, the matrix it mirrors.  Fitted to the times of all numbers of shares at
-// N = 512 .. 4352, K = 500 .. 50 000 in the three formats: the choice is 0.3 % above the fastest number on average and
-// 11 % at worst ([8300, 1536] fp16: 58 us with the ten it takes, 52 with eight), never more than 4 % above three shares.
+// goes over: the shares it adds up or, for one share, the matrix it mirrors.  Timed for all numbers of shares at
+// N = 512 .. 4096, K = 2000 .. 50 000: on 256 x 256 tiles, which one and two planes always take, the choice is at most 3 % above the fastest
+// number.  Of 16-bit rows in place and three planes, whose tiles gram_small_tiles chooses for the number that is fixed here, the pair is
+// 3 and 6 % above the fastest pair on average and up to 31 % ([20 000, 1024] fp32: 166 us in sixteen shares of 256 x 256 tiles, 126 in fourteen of 128 x 128).
 // N = 2048 takes seven (36 tiles: 252 workgroups; three gave 108), N = 512 at 2000 values of k sixteen, N = 4096 seven at
 // 50 000 values of k (952 workgroups, 3.7 rounds; three leave the second of two rounds 60 % full) and one at 2000 of 16 bits
 // (80 us; three 95).  A share has at least eight steps, and the shares together at most 512 MB.  Product and
 // sum against three shares, X^T X of [50 000, 2048] fp16 from its planes: 445 -> 248 us, of [50 000, 512] 371 -> 87.
-// (gram16_kernel takes the same numbers; where the tiles of the chosen shares leave CUs idle, see gram_small_tiles.)
+// (gram16_kernel takes the same numbers.)
 constexpr uint32_t kGramPartsMax = 16, kGramPartsFew = 3, kGramTilesMax = 170;
 uint32_t gram_parts(uint64_t N, uint64_t K, int dtype, bool two_planes, uint32_t most, size_t room = SIZE_MAX) {
     const uint64_t tiles = (N + BM - 1) / BM, lower = tiles * (tiles + 1) / 2;

@@ -653,7 +653,7 @@ __global__ __launch_bounds__(256) void abs_sum_kernel(const float* __restrict__ 
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-// The mean from the partial sums - every workgroup works it out for itself (4-16 KB from L2) instead of waiting for a
+// The mean from the partial sums - every workgroup works it out for itself (at most 8.3 KB from L2) instead of waiting for a
 // launch that does only that - and M /= mean, rows b, b + gridDim.x, ... for workgroup b.
 __global__ __launch_bounds__(256) void mean_scale_kernel(const float* __restrict__ partial, uint32_t count,
                                                          float* __restrict__ M, uint64_t ld, uint32_t n, int normalize,
