@@ -164,7 +164,7 @@ int trakhip_gemm_nt(const float* A_dev, uint64_t lda, const float* B_dev, uint64
 
 /* The same product for few rows or columns, on smaller tiles: K a multiple of 256, A_dev and B_dev 16-byte
  * aligned, lda and ldb multiples of 4 and below 2^23.  trakhip_gemm_nt_in_place_pays: 1 when it is expected
- * to take less time than trakhip_split_rows of both operands and trakhip_gemm_nt_split, else 0.  All of them
+ * to take less time than trakhip_split_rows of both operands and their product on 256 x 256 tiles, else 0.  All of them
  * have fp32 accuracy; they add up k in different orders, and so do the two shapes of tiles that this one has:
  * trakhip_gemm_nt_in_place_tile is the side of those it takes for a size, 32 or 64, or 0 for a size it does not take. */
 int trakhip_gemm_nt_in_place(const float* A_dev, uint64_t lda, const float* B_dev, uint64_t ldb, float* C_dev,

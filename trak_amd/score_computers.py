@@ -72,7 +72,10 @@ class BasicScoreComputer(AbstractScoreComputer):
     MFMA instruction directly; "split2" is an opt-in cheaper split for fp32 operands (rows scaled by a
     power of two, two fp16 planes, three MFMAs per k step: entries keep 22 significand bits relative
     to their row's largest magnitude instead of all 24; 1.75 times the speed of "split").  fp16 / bf16
-    operands are multiplied as they are (exact products) under "split" and "split2".
+    operands are multiplied as they are (exact products) under "split" and "split2".  Under "split", products of few
+    rows or columns read fp32 operands where they are, on the fp32 instruction (`utils.in_place_pays`); the order in which
+    k is added up goes with the numbers of rows and columns, so the last bits of an fp32 row's features or scores may
+    differ between calls of other sizes.  All rows of one `get_x_xtx_inv` are added up in one order.
 
     Differences from the reference that a caller can meet:
       * the device must be a GPU (the reference also runs on "cpu");

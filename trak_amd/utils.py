@@ -137,9 +137,9 @@ def _readable_in_place(a, b):
 
 
 def in_place_pays(a, b):
-    """Whether a @ b.T of two matrices that are multiplied from fp32 values is faster with `gemm_nt(in_place=True)`,
-    which reads them where they are (16-byte aligned rows, K % 256 == 0), than from splits: products of few rows or columns, for which the passes
-    that split the operands and 256 x 256 tiles cost more than the slower instruction."""
+    """Whether a @ b.T of two matrices that are multiplied from fp32 values goes through `gemm_nt(in_place=True)`,
+    which reads them where they are (16-byte aligned rows, K % 256 == 0), instead of splits: products of few rows or columns, for which the
+    passes that split the operands and 256 x 256 tiles cost more than the slower instruction (whose error is smaller)."""
     return _few_tiles(a, b) and _readable_in_place(a, b)
 
 
