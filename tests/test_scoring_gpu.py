@@ -695,6 +695,19 @@ def test_features_are_the_rounded_product_whatever_the_route(gpu, dtype):
         assert torch.equal(sc.get_x_xtx_inv(block.cpu(), xtx), want)               # from the host, block by block
 
 
+@pytest.mark.parametrize("cols", [512, 500])
+def test_gradients_on_the_host_cross_once(gpu, monkeypatch, cols):
+    x = torch.randn(3000, cols, generator=torch.Generator().manual_seed(cols)).half()
+    sc = BasicScoreComputer(dtype=torch.float16, device=gpu, lambda_reg=1.0)
+    want = sc.get_xtx(x.to(gpu))
+    crossed, move = [], torch.Tensor.to
+    monkeypatch.setattr(torch.Tensor, "to", lambda t, *args, **kw: (crossed.append(t.device.type), move(t, *args, **kw))[1])
+    assert torch.equal(sc.get_xtx(x), want) and crossed.count("cpu") == 1
+    crossed.clear()
+    sc.get_x_xtx_inv(x, want)
+    assert crossed.count("cpu") == 1
+
+
 def test_gemm_nt16_refuses_what_it_cannot_read_in_place(gpu):
     a = torch.randn(64, 128, device=gpu).half()
     b = torch.randn(32, 128, device=gpu).half()

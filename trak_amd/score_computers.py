@@ -145,9 +145,9 @@ class BasicScoreComputer(AbstractScoreComputer):
             return result
         blocks = self._blocks(grads)
         if len(blocks) == 1 and self.gemm != "fp32" and self.dtype in (ch.float16, ch.bfloat16):
-            block = blocks[0].to(self._dev)
-            if gram16_ok(block):
-                return gram16(block, out_dtype=self.dtype)
+            blocks = [blocks[0].to(self._dev)]
+            if gram16_ok(blocks[0]):
+                return gram16(blocks[0], out_dtype=self.dtype)
         result = ch.empty(self.proj_dim, self.proj_dim, dtype=ch.float32, device=self._dev)
         for i, block in enumerate(blocks):
             self._gram(block.to(self._dev), result, 0.0 if i == 0 else 1.0)
