@@ -1212,8 +1212,9 @@ int launch_split_tiles(const piece* a, uint64_t Rpa, uint64_t M, const piece* b,
 // Rows of a three-plane product that go to 256 x 256 tiles (the others to 128 x 128): as big_tile_rows, microseconds per 16 values
 // of k: 256 x 256 2.12 a round (a last one that leaves CUs idle 1.64, up to 2.1 as it fills), 128 x 128 tiles 0.82 for one on
 // a CU, 1.34 for two side by side, 1.8 for three.  196 products of M = 1000 .. 50 000, N = 100 .. 8000, K = 512 .. 4096: 0.2 %
-// above the fastest of the three on average, 5 % at worst, 27 % below 256 x 256 tiles alone and nowhere more than 3 % above: [4000 x 4096] by 1024 rows 427 ->
-// 210 us, [16 000 x 1024] by 300 117 -> 81, [50 000 x 2048] by 1024 1036 -> 975, [25 000 x 2048] by 4096 1851 -> 1790.
+// above the fastest of the three on average, 5 % at worst, 27 % below 256 x 256 tiles alone and nowhere more than 3 % above (6 %
+// at 64 values of k): [4000 x 4096] by 1024 rows 427 -> 210 us, [16 000 x 1024] by 300 117 -> 81, [50 000 x 2048] by 1024 1036 ->
+// 975, [25 000 x 2048] by 4096 1851 -> 1790.
 constexpr uint64_t kPlanCus = 256;
 double big_planes_us(uint64_t M, uint64_t N, uint64_t K) {
     if (M == 0) return 0.0;
@@ -1314,6 +1315,8 @@ int launch_nt16(const char* A, uint64_t lda, const void* B, uint64_t ldb, int dt
 // M = 1000 .. 50 000, N = 100 .. 8000, K = 512 .. 4096: on average 0.3 % above the fastest of the three, at worst 9 %, never
 // more than 2 % slower than 256 x 256 tiles alone and three quarters of their time on average: [50 000 x 2048] by 100 rows
 // 64 -> 43 us, by 2048 427 -> 410, [2000 x 512] by 512 21 -> 13, [4000 x 2048] by 1024 55 -> 28.
+// Less than 512 values of k, 280 products: 4 % above the fastest, at worst 39 % ([12 000 x 256] by 1500 rows 54 us, all on 128 x 128 39);
+// 16 % below 256 x 256 tiles alone, at worst 8 % above ([7000 x 128] by 3000 rows 46 us and 42).
 double big_tiles_us(uint64_t M, uint64_t N, uint64_t K, int cus) {
     if (M == 0) return 0.0;
     const uint64_t tiles = (M + 255) / 256 * ((N + 255) / 256), full = tiles / cus;
